@@ -21,6 +21,7 @@
 
 #include "bcx_batched.h"
 #include "bcx_small.h"
+#include "bcx_src.h"
 #include "bcx_runtime.h"
 
 using namespace bcx;
@@ -1270,6 +1271,7 @@ struct SmallState {
     // a pass started and not yet finished (persistent_start / _finish)
     bool pending = false, run_fp32 = false, run_graph = false;
     SmallArgs run{};
+    SrcArgs src{};  // (wave-per-source pass)
     std::vector<SmallTile> run_tiles;
     size_t run_narrow = 0;
     int run_grid = 0;
@@ -1336,46 +1338,26 @@ static int persistent_pass(bcx_ctx *ctx, SmallState &ss, bool wg, bool f64, bool
     return small_launch(ctx, ss, ss.run, wg, f64, ss.run_fp32, ss.run_grid, graph, ss.run_stream);
 }
 
-// One persistent launch over the tiles of `jobs`: the small-component kernel
-// (LDS state, n <= SMALL_N) or, with `wg`, the workgroup-per-tile kernel
-// (HBM slabs, n <= WG_N).  Tiles whose uint64 sigma overflows are rerun in
-// FP64 by a second launch.
-// Starts the pass on stream sp and returns without waiting for it;
-// persistent_finish waits, reruns the overflowed tiles and completes it.
-static int persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base,
-                            bcx_stats *st, bool wg, hipStream_t sp, bool probe) {
-    if (jobs.empty()) return BCX_OK;
-    if (!ctx->batched) ctx->batched = new BatchedState();
-    SmallState *&state = wg ? ctx->wgk : ctx->small;
-    if (!state) state = new SmallState();
-    SmallState &ss = *state;
-    int64_t nmax = 1, csr = 0;
-    for (const SmallJob &jb : jobs) {
-        nmax = std::max<int64_t>(nmax, jb.dc->n);
-        csr = std::max<int64_t>(csr, jb.dc->n + 1 + jb.dc->arcs);
-    }
-    // small kernel: a tile's CSR joins the LDS state when it fits beside the
-    // masks
-    csr = wg ? 0 : small_csr_words(nmax, csr);
-    std::vector<SmallComp> comps;
+// The tables of a persistent pass: its components, tiles of tw sources,
+// sources and weights, and eight zeroed counters, in device memory.
+struct PassTables {
     std::vector<SmallTile> tiles;
+    const SmallComp *comps = nullptr;
+    const SmallTile *d_tiles = nullptr;
+    const int32_t *srcs = nullptr;
+    const double *ws = nullptr;
+    int32_t *counters = nullptr;
+};
+
+static int stage_tables(bcx_ctx *ctx, SmallState &ss, const std::vector<const SmallJob *> &order, double *bc_base,
+                        size_t tw, PassTables &out) {
+    std::vector<SmallComp> comps;
+    std::vector<SmallTile> &tiles = out.tiles;
     std::vector<int32_t> srcs;
     std::vector<double> ws;
-    // workgroup kernel: components whose path counts from their highest-degree
-    // vertex already pass 2^62 start with FP64 sigma (their tiles would all
-    // overflow the 64-bit pass); their tiles go after the others
-    std::vector<const SmallJob *> order;
-    for (const SmallJob &jb : jobs) order.push_back(&jb);
-    auto wide = [&](const SmallJob *jb) { return wg && jb->dc->sigma_est > 4.6e18; };
-    std::stable_partition(order.begin(), order.end(), [&](const SmallJob *jb) { return !wide(jb); });
-    // tiles of 64 W sources (source k + 64 h on lane k); the small kernel's are 64
-    const int W = wg ? wg_spl(o) : 1;
-    const size_t TW = (size_t)BATCH_W * W;
-    size_t n_narrow_tiles = 0;
     for (const SmallJob *jbp : order) {
         const SmallJob &jb = *jbp;
         const DComp &dc = *jb.dc;
-        if (!wide(jbp)) n_narrow_tiles += (jb.srcs.size() + TW - 1) / TW;
         // (the workgroup kernel stays on the component's own ids: on the
         // BFS-ordered copy the 256x256 grid workload fetched 32% more bytes
         // and ran 8% slower)
@@ -1387,11 +1369,11 @@ static int persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, con
         c.bc = bc_base + dc.offset;
         const int32_t ci = (int32_t)comps.size();
         comps.push_back(c);
-        for (size_t i = 0; i < jb.srcs.size(); i += TW) {
+        for (size_t i = 0; i < jb.srcs.size(); i += tw) {
             SmallTile t{};
             t.comp = ci;
             t.src0 = (int32_t)srcs.size();
-            t.ns = (int32_t)std::min<size_t>(TW, jb.srcs.size() - i);
+            t.ns = (int32_t)std::min<size_t>(tw, jb.srcs.size() - i);
             tiles.push_back(t);
             for (int k = 0; k < t.ns; ++k) {
                 srcs.push_back(jb.srcs[i + k]);
@@ -1399,13 +1381,14 @@ static int persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, con
             }
         }
     }
-    // the four tables go up in one copy from pinned staging (the previous
-    // pass that used the staging has been waited for)
+    // the tables go up in one copy from pinned staging (the previous pass
+    // that used the staging has been waited for)
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const size_t o_tiles = al(sizeof(SmallComp) * comps.size());
     const size_t o_srcs = o_tiles + al(sizeof(SmallTile) * tiles.size());
     const size_t o_ws = o_srcs + al(4 * srcs.size());
-    const size_t t_bytes = o_ws + al(8 * ws.size());
+    const size_t o_ctr = o_ws + al(8 * ws.size());
+    const size_t t_bytes = o_ctr + 256;
     int rc;
     if (ss.pin_bytes < t_bytes) {
         if (ss.pin) (void)hipHostFree(ss.pin);
@@ -1430,10 +1413,59 @@ static int persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, con
     std::memcpy(stage + o_tiles, tiles.data(), sizeof(SmallTile) * tiles.size());
     std::memcpy(stage + o_srcs, srcs.data(), 4 * srcs.size());
     std::memcpy(stage + o_ws, ws.data(), 8 * ws.size());
+    std::memset(stage + o_ctr, 0, 256);
     if ((rc = ss.tables.ensure(ctx, t_bytes, "small tables")) ||
         (rc = ctx_hip(ctx, hipMemcpyAsync(ss.tables.p, stage, t_bytes, hipMemcpyHostToDevice, ctx->stream),
-                      "small tables")) ||
-        (rc = ss.counter.ensure(ctx, 64, "small counters")) ||
+                      "small tables")))
+        return rc;
+    unsigned char *d = (unsigned char *)ss.tables.p;
+    out.comps = (const SmallComp *)d;
+    out.d_tiles = (const SmallTile *)(d + o_tiles);
+    out.srcs = (const int32_t *)(d + o_srcs);
+    out.ws = (const double *)(d + o_ws);
+    out.counters = (int32_t *)(d + o_ctr);
+    return BCX_OK;
+}
+
+// One persistent launch over the tiles of `jobs`: the small-component kernel
+// (LDS state, n <= SMALL_N) or, with `wg`, the workgroup-per-tile kernel
+// (HBM slabs, n <= WG_N).  Tiles whose uint64 sigma overflows are rerun in
+// FP64 by a second launch.
+// Starts the pass on stream sp and returns without waiting for it;
+// persistent_finish waits, reruns the overflowed tiles and completes it.
+static int persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base,
+                            bcx_stats *st, bool wg, hipStream_t sp, bool probe) {
+    if (jobs.empty()) return BCX_OK;
+    if (!ctx->batched) ctx->batched = new BatchedState();
+    SmallState *&state = wg ? ctx->wgk : ctx->small;
+    if (!state) state = new SmallState();
+    SmallState &ss = *state;
+    int64_t nmax = 1, csr = 0;
+    for (const SmallJob &jb : jobs) {
+        nmax = std::max<int64_t>(nmax, jb.dc->n);
+        csr = std::max<int64_t>(csr, jb.dc->n + 1 + jb.dc->arcs);
+    }
+    // small kernel: a tile's CSR joins the LDS state when it fits beside the
+    // masks
+    csr = wg ? 0 : small_csr_words(nmax, csr);
+    // workgroup kernel: components whose path counts from their highest-degree
+    // vertex already pass 2^62 start with FP64 sigma (their tiles would all
+    // overflow the 64-bit pass); their tiles go after the others
+    std::vector<const SmallJob *> order;
+    for (const SmallJob &jb : jobs) order.push_back(&jb);
+    auto wide = [&](const SmallJob *jb) { return wg && jb->dc->sigma_est > 4.6e18; };
+    std::stable_partition(order.begin(), order.end(), [&](const SmallJob *jb) { return !wide(jb); });
+    // tiles of 64 W sources (source k + 64 h on lane k); the small kernel's are 64
+    const int W = wg ? wg_spl(o) : 1;
+    const size_t TW = (size_t)BATCH_W * W;
+    size_t n_narrow_tiles = 0;
+    for (const SmallJob *jb : order)
+        if (!wide(jb)) n_narrow_tiles += (jb->srcs.size() + TW - 1) / TW;
+    PassTables tb;
+    int rc = stage_tables(ctx, ss, order, bc_base, TW, tb);
+    if (rc) return rc;
+    std::vector<SmallTile> &tiles = tb.tiles;
+    if ((rc = ss.counter.ensure(ctx, 64, "small counters")) ||
         (rc = ss.redo.ensure(ctx, 4 * tiles.size(), "small redo list")))
         return rc;
     // as many small-kernel workgroups per CU as stay resident (LDS,
@@ -1467,12 +1499,11 @@ static int persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, con
                   (rc = ss.dbg.ensure(ctx, 8 * slab * grid, "probe delta"))))
         return rc;
     SmallArgs a{};
-    unsigned char *tb = (unsigned char *)ss.tables.p;
-    a.comps = (const SmallComp *)tb;
-    a.tiles = (const SmallTile *)(tb + o_tiles);
+    a.comps = tb.comps;
+    a.tiles = tb.d_tiles;
     a.n_tiles = (int32_t)tiles.size();
-    a.srcs = (const int32_t *)(tb + o_srcs);
-    a.ws = (const double *)(tb + o_ws);
+    a.srcs = tb.srcs;
+    a.ws = tb.ws;
     a.counter = (int32_t *)ss.counter.p;
     a.redo = (int32_t *)ss.redo.p;
     a.sig = (uint64_t *)ss.sig.p;
@@ -1561,17 +1592,141 @@ static int persistent_finish(bcx_ctx *ctx, bcx_stats *st, bool wg) {
     return BCX_OK;
 }
 
-int batched_persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base,
-                             bcx_stats *st, bool wg, hipStream_t sp) {
-    return persistent_start(ctx, jobs, o, bc_base, st, wg, sp, false);
+// ------------------------------------------------------------------------
+// wave-per-source pass (bcx_src.hip)
+// ------------------------------------------------------------------------
+
+// The wave-per-source kernel against the 64-source kernel (FP32C / FP64 terms,
+// us of a whole run over 20 components of n vertices and average degree d):
+// n 300, d 8 (16 sources in flight per workgroup): 267 / 179 against 429 / 438;
+// n 1200, d 8 (10): 1734 / 1517 against 3658 / 3921; n 2000, d 8 (5): 7509 /
+// 6507 against 9656 / 10431; n 2000, d 13 (4): 11855 / 9879 against 9969 /
+// 10863.  So it takes the components that leave LDS for five sources in flight
+// with FP32 terms (whose tiles of 64 sources stay on one workgroup), for four
+// with FP64 terms.
+bool src_takes(int64_t n, int64_t arcs, bool fp32) {
+    return n <= SRC_N && src_waves(n, arcs, SRC_LDS) >= (fp32 ? 5 : 4);
 }
 
-int batched_persistent_finish(bcx_ctx *ctx, bcx_stats *st, bool wg) { return persistent_finish(ctx, st, wg); }
+static bool run_fp32(const bcx_opts *o) { return o->path == BCX_PATH_BATCHED && o->precision == BCX_PREC_FP32C; }
+
+static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base,
+                     bcx_stats *st, hipStream_t sp, bool probe) {
+    if (jobs.empty()) return BCX_OK;
+    if (!ctx->srck) ctx->srck = new SmallState();
+    SmallState &ss = *ctx->srck;
+    // the costliest components first, so that the last tiles are short ones
+    std::vector<const SmallJob *> order;
+    size_t n_src = 0;
+    int64_t lds = 0;
+    for (const SmallJob &jb : jobs) {
+        order.push_back(&jb);
+        n_src += jb.srcs.size();
+        const int64_t shared = src_shared_bytes(jb.dc->n, jb.dc->arcs), wave = src_wave_bytes(jb.dc->n);
+        lds = std::max(lds, std::min(SRC_LDS, shared + SRC_WAVES * wave));
+    }
+    std::stable_sort(order.begin(), order.end(),
+                     [](const SmallJob *x, const SmallJob *y) { return x->dc->arcs > y->dc->arcs; });
+    // FP32 terms: tiles of 64 sources, the unit that a count overflow turns
+    // to FP64 terms; FP64 terms: as few as leave four tiles per compute unit
+    const bool fp32 = run_fp32(o);
+    size_t tw = BATCH_W;
+    if (!fp32 && !probe)
+        tw = std::min<size_t>(BATCH_W, std::max<size_t>(16, (n_src / (4 * (size_t)std::max(1, ctx->n_cu)) + 7) & ~(size_t)7));
+    PassTables tb;
+    int rc = stage_tables(ctx, ss, order, bc_base, tw, tb);
+    if (rc || (rc = ss.redo.ensure(ctx, 4 * tb.tiles.size(), "source redo list"))) return rc;
+    if (probe) {
+        size_t cells = 0;
+        for (const SmallJob &jb : jobs) cells = std::max(cells, (size_t)jb.dc->n * BATCH_W);
+        if ((rc = ss.psig.ensure(ctx, 8 * cells, "probe path counts")) ||
+            (rc = ss.lvl.ensure(ctx, 4 * cells, "probe levels")) || (rc = ss.dbg.ensure(ctx, 8 * cells, "probe delta")))
+            return rc;
+    }
+    SrcArgs a{};
+    a.comps = tb.comps;
+    a.tiles = tb.d_tiles;
+    a.n_tiles = (int32_t)tb.tiles.size();
+    a.lds = (int32_t)lds;
+    a.srcs = tb.srcs;
+    a.ws = tb.ws;
+    a.counter = tb.counters;
+    a.redo = (int32_t *)ss.redo.p;
+    a.limit = (o->sigma_f64_threshold_log2 > 0 && o->sigma_f64_threshold_log2 < 64)
+                  ? (1ull << o->sigma_f64_threshold_log2) : 0;
+    a.psig = probe ? (uint64_t *)ss.psig.p : nullptr;
+    a.lvl = probe ? (int32_t *)ss.lvl.p : nullptr;
+    a.dbg = probe ? (double *)ss.dbg.p : nullptr;
+    ss.src = a;
+    ss.run_fp32 = fp32;
+    ss.run_tiles = std::move(tb.tiles);
+    ss.run_grid = (int)std::min<int64_t>(a.n_tiles, (int64_t)src_blocks_per_cu(a.lds) * std::max(1, ctx->n_cu));
+    ss.run_stream = sp;
+    ss.pending = true;
+    if ((rc = follow_ctx_stream(ctx, sp))) return rc;
+    ctx->timer.begin(ctx);
+    rc = ctx_hip(ctx, launch_src(a, false, fp32, ss.run_grid, sp), "source kernel");
+    ctx->timer.end(ctx);
+    if (st) st->n_launches++;
+    return rc;
+}
+
+static int src_finish(bcx_ctx *ctx, bcx_stats *st) {
+    if (!ctx->srck || !ctx->srck->pending) return BCX_OK;
+    SmallState &ss = *ctx->srck;
+    ss.pending = false;
+    const hipStream_t sp = ss.run_stream;
+    SrcArgs a = ss.src;
+    int rc;
+    int32_t h[3];
+    if ((rc = ctx_hip(ctx, hipMemcpyAsync(h, a.counter, sizeof(h), hipMemcpyDeviceToHost, sp), "counter")) ||
+        (rc = ctx_hip(ctx, hipStreamSynchronize(sp), "source kernel")))
+        return rc;
+    if (h[1] > 0) {
+        // tiles with a uint64 overflow added nothing: rerun them in FP64
+        std::vector<int32_t> redo((size_t)h[1]);
+        if ((rc = ctx_hip(ctx, hipMemcpyAsync(redo.data(), a.redo, 4 * redo.size(), hipMemcpyDeviceToHost, sp), "redo")) ||
+            (rc = ctx_hip(ctx, hipStreamSynchronize(sp), "redo")))
+            return rc;
+        std::sort(redo.begin(), redo.end());
+        std::vector<SmallTile> again;
+        for (int32_t t : redo) again.push_back(ss.run_tiles[(size_t)t]);
+        if ((rc = upload(ctx, again.data(), sizeof(SmallTile) * again.size(), ss.tiles, "source tiles"))) return rc;
+        a.tiles = (const SmallTile *)ss.tiles.p;
+        a.n_tiles = (int32_t)again.size();
+        a.limit = 0;
+        a.counter += 4;
+        if (st) for (auto &t : again) st->n_f64_sigma += t.ns;
+        if ((rc = follow_ctx_stream(ctx, sp))) return rc;
+        ctx->timer.begin(ctx);
+        rc = ctx_hip(ctx, launch_src(a, true, ss.run_fp32, std::min(ss.run_grid, a.n_tiles), sp), "source kernel");
+        ctx->timer.end(ctx);
+        if (st) st->n_launches++;
+        int32_t h2[3];
+        if (rc || (rc = ctx_hip(ctx, hipMemcpyAsync(h2, a.counter, sizeof(h2), hipMemcpyDeviceToHost, sp), "counter")) ||
+            (rc = ctx_hip(ctx, hipStreamSynchronize(sp), "source kernel")))
+            return rc;
+        h[2] = std::max(h[2], h2[2]);
+    }
+    if (st && h[2] > st->max_level) st->max_level = h[2];
+    return BCX_OK;
+}
+
+int batched_persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base,
+                             bcx_stats *st, int pass, hipStream_t sp) {
+    if (pass == PASS_SRC) return src_start(ctx, jobs, o, bc_base, st, sp, false);
+    return persistent_start(ctx, jobs, o, bc_base, st, pass == PASS_WG, sp, false);
+}
+
+int batched_persistent_finish(bcx_ctx *ctx, bcx_stats *st, int pass) {
+    return pass == PASS_SRC ? src_finish(ctx, st) : persistent_finish(ctx, st, pass == PASS_WG);
+}
 
 void batched_persistent_reset(bcx_ctx *ctx) {
     if (ctx->side) (void)hipStreamSynchronize(ctx->side);
     if (ctx->small) ctx->small->pending = false;
     if (ctx->wgk) ctx->wgk->pending = false;
+    if (ctx->srck) ctx->srck->pending = false;
 }
 
 static void release_state(bcx_ctx *ctx, SmallState *&state) {
@@ -1589,6 +1744,7 @@ static void release_state(bcx_ctx *ctx, SmallState *&state) {
 void small_release(bcx_ctx *ctx) {
     release_state(ctx, ctx->small);
     release_state(ctx, ctx->wgk);
+    release_state(ctx, ctx->srck);
 }
 
 // Kernel the batched path runs component dc on, from the bcx_opts flags.
@@ -1759,20 +1915,23 @@ int batched_debug_tile(bcx_ctx *ctx, const bcx_component *comp, const int32_t *s
     }
     if (!rc && kind != BCX_KERNEL_MULTI) {
         const bool wg = kind == BCX_KERNEL_WG;
+        const bool by_src = kind == BCX_KERNEL_SMALL && src_takes(dc.n, dc.arcs, run_fp32(o));
         bcx_stats st{};
         if (!rc) {
             for (int32_t v = 0; v < n; ++v) at[v] = v;
             std::vector<SmallJob> jobs{{&dc, std::vector<int32_t>(srcs, srcs + ns)}};
-            rc = persistent_start(ctx, jobs, o, bc, &st, wg, ctx->stream, true);
-            if (!rc) rc = persistent_finish(ctx, &st, wg);
+            rc = by_src ? src_start(ctx, jobs, o, bc, &st, ctx->stream, true)
+                        : persistent_start(ctx, jobs, o, bc, &st, wg, ctx->stream, true);
+            if (!rc) rc = by_src ? src_finish(ctx, &st) : persistent_finish(ctx, &st, wg);
         }
         f64 = st.n_f64_sigma > 0;
         // one tile, so one workgroup: its slab is the start of every array
-        // (the workgroup kernel keeps lane-compacted records: its probe writes
-        // the path counts per (vertex, lane) beside them)
-        const SmallState *ss = wg ? ctx->wgk : ctx->small;
+        // (the workgroup kernel keeps lane-compacted records and the
+        // wave-per-source kernel its state in LDS: their probes write the path
+        // counts per (vertex, source) beside them)
+        const SmallState *ss = wg ? ctx->wgk : (by_src ? ctx->srck : ctx->small);
         if (!rc && ss) {
-            const void *sg_src = wg ? ss->psig.p : ss->sig.p;
+            const void *sg_src = wg || by_src ? ss->psig.p : ss->sig.p;
             rc = ctx_hip(ctx, hipMemcpyAsync(lv.data(), ss->lvl.p, 4 * cells, hipMemcpyDeviceToHost, ctx->stream),
                          "copy");
             if (!rc) rc = ctx_hip(ctx, hipMemcpyAsync(sg.data(), sg_src, 8 * cells, hipMemcpyDeviceToHost,

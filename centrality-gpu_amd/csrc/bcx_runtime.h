@@ -126,6 +126,7 @@ struct bcx_ctx {
     BatchedState *batched = nullptr;
     SmallState *small = nullptr;
     SmallState *wgk = nullptr;  // workgroup-per-tile kernel buffers
+    SmallState *srck = nullptr;  // wave-per-source kernel buffers
     std::vector<bcx::DBuf *> all_bufs() {
         return {&counters, &bc_acc, &plain_scratch, &rows_buf, &w_src, &w_aux, &w_mode, &w_slots, &bc_pack, &bc_chunks};
     }
@@ -164,12 +165,16 @@ std::vector<int32_t> tuned_sources(bcx::DComp &dc, const std::vector<int32_t> &s
 // Every vertex of the component in the order a full batched run tiles its
 // sources (64 consecutive entries per tile).
 std::vector<int32_t> batched_order(bcx::DComp &dc);
-// One persistent launch over the tiles of `jobs` (the small-component
-// kernel, or with `wg` the workgroup-per-tile kernel), started on stream sp
+// One persistent launch over the tiles of `jobs`, started on stream sp
 // without waiting; _finish waits for it and reruns overflowed tiles in FP64.
+// The passes: 64-source tiles of small components, the workgroup-per-tile
+// kernel, and the wave-per-source kernel (components that src_takes accepts).
+enum { PASS_SMALL = 0, PASS_WG = 1, PASS_SRC = 2 };
 int batched_persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base,
-                             bcx_stats *st, bool wg, hipStream_t sp);
-int batched_persistent_finish(bcx_ctx *ctx, bcx_stats *st, bool wg);
+                             bcx_stats *st, int pass, hipStream_t sp);
+int batched_persistent_finish(bcx_ctx *ctx, bcx_stats *st, int pass);
+// Whether the wave-per-source kernel takes a component, with FP32 or FP64 terms.
+bool src_takes(int64_t n, int64_t arcs, bool fp32);
 // Drops passes left unfinished by an earlier failed run (after waiting for them).
 void batched_persistent_reset(bcx_ctx *ctx);
 bool batched_narrow(bcx::DComp &dc);

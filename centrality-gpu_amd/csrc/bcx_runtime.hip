@@ -275,9 +275,18 @@ static int grid_for(bcx_ctx *ctx, int64_t count) {
     return (int)std::max<int64_t>(g, 1);
 }
 
+static int64_t plain_stride(int32_t n) { return ((int64_t)n + 2 + 63) & ~(int64_t)63; }
+constexpr size_t PLAIN_WORD_BYTES = 4 + 8 + 8 + 4 + 4;  // d, sig, dl, S, off
+
+// Whether the context's cap leaves room for the rows of `count` sources.
+static bool plain_scratch_fits(bcx_ctx *ctx, int32_t n, int64_t count) {
+    const size_t need = (size_t)plain_stride(n) * PLAIN_WORD_BYTES * (size_t)grid_for(ctx, count);
+    return need <= ctx->plain_scratch.bytes || ctx->mem_used - ctx->plain_scratch.bytes + need <= ctx->mem_cap;
+}
+
 static int ensure_plain_scratch(bcx_ctx *ctx, int32_t n, int grid, PlainScratch &sc) {
-    const int64_t stride = ((int64_t)n + 2 + 63) & ~(int64_t)63;
-    const size_t per = (size_t)stride * (4 + 8 + 8 + 4 + 4);
+    const int64_t stride = plain_stride(n);
+    const size_t per = (size_t)stride * PLAIN_WORD_BYTES;
     int rc = ctx->plain_scratch.ensure(ctx, per * (size_t)grid, "plain scratch");
     if (rc) return rc;
     char *p = (char *)ctx->plain_scratch.p;
@@ -691,6 +700,7 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
             sub[ci - 1].push_back((int32_t)(slot - dc.offset));
         }
     }
+    std::vector<SmallJob> srck;   // small components for the wave-per-source kernel (both paths)
     std::vector<SmallJob> small;  // batched path: components for the one-launch small kernel
     std::vector<SmallJob> wg;     // batched path: deep components for the workgroup-per-tile kernel
     std::vector<SmallJob> multi;  // batched path: components for the multi-launch tiles
@@ -709,6 +719,24 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
                             (double)n_chain * (8.0 * dc.arcs + 100.0 * dc.n);
             s->teps_work += (double)(n_bfs + n_chain) * (double)dc.arcs * 0.5;
         };
+        if (o.path == BCX_PATH_PLAIN && o.row_cap_bytes <= 0 && src_takes(dc.n, dc.arcs, false) &&
+            plain_scratch_fits(ctx, dc.n, sp ? sn : dc.n)) {
+            // every source runs on its own, chain vertices included: with the
+            // state in LDS a traversal costs less than the combine of two
+            // endpoint rows (a caller who sizes the row slab gets the rows,
+            // and a cap below the per-source rows is refused as before)
+            std::vector<uint8_t> want((size_t)dc.n, sp ? 0 : 1);
+            for (int64_t i = 0; i < sn; ++i) want[(size_t)sp[i]] = 1;
+            std::vector<int32_t> srcs;
+            for (int32_t v = 0; v < dc.n; ++v)
+                if (want[(size_t)v]) srcs.push_back(v);
+            int64_t n_chain = 0;
+            if (o.use_chains)
+                for (int32_t v : dc.host.ch_nodes) n_chain += want[(size_t)v];
+            account((int64_t)srcs.size() - n_chain, n_chain);
+            srck.push_back({&dc, std::move(srcs)});
+            continue;
+        }
         if (o.path == BCX_PATH_PLAIN) {
             Plan plan;
             rc = make_plan(dc.host, sp, sn, o.use_chains != 0, row_capacity(ctx, dc.n, &o), plan);
@@ -726,7 +754,7 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
         if (kind < 0) return kind;
         if (kind == BCX_KERNEL_SMALL) {
             s->n_comp_small++;
-            small.push_back({&dc, std::move(srcs)});
+            (src_takes(dc.n, dc.arcs, o.precision == BCX_PREC_FP32C) ? srck : small).push_back({&dc, std::move(srcs)});
             continue;
         }
         // larger components: tile order from the tuner (BFS ranks or balls)
@@ -745,22 +773,25 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
             multi.push_back({&dc, std::move(tiles)});
         }
     }
-    if (o.path == BCX_PATH_BATCHED && (!small.empty() || !wg.empty() || !multi.empty())) {
+    if (!srck.empty() || !small.empty() || !wg.empty() || !multi.empty()) {
         // the persistent passes (small components, deep components) run on a
         // side stream while the multi-launch tiles run on theirs; the run is
         // timed as one interval on the context stream around both
-        const bool overlap = !multi.empty() && (!small.empty() || !wg.empty());
+        const bool overlap = !multi.empty() && (!srck.empty() || !small.empty() || !wg.empty());
         if (overlap && !ctx->side &&
             (rc = ctx_hip(ctx, hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking), "side stream")))
             return rc;
         const hipStream_t sp = overlap ? ctx->side : ctx->stream;
         ctx->timer.begin(ctx);
-        if (!small.empty() && (rc = batched_persistent_start(ctx, small, &o, bc, s, false, sp))) return rc;
-        if (!wg.empty() && (rc = batched_persistent_start(ctx, wg, &o, bc, s, true, sp))) return rc;
+        if ((rc = batched_persistent_start(ctx, srck, &o, bc, s, PASS_SRC, sp)) ||
+            (rc = batched_persistent_start(ctx, small, &o, bc, s, PASS_SMALL, sp)) ||
+            (rc = batched_persistent_start(ctx, wg, &o, bc, s, PASS_WG, sp)))
+            return rc;
         for (SmallJob &jb : multi)
             if ((rc = batched_component(ctx, *const_cast<DComp *>(jb.dc), jb.srcs, &o, bc + jb.dc->offset, s)))
                 return rc;
-        if ((rc = batched_persistent_finish(ctx, s, false)) || (rc = batched_persistent_finish(ctx, s, true)))
+        if ((rc = batched_persistent_finish(ctx, s, PASS_SRC)) || (rc = batched_persistent_finish(ctx, s, PASS_SMALL)) ||
+            (rc = batched_persistent_finish(ctx, s, PASS_WG)))
             return rc;
         if (overlap) {
             hipEvent_t ev;
