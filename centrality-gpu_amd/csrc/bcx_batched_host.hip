@@ -1273,6 +1273,7 @@ struct SmallState {
     SmallArgs run{};
     SrcArgs src{};  // (wave-per-source pass)
     std::vector<SmallTile> run_tiles;
+    std::vector<std::pair<double *, int32_t>> run_slices;  // (wave-per-source pass) BC slice of each component
     size_t run_narrow = 0;
     int run_grid = 0;
     hipStream_t run_stream = nullptr;
@@ -1597,15 +1598,14 @@ static int persistent_finish(bcx_ctx *ctx, bcx_stats *st, bool wg) {
 // ------------------------------------------------------------------------
 
 // The wave-per-source kernel against the 64-source kernel (FP32C / FP64 terms,
-// us of a whole run over 20 components of n vertices and average degree d):
-// n 300, d 8 (16 sources in flight per workgroup): 267 / 179 against 429 / 438;
-// n 1200, d 8 (10): 1734 / 1517 against 3658 / 3921; n 2000, d 8 (5): 7509 /
-// 6507 against 9656 / 10431; n 2000, d 13 (4): 11855 / 9879 against 9969 /
-// 10863.  So it takes the components that leave LDS for five sources in flight
-// with FP32 terms (whose tiles of 64 sources stay on one workgroup), for four
-// with FP64 terms.
-bool src_takes(int64_t n, int64_t arcs, bool fp32) {
-    return n <= SRC_N && src_waves(n, arcs, SRC_LDS) >= (fp32 ? 5 : 4);
+// us of a whole run over 20 components of n vertices and average degree d; w:
+// sources in flight that their LDS leaves room for): n 300, d 8, w 16: 206 /
+// 153 against 429 / 438; n 1200, d 8, w 9: 1226 / 1018 against 3658 / 3921;
+// n 2000, d 8, w 4: 5268 / 4277 against 9639 / 10480; n 2000, d 13, w 3: 8336 /
+// 6754 against 10013 / 10866; n 2048, d 20, w 2: 16386 / 13395 against 12942 /
+// 13690 (one such component: 5417 / 1346 against 3561 / 3678).
+bool src_takes(const DComp &dc, bool fp32) {
+    return dc.n <= SRC_N && src_waves(dc.n, dc.groups, SRC_LDS) >= (fp32 ? 3 : 2);
 }
 
 static bool run_fp32(const bcx_opts *o) { return o->path == BCX_PATH_BATCHED && o->precision == BCX_PREC_FP32C; }
@@ -1622,17 +1622,18 @@ static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_
     for (const SmallJob &jb : jobs) {
         order.push_back(&jb);
         n_src += jb.srcs.size();
-        const int64_t shared = src_shared_bytes(jb.dc->n, jb.dc->arcs), wave = src_wave_bytes(jb.dc->n);
+        const int64_t shared = src_shared_bytes(jb.dc->n, jb.dc->groups), wave = src_wave_bytes(jb.dc->n);
         lds = std::max(lds, std::min(SRC_LDS, shared + SRC_WAVES * wave));
     }
     std::stable_sort(order.begin(), order.end(),
                      [](const SmallJob *x, const SmallJob *y) { return x->dc->arcs > y->dc->arcs; });
-    // FP32 terms: tiles of 64 sources, the unit that a count overflow turns
-    // to FP64 terms; FP64 terms: as few as leave four tiles per compute unit
+    // as few sources per tile as leave four tiles per compute unit.  With FP32
+    // terms a count overflow turns the 64 consecutive sources around it to FP64
+    // terms, so smaller tiles are a first try: an overflow (rare in components
+    // of this size) ends it and the pass is repeated in tiles of 64
     const bool fp32 = run_fp32(o);
-    size_t tw = BATCH_W;
-    if (!fp32 && !probe)
-        tw = std::min<size_t>(BATCH_W, std::max<size_t>(16, (n_src / (4 * (size_t)std::max(1, ctx->n_cu)) + 7) & ~(size_t)7));
+    const size_t per = n_src / (4 * (size_t)std::max(1, ctx->n_cu));
+    const size_t tw = probe || per > 32 ? BATCH_W : (per > 16 ? 32 : 16);
     PassTables tb;
     int rc = stage_tables(ctx, ss, order, bc_base, tw, tb);
     if (rc || (rc = ss.redo.ensure(ctx, 4 * tb.tiles.size(), "source redo list"))) return rc;
@@ -1654,10 +1655,13 @@ static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_
     a.redo = (int32_t *)ss.redo.p;
     a.limit = (o->sigma_f64_threshold_log2 > 0 && o->sigma_f64_threshold_log2 < 64)
                   ? (1ull << o->sigma_f64_threshold_log2) : 0;
+    a.stop = fp32 && tw < BATCH_W;
     a.psig = probe ? (uint64_t *)ss.psig.p : nullptr;
     a.lvl = probe ? (int32_t *)ss.lvl.p : nullptr;
     a.dbg = probe ? (double *)ss.dbg.p : nullptr;
     ss.src = a;
+    ss.run_slices.clear();
+    for (const SmallJob *jb : order) ss.run_slices.push_back({bc_base + jb->dc->offset, jb->dc->n});
     ss.run_fp32 = fp32;
     ss.run_tiles = std::move(tb.tiles);
     ss.run_grid = (int)std::min<int64_t>(a.n_tiles, (int64_t)src_blocks_per_cu(a.lds) * std::max(1, ctx->n_cu));
@@ -1678,10 +1682,42 @@ static int src_finish(bcx_ctx *ctx, bcx_stats *st) {
     const hipStream_t sp = ss.run_stream;
     SrcArgs a = ss.src;
     int rc;
-    int32_t h[3];
-    if ((rc = ctx_hip(ctx, hipMemcpyAsync(h, a.counter, sizeof(h), hipMemcpyDeviceToHost, sp), "counter")) ||
-        (rc = ctx_hip(ctx, hipStreamSynchronize(sp), "source kernel")))
-        return rc;
+    int32_t h[3] = {0, 0, 0};
+    auto counters = [&](const int32_t *from) {
+        int32_t c[3];
+        int r = ctx_hip(ctx, hipMemcpyAsync(c, from, sizeof(c), hipMemcpyDeviceToHost, sp), "counter");
+        if (!r) r = ctx_hip(ctx, hipStreamSynchronize(sp), "source kernel");
+        h[1] = c[1];
+        h[2] = std::max(h[2], c[2]);
+        return r;
+    };
+    // another launch over `tiles`, with counters of its own
+    auto again = [&](const std::vector<SmallTile> &tiles, bool f64) {
+        int r = upload(ctx, tiles.data(), sizeof(SmallTile) * tiles.size(), ss.tiles, "source tiles");
+        if (r || (r = follow_ctx_stream(ctx, sp))) return r;
+        a.tiles = (const SmallTile *)ss.tiles.p;
+        a.n_tiles = (int32_t)tiles.size();
+        a.counter += 4;
+        a.stop = 0;
+        ctx->timer.begin(ctx);
+        r = ctx_hip(ctx, launch_src(a, f64, ss.run_fp32, std::min(ss.run_grid, a.n_tiles), sp), "source kernel");
+        ctx->timer.end(ctx);
+        if (st) st->n_launches++;
+        return r ? r : counters(a.counter);
+    };
+    if ((rc = counters(a.counter))) return rc;
+    if (h[1] > 0 && a.stop) {
+        for (auto &s : ss.run_slices)
+            if ((rc = ctx_hip(ctx, hipMemsetAsync(s.first, 0, sizeof(double) * (size_t)s.second, ctx->stream), "memset")))
+                return rc;
+        std::vector<SmallTile> wide;
+        for (const SmallTile &t : ss.run_tiles) {
+            if (!wide.empty() && wide.back().comp == t.comp && wide.back().ns < BATCH_W) wide.back().ns += t.ns;
+            else wide.push_back(t);
+        }
+        ss.run_tiles.swap(wide);
+        if ((rc = again(ss.run_tiles, false))) return rc;
+    }
     if (h[1] > 0) {
         // tiles with a uint64 overflow added nothing: rerun them in FP64
         std::vector<int32_t> redo((size_t)h[1]);
@@ -1689,24 +1725,11 @@ static int src_finish(bcx_ctx *ctx, bcx_stats *st) {
             (rc = ctx_hip(ctx, hipStreamSynchronize(sp), "redo")))
             return rc;
         std::sort(redo.begin(), redo.end());
-        std::vector<SmallTile> again;
-        for (int32_t t : redo) again.push_back(ss.run_tiles[(size_t)t]);
-        if ((rc = upload(ctx, again.data(), sizeof(SmallTile) * again.size(), ss.tiles, "source tiles"))) return rc;
-        a.tiles = (const SmallTile *)ss.tiles.p;
-        a.n_tiles = (int32_t)again.size();
+        std::vector<SmallTile> wide;
+        for (int32_t t : redo) wide.push_back(ss.run_tiles[(size_t)t]);
+        if (st) for (auto &t : wide) st->n_f64_sigma += t.ns;
         a.limit = 0;
-        a.counter += 4;
-        if (st) for (auto &t : again) st->n_f64_sigma += t.ns;
-        if ((rc = follow_ctx_stream(ctx, sp))) return rc;
-        ctx->timer.begin(ctx);
-        rc = ctx_hip(ctx, launch_src(a, true, ss.run_fp32, std::min(ss.run_grid, a.n_tiles), sp), "source kernel");
-        ctx->timer.end(ctx);
-        if (st) st->n_launches++;
-        int32_t h2[3];
-        if (rc || (rc = ctx_hip(ctx, hipMemcpyAsync(h2, a.counter, sizeof(h2), hipMemcpyDeviceToHost, sp), "counter")) ||
-            (rc = ctx_hip(ctx, hipStreamSynchronize(sp), "source kernel")))
-            return rc;
-        h[2] = std::max(h[2], h2[2]);
+        if ((rc = again(wide, true))) return rc;
     }
     if (st && h[2] > st->max_level) st->max_level = h[2];
     return BCX_OK;
@@ -1915,7 +1938,7 @@ int batched_debug_tile(bcx_ctx *ctx, const bcx_component *comp, const int32_t *s
     }
     if (!rc && kind != BCX_KERNEL_MULTI) {
         const bool wg = kind == BCX_KERNEL_WG;
-        const bool by_src = kind == BCX_KERNEL_SMALL && src_takes(dc.n, dc.arcs, run_fp32(o));
+        const bool by_src = kind == BCX_KERNEL_SMALL && src_takes(dc, run_fp32(o));
         bcx_stats st{};
         if (!rc) {
             for (int32_t v = 0; v < n; ++v) at[v] = v;

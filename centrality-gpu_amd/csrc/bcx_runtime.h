@@ -58,6 +58,7 @@ struct DComp {
     std::vector<int32_t> ball;      // batched path: every vertex in ball-tile order (built on first use)
     int8_t tile_order = -1;         // batched path: 0 BFS-rank, 1 ball, 2 landmark tiles (tuned on first use)
     std::vector<int32_t> lm_pos;    // batched path: position of each vertex in the landmark order
+    int64_t groups = 0;             // sum over the rows of ceil(arcs / 4) (wave-per-source kernel)
     HostComp host;
     DBuf b_rp, b_col, b_reach, b_chp, b_chn, b_che;
     CompDev dev{};
@@ -174,7 +175,7 @@ int batched_persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, co
                              bcx_stats *st, int pass, hipStream_t sp);
 int batched_persistent_finish(bcx_ctx *ctx, bcx_stats *st, int pass);
 // Whether the wave-per-source kernel takes a component, with FP32 or FP64 terms.
-bool src_takes(int64_t n, int64_t arcs, bool fp32);
+bool src_takes(const bcx::DComp &dc, bool fp32);
 // Drops passes left unfinished by an earlier failed run (after waiting for them).
 void batched_persistent_reset(bcx_ctx *ctx);
 bool batched_narrow(bcx::DComp &dc);

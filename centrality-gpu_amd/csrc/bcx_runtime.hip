@@ -513,6 +513,7 @@ int bcx_upload(bcx_ctx *ctx, const bcx_component *comps, int32_t n_comps, bcx_dg
         hc.n = c.n;
         hc.arcs = c.arcs;
         hc.rp.assign(c.row_ptr, c.row_ptr + c.n + 1);
+        for (int32_t v = 0; v < c.n; ++v) dc.groups += (hc.rp[v + 1] - hc.rp[v] + 3) / 4;
         hc.col.assign(c.col, c.col + c.arcs);
         hc.reach.assign(c.reach, c.reach + c.n);
         hc.n_chains = std::max(c.n_chains, 0);
@@ -719,7 +720,7 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
                             (double)n_chain * (8.0 * dc.arcs + 100.0 * dc.n);
             s->teps_work += (double)(n_bfs + n_chain) * (double)dc.arcs * 0.5;
         };
-        if (o.path == BCX_PATH_PLAIN && o.row_cap_bytes <= 0 && src_takes(dc.n, dc.arcs, false) &&
+        if (o.path == BCX_PATH_PLAIN && o.row_cap_bytes <= 0 && src_takes(dc, false) &&
             plain_scratch_fits(ctx, dc.n, sp ? sn : dc.n)) {
             // every source runs on its own, chain vertices included: with the
             // state in LDS a traversal costs less than the combine of two
@@ -754,7 +755,7 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
         if (kind < 0) return kind;
         if (kind == BCX_KERNEL_SMALL) {
             s->n_comp_small++;
-            (src_takes(dc.n, dc.arcs, o.precision == BCX_PREC_FP32C) ? srck : small).push_back({&dc, std::move(srcs)});
+            (src_takes(dc, o.precision == BCX_PREC_FP32C) ? srck : small).push_back({&dc, std::move(srcs)});
             continue;
         }
         // larger components: tile order from the tuner (BFS ranks or balls)

@@ -8,24 +8,27 @@
 namespace bcx {
 
 // LDS of a workgroup.  Shared by its waves: the component's BC accumulator
-// (8 B per vertex), row pointers (4 B) and columns (2 B per arc).  Per wave,
-// i.e. per source in flight: one 8-byte word per vertex (the path count, which
-// the backward overwrites with the vertex's term), the level codes (2 bits)
-// and the level-ordered vertex list (2 B).
+// (8 B per vertex), row pointers (4 B) and columns (2 B per arc), rows padded to
+// groups of four arcs with one empty group at the end.
+// Per wave, i.e. per source in flight: one 8-byte word per vertex (the path
+// count, which the backward overwrites with the vertex's term), a level code
+// (1 B) and the level-ordered vertex list (2 B), each with two more entries
+// that lanes without an arc of their own read and write.
 constexpr int SRC_N = 2048;                 // largest component (list entries are 15-bit ids and a flag)
 constexpr int SRC_WAVES = 16;               // waves of a workgroup
 constexpr int64_t SRC_LDS = 160 * 1024 - 512;  // dynamic LDS of a workgroup at most
 
 __host__ __device__ constexpr int64_t src_up16(int64_t x) { return (x + 15) & ~(int64_t)15; }
-__host__ __device__ constexpr int64_t src_shared_bytes(int64_t n, int64_t arcs) {
-    return src_up16(8 * n) + src_up16(4 * (n + 1)) + src_up16(2 * arcs);
+// (groups: sum over the rows of ceil(arcs / 4))
+__host__ __device__ constexpr int64_t src_shared_bytes(int64_t n, int64_t groups) {
+    return src_up16(8 * n) + src_up16(4 * (n + 1)) + src_up16(8 * (groups + 1));
 }
 __host__ __device__ constexpr int64_t src_wave_bytes(int64_t n) {
-    return src_up16(8 * n) + src_up16(4 * ((n + 15) / 16)) + src_up16(2 * n);
+    return src_up16(8 * (n + 2)) + src_up16(n + 2) + src_up16(2 * (n + 2));
 }
 // Sources in flight in a workgroup of `lds` dynamic bytes.
-__host__ __device__ constexpr int64_t src_waves(int64_t n, int64_t arcs, int64_t lds) {
-    const int64_t w = (lds - src_shared_bytes(n, arcs)) / src_wave_bytes(n);
+__host__ __device__ constexpr int64_t src_waves(int64_t n, int64_t groups, int64_t lds) {
+    const int64_t w = (lds - src_shared_bytes(n, groups)) / src_wave_bytes(n);
     return w < 0 ? 0 : (w > SRC_WAVES ? SRC_WAVES : w);
 }
 
@@ -39,6 +42,7 @@ struct SrcArgs {
     int32_t *counter;        // [0] work counter, [1] tiles listed for an FP64 rerun, [2] deepest level
     int32_t *redo;           // [n_tiles] those tiles
     uint64_t limit;          // u64 path-count threshold (0 = 2^64)
+    int32_t stop;            // take no further tile once one has overflowed
     // probe only (null in runs): [n][64] per (vertex, source) of the last tile
     uint64_t *psig;
     int32_t *lvl;
