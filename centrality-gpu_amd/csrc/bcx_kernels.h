@@ -47,11 +47,20 @@ struct PlainArgs {
     uint64_t limit;        // u64 overflow threshold (0 = 2^64)
     int32_t *counters;
     double *bc;            // component slice of the BC accumulator
+    double *probe;         // probe only: [2n] dependencies, then (chain sources) the terms
 };
 
+// Launch shape of a component: waves per workgroup, workgroups per compute
+// unit, dynamic LDS, and whether a source's level codes fit in LDS.
+struct PlainShape {
+    int waves, per_cu, lds;
+    bool lds_codes;
+};
+PlainShape plain_shape(int32_t n);
+
 hipError_t launch_plain_bfs(const CompDev &c, const PlainArgs &a, const PlainScratch &sc,
-                            const Rows &rows, int grid, hipStream_t st);
+                            const Rows &rows, const PlainShape &p, int grid, hipStream_t st);
 hipError_t launch_plain_chain(const CompDev &c, const ChainDev &ch, const PlainArgs &a,
-                              const PlainScratch &sc, const Rows &rows, int grid, hipStream_t st);
+                              const PlainScratch &sc, const Rows &rows, const PlainShape &p, int grid, hipStream_t st);
 
 }  // namespace bcx

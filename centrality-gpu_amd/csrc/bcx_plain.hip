@@ -2,221 +2,497 @@
 // atomic work counter (the schedule of Codes/kernels_free.cu:154-473 and
 // Codes/kernels_active.cu:263-602), written for wave64 gfx950.
 //
-// Forward: level-synchronous top-down BFS.  A frontier vertex of degree <= 64
-// is expanded by one lane, a hub by a whole wave (lanes stride its arcs).
-// Discovery by CAS on the level word, sigma pushed with 64-bit atomics (exact
-// integer sums, order free) and the wrap of any partial sum flagged; in FP64
-// mode sigma is pulled per vertex in CSR order instead (the oracle's order,
-// so FP64 sigma is bit-exact).
-// Backward: successor method, delta_w = sum_v sigma_w/sigma_v (r(v)+1+delta_v)
-// in FP64, pulled per vertex (Codes/kernels_free.cu:378-421); BC[w] gets
-// (r(s)+1) delta_w through FP64 atomics (Codes/kernels_free.cu:423-426).
+// A level code of two bits per vertex (0: not reached, else 1 + level mod 3) is
+// all that an arc needs to know about its far end, because an arc joins levels
+// that differ by at most one.  The codes of a source sit in LDS (n / 4 bytes),
+// so an arc that leads nowhere costs no access to global memory.
+//
+// Forward, one walk over the arcs of each level's vertices: an arc to the level
+// below adds its path count (exact uint64 with the wrap of any sum flagged; in
+// FP64 mode the sum runs in CSR order, the oracle's, so FP64 counts are
+// bit-exact), an arc to an unreached vertex takes it by an LDS atomic and
+// appends it to the level-ordered list.  Backward, one walk: rho_v = sum of t_w
+// over successors, t_v = (r(v)+1)/sigma_v + rho_v, delta_v = sigma_v rho_v
+// (Codes/kernels_free.cu:378-421 computes the same with a division and three
+// gathers per arc); BC[v] gets (r(s)+1) delta_v through FP64 atomics
+// (Codes/kernels_free.cu:423-426).  t_v takes the place of sigma_v.
+//
+// What bounds it: the gathers of counts and terms along shortest-path arcs,
+// whose lines miss L2 on cores of 10^5 vertices (12.7 us per source of an 84k
+// core, the same with 256 and 512 sources in flight), and the dependent loads
+// per level on deep graphs.  Against level words, list marks and count atomics
+// in global memory with a lane per vertex: 1000 sources of the 84k core 165 ->
+// 19 ms, 2049 sources of an 18.6k grid 27.4 -> 5.1 ms.
+//
+// A wave takes 64 vertices of a level.  Short rows are walked by a lane each,
+// four arcs per step; longer ones as one flat range with a lane per arc, whose
+// row is found by a search over the rows' first arcs in LDS and whose value is
+// added to the row's sum in LDS; rows above HUB arcs by the whole wave.
+//
 // Chain sources: combine of two endpoint rows (Codes/postprocesses.cu:276-363)
-// and level buckets by an LDS counting sort in place of the CUB radix sort
+// and level buckets by a counting sort in place of the CUB radix sort
 // (Codes/postprocesses.cu:143-155), then the same backward.
 #include "bcx_device.h"
 #include "bcx_kernels.h"
 
+#include <algorithm>
+
 namespace bcx {
 
-constexpr int PB = 256;            // threads per workgroup
-constexpr int PW = PB / 64;        // waves per workgroup
-constexpr int HUB = 64;            // degree above which a wave expands a vertex
-constexpr int LDS_LEVELS = 4096;   // level histogram held in LDS
+namespace {
 
-struct FwdShared {
-    int cnt;
-    int ovf;
+constexpr int SHORT = 8;          // rows of a wave's vertices up to which a lane walks its own
+constexpr int HUB = 256;          // degree above which a wave walks a row alone
+constexpr int LDS_LEVELS = 1024;  // level offsets (chain kernel: level histogram) held in LDS
+constexpr int PMAXW = 16;         // waves of a workgroup at most
+// vertices whose level codes fit in LDS beside a workgroup's other arrays;
+// above, the codes live in the workgroup's rows in global memory
+constexpr int LV_LDS_N = 400000;
+
+// LDS of one wave: the flat walk's first arcs, their offset into the CSR and
+// the rows' sums
+struct WaveRows {
+    int P[64], A[64];
+    uint64_t acc[64];
+};
+
+struct PlainShared {
+    int cnt[3];  // vertices appended at a level, by level mod 3
+    int ovf[3];  // a count of the level overflowed, likewise
+    int item, stop, top;
+    int off[LDS_LEVELS];
 };
 
 __device__ __forceinline__ uint64_t sig_one(bool f64) { return f64 ? d2u(1.0) : 1ull; }
+__device__ __forceinline__ uint64_t pbal(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+__device__ __forceinline__ int prank(uint64_t b, int from) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, (uint32_t)from));
+}
+__device__ __forceinline__ uint64_t prl64(uint64_t x, int src) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, src);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), src);
+    return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ void psync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
-__device__ __forceinline__ void visit(const CompDev &c, int32_t *d, uint64_t *sg, int32_t *S,
-                                      int w, int lvl, int tail, uint64_t sv, bool f64,
-                                      uint64_t limit, FwdShared *sh) {
-    int dw = ald(&d[w]);
-    if (dw == BCX_INF) {
-        int old = atomicCAS(&d[w], BCX_INF, lvl + 1);
-        if (old == BCX_INF) {
-            int pos = atomicAdd(&sh->cnt, 1);
-            S[tail + pos] = w;
-            dw = lvl + 1;
-        } else {
-            dw = old;
-        }
+// Workgroup barrier after every outstanding memory access of the wave.
+__device__ __forceinline__ void pbarrier() {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+}
+
+// Level codes, 16 per word, in LDS or (LG) in global memory, where they are
+// set by L2 atomics and read past the vector L1.
+template <bool LG>
+struct Codes {
+    uint32_t *w;
+    __device__ __forceinline__ uint32_t get(int v) const {
+        const uint32_t x = LG ? (uint32_t)ald((const int32_t *)&w[v >> 4]) : w[v >> 4];
+        return (x >> (2 * (v & 15))) & 3u;
     }
-    if (!f64 && dw == lvl + 1) {
-        uint64_t old = atomicAdd((unsigned long long *)&sg[w], (unsigned long long)sv);
-        uint64_t nw = old + sv;
-        if (nw < old || (limit && nw >= limit)) sh->ovf = 1;
+    // sets an unset code; true for the one that did
+    __device__ __forceinline__ bool take(int v, uint32_t c) const {
+        const int sh = 2 * (v & 15);
+        return ((atomicOr(&w[v >> 4], c << sh) >> sh) & 3u) == 0;
+    }
+};
+
+// What a workgroup works on: its source's arrays.
+template <bool LG>
+struct PlainCtx {
+    const gint *rp, *col, *reach;
+    int n;
+    Codes<LG> lv;
+    uint64_t *sg;   // path counts
+    double *tt;     // terms (the same words as sg, unless sg is kept)
+    int32_t *S;     // vertices in level order
+    int32_t *off;   // level offsets past LDS_LEVELS
+    int32_t *drow;  // levels, when the source's row is kept
+    PlainShared *sh;
+    WaveRows *wr;   // this wave's
+    __device__ __forceinline__ int level_off(int l) const { return l < LDS_LEVELS ? sh->off[l] : off[l]; }
+    __device__ __forceinline__ void set_off(int l, int x) const {
+        if (l < LDS_LEVELS) sh->off[l] = x;
+        else off[l] = x;
+    }
+};
+
+// Row of flat arc g: the last k with P[k] <= g.
+__device__ __forceinline__ int row_of(const WaveRows &r, int g) {
+    int k = 0;
+#pragma unroll
+    for (int h = 32; h > 0; h >>= 1)
+        if (r.P[k + h] <= g) k += h;
+    return k;
+}
+
+// Lays the wave's rows (d arcs from j0 on each lane) out as one flat range;
+// returns its length.
+__device__ __forceinline__ int flat_rows(WaveRows &r, int j0, int d) {
+    const int lane = threadIdx.x & 63;
+    int inc = d;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += y;
+    }
+    r.P[lane] = inc - d;
+    r.A[lane] = j0 - (inc - d);
+    r.acc[lane] = 0;
+    psync();
+    return __builtin_amdgcn_readlane(inc, 63);
+}
+
+// Appends the vertices that the wave's lanes took to level l+1's list.
+template <int U, bool LG>
+__device__ __forceinline__ void append(const PlainCtx<LG> &x, const int (&w)[U], const bool (&mine)[U], int q1,
+                                       int *cnt) {
+    uint64_t b[U];
+    int tot = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        b[u] = pbal(mine[u]);
+        tot += __popcll(b[u]);
+    }
+    if (tot == 0) return;
+    int pos = 0;
+    if ((threadIdx.x & 63) == 0) pos = atomicAdd(cnt, tot);
+    pos = q1 + __builtin_amdgcn_readlane(pos, 0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (mine[u]) x.S[prank(b[u], pos)] = w[u];
+        pos += __popcll(b[u]);
     }
 }
 
-// Forward BFS from s.  Returns the deepest level; S holds the vertices in
-// level order with off[l]..off[l+1] the range of level l.
-__device__ int plain_forward(const CompDev &c, int32_t s, int32_t *d, uint64_t *sg, int32_t *S,
-                             int32_t *off, bool f64, uint64_t limit, FwdShared *sh) {
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    for (int k = tid; k < c.n; k += PB) {
-        ast(&d[k], BCX_INF);
-        ast(&sg[k], (uint64_t)0);
-    }
-    __syncthreads();
+constexpr int PU = 4;  // arcs of a lane in flight
+
+// Forward BFS from s.  Returns the deepest level, -1 when a uint64 count
+// overflowed.
+template <bool F64, bool LG>
+__device__ __forceinline__ int plain_forward(const PlainCtx<LG> &x, int s, uint64_t limit) {
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wv = tid >> 6;
+    PlainShared *sh = x.sh;
+    for (int k = tid; k < (x.n + 15) / 16; k += nt) x.lv.w[k] = 0;
+    if (tid < 3) sh->cnt[tid] = sh->ovf[tid] = 0;
+    pbarrier();
     if (tid == 0) {
-        ast(&d[s], 0);
-        ast(&sg[s], sig_one(f64));
-        S[0] = s;
-        off[0] = 0;
-        off[1] = 1;
-        sh->cnt = 0;
+        x.lv.take(s, 1);
+        x.sg[s] = sig_one(F64);
+        x.S[0] = s;
+        x.set_off(0, 0);
+        x.set_off(1, 1);
     }
-    __syncthreads();
-    int head = 0, tail = 1, lvl = 0;
+    pbarrier();
+    int q0 = 0, q1 = 1, l = 0;
+    uint32_t cprev = 3, cnext = 2;  // codes of levels l-1 (l = 0: none set) and l+1
     while (true) {
-        for (int i = head + tid; i < tail; i += PB) {
-            int v = S[i];
-            int j0 = c.rp[v], j1 = c.rp[v + 1];
-            if (j1 - j0 > HUB) continue;
-            uint64_t sv = f64 ? 0 : ald(&sg[v]);
-            for (int j = j0; j < j1; ++j) visit(c, d, sg, S, c.col[j], lvl, tail, sv, f64, limit, sh);
-        }
-        for (int i = head + wave; i < tail; i += PW) {
-            int v = S[i];
-            int j0 = c.rp[v], j1 = c.rp[v + 1];
-            if (j1 - j0 <= HUB) continue;
-            uint64_t sv = f64 ? 0 : ald(&sg[v]);
-            for (int j = j0 + lane; j < j1; j += 64) visit(c, d, sg, S, c.col[j], lvl, tail, sv, f64, limit, sh);
-        }
-        __syncthreads();
-        const int cnt = sh->cnt;
-        __syncthreads();
-        if (cnt == 0) break;
-        if (tid == 0) {
-            sh->cnt = 0;
-            off[lvl + 2] = tail + cnt;
-        }
-        head = tail;
-        tail += cnt;
-        lvl++;
-        if (f64) {
-            // pull: sigma_w = sum over predecessors in CSR order
-            for (int i = head + tid; i < tail; i += PB) {
-                int w = S[i];
-                double acc = 0.0;
-                for (int j = c.rp[w]; j < c.rp[w + 1]; ++j) {
-                    int v = c.col[j];
-                    if (ald(&d[v]) == lvl - 1) acc += u2d(ald(&sg[v]));
+        int *cnt = &sh->cnt[l % 3];
+        // (last read two levels ago)
+        if (tid == 0) sh->cnt[(l + 1) % 3] = sh->ovf[(l + 1) % 3] = 0;
+        for (int base = q0 + wv * 64; base < q1; base += nt) {
+            const int e = base + lane;
+            int v = 0, j0 = 0, j1 = 0;
+            if (e < q1) {
+                v = x.S[e];
+                j0 = x.rp[v];
+                j1 = x.rp[v + 1];
+            }
+            const int d = j1 - j0;
+            const uint64_t hubs = pbal(d > HUB);
+            const int je = d > HUB ? j0 : j1;
+            uint64_t acc = 0;
+            double facc = 0.0;
+            bool ovf = false;
+            if (F64 || !pbal(d > SHORT)) {
+                for (int j = j0; pbal(j < je); j += PU) {
+                    int w[PU];
+                    uint32_t f[PU];
+                    uint64_t y[PU];
+                    bool mine[PU];
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) w[u] = j + u < je ? x.col[j + u] : -1;
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) f[u] = x.lv.get(max(w[u], 0));
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) y[u] = w[u] >= 0 && f[u] == cprev ? x.sg[w[u]] : 0;
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) mine[u] = w[u] >= 0 && f[u] == 0 && x.lv.take(w[u], cnext);
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) {
+                        if (F64) facc += u2d(y[u]);
+                        else ovf |= __builtin_add_overflow(acc, y[u], &acc);
+                    }
+                    append<PU>(x, w, mine, q1, cnt);
                 }
-                ast(&sg[w], d2u(acc));
+            } else {
+                WaveRows &r = *x.wr;
+                const int T = flat_rows(r, j0, je - j0);
+                for (int g0 = 0; g0 < T; g0 += 64 * PU) {
+                    int w[PU], k[PU];
+                    uint32_t f[PU];
+                    uint64_t y[PU];
+                    bool mine[PU];
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) {
+                        const int g = g0 + 64 * u + lane;
+                        k[u] = row_of(r, g);
+                        w[u] = g < T ? x.col[r.A[k[u]] + g] : -1;
+                    }
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) f[u] = x.lv.get(max(w[u], 0));
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) y[u] = w[u] >= 0 && f[u] == cprev ? x.sg[w[u]] : 0;
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) mine[u] = w[u] >= 0 && f[u] == 0 && x.lv.take(w[u], cnext);
+                    append<PU>(x, w, mine, q1, cnt);
+#pragma unroll
+                    for (int u = 0; u < PU; ++u)
+                        if (y[u]) {
+                            const uint64_t old = atomicAdd((unsigned long long *)&r.acc[k[u]], (unsigned long long)y[u]);
+                            ovf |= old + y[u] < old;
+                        }
+                }
+                psync();
+                acc = r.acc[lane];
+                psync();
             }
+            for (uint64_t m = hubs; m; m &= m - 1) {
+                const int src = __ffsll((long long)m) - 1;
+                const int a0 = __builtin_amdgcn_readlane(j0, src), a1 = __builtin_amdgcn_readlane(j1, src);
+                uint64_t part = 0;
+                double fsum = 0.0;
+                for (int c = a0; c < a1; c += 64 * PU) {
+                    int w[PU];
+                    uint32_t f[PU];
+                    uint64_t y[PU];
+                    bool mine[PU];
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) w[u] = c + 64 * u + lane < a1 ? x.col[c + 64 * u + lane] : -1;
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) f[u] = x.lv.get(max(w[u], 0));
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) y[u] = w[u] >= 0 && f[u] == cprev ? x.sg[w[u]] : 0;
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) mine[u] = w[u] >= 0 && f[u] == 0 && x.lv.take(w[u], cnext);
+                    append<PU>(x, w, mine, q1, cnt);
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) {
+                        if (F64) {  // in CSR order
+                            for (uint64_t b = pbal(y[u] != 0); b; b &= b - 1)
+                                fsum += u2d(prl64(y[u], __ffsll((long long)b) - 1));
+                        } else {
+                            ovf |= __builtin_add_overflow(part, y[u], &part);
+                        }
+                    }
+                }
+                if (!F64) {
+#pragma unroll
+                    for (int o = 32; o > 0; o >>= 1)
+                        ovf |= __builtin_add_overflow(part, (uint64_t)__shfl_xor((unsigned long long)part, o, 64), &part);
+                }
+                if (lane == src) {
+                    acc = part;
+                    facc = fsum;
+                }
+            }
+            if (e < q1) {
+                if (l > 0) x.sg[v] = F64 ? d2u(facc) : acc;
+                if (x.drow) x.drow[v] = l;
+            }
+            if (!F64 && pbal(ovf || (limit && acc >= limit && l > 0)) && lane == 0) sh->ovf[l % 3] = 1;
         }
-        __syncthreads();
+        pbarrier();
+        const int tail = q1 + *cnt;
+        if (!F64 && sh->ovf[l % 3]) return -1;
+        if (tail == q1) break;
+        if (tid == 0) x.set_off(l + 2, tail);
+        q0 = q1;
+        q1 = tail;
+        l++;
+        const uint32_t c = cprev;  // l-1 <- l, l+1 <- l+2, whose code is the old l-1's
+        cprev = 6 - cprev - cnext;
+        cnext = c;
     }
-    return lvl;
+    return l;
 }
 
-__device__ __forceinline__ double sigd(const uint64_t *sg, int v, bool f64) {
-    uint64_t x = ald(&sg[v]);
-    return f64 ? u2d(x) : (double)x;
-}
-
-// Successor-method dependency, FP64, levels maxlvl-1 .. 1; adds ws*delta to bc.
-__device__ void plain_backward(const CompDev &c, int maxlvl, const int32_t *d, const uint64_t *sg,
-                               double *dl, const int32_t *S, const int32_t *off, bool f64,
-                               double ws, double *bc) {
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    for (int i = off[maxlvl] + tid; i < off[maxlvl + 1]; i += PB) dl[S[i]] = 0.0;
-    __syncthreads();
-    for (int l = maxlvl - 1; l >= 1; --l) {
-        const int a = off[l], b = off[l + 1];
-        for (int i = a + tid; i < b; i += PB) {
-            int w = S[i];
-            int j0 = c.rp[w], j1 = c.rp[w + 1];
-            if (j1 - j0 > HUB) continue;
-            double sw = sigd(sg, w, f64), acc = 0.0;
-            for (int j = j0; j < j1; ++j) {
-                int v = c.col[j];
-                if (ald(&d[v]) == l + 1)
-                    acc += sw / sigd(sg, v, f64) * ((double)c.reach[v] + 1.0 + dl[v]);
+// Successor-method dependency, FP64, levels maxlvl .. 1; adds ws*delta to bc
+// (and stores delta in probe, when given).
+template <bool F64, bool LG>
+__device__ __forceinline__ void plain_backward(const PlainCtx<LG> &x, int maxlvl, double ws, double *bc,
+                                               double *probe) {
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wv = tid >> 6;
+    for (int l = maxlvl; l >= 1; --l) {
+        const int q0 = x.level_off(l), q1 = x.level_off(l + 1);
+        const uint32_t csucc = 1 + (uint32_t)((l + 1) % 3);
+        for (int base = q0 + wv * 64; base < q1; base += nt) {
+            const int e = base + lane;
+            int v = 0, j0 = 0, j1 = 0, rv = 0;
+            uint64_t sx = 0;
+            if (e < q1) {
+                v = x.S[e];
+                j0 = x.rp[v];
+                j1 = x.rp[v + 1];
+                rv = x.reach[v];
+                sx = x.sg[v];
             }
-            dl[w] = acc;
-            if (acc != 0.0) unsafeAtomicAdd(&bc[w], ws * acc);
+            double rho = 0.0;
+            if (l < maxlvl) {
+                const int d = j1 - j0;
+                const uint64_t hubs = pbal(d > HUB);
+                const int je = d > HUB ? j0 : j1;
+                if (!pbal(d > SHORT)) {
+                    for (int j = j0; pbal(j < je); j += PU) {
+                        int w[PU];
+                        double t[PU];
+#pragma unroll
+                        for (int u = 0; u < PU; ++u) w[u] = j + u < je ? x.col[j + u] : -1;
+#pragma unroll
+                        for (int u = 0; u < PU; ++u)
+                            t[u] = w[u] >= 0 && x.lv.get(max(w[u], 0)) == csucc ? x.tt[w[u]] : 0.0;
+#pragma unroll
+                        for (int u = 0; u < PU; ++u) rho += t[u];
+                    }
+                } else {
+                    WaveRows &r = *x.wr;
+                    double *acc = (double *)r.acc;
+                    const int T = flat_rows(r, j0, je - j0);
+                    for (int g0 = 0; g0 < T; g0 += 64 * PU) {
+                        int w[PU], k[PU];
+                        double t[PU];
+#pragma unroll
+                        for (int u = 0; u < PU; ++u) {
+                            const int g = g0 + 64 * u + lane;
+                            k[u] = row_of(r, g);
+                            w[u] = g < T ? x.col[r.A[k[u]] + g] : -1;
+                        }
+#pragma unroll
+                        for (int u = 0; u < PU; ++u)
+                            t[u] = w[u] >= 0 && x.lv.get(max(w[u], 0)) == csucc ? x.tt[w[u]] : 0.0;
+#pragma unroll
+                        for (int u = 0; u < PU; ++u)
+                            if (t[u] != 0.0) unsafeAtomicAdd(&acc[k[u]], t[u]);
+                    }
+                    psync();
+                    rho = acc[lane];
+                    psync();
+                }
+                for (uint64_t m = hubs; m; m &= m - 1) {
+                    const int src = __ffsll((long long)m) - 1;
+                    const int a0 = __builtin_amdgcn_readlane(j0, src), a1 = __builtin_amdgcn_readlane(j1, src);
+                    double part = 0.0;
+                    for (int c = a0; c < a1; c += 64 * PU) {
+                        int w[PU];
+                        double t[PU];
+#pragma unroll
+                        for (int u = 0; u < PU; ++u) w[u] = c + 64 * u + lane < a1 ? x.col[c + 64 * u + lane] : -1;
+#pragma unroll
+                        for (int u = 0; u < PU; ++u)
+                            t[u] = w[u] >= 0 && x.lv.get(max(w[u], 0)) == csucc ? x.tt[w[u]] : 0.0;
+#pragma unroll
+                        for (int u = 0; u < PU; ++u) part += t[u];
+                    }
+                    part = wave_sum(part);
+                    if (lane == src) rho = part;
+                }
+            }
+            if (e < q1) {
+                const double sv = F64 ? u2d(sx) : (double)sx;
+                const double delta = sv * rho;
+                x.tt[v] = ((double)rv + 1.0) / sv + rho;
+                if (delta != 0.0) unsafeAtomicAdd(&bc[v], ws * delta);
+                if (probe) probe[v] = delta;
+            }
         }
-        for (int i = a + wave; i < b; i += PW) {
-            int w = S[i];
-            int j0 = c.rp[w], j1 = c.rp[w + 1];
-            if (j1 - j0 <= HUB) continue;
-            double sw = sigd(sg, w, f64), acc = 0.0;
-            for (int j = j0 + lane; j < j1; j += 64) {
-                int v = c.col[j];
-                if (ald(&d[v]) == l + 1)
-                    acc += sw / sigd(sg, v, f64) * ((double)c.reach[v] + 1.0 + dl[v]);
-            }
-            acc = wave_sum(acc);
-            if (lane == 0) {
-                dl[w] = acc;
-                if (acc != 0.0) unsafeAtomicAdd(&bc[w], ws * acc);
-            }
-        }
-        __syncthreads();
+        pbarrier();
     }
 }
 
-__global__ __launch_bounds__(PB) void k_plain_bfs(CompDev c, PlainArgs a, PlainScratch sc, Rows rows) {
-    __shared__ FwdShared sh;
-    __shared__ int s_item, s_stop;
+// LDS of a workgroup past its static part: the waves' rows, then the codes
+template <bool LG>
+__device__ __forceinline__ void carve(PlainCtx<LG> &x, unsigned char *lds, const CompDev &c, uint32_t *lv_rows) {
+    x.wr = (WaveRows *)lds + (threadIdx.x >> 6);
+    x.lv.w = LG ? lv_rows : (uint32_t *)((WaveRows *)lds + (blockDim.x >> 6));
+    x.rp = glb(c.rp);
+    x.col = glb(c.col);
+    x.reach = glb(c.reach);
+    x.n = c.n;
+}
+
+}  // namespace
+
+template <bool F64, bool LG>
+__global__ __launch_bounds__(64 * PMAXW) void k_plain_bfs(CompDev c, PlainArgs a, PlainScratch sc, Rows rows) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ PlainShared sh;
     const int tid = threadIdx.x;
     const int64_t base = (int64_t)blockIdx.x * sc.stride;
-    const bool f64 = a.sigma_f64 != 0;
-    if (tid == 0) sh.ovf = 0;
+    PlainCtx<LG> x;
+    // (a kept row holds its levels itself, so the workgroup's d row is free)
+    carve<LG>(x, lds, c, (uint32_t *)(sc.d + base));
+    x.S = sc.S + base;
+    x.off = sc.off + base;
+    x.sh = &sh;
     while (true) {
         if (tid == 0) {
-            s_item = atomicAdd(&a.counters[0], 1);
-            s_stop = (!f64 && ald(&a.counters[1]) != 0) ? 1 : 0;
+            sh.item = atomicAdd(&a.counters[0], 1);
+            sh.stop = (!F64 && ald(&a.counters[1]) != 0) ? 1 : 0;
         }
-        __syncthreads();
-        const int item = s_item;
-        if (item >= a.count || s_stop) break;
+        pbarrier();
+        const int item = sh.item;
+        if (item >= a.count || sh.stop) break;
         const int s = a.src[item];
         const int slot = a.aux[item];
         const int mode = a.mode[item];
-        int32_t *d = (mode & MODE_ROW) ? rows.d + (int64_t)slot * rows.stride : sc.d + base;
-        uint64_t *sg = (mode & MODE_ROW) ? rows.sig + (int64_t)slot * rows.stride : sc.sig + base;
-        int32_t *S = sc.S + base, *off = sc.off + base;
-        int maxlvl = plain_forward(c, s, d, sg, S, off, f64, a.limit, &sh);
-        if (tid == 0 && sh.ovf) {
-            atomicExch(&a.counters[1], 1);
+        const bool row = mode & MODE_ROW;
+        x.sg = row ? rows.sig + (int64_t)slot * rows.stride : sc.sig + base;
+        x.tt = row ? sc.dl + base : (double *)x.sg;
+        x.drow = row ? rows.d + (int64_t)slot * rows.stride : nullptr;
+        const int maxlvl = plain_forward<F64, LG>(x, s, a.limit);
+        if (!F64 && maxlvl < 0) {
+            if (tid == 0) atomicExch(&a.counters[1], 1);
+            break;
         }
-        __syncthreads();
-        const int ovf = sh.ovf;
-        if (ovf) break;
         if (tid == 0) atomicMax(&a.counters[2], maxlvl);
         if (mode & MODE_BC)
-            plain_backward(c, maxlvl, d, sg, sc.dl + base, S, off, f64, (double)c.reach[s] + 1.0, a.bc);
-        __syncthreads();
+            plain_backward<F64, LG>(x, maxlvl, (double)c.reach[s] + 1.0, a.bc, a.probe);
+        pbarrier();
     }
 }
 
-__global__ __launch_bounds__(PB) void k_plain_chain(CompDev c, ChainDev ch, PlainArgs a,
-                                                    PlainScratch sc, Rows rows) {
-    __shared__ int s_item, s_max;
-    __shared__ int hist[LDS_LEVELS];
-    const int tid = threadIdx.x, lane = tid & 63;
+template <bool F64, bool LG>
+__global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev ch, PlainArgs a, PlainScratch sc,
+                                                            Rows rows) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ PlainShared sh;
+    __shared__ int hist[LDS_LEVELS + 2];
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63;
     const int64_t base = (int64_t)blockIdx.x * sc.stride;
-    const bool f64 = a.sigma_f64 != 0;
-    int32_t *d = sc.d + base, *S = sc.S + base, *off = sc.off + base;
+    int32_t *d = sc.d + base, *off = sc.off + base;
     uint64_t *sg = sc.sig + base;
+    PlainCtx<LG> x;
+    carve<LG>(x, lds, c, (uint32_t *)(sc.dl + base));
+    x.S = sc.S + base;
+    x.off = off;
+    x.sh = &sh;
+    x.sg = sg;
+    x.tt = a.probe ? a.probe + c.n : (double *)sg;
+    x.drow = nullptr;
     while (true) {
         if (tid == 0) {
-            s_item = atomicAdd(&a.counters[0], 1);
-            s_max = 0;
+            sh.item = atomicAdd(&a.counters[0], 1);
+            sh.top = 0;
         }
-        __syncthreads();
-        const int item = s_item;
+        pbarrier();
+        const int item = sh.item;
         if (item >= a.count) break;
         const int ci = a.src[item], pos = a.aux[item];
         const int p0 = ch.ptr[ci], cnt = ch.ptr[ci + 1] - p0;
-        const int x = ch.nodes[p0 + pos];
+        const int s = ch.nodes[p0 + pos];
         const int ld = pos + 1, rd = cnt - pos;
         const int32_t *dL = rows.d + (int64_t)a.slots[2 * item] * rows.stride;
         const int32_t *dR = rows.d + (int64_t)a.slots[2 * item + 1] * rows.stride;
@@ -224,93 +500,149 @@ __global__ __launch_bounds__(PB) void k_plain_chain(CompDev c, ChainDev ch, Plai
         const uint64_t *sR = rows.sig + (int64_t)a.slots[2 * item + 1] * rows.stride;
         // combine (Codes/postprocesses.cu:329-351)
         int mymax = 0;
-        for (int k = tid; k < c.n; k += PB) {
-            int la = dL[k] + ld, lb = dR[k] + rd;
+        for (int k = tid; k < c.n; k += nt) {
+            const int la = dL[k] + ld, lb = dR[k] + rd;
             int lv;
             uint64_t sv;
             if (la < lb) { lv = la; sv = sL[k]; }
             else if (la > lb) { lv = lb; sv = sR[k]; }
-            else { lv = lb; sv = f64 ? d2u(u2d(sL[k]) + u2d(sR[k])) : sL[k] + sR[k]; }
-            ast(&d[k], lv);
-            ast(&sg[k], sv);
+            else { lv = lb; sv = F64 ? d2u(u2d(sL[k]) + u2d(sR[k])) : sL[k] + sR[k]; }
+            d[k] = lv;
+            sg[k] = sv;
             mymax = max(mymax, lv);
         }
         mymax = wave_max(mymax);
-        if (lane == 0) atomicMax(&s_max, mymax);
-        __syncthreads();
+        if (lane == 0) atomicMax(&sh.top, mymax);
+        for (int k = tid; k < (c.n + 15) / 16; k += nt) x.lv.w[k] = 0;
+        pbarrier();
         // own chain: direct distances (Codes/postprocesses.cu:205-274, 354-360)
-        for (int j = tid; j < cnt; j += PB) {
-            int y = ch.nodes[p0 + j];
+        for (int j = tid; j < cnt; j += nt) {
+            const int y = ch.nodes[p0 + j];
             if (j == pos) {
-                ast(&d[y], 0);
-                ast(&sg[y], sig_one(f64));
+                d[y] = 0;
+                sg[y] = sig_one(F64);
                 continue;
             }
-            int dist = j > pos ? j - pos : pos - j;
-            int dy = ald(&d[y]);
-            if (dy > dist) {
-                ast(&d[y], dist);
-                ast(&sg[y], sig_one(f64));
-            } else if (dy == dist) {
-                uint64_t sy = ald(&sg[y]);
-                ast(&sg[y], f64 ? d2u(u2d(sy) + 1.0) : sy + 1);
+            const int dist = j > pos ? j - pos : pos - j;
+            if (d[y] > dist) {
+                d[y] = dist;
+                sg[y] = sig_one(F64);
+            } else if (d[y] == dist) {
+                sg[y] = F64 ? d2u(u2d(sg[y]) + 1.0) : sg[y] + 1;
             }
         }
         // final levels are BFS distances (< n); the combine maximum can be
         // larger on the source's own chain before the walk above fixes it
-        const int maxl = min(s_max, c.n - 1);
-        const bool lds = maxl + 2 <= LDS_LEVELS;
-        int *h = lds ? hist : off;  // off doubles as the histogram when deep
-        for (int l = tid; l < maxl + 2; l += PB) h[l] = 0;
-        __syncthreads();
-        for (int k = tid; k < c.n; k += PB) atomicAdd(&h[ald(&d[k]) + 1], 1);
-        __syncthreads();
+        const int maxl = min(sh.top, c.n - 1);
+        const bool in_lds = maxl + 2 <= LDS_LEVELS;
+        int *h = in_lds ? hist : off;  // off doubles as the histogram when deep
+        for (int l = tid; l < maxl + 2; l += nt) h[l] = 0;
+        pbarrier();
+        // level codes and histogram; the lanes of a wave that share a level add
+        // once (most of a small-world component sits on a few levels)
+        for (int k0 = 0; k0 < c.n; k0 += nt) {
+            const int k = k0 + tid;
+            const int l = k < c.n ? d[k] : -1;
+            if (l >= 0) x.lv.take(k, 1 + (uint32_t)(l % 3));
+            for (uint64_t m = pbal(l >= 0); m;) {
+                const int src = __ffsll((long long)m) - 1;
+                const int l0 = __builtin_amdgcn_readlane(l, src);
+                const uint64_t same = pbal(l == l0);
+                if (lane == src) atomicAdd(&h[l0 + 1], __popcll(same));
+                m &= ~same;
+            }
+        }
+        pbarrier();
         if (tid == 0) {
             int run = 0;
             for (int l = 0; l < maxl + 2; ++l) {
-                run += h[l];
-                h[l] = run;        // h[l] = start of level l (exclusive prefix over l+1 bins)
-                off[l] = run;
+                run += in_lds ? h[l] : ald(&h[l]);
+                // start of level l (exclusive prefix over l+1 bins); the
+                // cursors of a deep source overwrite off, which the sorted
+                // list then gives back
+                if (in_lds) {
+                    h[l] = run;
+                    x.set_off(l, run);
+                } else {
+                    ast(&h[l], run);
+                }
             }
         }
-        __syncthreads();
+        pbarrier();
         // h[l] now = number of vertices with level < l; use as cursors
-        for (int k = tid; k < c.n; k += PB) {
-            int l = ald(&d[k]);
-            int p = atomicAdd(&h[l], 1);
-            S[p] = k;
-        }
-        __syncthreads();
-        if (!lds) {
-            // off was consumed as cursors; rebuild it from the sorted levels
-            if (tid == 0) off[0] = 0;
-            for (int i = tid; i < c.n; i += PB) {
-                int li = ald(&d[S[i]]);
-                int lp = i ? ald(&d[S[i - 1]]) : -1;
-                for (int l = lp + 1; l <= li; ++l) off[l] = i;
-                if (i == c.n - 1)
-                    for (int l = li + 1; l <= maxl + 1; ++l) off[l] = c.n;
+        for (int k0 = 0; k0 < c.n; k0 += nt) {
+            const int k = k0 + tid;
+            const int l = k < c.n ? d[k] : -1;
+            for (uint64_t m = pbal(l >= 0); m;) {
+                const int src = __ffsll((long long)m) - 1;
+                const int l0 = __builtin_amdgcn_readlane(l, src);
+                const uint64_t same = pbal(l == l0);
+                int at = 0;
+                if (lane == src) at = atomicAdd(&h[l0], __popcll(same));
+                at = __builtin_amdgcn_readlane(at, src);
+                if (l == l0) x.S[prank(same, at)] = k;
+                m &= ~same;
             }
-            __syncthreads();
+        }
+        pbarrier();
+        if (!in_lds) {
+            // every level's offset again from the sorted levels (the first
+            // LDS_LEVELS of them in LDS)
+            if (tid == 0) x.set_off(0, 0);
+            for (int i = tid; i < c.n; i += nt) {
+                const int li = d[x.S[i]];
+                const int lp = i ? d[x.S[i - 1]] : -1;
+                for (int l = lp + 1; l <= li; ++l) x.set_off(l, i);
+                if (i == c.n - 1)
+                    for (int l = li + 1; l <= maxl + 1; ++l) x.set_off(l, c.n);
+            }
+            pbarrier();
         }
         // the deepest non-empty level
         int top = maxl;
-        while (top > 0 && off[top] == off[top + 1]) --top;
+        while (top > 0 && x.level_off(top) == x.level_off(top + 1)) --top;
         if (tid == 0) atomicMax(&a.counters[2], top);
-        plain_backward(c, top, d, sg, sc.dl + base, S, off, f64, (double)c.reach[x] + 1.0, a.bc);
-        __syncthreads();
+        plain_backward<F64, LG>(x, top, (double)c.reach[s] + 1.0, a.bc, a.probe);
+        pbarrier();
     }
 }
 
-hipError_t launch_plain_bfs(const CompDev &c, const PlainArgs &a, const PlainScratch &sc,
-                            const Rows &rows, int grid, hipStream_t st) {
-    hipLaunchKernelGGL(k_plain_bfs, dim3(grid), dim3(PB), 0, st, c, a, sc, rows);
+// Waves per source by the component's size: a barrier per level against the
+// vertices a level gives the waves.  4 / 8 / 16 waves (us; k sources): grid of
+// 3.7k vertices, k 2049: 1370 / 1485 / 2654; grid of 18.6k, k 2049: 5150 / 5100 /
+// 7540; power-law core of 21k, k 2000: 6837 / 5351 / 6150, of 84k, k 1000: 26150 /
+// 21440 / 18950, of 335k, k 600: 82052 / 56163 / 46738; R-MAT core of 86k, k 1000:
+// 31553 / 30536 / 25703; grid of 74k, k 2049: 15381 / 14186 / 14663.  One or two
+// 16-wave workgroups per compute unit run the same.
+PlainShape plain_shape(int32_t n) {
+    PlainShape p;
+    p.waves = n <= 8192 ? 4 : (n <= 49152 ? 8 : 16);
+    p.lds_codes = n <= LV_LDS_N;
+    const int64_t codes = p.lds_codes ? 4 * (((int64_t)n + 15) / 16) : 0;
+    p.lds = (int)(codes + p.waves * (int64_t)sizeof(WaveRows));
+    const int64_t fit = 160 * 1024 / (p.lds + (int64_t)sizeof(PlainShared) + 4 * (LDS_LEVELS + 2) + 512);
+    p.per_cu = (int)std::max<int64_t>(1, std::min<int64_t>(fit, 24 / p.waves));
+    return p;
+}
+
+hipError_t launch_plain_bfs(const CompDev &c, const PlainArgs &a, const PlainScratch &sc, const Rows &rows,
+                            const PlainShape &p, int grid, hipStream_t st) {
+    const dim3 g(grid), b(64 * p.waves);
+    if (p.lds_codes && a.sigma_f64) hipLaunchKernelGGL((k_plain_bfs<true, false>), g, b, p.lds, st, c, a, sc, rows);
+    else if (p.lds_codes) hipLaunchKernelGGL((k_plain_bfs<false, false>), g, b, p.lds, st, c, a, sc, rows);
+    else if (a.sigma_f64) hipLaunchKernelGGL((k_plain_bfs<true, true>), g, b, p.lds, st, c, a, sc, rows);
+    else hipLaunchKernelGGL((k_plain_bfs<false, true>), g, b, p.lds, st, c, a, sc, rows);
     return hipGetLastError();
 }
 
-hipError_t launch_plain_chain(const CompDev &c, const ChainDev &ch, const PlainArgs &a,
-                              const PlainScratch &sc, const Rows &rows, int grid, hipStream_t st) {
-    hipLaunchKernelGGL(k_plain_chain, dim3(grid), dim3(PB), 0, st, c, ch, a, sc, rows);
+hipError_t launch_plain_chain(const CompDev &c, const ChainDev &ch, const PlainArgs &a, const PlainScratch &sc,
+                              const Rows &rows, const PlainShape &p, int grid, hipStream_t st) {
+    const dim3 g(grid), b(64 * p.waves);
+    if (p.lds_codes && a.sigma_f64)
+        hipLaunchKernelGGL((k_plain_chain<true, false>), g, b, p.lds, st, c, ch, a, sc, rows);
+    else if (p.lds_codes) hipLaunchKernelGGL((k_plain_chain<false, false>), g, b, p.lds, st, c, ch, a, sc, rows);
+    else if (a.sigma_f64) hipLaunchKernelGGL((k_plain_chain<true, true>), g, b, p.lds, st, c, ch, a, sc, rows);
+    else hipLaunchKernelGGL((k_plain_chain<false, true>), g, b, p.lds, st, c, ch, a, sc, rows);
     return hipGetLastError();
 }
 

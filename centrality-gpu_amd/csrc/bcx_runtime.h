@@ -117,7 +117,6 @@ struct bcx_ctx {
     hipStream_t side = nullptr;  // batched: persistent passes beside the multi-launch tiles
     std::string err;
     bool overflow = false;
-    int plain_wg_per_cu = 2;
     bcx::Timer timer, timer_chain;
     bcx::DBuf counters, bc_acc, plain_scratch, rows_buf;
     bcx::DBuf w_src, w_aux, w_mode, w_slots;

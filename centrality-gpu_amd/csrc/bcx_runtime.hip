@@ -269,19 +269,31 @@ int bcx::make_plan(const HostComp &hc, const int32_t *subset, int64_t n_sub, boo
 // plain path
 // ------------------------------------------------------------------------
 
-static int grid_for(bcx_ctx *ctx, int64_t count) {
-    int64_t g = (int64_t)ctx->n_cu * ctx->plain_wg_per_cu;
-    if (count < g) g = count;
-    return (int)std::max<int64_t>(g, 1);
-}
-
 static int64_t plain_stride(int32_t n) { return ((int64_t)n + 2 + 63) & ~(int64_t)63; }
 constexpr size_t PLAIN_WORD_BYTES = 4 + 8 + 8 + 4 + 4;  // d, sig, dl, S, off
 
-// Whether the context's cap leaves room for the rows of `count` sources.
+// Device memory for the workgroups' rows: what they hold now plus what the cap leaves.
+static size_t plain_room(bcx_ctx *ctx) {
+    const size_t others = ctx->mem_used - ctx->plain_scratch.bytes;
+    return std::max(ctx->plain_scratch.bytes, ctx->mem_cap > others ? ctx->mem_cap - others : 0);
+}
+
+// Fewest workgroups a run of `count` sources takes: with less memory than
+// their rows it is refused.
+static int64_t plain_min_grid(bcx_ctx *ctx, int64_t count) {
+    return std::max<int64_t>(1, std::min<int64_t>(count, 2 * (int64_t)ctx->n_cu));
+}
+
 static bool plain_scratch_fits(bcx_ctx *ctx, int32_t n, int64_t count) {
-    const size_t need = (size_t)plain_stride(n) * PLAIN_WORD_BYTES * (size_t)grid_for(ctx, count);
-    return need <= ctx->plain_scratch.bytes || ctx->mem_used - ctx->plain_scratch.bytes + need <= ctx->mem_cap;
+    return (size_t)plain_stride(n) * PLAIN_WORD_BYTES * (size_t)plain_min_grid(ctx, count) <= plain_room(ctx);
+}
+
+// Workgroups of a launch: what the compute units hold, within the sources and
+// half of the device memory that is left.
+static int plain_grid(bcx_ctx *ctx, int32_t n, int64_t count, const PlainShape &p) {
+    const int64_t fit = (int64_t)(plain_room(ctx) / 2 / ((size_t)plain_stride(n) * PLAIN_WORD_BYTES));
+    const int64_t g = std::min<int64_t>({count, (int64_t)ctx->n_cu * p.per_cu, fit});
+    return (int)std::max(g, plain_min_grid(ctx, count));
 }
 
 static int ensure_plain_scratch(bcx_ctx *ctx, int32_t n, int grid, PlainScratch &sc) {
@@ -320,7 +332,8 @@ int64_t row_capacity(bcx_ctx *ctx, int32_t n, const bcx_opts *o) {
 
 static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t> &src,
                         const std::vector<int32_t> &slot, const std::vector<int8_t> &mode,
-                        bool f64, uint64_t limit, double *bc, const Rows &rows, bcx_stats *st) {
+                        bool f64, uint64_t limit, double *bc, const Rows &rows, bcx_stats *st,
+                        double *probe = nullptr) {
     if (src.empty()) return BCX_OK;
     int rc;
     if ((rc = upload(ctx, src.data(), src.size() * 4, ctx->w_src, "work list"))) return rc;
@@ -328,7 +341,8 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
     if ((rc = upload(ctx, mode.data(), mode.size(), ctx->w_mode, "work list"))) return rc;
     rc = ctx_hip(ctx, hipMemsetAsync(ctx->counters.p, 0, 4 * sizeof(int32_t), ctx->stream), "memset");
     if (rc) return rc;
-    const int grid = grid_for(ctx, (int64_t)src.size());
+    const PlainShape shape = plain_shape(dc.n);
+    const int grid = plain_grid(ctx, dc.n, (int64_t)src.size(), shape);
     PlainScratch sc;
     if ((rc = ensure_plain_scratch(ctx, dc.n, grid, sc))) return rc;
     PlainArgs a{};
@@ -340,8 +354,9 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
     a.limit = limit;
     a.counters = (int32_t *)ctx->counters.p;
     a.bc = bc;
+    a.probe = probe;
     ctx->timer.begin(ctx);
-    hipError_t e = launch_plain_bfs(dc.dev, a, sc, rows, grid, ctx->stream);
+    hipError_t e = launch_plain_bfs(dc.dev, a, sc, rows, shape, grid, ctx->stream);
     ctx->timer.end(ctx);
     if (st) st->n_launches++;
     rc = ctx_hip(ctx, e, "k_plain_bfs launch");
@@ -362,7 +377,7 @@ int read_counters(bcx_ctx *ctx, bcx_stats *st) {
 }
 
 static int run_chain_list(bcx_ctx *ctx, const DComp &dc, const PlanBatch &b, bool f64, double *bc,
-                          const Rows &rows, bcx_stats *st) {
+                          const Rows &rows, bcx_stats *st, double *probe = nullptr) {
     if (b.cci.empty()) return BCX_OK;
     int rc;
     if ((rc = upload(ctx, b.cci.data(), b.cci.size() * 4, ctx->w_src, "chain list"))) return rc;
@@ -370,7 +385,8 @@ static int run_chain_list(bcx_ctx *ctx, const DComp &dc, const PlanBatch &b, boo
     if ((rc = upload(ctx, b.cslots.data(), b.cslots.size() * 4, ctx->w_slots, "chain list"))) return rc;
     rc = ctx_hip(ctx, hipMemsetAsync(ctx->counters.p, 0, 4 * sizeof(int32_t), ctx->stream), "memset");
     if (rc) return rc;
-    const int grid = grid_for(ctx, (int64_t)b.cci.size());
+    const PlainShape shape = plain_shape(dc.n);
+    const int grid = plain_grid(ctx, dc.n, (int64_t)b.cci.size(), shape);
     PlainScratch sc;
     if ((rc = ensure_plain_scratch(ctx, dc.n, grid, sc))) return rc;
     PlainArgs a{};
@@ -381,8 +397,9 @@ static int run_chain_list(bcx_ctx *ctx, const DComp &dc, const PlanBatch &b, boo
     a.sigma_f64 = f64;
     a.counters = (int32_t *)ctx->counters.p;
     a.bc = bc;
+    a.probe = probe;
     ctx->timer_chain.begin(ctx);
-    hipError_t e = launch_plain_chain(dc.dev, dc.chains, a, sc, rows, grid, ctx->stream);
+    hipError_t e = launch_plain_chain(dc.dev, dc.chains, a, sc, rows, shape, grid, ctx->stream);
     ctx->timer_chain.end(ctx);
     if (st) st->n_launches++;
     rc = ctx_hip(ctx, e, "k_plain_chain launch");
@@ -874,19 +891,21 @@ int bcx_debug_source(bcx_ctx *ctx, const bcx_component *comp, int32_t src, const
             for (int32_t j = dc.host.ch_ptr[c]; j < dc.host.ch_ptr[c + 1]; ++j)
                 if (dc.host.ch_nodes[j] == src) { ci = c; pos = j - dc.host.ch_ptr[c]; break; }
     rc = ctx->bc_acc.ensure(ctx, sizeof(double) * n, "bc accumulator");
+    DBuf probe;
+    if (!rc) rc = probe.ensure(ctx, 2 * sizeof(double) * (size_t)n, "probe delta");
     for (int attempt = 0; attempt < 2 && !rc; ++attempt) {
         ctx->overflow = false;
         Rows rows{};
         if ((rc = ensure_rows(ctx, n, 2, rows))) break;
         PlainScratch sc;
-        double *bc = (double *)ctx->bc_acc.p;
+        double *bc = (double *)ctx->bc_acc.p, *pd = (double *)probe.p;
+        if ((rc = ctx_hip(ctx, hipMemsetAsync(pd, 0, sizeof(double) * (size_t)n, ctx->stream), "memset"))) break;
         if (ci < 0) {
             std::vector<int32_t> s{src}, sl{0};
             std::vector<int8_t> m{(int8_t)(MODE_BC | MODE_ROW)};
-            rc = run_bfs_list(ctx, dc, s, sl, m, f64, limit, bc, rows, nullptr);
+            rc = run_bfs_list(ctx, dc, s, sl, m, f64, limit, bc, rows, nullptr, pd);
             if (rc) break;
             if (ctx->overflow && !f64) { f64 = true; continue; }
-            if ((rc = ensure_plain_scratch(ctx, n, 1, sc))) break;
             rc = ctx_hip(ctx, hipMemcpyAsync(lv.data(), rows.d, 4 * n, hipMemcpyDeviceToHost, ctx->stream), "copy");
             if (!rc) rc = ctx_hip(ctx, hipMemcpyAsync(sg.data(), rows.sig, 8 * n, hipMemcpyDeviceToHost, ctx->stream), "copy");
         } else {
@@ -899,19 +918,20 @@ int bcx_debug_source(bcx_ctx *ctx, const bcx_component *comp, int32_t src, const
             b.cci = {ci};
             b.cpos = {pos};
             b.cslots = {0, 1};
-            rc = run_chain_list(ctx, dc, b, f64, bc, rows, nullptr);
+            rc = run_chain_list(ctx, dc, b, f64, bc, rows, nullptr, pd);
             if (rc) break;
             // the chain launch ran one workgroup: its rows start at offset 0
             if ((rc = ensure_plain_scratch(ctx, n, 1, sc))) break;
             rc = ctx_hip(ctx, hipMemcpyAsync(lv.data(), sc.d, 4 * n, hipMemcpyDeviceToHost, ctx->stream), "copy");
             if (!rc) rc = ctx_hip(ctx, hipMemcpyAsync(sg.data(), sc.sig, 8 * n, hipMemcpyDeviceToHost, ctx->stream), "copy");
         }
-        if (!rc) rc = ctx_hip(ctx, hipMemcpyAsync(dl.data(), sc.dl, 8 * n, hipMemcpyDeviceToHost, ctx->stream), "copy");
+        if (!rc) rc = ctx_hip(ctx, hipMemcpyAsync(dl.data(), pd, 8 * n, hipMemcpyDeviceToHost, ctx->stream), "copy");
         if (!rc) rc = ctx_hip(ctx, hipStreamSynchronize(ctx->stream), "copy");
         break;
     }
     (void)ctx->timer.collect();
     (void)ctx->timer_chain.collect();
+    probe.release(ctx);
     bcx_dgraph_free(ctx, g);
     if (rc) return rc;
     dl[src] = 0.0;
