@@ -15,6 +15,7 @@
 // event; the host never waits on a single tile.
 #include <algorithm>
 #include <array>
+#include <cmath>
 #include <cstring>
 #include <thread>
 #include <vector>
@@ -1780,22 +1781,28 @@ int batched_kind(DComp &dc, int flags) {
 
 // ------------------------------------------------------------------------
 // Schedule tuner.  A component of at least TUNE_N vertices is run once on
-// sample tiles (evenly spaced over its tile order, BC into a scratch
+// sample sources (evenly spaced over its tile order, BC into a scratch
 // accumulator, timed with HIP events, outside the run's timing) under each
-// candidate schedule, and the fastest is cached for every later run:
-//  * kernel, for components the workgroup kernel can take (<= WG_N vertices):
-//    the workgroup kernel over min(tiles, CUs) sample tiles (its concurrent
-//    width) against the multi-launch tiles over TUNE_TILES;
+// candidate schedule, and what was measured is cached for every later run:
+//  * kernel: the multi-launch tiles over TUNE_TILES tiles, the per-source
+//    kernel over TUNE_SOURCES sources and, for components it can take (<= WG_N
+//    vertices), the workgroup kernel over min(tiles, CUs) tiles (its
+//    concurrent width).  A run takes the kernel with the least estimated time
+//    for its number of sources: a sample of sources that leaves most CUs
+//    without a workgroup tile still fills the chip source by source (2000
+//    sources of an 84k power-law core: 158 ms on the workgroup kernel, 26 ms
+//    per source; 2049 of an 18.6k grid: 65 ms against 5 ms);
 //  * multi-launch: 8 / 4 / 16 level-kernel blocks per CU, 8 / 4 tiles in
-//    flight, chain contraction on / off.
-// Each candidate runs twice (the first run captures its graphs) and is timed
-// on the second; a candidate replaces the default only when its rate
-// (sources per second) is at least 3% higher.  Options that fix a choice are
-// kept.  (The reference picks its schedule from sampled BFS depths and
-// frontier sizes, Codes/kernels_free.cu:447-470, 288, 381.)
+//    flight, chain contraction on / off, once a run takes them.
+// Each tiled candidate runs twice (the first run captures its graphs) and is
+// timed on the second; a multi-launch candidate replaces the default only when
+// its rate (sources per second) is at least 3% higher.  Options that fix a
+// choice are kept.  (The reference picks its schedule from sampled BFS depths
+// and frontier sizes, Codes/kernels_free.cu:447-470, 288, 381.)
 // ------------------------------------------------------------------------
 constexpr int32_t TUNE_N = 16384;
 constexpr int TUNE_TILES = 24;
+constexpr int64_t TUNE_SOURCES = 1024;
 
 // Sources of k tiles of `width` evenly spaced over the component's tile order.
 static std::vector<int32_t> sample_tiles(DComp &dc, int64_t k, int64_t width) {
@@ -1811,13 +1818,36 @@ static std::vector<int32_t> sample_tiles(DComp &dc, int64_t k, int64_t width) {
     return out;
 }
 
-int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, bcx_stats *st) {
+// The kernel with the least estimated time for n_src sources, from the rates
+// measured on the samples.
+static int measured_kind(bcx_ctx *ctx, const DComp &dc, int64_t n_src) {
+    const double cus = std::max(1, ctx->n_cu), s = (double)n_src;
+    int kind = BCX_KERNEL_MULTI;
+    // (one tile alone runs at 0.7 of the rate of eight)
+    double best = dc.rate_multi > 0 ? s / dc.rate_multi * (n_src < 8 * BATCH_W * MAX_SPL ? 1.4 : 1.0) : 1e30;
+    if (dc.rate_wg > 0) {
+        const double t = std::ceil(std::ceil(s / BATCH_W) / cus) * dc.round_wg / dc.rate_wg;
+        if (t < best) {
+            best = t;
+            kind = BCX_KERNEL_WG;
+        }
+    }
+    if (dc.rate_src > 0 && std::max(s, cus) / dc.rate_src < best) kind = KIND_SOURCE;
+    return kind;
+}
+
+int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, int64_t n_src, bcx_stats *st) {
     const int kind0 = batched_kind(dc, o->flags);
     if (kind0 == BCX_KERNEL_SMALL) return kind0;
-    if ((o->flags & BCX_FLAG_NO_TUNE) || dc.n < TUNE_N) return kind0;
-    const bool kind_fixed = (o->flags & (BCX_FLAG_NO_WG_KERNEL | BCX_FLAG_WG_KERNEL)) || dc.n > WG_N;
-    int kind = kind_fixed ? kind0 : dc.sched_kind;
-    const bool need_kind = kind < 0;
+    const bool kind_fixed = (o->flags & (BCX_FLAG_NO_WG_KERNEL | BCX_FLAG_WG_KERNEL)) != 0;
+    // (the rows of the per-source kernel have to fit beside the tiles' buffers)
+    const bool source_fits = plain_scratch_fits(ctx, dc.n, n_src);
+    if ((o->flags & BCX_FLAG_NO_TUNE) || dc.n < TUNE_N)
+        return kind0 == BCX_KERNEL_WG && !kind_fixed && source_fits && !valid_spl(o->sources_per_lane) ? KIND_SOURCE
+                                                                                                       : kind0;
+    const bool need_kind = !kind_fixed && !dc.kind_measured;
+    int kind = kind_fixed ? kind0 : (dc.kind_measured ? measured_kind(ctx, dc, n_src) : -1);
+    if (kind == KIND_SOURCE && !source_fits) kind = kind0;
     const bool need_multi = !dc.sched_multi && (need_kind || kind == BCX_KERNEL_MULTI);
     if (!need_kind && !need_multi) return kind;
     // the run's timer is set aside: the samples are timed on their own
@@ -1861,9 +1891,23 @@ int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, bcx_stats *st) 
     double r_multi = 0.0;
     if (!rc) rc = time_multi(samp, base, &r_multi);
     if (!rc && need_kind) {
-        double r_wg = 0.0;
-        rc = time_wg(sample_tiles(dc, std::max(1, ctx->n_cu), (int64_t)BATCH_W * wg_spl(o)), &r_wg);
-        kind = r_wg >= r_multi ? BCX_KERNEL_WG : BCX_KERNEL_MULTI;
+        dc.rate_multi = r_multi;
+        if (dc.n <= WG_N) {
+            const std::vector<int32_t> ws = sample_tiles(dc, std::max(1, ctx->n_cu), (int64_t)BATCH_W * wg_spl(o));
+            rc = time_wg(ws, &dc.rate_wg);
+            dc.round_wg = (double)ws.size();
+        }
+        if (!rc && source_fits && !valid_spl(o->sources_per_lane)) {
+            std::vector<int32_t> order = batched_order(dc), ss;
+            const int64_t k = std::min<int64_t>(dc.n <= WG_N ? TUNE_SOURCES : TUNE_SOURCES / 4, dc.n);
+            for (int64_t i = 0; i < k; ++i) ss.push_back(order[(size_t)(i * dc.n / k)]);
+            bool overflow = false;
+            rc = source_component(ctx, dc, ss, &to, bc + dc.offset, nullptr, &overflow);
+            const double t = ctx->timer.collect();
+            dc.rate_src = t > 0 && !overflow ? (double)k / t : 0.0;
+        }
+        dc.kind_measured = !rc;
+        kind = measured_kind(ctx, dc, n_src);
     }
     MultiSched best = base;
     const bool tune_multi = need_multi && kind == BCX_KERNEL_MULTI;
@@ -1890,7 +1934,6 @@ int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, bcx_stats *st) 
     keep.destroy();
     scratch.release(ctx);
     if (rc) return rc;
-    if (need_kind) dc.sched_kind = (int8_t)kind;
     if (tune_multi) {
         // (a choice the options fixed is not cached: later runs may leave it free)
         dc.sched_multi = true;

@@ -43,7 +43,9 @@ struct PlainArgs {
     const int8_t *mode;    // bfs only: MODE_* bits
     const int32_t *slots;  // chain only: [2*count] row slots of L and R
     int32_t count;
+    int32_t split;         // bfs: copies of the BC accumulator (bc holds split * n words)
     int32_t sigma_f64;     // 1: FP64 sigma by pull
+    int32_t fp32;          // bfs: compensated FP32 terms (with integer sigma; no MODE_ROW)
     uint64_t limit;        // u64 overflow threshold (0 = 2^64)
     int32_t *counters;
     double *bc;            // component slice of the BC accumulator
@@ -56,10 +58,11 @@ struct PlainShape {
     int waves, per_cu, lds;
     bool lds_codes;
 };
-PlainShape plain_shape(int32_t n);
+PlainShape plain_shape(int32_t n, bool fp32);
 
 hipError_t launch_plain_bfs(const CompDev &c, const PlainArgs &a, const PlainScratch &sc,
                             const Rows &rows, const PlainShape &p, int grid, hipStream_t st);
+hipError_t launch_plain_fold(double *bc, const double *copies, int n, int split, hipStream_t st);
 hipError_t launch_plain_chain(const CompDev &c, const ChainDev &ch, const PlainArgs &a,
                               const PlainScratch &sc, const Rows &rows, const PlainShape &p, int grid, hipStream_t st);
 

@@ -55,6 +55,32 @@ struct WaveRows {
     int P[64], A[64];
     uint64_t acc[64];
 };
+// with compensated FP32 terms, also a step's terms in arc order and the number
+// of them before each arc
+struct WaveTerms {
+    float t[64 * 4];
+    uint16_t before[64 * 4 + 4];  // (the waves' parts stay 8-byte aligned)
+};
+template <typename TT>
+__host__ __device__ constexpr int wave_lds() {
+    return (int)(sizeof(WaveRows) + (sizeof(TT) == 4 ? sizeof(WaveTerms) : 0));
+}
+
+struct KahanP {
+    float s = 0.f, c = 0.f;
+    __device__ __forceinline__ void add(float x) {
+        const float y = x - c;
+        const float t = s + y;
+        c = (t - s) - y;
+        s = t;
+    }
+    __device__ __forceinline__ double value() const { return (double)s - (double)c; }
+};
+struct SumP {
+    double s = 0.0;
+    __device__ __forceinline__ void add(double x) { s += x; }
+    __device__ __forceinline__ double value() const { return s; }
+};
 
 struct PlainShared {
     int cnt[3];  // vertices appended at a level, by level mod 3
@@ -101,18 +127,19 @@ struct Codes {
 };
 
 // What a workgroup works on: its source's arrays.
-template <bool LG>
+template <bool LG, typename TT>
 struct PlainCtx {
     const gint *rp, *col, *reach;
     int n;
     Codes<LG> lv;
     uint64_t *sg;   // path counts
-    double *tt;     // terms (the same words as sg, unless sg is kept)
+    TT *tt;         // terms (FP64: the same words as sg, unless sg is kept)
     int32_t *S;     // vertices in level order
     int32_t *off;   // level offsets past LDS_LEVELS
     int32_t *drow;  // levels, when the source's row is kept
     PlainShared *sh;
     WaveRows *wr;   // this wave's
+    WaveTerms *wt;
     __device__ __forceinline__ int level_off(int l) const { return l < LDS_LEVELS ? sh->off[l] : off[l]; }
     __device__ __forceinline__ void set_off(int l, int x) const {
         if (l < LDS_LEVELS) sh->off[l] = x;
@@ -147,8 +174,8 @@ __device__ __forceinline__ int flat_rows(WaveRows &r, int j0, int d) {
 }
 
 // Appends the vertices that the wave's lanes took to level l+1's list.
-template <int U, bool LG>
-__device__ __forceinline__ void append(const PlainCtx<LG> &x, const int (&w)[U], const bool (&mine)[U], int q1,
+template <int U, typename Ctx>
+__device__ __forceinline__ void append(const Ctx &x, const int (&w)[U], const bool (&mine)[U], int q1,
                                        int *cnt) {
     uint64_t b[U];
     int tot = 0;
@@ -169,11 +196,12 @@ __device__ __forceinline__ void append(const PlainCtx<LG> &x, const int (&w)[U],
 }
 
 constexpr int PU = 4;  // arcs of a lane in flight
+static_assert(sizeof(WaveTerms::t) == 4 * 64 * PU, "a step's terms");
 
 // Forward BFS from s.  Returns the deepest level, -1 when a uint64 count
 // overflowed.
-template <bool F64, bool LG>
-__device__ __forceinline__ int plain_forward(const PlainCtx<LG> &x, int s, uint64_t limit) {
+template <bool F64, typename Ctx>
+__device__ __forceinline__ int plain_forward(const Ctx &x, int s, uint64_t limit) {
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wv = tid >> 6;
     PlainShared *sh = x.sh;
     for (int k = tid; k < (x.n + 15) / 16; k += nt) x.lv.w[k] = 0;
@@ -320,11 +348,14 @@ __device__ __forceinline__ int plain_forward(const PlainCtx<LG> &x, int s, uint6
     return l;
 }
 
-// Successor-method dependency, FP64, levels maxlvl .. 1; adds ws*delta to bc
-// (and stores delta in probe, when given).
-template <bool F64, bool LG>
-__device__ __forceinline__ void plain_backward(const PlainCtx<LG> &x, int maxlvl, double ws, double *bc,
+// Successor-method dependency, levels maxlvl .. 1; adds ws*delta to bc (and
+// stores delta in probe, when given).  FP64 terms are summed in any order;
+// compensated FP32 terms in CSR order, as every kernel of that precision does.
+template <bool F64, bool LG, typename TT>
+__device__ __forceinline__ void plain_backward(const PlainCtx<LG, TT> &x, int maxlvl, double ws, double *bc,
                                                double *probe) {
+    constexpr bool ORD = sizeof(TT) == 4;
+    using Acc = typename std::conditional<ORD, KahanP, SumP>::type;
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wv = tid >> 6;
     for (int l = maxlvl; l >= 1; --l) {
         const int q0 = x.level_off(l), q1 = x.level_off(l + 1);
@@ -340,7 +371,7 @@ __device__ __forceinline__ void plain_backward(const PlainCtx<LG> &x, int maxlvl
                 rv = x.reach[v];
                 sx = x.sg[v];
             }
-            double rho = 0.0;
+            Acc rho;
             if (l < maxlvl) {
                 const int d = j1 - j0;
                 const uint64_t hubs = pbal(d > HUB);
@@ -348,22 +379,25 @@ __device__ __forceinline__ void plain_backward(const PlainCtx<LG> &x, int maxlvl
                 if (!pbal(d > SHORT)) {
                     for (int j = j0; pbal(j < je); j += PU) {
                         int w[PU];
-                        double t[PU];
+                        bool use[PU];
+                        TT t[PU];
 #pragma unroll
                         for (int u = 0; u < PU; ++u) w[u] = j + u < je ? x.col[j + u] : -1;
 #pragma unroll
-                        for (int u = 0; u < PU; ++u)
-                            t[u] = w[u] >= 0 && x.lv.get(max(w[u], 0)) == csucc ? x.tt[w[u]] : 0.0;
+                        for (int u = 0; u < PU; ++u) use[u] = w[u] >= 0 && x.lv.get(max(w[u], 0)) == csucc;
 #pragma unroll
-                        for (int u = 0; u < PU; ++u) rho += t[u];
+                        for (int u = 0; u < PU; ++u) t[u] = use[u] ? x.tt[w[u]] : (TT)0;
+#pragma unroll
+                        for (int u = 0; u < PU; ++u)
+                            if (use[u]) rho.add(t[u]);
                     }
                 } else {
                     WaveRows &r = *x.wr;
-                    double *acc = (double *)r.acc;
                     const int T = flat_rows(r, j0, je - j0);
                     for (int g0 = 0; g0 < T; g0 += 64 * PU) {
                         int w[PU], k[PU];
-                        double t[PU];
+                        bool use[PU];
+                        TT t[PU];
 #pragma unroll
                         for (int u = 0; u < PU; ++u) {
                             const int g = g0 + 64 * u + lane;
@@ -371,39 +405,80 @@ __device__ __forceinline__ void plain_backward(const PlainCtx<LG> &x, int maxlvl
                             w[u] = g < T ? x.col[r.A[k[u]] + g] : -1;
                         }
 #pragma unroll
-                        for (int u = 0; u < PU; ++u)
-                            t[u] = w[u] >= 0 && x.lv.get(max(w[u], 0)) == csucc ? x.tt[w[u]] : 0.0;
+                        for (int u = 0; u < PU; ++u) use[u] = w[u] >= 0 && x.lv.get(max(w[u], 0)) == csucc;
 #pragma unroll
-                        for (int u = 0; u < PU; ++u)
-                            if (t[u] != 0.0) unsafeAtomicAdd(&acc[k[u]], t[u]);
+                        for (int u = 0; u < PU; ++u) t[u] = use[u] ? x.tt[w[u]] : (TT)0;
+                        if constexpr (ORD) {
+                            // the step's terms compacted in arc order, then
+                            // each lane adds its row's
+                            WaveTerms &q = *x.wt;
+                            int tot = 0;
+#pragma unroll
+                            for (int u = 0; u < PU; ++u) {
+                                const uint64_t b = pbal(use[u]);
+                                const int at = prank(b, tot);
+                                q.before[64 * u + lane] = (uint16_t)at;
+                                if (use[u]) q.t[at] = t[u];
+                                tot += __popcll(b);
+                            }
+                            if (lane == 0) q.before[64 * PU] = (uint16_t)tot;
+                            psync();
+                            const int p = r.P[lane], a0 = max(p - g0, 0), a1 = min(p + (je - j0) - g0, 64 * PU);
+                            int i = 0, ie = 0;
+                            if (a0 < a1) {
+                                i = q.before[a0];
+                                ie = q.before[a1];
+                            }
+                            for (; pbal(i < ie); ++i)
+                                if (i < ie) rho.add(q.t[i]);
+                            psync();
+                        } else {
+                            double *acc = (double *)r.acc;
+#pragma unroll
+                            for (int u = 0; u < PU; ++u)
+                                if (use[u]) unsafeAtomicAdd(&acc[k[u]], (double)t[u]);
+                        }
                     }
-                    psync();
-                    rho = acc[lane];
-                    psync();
+                    if constexpr (!ORD) {
+                        psync();
+                        rho.s = ((const double *)r.acc)[lane];
+                        psync();
+                    }
                 }
                 for (uint64_t m = hubs; m; m &= m - 1) {
                     const int src = __ffsll((long long)m) - 1;
                     const int a0 = __builtin_amdgcn_readlane(j0, src), a1 = __builtin_amdgcn_readlane(j1, src);
-                    double part = 0.0;
+                    Acc part;
                     for (int c = a0; c < a1; c += 64 * PU) {
                         int w[PU];
-                        double t[PU];
+                        bool use[PU];
+                        TT t[PU];
 #pragma unroll
                         for (int u = 0; u < PU; ++u) w[u] = c + 64 * u + lane < a1 ? x.col[c + 64 * u + lane] : -1;
 #pragma unroll
-                        for (int u = 0; u < PU; ++u)
-                            t[u] = w[u] >= 0 && x.lv.get(max(w[u], 0)) == csucc ? x.tt[w[u]] : 0.0;
+                        for (int u = 0; u < PU; ++u) use[u] = w[u] >= 0 && x.lv.get(max(w[u], 0)) == csucc;
 #pragma unroll
-                        for (int u = 0; u < PU; ++u) part += t[u];
+                        for (int u = 0; u < PU; ++u) t[u] = use[u] ? x.tt[w[u]] : (TT)0;
+#pragma unroll
+                        for (int u = 0; u < PU; ++u) {
+                            if constexpr (ORD) {
+                                for (uint64_t b = pbal(use[u]); b; b &= b - 1)
+                                    part.add(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(t[u]),
+                                                                                      __ffsll((long long)b) - 1)));
+                            } else {
+                                part.add((double)t[u]);
+                            }
+                        }
                     }
-                    part = wave_sum(part);
+                    if constexpr (!ORD) part.s = wave_sum(part.s);
                     if (lane == src) rho = part;
                 }
             }
             if (e < q1) {
                 const double sv = F64 ? u2d(sx) : (double)sx;
-                const double delta = sv * rho;
-                x.tt[v] = ((double)rv + 1.0) / sv + rho;
+                const double sum = rho.value();
+                const double delta = sv * sum;
+                x.tt[v] = (TT)(((double)rv + 1.0) / sv + sum);
                 if (delta != 0.0) unsafeAtomicAdd(&bc[v], ws * delta);
                 if (probe) probe[v] = delta;
             }
@@ -413,10 +488,11 @@ __device__ __forceinline__ void plain_backward(const PlainCtx<LG> &x, int maxlvl
 }
 
 // LDS of a workgroup past its static part: the waves' rows, then the codes
-template <bool LG>
-__device__ __forceinline__ void carve(PlainCtx<LG> &x, unsigned char *lds, const CompDev &c, uint32_t *lv_rows) {
-    x.wr = (WaveRows *)lds + (threadIdx.x >> 6);
-    x.lv.w = LG ? lv_rows : (uint32_t *)((WaveRows *)lds + (blockDim.x >> 6));
+template <bool LG, typename TT>
+__device__ __forceinline__ void carve(PlainCtx<LG, TT> &x, unsigned char *lds, const CompDev &c, uint32_t *lv_rows) {
+    x.wr = (WaveRows *)(lds + (threadIdx.x >> 6) * wave_lds<TT>());
+    x.wt = (WaveTerms *)(x.wr + 1);
+    x.lv.w = LG ? lv_rows : (uint32_t *)(lds + (blockDim.x >> 6) * wave_lds<TT>());
     x.rp = glb(c.rp);
     x.col = glb(c.col);
     x.reach = glb(c.reach);
@@ -425,18 +501,19 @@ __device__ __forceinline__ void carve(PlainCtx<LG> &x, unsigned char *lds, const
 
 }  // namespace
 
-template <bool F64, bool LG>
+template <bool F64, bool LG, typename TT>
 __global__ __launch_bounds__(64 * PMAXW) void k_plain_bfs(CompDev c, PlainArgs a, PlainScratch sc, Rows rows) {
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ PlainShared sh;
     const int tid = threadIdx.x;
     const int64_t base = (int64_t)blockIdx.x * sc.stride;
-    PlainCtx<LG> x;
+    PlainCtx<LG, TT> x;
     // (a kept row holds its levels itself, so the workgroup's d row is free)
-    carve<LG>(x, lds, c, (uint32_t *)(sc.d + base));
+    carve<LG, TT>(x, lds, c, (uint32_t *)(sc.d + base));
     x.S = sc.S + base;
     x.off = sc.off + base;
     x.sh = &sh;
+    double *bc = a.bc + (int64_t)(blockIdx.x % (unsigned)a.split) * c.n;
     while (true) {
         if (tid == 0) {
             sh.item = atomicAdd(&a.counters[0], 1);
@@ -444,22 +521,23 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_bfs(CompDev c, PlainArgs a
         }
         pbarrier();
         const int item = sh.item;
-        if (item >= a.count || sh.stop) break;
+        if (sh.stop) return;  // (the component is redone)
+        if (item >= a.count) break;
         const int s = a.src[item];
         const int slot = a.aux[item];
         const int mode = a.mode[item];
         const bool row = mode & MODE_ROW;
         x.sg = row ? rows.sig + (int64_t)slot * rows.stride : sc.sig + base;
-        x.tt = row ? sc.dl + base : (double *)x.sg;
+        x.tt = row || sizeof(TT) == 4 ? (TT *)(sc.dl + base) : (TT *)x.sg;
         x.drow = row ? rows.d + (int64_t)slot * rows.stride : nullptr;
-        const int maxlvl = plain_forward<F64, LG>(x, s, a.limit);
+        const int maxlvl = plain_forward<F64>(x, s, a.limit);
         if (!F64 && maxlvl < 0) {
             if (tid == 0) atomicExch(&a.counters[1], 1);
-            break;
+            return;
         }
         if (tid == 0) atomicMax(&a.counters[2], maxlvl);
         if (mode & MODE_BC)
-            plain_backward<F64, LG>(x, maxlvl, (double)c.reach[s] + 1.0, a.bc, a.probe);
+            plain_backward<F64>(x, maxlvl, (double)c.reach[s] + 1.0, bc, a.probe);
         pbarrier();
     }
 }
@@ -474,8 +552,8 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev 
     const int64_t base = (int64_t)blockIdx.x * sc.stride;
     int32_t *d = sc.d + base, *off = sc.off + base;
     uint64_t *sg = sc.sig + base;
-    PlainCtx<LG> x;
-    carve<LG>(x, lds, c, (uint32_t *)(sc.dl + base));
+    PlainCtx<LG, double> x;
+    carve<LG, double>(x, lds, c, (uint32_t *)(sc.dl + base));
     x.S = sc.S + base;
     x.off = off;
     x.sh = &sh;
@@ -602,7 +680,7 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev 
         int top = maxl;
         while (top > 0 && x.level_off(top) == x.level_off(top + 1)) --top;
         if (tid == 0) atomicMax(&a.counters[2], top);
-        plain_backward<F64, LG>(x, top, (double)c.reach[s] + 1.0, a.bc, a.probe);
+        plain_backward<F64>(x, top, (double)c.reach[s] + 1.0, a.bc, a.probe);
         pbarrier();
     }
 }
@@ -614,12 +692,12 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev 
 // 21440 / 18950, of 335k, k 600: 82052 / 56163 / 46738; R-MAT core of 86k, k 1000:
 // 31553 / 30536 / 25703; grid of 74k, k 2049: 15381 / 14186 / 14663.  One or two
 // 16-wave workgroups per compute unit run the same.
-PlainShape plain_shape(int32_t n) {
+PlainShape plain_shape(int32_t n, bool fp32) {
     PlainShape p;
     p.waves = n <= 8192 ? 4 : (n <= 49152 ? 8 : 16);
     p.lds_codes = n <= LV_LDS_N;
     const int64_t codes = p.lds_codes ? 4 * (((int64_t)n + 15) / 16) : 0;
-    p.lds = (int)(codes + p.waves * (int64_t)sizeof(WaveRows));
+    p.lds = (int)codes + p.waves * (fp32 ? wave_lds<float>() : wave_lds<double>());
     const int64_t fit = 160 * 1024 / (p.lds + (int64_t)sizeof(PlainShared) + 4 * (LDS_LEVELS + 2) + 512);
     p.per_cu = (int)std::max<int64_t>(1, std::min<int64_t>(fit, 24 / p.waves));
     return p;
@@ -628,10 +706,30 @@ PlainShape plain_shape(int32_t n) {
 hipError_t launch_plain_bfs(const CompDev &c, const PlainArgs &a, const PlainScratch &sc, const Rows &rows,
                             const PlainShape &p, int grid, hipStream_t st) {
     const dim3 g(grid), b(64 * p.waves);
-    if (p.lds_codes && a.sigma_f64) hipLaunchKernelGGL((k_plain_bfs<true, false>), g, b, p.lds, st, c, a, sc, rows);
-    else if (p.lds_codes) hipLaunchKernelGGL((k_plain_bfs<false, false>), g, b, p.lds, st, c, a, sc, rows);
-    else if (a.sigma_f64) hipLaunchKernelGGL((k_plain_bfs<true, true>), g, b, p.lds, st, c, a, sc, rows);
-    else hipLaunchKernelGGL((k_plain_bfs<false, true>), g, b, p.lds, st, c, a, sc, rows);
+    if (a.fp32 && !a.sigma_f64) {
+        if (p.lds_codes) hipLaunchKernelGGL((k_plain_bfs<false, false, float>), g, b, p.lds, st, c, a, sc, rows);
+        else hipLaunchKernelGGL((k_plain_bfs<false, true, float>), g, b, p.lds, st, c, a, sc, rows);
+    } else if (a.sigma_f64) {
+        if (p.lds_codes) hipLaunchKernelGGL((k_plain_bfs<true, false, double>), g, b, p.lds, st, c, a, sc, rows);
+        else hipLaunchKernelGGL((k_plain_bfs<true, true, double>), g, b, p.lds, st, c, a, sc, rows);
+    } else {
+        if (p.lds_codes) hipLaunchKernelGGL((k_plain_bfs<false, false, double>), g, b, p.lds, st, c, a, sc, rows);
+        else hipLaunchKernelGGL((k_plain_bfs<false, true, double>), g, b, p.lds, st, c, a, sc, rows);
+    }
+    return hipGetLastError();
+}
+
+// Adds the copies of a split BC accumulator to the component's slice.
+__global__ void k_plain_fold(double *bc, const double *copies, int n, int split) {
+    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= n) return;
+    double s = 0.0;
+    for (int k = 0; k < split; ++k) s += copies[(int64_t)k * n + v];
+    bc[v] += s;
+}
+
+hipError_t launch_plain_fold(double *bc, const double *copies, int n, int split, hipStream_t st) {
+    hipLaunchKernelGGL(k_plain_fold, dim3((n + 255) / 256), dim3(256), 0, st, bc, copies, n, split);
     return hipGetLastError();
 }
 

@@ -73,10 +73,12 @@ struct DComp {
     // cut_state -1 not yet tried, 0 the component has too few such chains)
     ChainCut *cut = nullptr;
     int8_t cut_state = -1;
-    // batched path: the schedule measured on sample tiles, cached for every
-    // later run of the component (sched_kind -1: kernel not measured;
+    // batched path: the schedule measured on sample sources, cached for every
+    // later run of the component (sources per second on each kernel, 0: not a
+    // candidate; round_wg: sources of a full round of workgroup tiles;
     // sched_multi: the multi-launch fields below were measured)
-    int8_t sched_kind = -1;
+    bool kind_measured = false;
+    double rate_multi = 0.0, rate_wg = 0.0, rate_src = 0.0, round_wg = 0.0;
     bool sched_multi = false;
     int8_t sched_cut = 1;     // multi-launch: 1 contracted chains, 0 the relabelled copy
     int16_t sched_bpc = 0;    // multi-launch: level-kernel blocks per CU (0: default)
@@ -119,7 +121,7 @@ struct bcx_ctx {
     bool overflow = false;
     bcx::Timer timer, timer_chain;
     bcx::DBuf counters, bc_acc, plain_scratch, rows_buf;
-    bcx::DBuf w_src, w_aux, w_mode, w_slots;
+    bcx::DBuf w_src, w_aux, w_mode, w_slots, bc_split;
     bcx::DBuf bc_pack, bc_chunks;  // result download: packed slices and their chunk list
     double *bc_pin = nullptr;      // pinned host staging of the result download
     size_t bc_pin_bytes = 0;
@@ -128,7 +130,7 @@ struct bcx_ctx {
     SmallState *wgk = nullptr;  // workgroup-per-tile kernel buffers
     SmallState *srck = nullptr;  // wave-per-source kernel buffers
     std::vector<bcx::DBuf *> all_bufs() {
-        return {&counters, &bc_acc, &plain_scratch, &rows_buf, &w_src, &w_aux, &w_mode, &w_slots, &bc_pack, &bc_chunks};
+        return {&counters, &bc_acc, &plain_scratch, &rows_buf, &w_src, &w_aux, &w_mode, &w_slots, &bc_split, &bc_pack, &bc_chunks};
     }
 };
 
@@ -190,8 +192,18 @@ int batched_kind(bcx::DComp &dc, int flags);
 // The kernel and, for the multi-launch tiles, the schedule of a component of
 // the batched path: measured once on sample tiles for components of at least
 // TUNE_N vertices (unless the options fix it), else batched_kind's rule.
-// Returns a BCX_KERNEL_* or a negative BCX_E_* status.
-int batched_schedule(bcx_ctx *ctx, bcx::DComp &dc, const bcx_opts *o, bcx_stats *st);
+// Returns a BCX_KERNEL_*, KIND_SOURCE (the per-source kernel of the plain path,
+// sources one by one) or a negative BCX_E_* status.
+constexpr int KIND_SOURCE = 4;
+int batched_schedule(bcx_ctx *ctx, bcx::DComp &dc, const bcx_opts *o, int64_t n_src, bcx_stats *st);
+// The sources srcs of a component on the per-source kernel in the run's
+// precision.  *overflow: a uint64 count overflowed with FP32 terms; bc is as
+// before and the component is left to the tiled kernels, which turn to FP64
+// terms tile by tile.
+int source_component(bcx_ctx *ctx, bcx::DComp &dc, const std::vector<int32_t> &srcs, const bcx_opts *o, double *bc,
+                     bcx_stats *st, bool *overflow);
+// Whether the context's cap leaves room for the per-source kernel's rows.
+bool plain_scratch_fits(bcx_ctx *ctx, int32_t n, int64_t count);
 // Blocks per CU, tiles in flight and sources per lane a multi-launch run of
 // dc uses.
 void batched_sched_report(const bcx::DComp &dc, const bcx_opts *o, int32_t *bpc, int32_t *slots, int32_t *spl);

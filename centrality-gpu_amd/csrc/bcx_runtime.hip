@@ -284,7 +284,7 @@ static int64_t plain_min_grid(bcx_ctx *ctx, int64_t count) {
     return std::max<int64_t>(1, std::min<int64_t>(count, 2 * (int64_t)ctx->n_cu));
 }
 
-static bool plain_scratch_fits(bcx_ctx *ctx, int32_t n, int64_t count) {
+bool plain_scratch_fits(bcx_ctx *ctx, int32_t n, int64_t count) {
     return (size_t)plain_stride(n) * PLAIN_WORD_BYTES * (size_t)plain_min_grid(ctx, count) <= plain_room(ctx);
 }
 
@@ -333,7 +333,7 @@ int64_t row_capacity(bcx_ctx *ctx, int32_t n, const bcx_opts *o) {
 static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t> &src,
                         const std::vector<int32_t> &slot, const std::vector<int8_t> &mode,
                         bool f64, uint64_t limit, double *bc, const Rows &rows, bcx_stats *st,
-                        double *probe = nullptr) {
+                        double *probe = nullptr, bool fp32 = false) {
     if (src.empty()) return BCX_OK;
     int rc;
     if ((rc = upload(ctx, src.data(), src.size() * 4, ctx->w_src, "work list"))) return rc;
@@ -341,7 +341,7 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
     if ((rc = upload(ctx, mode.data(), mode.size(), ctx->w_mode, "work list"))) return rc;
     rc = ctx_hip(ctx, hipMemsetAsync(ctx->counters.p, 0, 4 * sizeof(int32_t), ctx->stream), "memset");
     if (rc) return rc;
-    const PlainShape shape = plain_shape(dc.n);
+    const PlainShape shape = plain_shape(dc.n, fp32);
     const int grid = plain_grid(ctx, dc.n, (int64_t)src.size(), shape);
     PlainScratch sc;
     if ((rc = ensure_plain_scratch(ctx, dc.n, grid, sc))) return rc;
@@ -355,10 +355,27 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
     a.counters = (int32_t *)ctx->counters.p;
     a.bc = bc;
     a.probe = probe;
+    a.fp32 = fp32;
+    // Thousands of sources add into SPLIT copies of the accumulator, folded
+    // afterwards: a vertex's sum is then SPLIT times shorter, and its rounding
+    // error what the tiled kernels' is, which add a tile's sources first (16384
+    // sources of a 26k grid, error against 64 bits 1.5e-15 on tiles, 5.7e-15
+    // with one accumulator).  Accumulators of the workgroups' own, without
+    // atomics, ran 20-30% slower (8000 sources of that grid 13.6 -> 16.0 ms).
+    constexpr int SPLIT = 16;
+    constexpr size_t SPLIT_SOURCES = 4096;
+    const size_t split_bytes = sizeof(double) * SPLIT * (size_t)dc.n;
+    a.split = 1;
+    if (src.size() >= SPLIT_SOURCES && ctx->bc_split.ensure(ctx, split_bytes, "split accumulator") == BCX_OK) {
+        a.split = SPLIT;
+        a.bc = (double *)ctx->bc_split.p;
+        if ((rc = ctx_hip(ctx, hipMemsetAsync(a.bc, 0, split_bytes, ctx->stream), "memset"))) return rc;
+    }
     ctx->timer.begin(ctx);
     hipError_t e = launch_plain_bfs(dc.dev, a, sc, rows, shape, grid, ctx->stream);
+    if (e == hipSuccess && a.split > 1) e = launch_plain_fold(bc, a.bc, dc.n, a.split, ctx->stream);
     ctx->timer.end(ctx);
-    if (st) st->n_launches++;
+    if (st) st->n_launches += a.split > 1 ? 2 : 1;
     rc = ctx_hip(ctx, e, "k_plain_bfs launch");
     if (rc) return rc;
     return read_counters(ctx, st);
@@ -385,7 +402,7 @@ static int run_chain_list(bcx_ctx *ctx, const DComp &dc, const PlanBatch &b, boo
     if ((rc = upload(ctx, b.cslots.data(), b.cslots.size() * 4, ctx->w_slots, "chain list"))) return rc;
     rc = ctx_hip(ctx, hipMemsetAsync(ctx->counters.p, 0, 4 * sizeof(int32_t), ctx->stream), "memset");
     if (rc) return rc;
-    const PlainShape shape = plain_shape(dc.n);
+    const PlainShape shape = plain_shape(dc.n, false);
     const int grid = plain_grid(ctx, dc.n, (int64_t)b.cci.size(), shape);
     PlainScratch sc;
     if ((rc = ensure_plain_scratch(ctx, dc.n, grid, sc))) return rc;
@@ -441,6 +458,32 @@ int plain_component(bcx_ctx *ctx, const DComp &dc, const Plan &plan, const bcx_o
     if (st) st->n_f64_sigma += plan.n_bfs + plan.n_chain;
     ctx->overflow = false;
     return plain_component_mode(ctx, dc, plan, true, 0, bc, st);
+}
+
+int source_component(bcx_ctx *ctx, DComp &dc, const std::vector<int32_t> &srcs, const bcx_opts *o, double *bc,
+                     bcx_stats *st, bool *overflow) {
+    const uint64_t limit = (o->sigma_f64_threshold_log2 > 0 && o->sigma_f64_threshold_log2 < 64)
+                               ? (1ull << o->sigma_f64_threshold_log2) : 0;
+    const bool fp32 = o->precision == BCX_PREC_FP32C;
+    const std::vector<int32_t> slots(srcs.size(), -1);
+    const std::vector<int8_t> modes(srcs.size(), MODE_BC);
+    const Rows rows{};
+    *overflow = false;
+    int rc;
+    // components whose counts from their highest-degree vertex pass 2^62 start
+    // with FP64 counts, as on the workgroup kernel
+    if (dc.sigma_est <= 4.6e18) {
+        ctx->overflow = false;
+        if ((rc = run_bfs_list(ctx, dc, srcs, slots, modes, false, limit, bc, rows, st, nullptr, fp32))) return rc;
+        if (!ctx->overflow) return BCX_OK;
+        rc = ctx_hip(ctx, hipMemsetAsync(bc, 0, sizeof(double) * (size_t)dc.n, ctx->stream), "memset");
+        if (rc || fp32) {
+            *overflow = true;
+            return rc;
+        }
+    }
+    if (st) st->n_f64_sigma += (int64_t)srcs.size();
+    return run_bfs_list(ctx, dc, srcs, slots, modes, true, 0, bc, rows, st);
 }
 
 // ------------------------------------------------------------------------
@@ -721,6 +764,7 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
     std::vector<SmallJob> srck;   // small components for the wave-per-source kernel (both paths)
     std::vector<SmallJob> small;  // batched path: components for the one-launch small kernel
     std::vector<SmallJob> wg;     // batched path: deep components for the workgroup-per-tile kernel
+    std::vector<SmallJob> single;  // batched path: components whose sources run one by one
     std::vector<SmallJob> multi;  // batched path: components for the multi-launch tiles
     int32_t largest_multi = -1;
     for (size_t ci = 0; ci < g->comps.size(); ++ci) {
@@ -768,7 +812,7 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
         int64_t n_chain = 0;
         std::vector<int32_t> srcs = batched_sources(dc, sp, sn, o.use_chains ? &n_chain : nullptr);
         account((int64_t)srcs.size() - n_chain, n_chain);
-        const int kind = batched_schedule(ctx, dc, &o, s);  // (one-time sample runs stay outside the timing)
+        const int kind = batched_schedule(ctx, dc, &o, (int64_t)srcs.size(), s);  // (one-time sample runs stay outside the timing)
         if (kind < 0) return kind;
         if (kind == BCX_KERNEL_SMALL) {
             s->n_comp_small++;
@@ -778,9 +822,9 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
         // larger components: tile order from the tuner (BFS ranks or balls)
         std::vector<int32_t> tiles = tuned_sources(dc, srcs);
         if (dc.tile_order == 1) s->n_ball_tiles++;
-        if (kind == BCX_KERNEL_WG) {
+        if (kind == BCX_KERNEL_WG || kind == KIND_SOURCE) {
             s->n_comp_wg++;
-            wg.push_back({&dc, std::move(tiles)});
+            (kind == KIND_SOURCE ? single : wg).push_back({&dc, std::move(tiles)});
         } else {
             if ((rc = batched_prepare(ctx, dc, &o))) return rc;  // one-time work stays outside the timing
             s->n_comp_multi++;
@@ -791,11 +835,11 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
             multi.push_back({&dc, std::move(tiles)});
         }
     }
-    if (!srck.empty() || !small.empty() || !wg.empty() || !multi.empty()) {
+    if (!srck.empty() || !small.empty() || !wg.empty() || !single.empty() || !multi.empty()) {
         // the persistent passes (small components, deep components) run on a
         // side stream while the multi-launch tiles run on theirs; the run is
         // timed as one interval on the context stream around both
-        const bool overlap = !multi.empty() && (!srck.empty() || !small.empty() || !wg.empty());
+        const bool overlap = (!multi.empty() || !single.empty()) && (!srck.empty() || !small.empty() || !wg.empty());
         if (overlap && !ctx->side &&
             (rc = ctx_hip(ctx, hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking), "side stream")))
             return rc;
@@ -808,9 +852,28 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
         for (SmallJob &jb : multi)
             if ((rc = batched_component(ctx, *const_cast<DComp *>(jb.dc), jb.srcs, &o, bc + jb.dc->offset, s)))
                 return rc;
+        std::vector<SmallJob> again;  // FP32 terms, overflowed counts
+        for (SmallJob &jb : single) {
+            bool overflow = false;
+            if ((rc = source_component(ctx, *const_cast<DComp *>(jb.dc), jb.srcs, &o, bc + jb.dc->offset, s, &overflow)))
+                return rc;
+            if (overflow) again.push_back(std::move(jb));
+        }
         if ((rc = batched_persistent_finish(ctx, s, PASS_SRC)) || (rc = batched_persistent_finish(ctx, s, PASS_SMALL)) ||
             (rc = batched_persistent_finish(ctx, s, PASS_WG)))
             return rc;
+        for (SmallJob &jb : again) {
+            DComp &dc = *const_cast<DComp *>(jb.dc);
+            if (dc.n > WG_N) {
+                if ((rc = batched_prepare(ctx, dc, &o)) ||
+                    (rc = batched_component(ctx, dc, jb.srcs, &o, bc + dc.offset, s)))
+                    return rc;
+                continue;
+            }
+            if ((rc = batched_persistent_start(ctx, {jb}, &o, bc, s, PASS_WG, ctx->stream)) ||
+                (rc = batched_persistent_finish(ctx, s, PASS_WG)))
+                return rc;
+        }
         if (overlap) {
             hipEvent_t ev;
             if ((rc = ctx_hip(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming), "event"))) return rc;
