@@ -1628,13 +1628,14 @@ static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_
     }
     std::stable_sort(order.begin(), order.end(),
                      [](const SmallJob *x, const SmallJob *y) { return x->dc->arcs > y->dc->arcs; });
-    // as few sources per tile as leave four tiles per compute unit.  With FP32
+    // few sources per tile while that gives every compute unit a tile, four
+    // tiles per compute unit for larger jobs.  With FP32
     // terms a count overflow turns the 64 consecutive sources around it to FP64
     // terms, so smaller tiles are a first try: an overflow (rare in components
     // of this size) ends it and the pass is repeated in tiles of 64
     const bool fp32 = run_fp32(o);
-    const size_t per = n_src / (4 * (size_t)std::max(1, ctx->n_cu));
-    const size_t tw = probe || per > 32 ? BATCH_W : (per > 16 ? 32 : 16);
+    const size_t per = n_src / (size_t)std::max(1, ctx->n_cu);
+    const size_t tw = probe || per > 128 ? BATCH_W : (per > 64 ? 32 : (per > 8 ? 16 : (per > 4 ? 8 : 4)));
     PassTables tb;
     int rc = stage_tables(ctx, ss, order, bc_base, tw, tb);
     if (rc || (rc = ss.redo.ensure(ctx, 4 * tb.tiles.size(), "source redo list"))) return rc;

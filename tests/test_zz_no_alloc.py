@@ -120,3 +120,21 @@ def test_noalloc_rejects_what_it_cannot_hold(engine):
     got = noalloc(engine, small, None, bcx.PREC_FP64)
     mx, _, zeros = relerr(got, oracle.component_bc(small.row_ptr, small.col, small.reach))
     assert mx < 1e-9 and zeros
+
+
+@pytest.mark.parametrize("prec", [bcx.PREC_FP64, bcx.PREC_FP32C])
+@pytest.mark.parametrize("n,m,k", [(3, 0, 3), (1024, 3000, 1024), (1025, 3000, 1025), (2048, 4000, 2048),
+                                   (2048, 4000, 5), (2048, 30000, 130), (700, 60000, 700)])
+def test_noalloc_sizes(engine, n, m, k, prec):
+    """Where the call changes its tiles (1024 sources) or its kernel (arcs past
+    the LDS of the wave-per-source kernel), and the smallest and largest
+    component: against the oracle."""
+    rng = np.random.default_rng(n + m)
+    e = [(i, (i + 1) % n) for i in range(n)] + [tuple(map(int, p)) for p in rng.integers(0, n, (m, 2))]
+    e = sorted({(min(p), max(p)) for p in e if p[0] != p[1]})
+    c = bcx.Host.from_edges(n, e).decompose().components()[0]
+    assert c.n == n
+    srcs = None if k == n else np.sort(rng.choice(n, size=k, replace=False)).astype(np.int32)
+    ref = oracle.component_bc(c.row_ptr, c.col, c.reach, sources=srcs)
+    mx, _, zeros = relerr(noalloc(engine, c, srcs, prec), ref)
+    assert mx < (1e-9 if prec == bcx.PREC_FP64 else 1e-6) and zeros, (n, m, k, prec, mx)
