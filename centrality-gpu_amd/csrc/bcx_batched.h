@@ -39,6 +39,10 @@ struct BatchDev {
     const int32_t *hub_nsl;           // [n_hub] slices per hub
     const int32_t *sl_hub;            // [n_slice] hub of each slice
     const int32_t *sl_j0, *sl_j1;     // [n_slice] arc range of each slice
+    // vertices [0, n) in chunks of at most 64 vertices and about PULL_ARCS
+    // arcs (hubs aside), one wave each in the pull
+    int32_t n_chunk;
+    const int32_t *chunk;             // [n_chunk + 1] first vertex of each chunk
     uint64_t *hub_mask;               // [n_hub * hub_stride][W] sources of hub at level l
     double *hub_acc;                  // [n_hub * 64 * W] backward partial sums
     int32_t *hub_cnt;                 // [n_hub] slices finished this level

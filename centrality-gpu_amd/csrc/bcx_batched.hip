@@ -20,7 +20,7 @@
 //   expand  pushes source masks from Q_l to neighbours, F & ~vis[w], with
 //           fire-and-forget 64-bit atomic ORs into mb[(l+1)%3] (a lane walks
 //           the arcs of a low-degree entry, a wave those of a larger one);
-//   pull    scans mb[(l+1)%3] in coalesced 64-vertex chunks; every non-zero
+//   pull    scans mb[(l+1)%3] in chunks of bounded vertices and arcs; every non-zero
 //           entry w joins Q_{l+1} and gets sigma_w = sum of sigma_v over
 //           neighbours v in CSR order for the sources where v is at level l
 //           -- no sigma atomics, and the FP64 order is the oracle's, so FP64
@@ -405,8 +405,13 @@ __global__ __launch_bounds__(BB) void k_b_expand(BatchDev b, int l) {
             if (K - j == l + 1) push<W>(b, dst, b.ch_R[c], mbit<W>(h, lane));
         }
     }
-    for (int base = q0 + gwave() * 64; base < q1; base += nwaves() * 64) {
-        const int e = base + lane;
+    // lane k of group g takes entry g + k G of the level: the list follows the
+    // vertex ids, whose heavy rows lie together, and a wave walks its entries
+    // above SMALL arcs one after another (168k-vertex power-law core, a tile's
+    // three big levels: 248, 395, 217 us in runs of 64 entries, 209, 286, 68 so)
+    const int G = (q1 - q0 + 63) / 64;
+    for (int g = gwave(); g < G; g += nwaves()) {
+        const int e = q0 + g + lane * G;
         int j0 = 0, j1 = 0;
         Msk<W> F = mzero<W>();
         if (e < q1) {
@@ -563,9 +568,9 @@ __global__ __launch_bounds__(BB) void k_b_pull(BatchDev b, int l) {
         if (K - j == l + 1) mR[h] = b.ch_R[myc[h]];
     }
     int cnt = 0;  // wave-uniform
-    for (int base = gwave() * 64; base < b.n; base += nwaves() * 64) {
-        const int w0 = base + lane;
-        const Msk<W> N0 = w0 < b.n ? mld<W>(nx, w0) : mzero<W>();
+    for (int c = gwave(); c < b.n_chunk; c += nwaves()) {
+        const int w0 = b.chunk[c] + lane;
+        const Msk<W> N0 = w0 < b.chunk[c + 1] ? mld<W>(nx, w0) : mzero<W>();
         const uint64_t bal = __ballot(many<W>(N0));
         if (!bal) continue;
         const int k0 = cnt;
