@@ -9,6 +9,7 @@
 namespace bcx {
 
 constexpr int BATCH_W = 64;  // lanes of a wave64; a tile holds W * 64 sources
+constexpr int TERM_CHAINS = 8;  // chains per wave in the endpoints' chain terms
 constexpr int MAX_SPL = 4;   // largest W: sources per lane of the multi-launch tiles
 
 // A tile of the multi-launch kernels holds W * 64 sources (W = spl: 1, 2 or 4):
@@ -68,6 +69,11 @@ struct BatchDev {
     const int32_t *ep_off;            // [n_ep + 1] chains attached to endpoint e:
     const int32_t *ep_list;           //   ep_list[ep_off[e] ..) = 2c + (0: e is L, 1: R)
     int32_t n_ep;                     // endpoints (vertices with an attached chain)
+    // an endpoint's chains in slices of at most TERM_CHAINS, one wave each;
+    // endpoints of several slices are summed into zeroed rows
+    int32_t n_ts, n_tm;
+    const int32_t *ts_ep, *ts_q;      // [n_ts] endpoint and first list entry of a slice
+    const int32_t *tm_ep;             // [n_tm] endpoints of several slices
     int32_t *ep_lvl;                  // [n_ep * 64 * W] the tile's level of each endpoint per source
     double *ep_rho;                   // [n_ep * 64 * W] the chain terms of each endpoint's rho per
                                       // source (made after the forward, added by the backward)

@@ -277,6 +277,7 @@ __global__ __launch_bounds__(BB) void k_b_clear_vis(BatchDev b, int sm) {
         b.hub_acc[i] = 0.0;
     }
     for (int64_t i = t0; i < b.n_hub; i += stride) b.hub_cnt[i] = 0;
+    for (int64_t i = t0; i < (int64_t)b.n_tm * ROW; i += stride) b.ep_rho[(int64_t)b.tm_ep[i / ROW] * ROW + i % ROW] = 0.0;
 }
 
 // Sources that are tile vertices start at level 0.  A source that is the
@@ -1085,15 +1086,20 @@ __global__ __launch_bounds__(BB) void k_b_chain_check(BatchDev b) {
 // rho for every source, which depend on the endpoints' levels and counts
 // alone, into ep_rho; the backward adds them when it finishes an endpoint
 // (inlined there, the closed forms raised the backward's register peak by a
-// wave per SIMD).  One wave per endpoint.
+// wave per SIMD).  One wave per slice of an endpoint's chains: the loads of a
+// chain depend on each other, and a hub can end hundreds of chains (R-MAT core
+// of 165k vertices, one wave per endpoint: 600 us a tile, of which all but the
+// hubs' waves took 40).
 template <int SM, int W>
 __global__ __launch_bounds__(BB) void k_b_chain_terms(BatchDev b) {
     constexpr bool F64 = SM == SIG_F64;
     if (ldi(&b.ctr[3]) < 0 || (!F64 && b.ctr[1]) || b.ctr[2]) return;
     const int lane = threadIdx.x & 63;
     const int ns = b.ctr[5];
-    for (int e = gwave(); e < b.n_ep; e += nwaves()) {
-        const int q0 = b.ep_off[e], q1 = b.ep_off[e + 1];
+    for (int i = gwave(); i < b.n_ts; i += nwaves()) {
+        const int e = b.ts_ep[i], q0 = b.ts_q[i], p0 = b.ep_off[e], p1 = b.ep_off[e + 1];
+        const int q1 = min(q0 + TERM_CHAINS, p1);
+        const bool whole = p1 - p0 <= TERM_CHAINS;
         const int code0 = b.ep_list[q0];  // (an endpoint has a chain: its vertex is that chain's end)
         const int v = (code0 & 1) ? b.ch_R[code0 >> 1] : b.ch_L[code0 >> 1];
         // per source slot k + 64 h: the endpoint's level and count, the
@@ -1138,7 +1144,11 @@ __global__ __launch_bounds__(BB) void k_b_chain_terms(BatchDev b) {
         }
 #pragma unroll
         for (int h = 0; h < W; ++h)
-            if (h * 64 + lane < ns) b.ep_rho[((int64_t)e * 64 + lane) * W + h] = rho[h];
+            if (h * 64 + lane < ns) {
+                double *to = &b.ep_rho[((int64_t)e * 64 + lane) * W + h];
+                if (whole) *to = rho[h];
+                else if (rho[h] != 0.0) unsafeAtomicAdd(to, rho[h]);
+            }
     }
 }
 
@@ -1429,10 +1439,10 @@ static void chain_terms_w(const BatchDev &b, int sm, int g, hipStream_t st) {
     else hipLaunchKernelGGL((k_b_chain_terms<SIG_F64, W>), dim3(g), dim3(BB), 0, st, b);
 }
 
-// one wave per endpoint
+// one wave per slice of an endpoint's chains
 hipError_t launch_b_chain_terms(const BatchDev &b, int sm, int grid, hipStream_t st) {
     (void)grid;
-    const int g = (int)std::max<int64_t>(1, std::min<int64_t>(((int64_t)b.n_ep + NW - 1) / NW, 1 << 16));
+    const int g = (int)std::max<int64_t>(1, std::min<int64_t>(((int64_t)b.n_ts + NW - 1) / NW, 1 << 16));
     if (b.spl == 4) chain_terms_w<4>(b, sm, g, st);
     else if (b.spl == 2) chain_terms_w<2>(b, sm, g, st);
     else chain_terms_w<1>(b, sm, g, st);

@@ -936,12 +936,13 @@ constexpr int CUT_LM = 8;
 
 struct bcx::ChainCut {
     DComp g;                   // the copy: [0, n_core) the tile graph in BFS order, then the interiors
-    int32_t n_core = 0, n_chain = 0, n_ep = 0;
+    int32_t n_core = 0, n_chain = 0, n_ep = 0, n_ts = 0, n_tm = 0;
     std::vector<int32_t> inv;  // component id -> copy id
     DBuf b_perm;               // copy id -> component id
     DBuf b_tab;                // the chain tables, one allocation
     const int32_t *ch_L = nullptr, *ch_R = nullptr, *ch_off = nullptr, *ch_of = nullptr;
     const int32_t *ep_idx = nullptr, *ep_off = nullptr, *ep_list = nullptr;
+    const int32_t *ts_ep = nullptr, *ts_q = nullptr, *tm_ep = nullptr;
     const double *ch_pre = nullptr;
 };
 
@@ -1099,14 +1100,25 @@ static int chain_cut(bcx_ctx *ctx, DComp &dc, ChainCut *&out) {
         }
     }
     cut->n_ep = n_ep;
+    // the endpoints' chains in slices
+    std::vector<int32_t> tsep, tsq, tmep;
+    for (int32_t e = 0; e < n_ep; ++e) {
+        for (int32_t q = epoff[(size_t)e]; q < epoff[(size_t)e + 1]; q += TERM_CHAINS) {
+            tsep.push_back(e);
+            tsq.push_back(q);
+        }
+        if (epoff[(size_t)e + 1] - epoff[(size_t)e] > TERM_CHAINS) tmep.push_back(e);
+    }
+    cut->n_ts = (int32_t)tsep.size();
+    cut->n_tm = (int32_t)tmep.size();
     // one allocation: the prefix sums (8-byte aligned at the start), then the int tables
     const size_t ints = 2 * (size_t)npc + ((size_t)npc + 1) + (size_t)n_in + (size_t)n_core + ((size_t)n_ep + 1) +
-                        2 * (size_t)npc;
+                        2 * (size_t)npc + tsep.size() + tsq.size() + tmep.size();
     std::vector<unsigned char> tab(8 * (size_t)n_in + 4 * ints);
     std::memcpy(tab.data(), pre.data(), 8 * (size_t)n_in);
     size_t at = 8 * (size_t)n_in;
     std::vector<size_t> pos;
-    for (const std::vector<int32_t> *t : {&chL, &chR, &off, &chof, &epidx, &epoff, &eplist}) {
+    for (const std::vector<int32_t> *t : {&chL, &chR, &off, &chof, &epidx, &epoff, &eplist, &tsep, &tsq, &tmep}) {
         pos.push_back(at);
         std::memcpy(tab.data() + at, t->data(), 4 * t->size());
         at += 4 * t->size();
@@ -1131,6 +1143,9 @@ static int chain_cut(bcx_ctx *ctx, DComp &dc, ChainCut *&out) {
     cut->ep_idx = (const int32_t *)(base + pos[4]);
     cut->ep_off = (const int32_t *)(base + pos[5]);
     cut->ep_list = (const int32_t *)(base + pos[6]);
+    cut->ts_ep = (const int32_t *)(base + pos[7]);
+    cut->ts_q = (const int32_t *)(base + pos[8]);
+    cut->tm_ep = (const int32_t *)(base + pos[9]);
     DComp &g = cut->g;
     g.n = n;
     g.arcs = q.arcs;
@@ -1160,6 +1175,11 @@ static void set_chains(BatchDev &b, Slot &s, const ChainCut *cut) {
     b.ep_off = cut->ep_off;
     b.ep_list = cut->ep_list;
     b.n_ep = cut->n_ep;
+    b.n_ts = cut->n_ts;
+    b.n_tm = cut->n_tm;
+    b.ts_ep = cut->ts_ep;
+    b.ts_q = cut->ts_q;
+    b.tm_ep = cut->tm_ep;
     b.ep_lvl = (int32_t *)s.eplv.p;
     b.ep_rho = (double *)s.eprho.p;
     b.lane_ch = (int32_t *)s.lanes.p;
