@@ -58,7 +58,7 @@ struct WaveRows {
 // with compensated FP32 terms, also a step's terms in arc order and the number
 // of them before each arc
 struct WaveTerms {
-    float t[64 * 4];
+    float t[64 * 4 + 4];  // (read four at a time)
     uint16_t before[64 * 4 + 4];  // (the waves' parts stay 8-byte aligned)
 };
 template <typename TT>
@@ -196,7 +196,7 @@ __device__ __forceinline__ void append(const Ctx &x, const int (&w)[U], const bo
 }
 
 constexpr int PU = 4;  // arcs of a lane in flight
-static_assert(sizeof(WaveTerms::t) == 4 * 64 * PU, "a step's terms");
+static_assert(sizeof(WaveTerms::t) >= 4 * 64 * PU, "a step's terms");
 
 // Forward BFS from s.  Returns the deepest level, -1 when a uint64 count
 // overflowed.
@@ -429,8 +429,18 @@ __device__ __forceinline__ void plain_backward(const PlainCtx<LG, TT> &x, int ma
                                 i = q.before[a0];
                                 ie = q.before[a1];
                             }
-                            for (; pbal(i < ie); ++i)
-                                if (i < ie) rho.add(q.t[i]);
+                            for (; pbal(i < ie); i += 4) {
+                                float y[4];
+                                const int at = i < ie ? i : 0;
+#pragma unroll
+                                for (int u = 0; u < 4; ++u) y[u] = q.t[at + u];
+#pragma unroll
+                                for (int u = 0; u < 4; ++u) {
+                                    Acc more = rho;
+                                    more.add(y[u]);
+                                    if (i + u < ie) rho = more;
+                                }
+                            }
                             psync();
                         } else {
                             double *acc = (double *)r.acc;

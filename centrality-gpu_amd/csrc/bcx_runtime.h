@@ -98,11 +98,13 @@ struct PlanBatch {
 struct Plan {
     std::vector<int32_t> free_src;     // BFS sources that need no row
     std::vector<PlanBatch> batches;
+    // sources by their role in the method: n_chain counts the chain vertices,
+    // those among free_src too
     int64_t n_bfs = 0, n_chain = 0, n_row_only = 0;
 };
 
 int make_plan(const HostComp &hc, const int32_t *subset, int64_t n_sub, bool use_chains,
-              int64_t row_cap, Plan &plan);
+              int64_t row_cap, bool direct, Plan &plan);
 
 }  // namespace bcx
 

@@ -145,8 +145,15 @@ void Timer::destroy() {
 // endpoint on the ear graph (endpoints as vertices, chains as edges), the
 // role of the ear-graph level batches of Codes/arrangelevels.cpp:56-109, and
 // packed greedily while the distinct endpoints fit in row_cap slots.
+// With `direct`, the sources of a chain whose endpoints' rows only it needs run
+// as BFS sources: on an 84k power-law core a kept row costs 10.2 us, a combined
+// source 9.5 us and a BFS source 13.4 us, so a row that no source wants for
+// itself pays from three chain sources on; and the combine's launches of their
+// own pay from an eighth of the sources on (1000 sampled sources 18.9 -> 13.5
+// ms, 2049 of an 18.6k grid 5.1 -> 3.5 ms; with every source of a 17k core
+// wanted, 37% of them on chains, the rows save 6%).
 int bcx::make_plan(const HostComp &hc, const int32_t *subset, int64_t n_sub, bool use_chains,
-              int64_t row_cap, Plan &plan) {
+              int64_t row_cap, bool direct, Plan &plan) {
     const int32_t n = hc.n;
     const int32_t nch = use_chains ? hc.n_chains : 0;
     plan = Plan();
@@ -162,8 +169,10 @@ int bcx::make_plan(const HostComp &hc, const int32_t *subset, int64_t n_sub, boo
     }
     std::vector<uint8_t> want_bfs((size_t)n, 0);
     std::vector<std::vector<int32_t>> chain_srcs((size_t)nch);
+    int64_t n_wanted = 0;
     auto add = [&](int32_t v) {
         if (v < 0 || v >= n) return;
+        n_wanted++;
         if (chain_of[v] >= 0) chain_srcs[chain_of[v]].push_back(pos_of[v]);
         else want_bfs[v] = 1;
     };
@@ -177,6 +186,28 @@ int bcx::make_plan(const HostComp &hc, const int32_t *subset, int64_t n_sub, boo
             chain_srcs[c].erase(std::unique(chain_srcs[c].begin(), chain_srcs[c].end()), chain_srcs[c].end());
             need.push_back(c);
         }
+    if (direct) {
+        auto pays = [&](int32_t c) {
+            const int32_t L = hc.ch_ends[2 * c], R = hc.ch_ends[2 * c + 1];
+            const size_t rows = (size_t)!want_bfs[L] + (size_t)(!want_bfs[R] && R != L);
+            return chain_srcs[c].size() >= 3 * rows;
+        };
+        int64_t combined = 0;
+        for (int32_t c : need)
+            if (pays(c)) combined += (int64_t)chain_srcs[c].size();
+        const bool none = combined < n_wanted / 8;
+        std::vector<int32_t> keep;
+        for (int32_t c : need) {
+            if (!none && pays(c)) {
+                keep.push_back(c);
+                continue;
+            }
+            for (int32_t p : chain_srcs[c]) plan.free_src.push_back(hc.ch_nodes[hc.ch_ptr[c] + p]);
+            plan.n_chain += (int64_t)chain_srcs[c].size();
+        }
+        need.swap(keep);
+    }
+    const int64_t n_direct = (int64_t)plan.free_src.size();
     // endpoints of needed chains
     std::vector<uint8_t> needed_end((size_t)n, 0);
     for (int32_t c : need) {
@@ -185,7 +216,7 @@ int bcx::make_plan(const HostComp &hc, const int32_t *subset, int64_t n_sub, boo
     }
     for (int32_t v = 0; v < n; ++v)
         if (want_bfs[v] && !needed_end[v]) plan.free_src.push_back(v);
-    plan.n_bfs = (int64_t)plan.free_src.size();
+    plan.n_bfs = (int64_t)plan.free_src.size() - n_direct;
     if (need.empty()) return BCX_OK;
 
     // ear graph BFS order over needed endpoints
@@ -801,7 +832,8 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
         }
         if (o.path == BCX_PATH_PLAIN) {
             Plan plan;
-            rc = make_plan(dc.host, sp, sn, o.use_chains != 0, row_capacity(ctx, dc.n, &o), plan);
+            // (a caller who sizes the row slab gets the rows)
+            rc = make_plan(dc.host, sp, sn, o.use_chains != 0, row_capacity(ctx, dc.n, &o), o.row_cap_bytes <= 0, plan);
             if (rc) return rc;
             account(plan.n_bfs, plan.n_chain);
             s->n_row_only += plan.n_row_only;
