@@ -62,7 +62,13 @@ PlainShape plain_shape(int32_t n, bool fp32);
 
 hipError_t launch_plain_bfs(const CompDev &c, const PlainArgs &a, const PlainScratch &sc,
                             const Rows &rows, const PlainShape &p, int grid, hipStream_t st);
-hipError_t launch_plain_fold(double *bc, const double *copies, int n, int split, hipStream_t st);
+// Adds `split` copies of an accumulator to bc (perm, optional: word v of a copy
+// belongs to bc[perm[v]]).
+hipError_t launch_plain_fold(double *bc, const double *copies, const int32_t *perm, int n, int split, hipStream_t st);
+// Fills to.col and to.reach: row i of `to` is row perm[i] of `from`, its columns
+// renumbered by inv.
+hipError_t launch_plain_reorder(const CompDev &from, const CompDev &to, const int32_t *perm, const int32_t *inv,
+                                hipStream_t st);
 hipError_t launch_plain_chain(const CompDev &c, const ChainDev &ch, const PlainArgs &a,
                               const PlainScratch &sc, const Rows &rows, const PlainShape &p, int grid, hipStream_t st);
 

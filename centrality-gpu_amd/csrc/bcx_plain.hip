@@ -729,17 +729,32 @@ hipError_t launch_plain_bfs(const CompDev &c, const PlainArgs &a, const PlainScr
     return hipGetLastError();
 }
 
-// Adds the copies of a split BC accumulator to the component's slice.
-__global__ void k_plain_fold(double *bc, const double *copies, int n, int split) {
+__global__ void k_plain_fold(double *bc, const double *copies, const int32_t *perm, int n, int split) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= n) return;
     double s = 0.0;
     for (int k = 0; k < split; ++k) s += copies[(int64_t)k * n + v];
-    bc[v] += s;
+    bc[perm ? perm[v] : v] += s;
 }
 
-hipError_t launch_plain_fold(double *bc, const double *copies, int n, int split, hipStream_t st) {
-    hipLaunchKernelGGL(k_plain_fold, dim3((n + 255) / 256), dim3(256), 0, st, bc, copies, n, split);
+hipError_t launch_plain_fold(double *bc, const double *copies, const int32_t *perm, int n, int split, hipStream_t st) {
+    hipLaunchKernelGGL(k_plain_fold, dim3((n + 255) / 256), dim3(256), 0, st, bc, copies, perm, n, split);
+    return hipGetLastError();
+}
+
+// One wave per row.
+__global__ __launch_bounds__(256) void k_plain_reorder(CompDev from, CompDev to, const int32_t *perm,
+                                                       const int32_t *inv) {
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (i >= from.n) return;
+    const int v = perm[i], a = from.rp[v], d = from.rp[v + 1] - a, at = to.rp[i];
+    for (int j = lane; j < d; j += 64) const_cast<int32_t *>(to.col)[at + j] = inv[from.col[a + j]];
+    if (lane == 0) const_cast<int32_t *>(to.reach)[i] = from.reach[v];
+}
+
+hipError_t launch_plain_reorder(const CompDev &from, const CompDev &to, const int32_t *perm, const int32_t *inv,
+                                hipStream_t st) {
+    hipLaunchKernelGGL(k_plain_reorder, dim3((from.n + 3) / 4), dim3(256), 0, st, from, to, perm, inv);
     return hipGetLastError();
 }
 

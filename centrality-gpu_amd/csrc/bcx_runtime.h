@@ -69,6 +69,14 @@ struct DComp {
     DComp *relabel = nullptr;
     DBuf b_perm;
     std::vector<int32_t> relabel_inv;
+    // per-source kernel: the component in BFS order from its highest-degree
+    // vertex (built on first use; ord_state -1 not yet looked at, 0 degrees too
+    // even, 1 built), ord_inv[old] = new, ord_perm[new] = old
+    int8_t ord_state = -1;
+    CompDev ord{};
+    DBuf b_ord;
+    const int32_t *ord_perm = nullptr;
+    std::vector<int32_t> ord_inv;
     // multi-launch batched path with contracted chains (built on first use;
     // cut_state -1 not yet tried, 0 the component has too few such chains)
     ChainCut *cut = nullptr;
@@ -151,7 +159,7 @@ void dev_free(bcx_ctx *ctx, void *p);
 int upload(bcx_ctx *ctx, const void *host, size_t bytes, bcx::DBuf &buf, const char *what);
 int read_counters(bcx_ctx *ctx, bcx_stats *st);
 int64_t row_capacity(bcx_ctx *ctx, int32_t n, const bcx_opts *o);
-int plain_component(bcx_ctx *ctx, const bcx::DComp &dc, const bcx::Plan &plan, const bcx_opts *o,
+int plain_component(bcx_ctx *ctx, bcx::DComp &dc, const bcx::Plan &plan, const bcx_opts *o,
                     double *bc, bcx_stats *st);
 
 // Device address of the no-allocation entry point's static scratch array on

@@ -361,13 +361,18 @@ int64_t row_capacity(bcx_ctx *ctx, int32_t n, const bcx_opts *o) {
     return std::max<int64_t>(2, std::min<int64_t>(r, 1 << 16));
 }
 
+// (ordered: on the ordered copy when there is one; no rows kept)
 static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t> &src,
                         const std::vector<int32_t> &slot, const std::vector<int8_t> &mode,
                         bool f64, uint64_t limit, double *bc, const Rows &rows, bcx_stats *st,
-                        double *probe = nullptr, bool fp32 = false) {
+                        double *probe = nullptr, bool fp32 = false, bool ordered = false) {
     if (src.empty()) return BCX_OK;
     int rc;
-    if ((rc = upload(ctx, src.data(), src.size() * 4, ctx->w_src, "work list"))) return rc;
+    ordered = ordered && dc.ord_state == 1;
+    std::vector<int32_t> ids;
+    if (ordered)
+        for (int32_t v : src) ids.push_back(dc.ord_inv[(size_t)v]);
+    if ((rc = upload(ctx, ordered ? ids.data() : src.data(), src.size() * 4, ctx->w_src, "work list"))) return rc;
     if ((rc = upload(ctx, slot.data(), slot.size() * 4, ctx->w_aux, "work list"))) return rc;
     if ((rc = upload(ctx, mode.data(), mode.size(), ctx->w_mode, "work list"))) return rc;
     rc = ctx_hip(ctx, hipMemsetAsync(ctx->counters.p, 0, 4 * sizeof(int32_t), ctx->stream), "memset");
@@ -395,21 +400,95 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
     // atomics, ran 20-30% slower (8000 sources of that grid 13.6 -> 16.0 ms).
     constexpr int SPLIT = 16;
     constexpr size_t SPLIT_SOURCES = 4096;
-    const size_t split_bytes = sizeof(double) * SPLIT * (size_t)dc.n;
-    a.split = 1;
-    if (src.size() >= SPLIT_SOURCES && ctx->bc_split.ensure(ctx, split_bytes, "split accumulator") == BCX_OK) {
-        a.split = SPLIT;
+    // (an ordered run folds its one copy back to the component's order)
+    a.split = src.size() >= SPLIT_SOURCES ? SPLIT : 1;
+    const size_t word = sizeof(double) * (size_t)dc.n;
+    bool fold = a.split > 1 || ordered;
+    if (fold && ctx->bc_split.ensure(ctx, word * a.split, "split accumulator") != BCX_OK) {
+        a.split = 1;
+        if (ordered && (rc = ctx->bc_split.ensure(ctx, word, "accumulator"))) return rc;
+        fold = ordered;
+    }
+    if (fold) {
         a.bc = (double *)ctx->bc_split.p;
-        if ((rc = ctx_hip(ctx, hipMemsetAsync(a.bc, 0, split_bytes, ctx->stream), "memset"))) return rc;
+        if ((rc = ctx_hip(ctx, hipMemsetAsync(a.bc, 0, word * a.split, ctx->stream), "memset"))) return rc;
     }
     ctx->timer.begin(ctx);
-    hipError_t e = launch_plain_bfs(dc.dev, a, sc, rows, shape, grid, ctx->stream);
-    if (e == hipSuccess && a.split > 1) e = launch_plain_fold(bc, a.bc, dc.n, a.split, ctx->stream);
+    hipError_t e = launch_plain_bfs(ordered ? dc.ord : dc.dev, a, sc, rows, shape, grid, ctx->stream);
+    if (e == hipSuccess && fold)
+        e = launch_plain_fold(bc, a.bc, ordered ? dc.ord_perm : nullptr, dc.n, a.split, ctx->stream);
     ctx->timer.end(ctx);
-    if (st) st->n_launches += a.split > 1 ? 2 : 1;
+    if (st) st->n_launches += fold ? 2 : 1;
     rc = ctx_hip(ctx, e, "k_plain_bfs launch");
     if (rc) return rc;
     return read_counters(ctx, st);
+}
+
+// A copy of the component numbered in BFS order from its highest-degree vertex,
+// for the per-source kernel: most gathers of a skewed graph go to few vertices,
+// and those and what a level reaches then share cache lines (1000 sources of an
+// 84k power-law core 13.5 -> 11.0 ms; ordered by degree class 12.4).  Rows keep
+// the order of their arcs, so FP64 counts keep the oracle's sums.  Made for
+// runs of ORDER_SOURCES sources or more, on components of ORDER_N vertices or
+// more a quarter of whose vertices take half of the arcs (on grids the
+// component's own order is as good).  The order is the vertex list that the
+// kernel itself leaves behind for that source.
+constexpr int32_t ORDER_N = 4096;
+constexpr int64_t ORDER_SOURCES = 512;
+static int order_copy(bcx_ctx *ctx, DComp &dc) {
+    if (dc.ord_state >= 0) return BCX_OK;
+    dc.ord_state = 0;
+    const HostComp &h = dc.host;
+    const int32_t n = h.n;
+    if (n < ORDER_N) return BCX_OK;
+    int64_t of[33] = {0}, arcs[33] = {0};  // vertices and arcs by degree class (powers of two)
+    int32_t root = 0;
+    for (int32_t v = 0; v < n; ++v) {
+        const int32_t d = h.rp[v + 1] - h.rp[v];
+        const int k = d > 0 ? 32 - __builtin_clz((unsigned)d) : 0;
+        of[k]++;
+        arcs[k] += d;
+        if (d > h.rp[root + 1] - h.rp[root]) root = v;
+    }
+    int64_t top = 0, top_arcs = 0;
+    for (int k = 32; k >= 0 && top + of[k] <= n / 4; --k) {
+        top += of[k];
+        top_arcs += arcs[k];
+    }
+    if (2 * top_arcs < h.arcs) return BCX_OK;
+    int rc = run_bfs_list(ctx, dc, {root}, {-1}, {0}, true, 0, nullptr, Rows{}, nullptr);  // (forward only)
+    PlainScratch sc;
+    if (rc || (rc = ensure_plain_scratch(ctx, n, 1, sc))) return rc;
+    // row pointers, permutation and its inverse from the host; columns and
+    // reach weights are filled in on the device
+    std::vector<int32_t> t(3 * (size_t)n + 1);
+    int32_t *rp = t.data(), *perm = rp + n + 1, *inv = perm + n;
+    if ((rc = ctx_hip(ctx, hipMemcpyAsync(perm, sc.S, 4 * (size_t)n, hipMemcpyDeviceToHost, ctx->stream), "copy")) ||
+        (rc = ctx_hip(ctx, hipStreamSynchronize(ctx->stream), "copy")))
+        return rc;
+    std::fill(inv, inv + n, -1);
+    rp[0] = 0;
+    for (int32_t i = 0; i < n; ++i) {
+        const int32_t v = perm[i];
+        if (v < 0 || v >= n || inv[v] >= 0) return BCX_OK;  // (not connected: the list is short)
+        inv[v] = i;
+        rp[i + 1] = rp[i] + (h.rp[v + 1] - h.rp[v]);
+    }
+    // (no room under the cap: the component's own order does as well)
+    if (dc.b_ord.ensure(ctx, 4 * (t.size() + (size_t)n + h.col.size()), "ordered component") != BCX_OK) return BCX_OK;
+    int32_t *d = (int32_t *)dc.b_ord.p;
+    dc.ord.n = n;
+    dc.ord.arcs = dc.arcs;
+    dc.ord.rp = d;
+    dc.ord_perm = d + n + 1;
+    dc.ord.reach = d + t.size();
+    dc.ord.col = dc.ord.reach + n;
+    dc.ord_inv.assign(inv, inv + n);
+    rc = upload(ctx, t.data(), 4 * t.size(), dc.b_ord, "ordered component");
+    if (!rc) rc = ctx_hip(ctx, launch_plain_reorder(dc.dev, dc.ord, dc.ord_perm, dc.ord_perm + n, ctx->stream), "reorder");
+    if (!rc) rc = ctx_hip(ctx, hipStreamSynchronize(ctx->stream), "ordered component");
+    if (!rc) dc.ord_state = 1;
+    return rc;
 }
 
 int read_counters(bcx_ctx *ctx, bcx_stats *st) {
@@ -465,7 +544,8 @@ static int plain_component_mode(bcx_ctx *ctx, const DComp &dc, const Plan &plan,
     if ((rc = ensure_rows(ctx, dc.n, max_rows, rows))) return rc;
     std::vector<int32_t> slots(plan.free_src.size(), -1);
     std::vector<int8_t> modes(plan.free_src.size(), MODE_BC);
-    if ((rc = run_bfs_list(ctx, dc, plan.free_src, slots, modes, f64, limit, bc, rows, st))) return rc;
+    if ((rc = run_bfs_list(ctx, dc, plan.free_src, slots, modes, f64, limit, bc, rows, st, nullptr, false, true)))
+        return rc;
     if (ctx->overflow && !f64) return BCX_OK;
     for (auto &b : plan.batches) {
         if ((rc = run_bfs_list(ctx, dc, b.bsrc, b.bslot, b.bmode, f64, limit, bc, rows, st))) return rc;
@@ -475,12 +555,14 @@ static int plain_component_mode(bcx_ctx *ctx, const DComp &dc, const Plan &plan,
     return BCX_OK;
 }
 
-int plain_component(bcx_ctx *ctx, const DComp &dc, const Plan &plan, const bcx_opts *o,
+int plain_component(bcx_ctx *ctx, DComp &dc, const Plan &plan, const bcx_opts *o,
                     double *bc, bcx_stats *st) {
     const uint64_t limit = (o && o->sigma_f64_threshold_log2 > 0 && o->sigma_f64_threshold_log2 < 64)
                                ? (1ull << o->sigma_f64_threshold_log2) : 0;
     ctx->overflow = false;
-    int rc = plain_component_mode(ctx, dc, plan, false, limit, bc, st);
+    int rc = (int64_t)plan.free_src.size() >= ORDER_SOURCES ? order_copy(ctx, dc) : BCX_OK;
+    if (rc) return rc;
+    rc = plain_component_mode(ctx, dc, plan, false, limit, bc, st);
     if (rc) return rc;
     if (!ctx->overflow) return BCX_OK;
     // sigma left uint64: redo the component with FP64 sigma (pull order)
@@ -501,11 +583,13 @@ int source_component(bcx_ctx *ctx, DComp &dc, const std::vector<int32_t> &srcs, 
     const Rows rows{};
     *overflow = false;
     int rc;
+    if ((int64_t)srcs.size() >= ORDER_SOURCES && (rc = order_copy(ctx, dc))) return rc;
     // components whose counts from their highest-degree vertex pass 2^62 start
     // with FP64 counts, as on the workgroup kernel
     if (dc.sigma_est <= 4.6e18) {
         ctx->overflow = false;
-        if ((rc = run_bfs_list(ctx, dc, srcs, slots, modes, false, limit, bc, rows, st, nullptr, fp32))) return rc;
+        if ((rc = run_bfs_list(ctx, dc, srcs, slots, modes, false, limit, bc, rows, st, nullptr, fp32, true)))
+            return rc;
         if (!ctx->overflow) return BCX_OK;
         rc = ctx_hip(ctx, hipMemsetAsync(bc, 0, sizeof(double) * (size_t)dc.n, ctx->stream), "memset");
         if (rc || fp32) {
@@ -514,7 +598,7 @@ int source_component(bcx_ctx *ctx, DComp &dc, const std::vector<int32_t> &srcs, 
         }
     }
     if (st) st->n_f64_sigma += (int64_t)srcs.size();
-    return run_bfs_list(ctx, dc, srcs, slots, modes, true, 0, bc, rows, st);
+    return run_bfs_list(ctx, dc, srcs, slots, modes, true, 0, bc, rows, st, nullptr, false, true);
 }
 
 // ------------------------------------------------------------------------
@@ -673,7 +757,7 @@ void bcx_dgraph_free(bcx_ctx *ctx, bcx_dgraph *g) {
     if (ctx) {
         (void)hipStreamSynchronize(ctx->stream);
         for (auto &dc : g->comps)
-            for (DBuf *b : {&dc.b_rp, &dc.b_col, &dc.b_reach, &dc.b_chp, &dc.b_chn, &dc.b_che}) b->release(ctx);
+            for (DBuf *b : {&dc.b_rp, &dc.b_col, &dc.b_reach, &dc.b_chp, &dc.b_chn, &dc.b_che, &dc.b_ord}) b->release(ctx);
         batched_graph_release(ctx, g);
         g->pool.release(ctx);
     }
