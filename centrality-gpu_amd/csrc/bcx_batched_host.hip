@@ -1830,14 +1830,16 @@ int batched_kind(DComp &dc, int flags) {
 // sample sources (evenly spaced over its tile order, BC into a scratch
 // accumulator, timed with HIP events, outside the run's timing) under each
 // candidate schedule, and what was measured is cached for every later run:
-//  * kernel: the multi-launch tiles over TUNE_TILES tiles, the per-source
-//    kernel over TUNE_SOURCES sources and, for components it can take (<= WG_N
-//    vertices), the workgroup kernel over min(tiles, CUs) tiles (its
-//    concurrent width).  A run takes the kernel with the least estimated time
-//    for its number of sources: a sample of sources that leaves most CUs
-//    without a workgroup tile still fills the chip source by source (2000
-//    sources of an 84k power-law core: 158 ms on the workgroup kernel, 26 ms
-//    per source; 2049 of an 18.6k grid: 65 ms against 5 ms);
+//  * kernel: the per-source kernel over TUNE_SOURCES sources and the
+//    multi-launch tiles over TUNE_TILES tiles, unless three launches per level
+//    alone would take those longer than half of what the per-source kernel
+//    takes (deep components); the workgroup kernel over min(tiles, CUs) tiles
+//    (its concurrent width) only where counts overflow the per-source kernel
+//    with FP32 terms.  A run takes the kernel with the least estimated time for
+//    its number of sources.  All sources, per source / multi-launch / workgroup
+//    (ms): 18.6k grid 22 / - / 97; 10.6k power-law core 11 / 26 / 40, 42k core
+//    - / 131 / 220, 84k core (20000 sources) - / 93 / 207; 2000 sources of the
+//    84k core 24 / 23 / 158;
 //  * multi-launch: 8 / 4 / 16 level-kernel blocks per CU, 8 / 4 tiles in
 //    flight, chain contraction on / off, once a run takes them.
 // Each tiled candidate runs twice (the first run captures its graphs) and is
@@ -1848,7 +1850,8 @@ int batched_kind(DComp &dc, int flags) {
 // ------------------------------------------------------------------------
 constexpr int32_t TUNE_N = 16384;
 constexpr int TUNE_TILES = 24;
-constexpr int64_t TUNE_SOURCES = 1024;
+constexpr int64_t TUNE_SOURCES = 4096;
+constexpr double LAUNCH_S = 4e-6;  // of a level kernel that finds next to nothing to do
 
 // Sources of k tiles of `width` evenly spaced over the component's tile order.
 static std::vector<int32_t> sample_tiles(DComp &dc, int64_t k, int64_t width) {
@@ -1865,7 +1868,7 @@ static std::vector<int32_t> sample_tiles(DComp &dc, int64_t k, int64_t width) {
 }
 
 // The kernel with the least estimated time for n_src sources, from the rates
-// measured on the samples.
+// measured on the samples (0: not measured).
 static int measured_kind(bcx_ctx *ctx, const DComp &dc, int64_t n_src) {
     const double cus = std::max(1, ctx->n_cu), s = (double)n_src;
     int kind = BCX_KERNEL_MULTI;
@@ -1935,24 +1938,30 @@ int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, int64_t n_src, 
     const std::vector<int32_t> samp =
         rc ? std::vector<int32_t>() : sample_tiles(dc, TUNE_TILES, (int64_t)BATCH_W * MAX_SPL);
     double r_multi = 0.0;
-    if (!rc) rc = time_multi(samp, base, &r_multi);
     if (!rc && need_kind) {
-        dc.rate_multi = r_multi;
-        if (dc.n <= WG_N) {
-            const std::vector<int32_t> ws = sample_tiles(dc, std::max(1, ctx->n_cu), (int64_t)BATCH_W * wg_spl(o));
-            rc = time_wg(ws, &dc.rate_wg);
-            dc.round_wg = (double)ws.size();
-        }
-        if (!rc && source_fits && !valid_spl(o->sources_per_lane)) {
-            std::vector<int32_t> order = batched_order(dc), ss;
-            const int64_t k = std::min<int64_t>(dc.n <= WG_N ? TUNE_SOURCES : TUNE_SOURCES / 4, dc.n);
+        dc.rate_src = dc.rate_wg = dc.rate_multi = 0.0;
+        if (source_fits && !valid_spl(o->sources_per_lane)) {
+            const std::vector<int32_t> order = batched_order(dc);
+            std::vector<int32_t> ss;
+            const int64_t k = std::min<int64_t>(dc.n <= WG_N ? TUNE_SOURCES : TUNE_SOURCES / 8, dc.n);
             for (int64_t i = 0; i < k; ++i) ss.push_back(order[(size_t)(i * dc.n / k)]);
             bool overflow = false;
             rc = source_component(ctx, dc, ss, &to, bc + dc.offset, nullptr, &overflow);
             const double t = ctx->timer.collect();
             dc.rate_src = t > 0 && !overflow ? (double)k / t : 0.0;
         }
-        dc.kind_measured = !rc;
+        if (!rc && dc.rate_src == 0.0 && dc.n <= WG_N) {
+            const std::vector<int32_t> ws = sample_tiles(dc, std::max(1, ctx->n_cu), (int64_t)BATCH_W * wg_spl(o));
+            rc = time_wg(ws, &dc.rate_wg);
+            dc.round_wg = (double)ws.size();
+        }
+    }
+    const double per_src = need_kind && dc.rate_src > 0 ? 1.0 / dc.rate_src : 0.0;
+    const double launches = 3.0 * (dc.depth + 1) * LAUNCH_S / (MAX_SLOTS * BATCH_W * MAX_SPL);
+    if (!rc && !(per_src > 0 && dc.depth >= 0 && per_src < 2 * launches)) rc = time_multi(samp, base, &r_multi);
+    if (!rc && need_kind) {
+        dc.rate_multi = r_multi;
+        dc.kind_measured = true;
         kind = measured_kind(ctx, dc, n_src);
     }
     MultiSched best = base;
