@@ -1312,6 +1312,9 @@ struct SmallState {
     // tiles: the tiles of an FP64 rerun
     DBuf tables, tiles, counter, redo, sig, tt, Q, Qm, masks, qoffs, qr, ro, tag, lvl, dbg, psig;
     unsigned char *pin = nullptr;  // pinned host staging of the tables
+    // (wave-per-source pass) a launch's counters come back here
+    int32_t *ctr_pin = nullptr, *ctr_back = nullptr, ctr_host[4] = {0, 0, 0, 0};
+    int occ_lds = -1, occ = 1;     // workgroups per compute unit at that much LDS
     size_t pin_bytes = 0;
     int grid = 0;
     // a pass started and not yet finished (persistent_start / _finish)
@@ -1656,6 +1659,16 @@ bool src_takes(const DComp &dc, bool fp32) {
 
 static bool run_fp32(const bcx_opts *o) { return o->path == BCX_PATH_BATCHED && o->precision == BCX_PREC_FP32C; }
 
+// Queues the read-back of a launch's counters behind it.
+static int src_counters(bcx_ctx *ctx, SmallState &ss, const int32_t *from, hipStream_t sp) {
+    if (!ss.ctr_pin && hipHostMalloc((void **)&ss.ctr_pin, 64, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        ss.ctr_pin = nullptr;
+    }
+    ss.ctr_back = ss.ctr_pin ? ss.ctr_pin : ss.ctr_host;
+    return ctx_hip(ctx, hipMemcpyAsync(ss.ctr_back, from, 3 * sizeof(int32_t), hipMemcpyDeviceToHost, sp), "counter");
+}
+
 static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base,
                      bcx_stats *st, hipStream_t sp, bool probe) {
     if (jobs.empty()) return BCX_OK;
@@ -1674,10 +1687,10 @@ static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_
     std::stable_sort(order.begin(), order.end(),
                      [](const SmallJob *x, const SmallJob *y) { return x->dc->arcs > y->dc->arcs; });
     // few sources per tile while that gives every compute unit a tile, four
-    // tiles per compute unit for larger jobs.  With FP32
-    // terms a count overflow turns the 64 consecutive sources around it to FP64
-    // terms, so smaller tiles are a first try: an overflow (rare in components
-    // of this size) ends it and the pass is repeated in tiles of 64
+    // tiles per compute unit for larger jobs.  With FP32 terms a count overflow
+    // turns the 64 consecutive sources around it to FP64 terms, so smaller
+    // tiles are a first try: an overflow (rare in components of this size) ends
+    // it and the pass is repeated in tiles of 64
     const bool fp32 = run_fp32(o);
     const size_t per = n_src / (size_t)std::max(1, ctx->n_cu);
     const size_t tw = probe || per > 128 ? BATCH_W : (per > 64 ? 32 : (per > 8 ? 16 : (per > 4 ? 8 : 4)));
@@ -1711,7 +1724,11 @@ static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_
     for (const SmallJob *jb : order) ss.run_slices.push_back({bc_base + jb->dc->offset, jb->dc->n});
     ss.run_fp32 = fp32;
     ss.run_tiles = std::move(tb.tiles);
-    ss.run_grid = (int)std::min<int64_t>(a.n_tiles, (int64_t)src_blocks_per_cu(a.lds) * std::max(1, ctx->n_cu));
+    if (ss.occ_lds != a.lds) {
+        ss.occ = src_blocks_per_cu(a.lds);
+        ss.occ_lds = a.lds;
+    }
+    ss.run_grid = (int)std::min<int64_t>(a.n_tiles, (int64_t)ss.occ * std::max(1, ctx->n_cu));
     ss.run_stream = sp;
     ss.pending = true;
     if ((rc = follow_ctx_stream(ctx, sp))) return rc;
@@ -1719,10 +1736,10 @@ static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_
     rc = ctx_hip(ctx, launch_src(a, false, fp32, ss.run_grid, sp), "source kernel");
     ctx->timer.end(ctx);
     if (st) st->n_launches++;
-    return rc;
+    return rc ? rc : src_counters(ctx, ss, a.counter, sp);
 }
 
-static int src_finish(bcx_ctx *ctx, bcx_stats *st) {
+static int src_finish(bcx_ctx *ctx, bcx_stats *st, bool *reran = nullptr) {
     if (!ctx->srck || !ctx->srck->pending) return BCX_OK;
     SmallState &ss = *ctx->srck;
     ss.pending = false;
@@ -1730,12 +1747,10 @@ static int src_finish(bcx_ctx *ctx, bcx_stats *st) {
     SrcArgs a = ss.src;
     int rc;
     int32_t h[3] = {0, 0, 0};
-    auto counters = [&](const int32_t *from) {
-        int32_t c[3];
-        int r = ctx_hip(ctx, hipMemcpyAsync(c, from, sizeof(c), hipMemcpyDeviceToHost, sp), "counter");
-        if (!r) r = ctx_hip(ctx, hipStreamSynchronize(sp), "source kernel");
-        h[1] = c[1];
-        h[2] = std::max(h[2], c[2]);
+    auto counters = [&]() {
+        const int r = ctx_hip(ctx, hipStreamSynchronize(sp), "source kernel");
+        h[1] = ss.ctr_back[1];
+        h[2] = std::max(h[2], ss.ctr_back[2]);
         return r;
     };
     // another launch over `tiles`, with counters of its own
@@ -1750,9 +1765,11 @@ static int src_finish(bcx_ctx *ctx, bcx_stats *st) {
         r = ctx_hip(ctx, launch_src(a, f64, ss.run_fp32, std::min(ss.run_grid, a.n_tiles), sp), "source kernel");
         ctx->timer.end(ctx);
         if (st) st->n_launches++;
-        return r ? r : counters(a.counter);
+        if (reran) *reran = true;
+        if (r || (r = src_counters(ctx, ss, a.counter, sp))) return r;
+        return counters();
     };
-    if ((rc = counters(a.counter))) return rc;
+    if ((rc = counters())) return rc;
     if (h[1] > 0 && a.stop) {
         for (auto &s : ss.run_slices)
             if ((rc = ctx_hip(ctx, hipMemsetAsync(s.first, 0, sizeof(double) * (size_t)s.second, ctx->stream), "memset")))
@@ -1788,8 +1805,8 @@ int batched_persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, co
     return persistent_start(ctx, jobs, o, bc_base, st, pass == PASS_WG, sp, false);
 }
 
-int batched_persistent_finish(bcx_ctx *ctx, bcx_stats *st, int pass) {
-    return pass == PASS_SRC ? src_finish(ctx, st) : persistent_finish(ctx, st, pass == PASS_WG);
+int batched_persistent_finish(bcx_ctx *ctx, bcx_stats *st, int pass, bool *again) {
+    return pass == PASS_SRC ? src_finish(ctx, st, again) : persistent_finish(ctx, st, pass == PASS_WG);
 }
 
 void batched_persistent_reset(bcx_ctx *ctx) {
@@ -1804,6 +1821,7 @@ static void release_state(bcx_ctx *ctx, SmallState *&state) {
     SmallState &ss = *state;
     if (ss.exec) (void)hipGraphExecDestroy(ss.exec);
     if (ss.pin) (void)hipHostFree(ss.pin);
+    if (ss.ctr_pin) (void)hipHostFree(ss.ctr_pin);
     for (DBuf *b : {&ss.tables, &ss.tiles, &ss.counter, &ss.redo, &ss.sig, &ss.tt, &ss.Q, &ss.Qm, &ss.masks,
                     &ss.qoffs, &ss.qr, &ss.ro, &ss.tag, &ss.lvl, &ss.dbg, &ss.psig})
         b->release(ctx);

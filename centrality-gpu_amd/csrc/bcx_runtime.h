@@ -135,6 +135,8 @@ struct bcx_ctx {
     bcx::DBuf bc_pack, bc_chunks;  // result download: packed slices and their chunk list
     double *bc_pin = nullptr;      // pinned host staging of the result download
     size_t bc_pin_bytes = 0;
+    int32_t *up_pin = nullptr;     // pinned host staging of small uploads
+    bool busy = true;              // work may be in flight on the context stream
     BatchedState *batched = nullptr;
     SmallState *small = nullptr;
     SmallState *wgk = nullptr;  // workgroup-per-tile kernel buffers
@@ -184,7 +186,8 @@ std::vector<int32_t> batched_order(bcx::DComp &dc);
 enum { PASS_SMALL = 0, PASS_WG = 1, PASS_SRC = 2 };
 int batched_persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base,
                              bcx_stats *st, int pass, hipStream_t sp);
-int batched_persistent_finish(bcx_ctx *ctx, bcx_stats *st, int pass);
+// (*again, optional: some of it was rerun after the first launch)
+int batched_persistent_finish(bcx_ctx *ctx, bcx_stats *st, int pass, bool *again = nullptr);
 // Whether the wave-per-source kernel takes a component, with FP32 or FP64 terms.
 bool src_takes(const bcx::DComp &dc, bool fp32);
 // Drops passes left unfinished by an earlier failed run (after waiting for them).

@@ -372,9 +372,12 @@ __global__ __launch_bounds__(XB) void k_src(SrcArgs a) {
     __shared__ int s_item, s_next, s_ovf, s_depth, s_scan[SRC_WAVES];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int n_tiles = a.n_tiles_dev ? *a.n_tiles_dev : a.n_tiles;
-    while (true) {
+    // the first tile is the workgroup's own, the work counter hands out the rest
+    for (bool first = true;; first = false) {
         if (tid == 0) {
-            s_item = a.stop && ald(&a.counter[1]) != 0 ? n_tiles : atomicAdd(&a.counter[0], 1);
+            if (a.stop && ald(&a.counter[1]) != 0) s_item = n_tiles;
+            else if (first) s_item = blockIdx.x;
+            else s_item = (int)gridDim.x < n_tiles ? (int)gridDim.x + atomicAdd(&a.counter[0], 1) : n_tiles;
             s_next = 0;
             s_ovf = 0;
             s_depth = 0;
