@@ -26,6 +26,9 @@
 //           -- no sigma atomics, and the FP64 order is the oracle's, so FP64
 //           sigma is bit-exact.  (Codes/kernels_free.cu:286-362 computes the
 //           same quantities one source per block with atomics.)
+// From a wide frontier (bottom_up) the expand makes the hubs' masks alone; the
+// pull takes every vertex with sources left to reach and keeps those that have
+// a neighbour at level l.
 // Backward level l: rho_v = sum over successors w of t_w, with
 // rho = delta / sigma, so the successor-method term
 // sigma_v/sigma_w (r(w)+1 + delta_w) (Codes/kernels_free.cu:378-421) becomes a
@@ -370,6 +373,17 @@ __device__ __forceinline__ bool seed_pending(const BatchDev &b, int l) {
     return __ballot(p) != 0;
 }
 
+// Whether level l+1 is found bottom-up: from a frontier of more than a
+// sixteenth of the vertices a tile reaches most vertices on the next level, so
+// the pull would walk their arcs anyway, and the expand's atomics (up to W per
+// arc) are saved.  Per tile on a 168k-vertex power-law core and an R-MAT core
+// of 165k (expands, pulls): 710 + 1293 us and 1223 + 1615 pushed, 186 + 1333
+// and 231 + 1626 so; 6144 sources 53.4 -> 44.7 ms and 100.9 -> 87.4.  Line at
+// n / 4: 45.4 and 90.8 ms, n / 8: 44.9 and 88.5, n / 32: 44.4 and 86.9, where
+// a frontier that stays narrow for many levels would be walked for too long.
+constexpr int UP_FRONTIER = 16;
+__device__ __forceinline__ bool bottom_up(const BatchDev &b, int q0, int q1) { return q1 - q0 > b.n / UP_FRONTIER; }
+
 // Level l: Q_l = Q[qoff[l], ctr[0]).  Records qoff[l+1]; an empty Q_l with
 // no pending injection ends the forward with depth l-1.  Clears Q_{l-1} from
 // mask array (l+2)%3.
@@ -406,6 +420,28 @@ __global__ __launch_bounds__(BB) void k_b_expand(BatchDev b, int l) {
             if (K - j == l + 1) push<W>(b, dst, b.ch_R[c], mbit<W>(h, lane));
         }
     }
+    const uint64_t *cur = mbuf(b, l);
+    if (bottom_up(b, q0, q1)) {
+        // the pull finds the sources of the other vertices; a hub's are found
+        // here, as its slices share them
+        for (int s = gwave(); s < b.n_slice; s += nwaves()) {
+            const int v = b.hub_v[b.sl_hub[s]];
+            Msk<W> F = mzero<W>();
+            for (int j = b.sl_j0[s] + lane; j < b.sl_j1[s]; j += 64) {
+                const int w = b.col[j];
+                if (w < 0) continue;
+                const Msk<W> x = mld<W>(cur, w);
+#pragma unroll
+                for (int h = 0; h < W; ++h) F.m[h] |= x.m[h];
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+                for (int h = 0; h < W; ++h) F.m[h] |= __shfl_xor((unsigned long long)F.m[h], o, 64);
+            if (lane == 0) push<W>(b, dst, v, F);
+        }
+        return;
+    }
     // lane k of group g takes entry g + k G of the level: the list follows the
     // vertex ids, whose heavy rows lie together, and a wave walks its entries
     // above SMALL arcs one after another (168k-vertex power-law core, a tile's
@@ -440,7 +476,6 @@ __global__ __launch_bounds__(BB) void k_b_expand(BatchDev b, int l) {
         }
     }
     // hub slices: the hub's level-l sources are its mask in mb[l%3]
-    const uint64_t *cur = mbuf(b, l);
     for (int s = gwave(); s < b.n_slice; s += nwaves()) {
         const int v = b.hub_v[b.sl_hub[s]];
         const Msk<W> F = mld<W>(cur, v);
@@ -454,13 +489,13 @@ __global__ __launch_bounds__(BB) void k_b_expand(BatchDev b, int l) {
 
 // --------------------------------------------------------------- pull ---
 // sigma_w for the sources N of entry w: the sum over neighbours at level l
-// (fr) in CSR order.  A contracted chain's arc (~c) counts 1 for the source
+// (fr) in CSR order; `seen` gets the lane's sources that had one.  A contracted chain's arc (~c) counts 1 for the source
 // of word h whose chain is c and that is injected at w on this level
 // (sc[h] == c); cm holds the tile's chain sources.
 template <int SM, int W>
 __device__ __forceinline__ void sigma_sum(const BatchDev &b, const uint64_t *fr, const Msk<W> &N, int a0, int a1,
-                                          SgW<SM> (&acc)[W], double (&facc)[W], bool &ovf, const int (&sc)[W],
-                                          const Msk<W> &cm) {
+                                          SgW<SM> (&acc)[W], double (&facc)[W], bool &ovf, int &seen,
+                                          const int (&sc)[W], const Msk<W> &cm) {
     // gathers in flight (W words each): 2 at W = 4, where 4 in flight cost
     // the pull a wave per SIMD (measured 165.0k against 175.2k MTEPS on the
     // 1M-vertex mixed graph, 276.9k against 295.2k on R-MAT)
@@ -503,6 +538,8 @@ __device__ __forceinline__ void sigma_sum(const BatchDev &b, const uint64_t *fr,
                     }
                 }
             }
+#pragma unroll
+            for (int u = 0; u < UW; ++u) seen |= use[u];
 #pragma unroll
             for (int u = 0; u < UW; ++u)
 #pragma unroll
@@ -548,7 +585,7 @@ __global__ __launch_bounds__(BB) void k_b_pull(BatchDev b, int l) {
     __shared__ Msk<W> s_m[NW][STAGE];
     if (ldi(&b.ctr[3]) >= 0) return;
     const uint64_t *fr = mbuf(b, l);
-    const uint64_t *nx = mbuf(b, l + 1);
+    uint64_t *nx = mbuf(b, l + 1);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const uint64_t me = 1ull << lane;
     const bool split = !F64 && b.n_hub > 0;
@@ -568,10 +605,23 @@ __global__ __launch_bounds__(BB) void k_b_pull(BatchDev b, int l) {
         if (j == l + 1) mL[h] = b.ch_L[myc[h]];
         if (K - j == l + 1) mR[h] = b.ch_R[myc[h]];
     }
+    // bottom-up, a vertex's candidates are the tile's sources that have not
+    // reached it, and those that had a neighbour at level l remain
+    const bool up = bottom_up(b, b.qoff[l], b.qoff[l + 1]);
+    const int ns = b.ctr[5];
     int cnt = 0;  // wave-uniform
     for (int c = gwave(); c < b.n_chunk; c += nwaves()) {
         const int w0 = b.chunk[c] + lane;
-        const Msk<W> N0 = w0 < b.chunk[c + 1] ? mld<W>(nx, w0) : mzero<W>();
+        const bool in = w0 < b.chunk[c + 1];
+        Msk<W> N0 = in ? mld<W>(nx, w0) : mzero<W>();
+        if (up && in && !is_hub(b, b.rp[w0 + 1] - b.rp[w0])) {
+            const Msk<W> vis = mld<W>(b.vis, w0);
+#pragma unroll
+            for (int h = 0; h < W; ++h) {
+                const int m = ns - 64 * h;
+                N0.m[h] = ~vis.m[h] & (m >= 64 ? ~0ull : (m > 0 ? (1ull << m) - 1 : 0ull));
+            }
+        }
         const uint64_t bal = __ballot(many<W>(N0));
         if (!bal) continue;
         const int k0 = cnt;
@@ -588,6 +638,7 @@ __global__ __launch_bounds__(BB) void k_b_pull(BatchDev b, int l) {
         cnt += __popcll(bal);
         __builtin_amdgcn_wave_barrier();
         uint64_t rest = bal;
+        int out = k0;
         for (int k = k0; k < cnt; ++k) {
             const int src = __ffsll((long long)rest) - 1;
             rest &= rest - 1;
@@ -599,9 +650,10 @@ __global__ __launch_bounds__(BB) void k_b_pull(BatchDev b, int l) {
             for (int h = 0; h < W; ++h) N.m[h] = uni64(s_m[wv][k].m[h]);
             const int a0 = bcast(r0, src), a1 = bcast(r1, src);
             const int ew = bcast(e0, src);
-            const int pb = mbits<W>(N, lane);
+            const bool hub = is_hub(b, a1 - a0);
+            int pb = mbits<W>(N, lane);
             const int64_t cell = ((int64_t)w * 64 + lane) * W;
-            if (!(split && is_hub(b, a1 - a0))) {
+            if (!(split && hub)) {
                 SgW<SM> acc[W];
                 double facc[W];
                 int sc[W];
@@ -612,7 +664,15 @@ __global__ __launch_bounds__(BB) void k_b_pull(BatchDev b, int l) {
                     sc[h] = (w == mL[h] || w == mR[h]) ? myc[h] : -1;
                 }
                 bool ovf = false;
-                sigma_sum<SM, W>(b, fr, N, a0, a1, acc, facc, ovf, sc, cm);
+                int seen = 0;
+                sigma_sum<SM, W>(b, fr, N, a0, a1, acc, facc, ovf, seen, sc, cm);
+                if (up && !hub) {
+                    pb = seen;
+#pragma unroll
+                    for (int h = 0; h < W; ++h) N.m[h] = __ballot((seen >> h) & 1);
+                    if (!many<W>(N)) continue;
+                    if (lane == 0) mst<W>(nx, w, N);
+                }
 #pragma unroll
                 for (int h = 0; h < W; ++h) {
                     if (!((pb >> h) & 1)) continue;
@@ -629,7 +689,14 @@ __global__ __launch_bounds__(BB) void k_b_pull(BatchDev b, int l) {
             if (lane == 0)
 #pragma unroll
                 for (int h = 0; h < W; ++h) b.vis[(int64_t)w * W + h] |= N.m[h];
+            if (up && lane == 0) {  // (candidates without a neighbour drop out)
+                s_w[wv][out] = w;
+                s_m[wv][out] = N;
+            }
+            ++out;
         }
+        cnt = out;
+        __builtin_amdgcn_wave_barrier();
         if (cnt >= STAGE_FLUSH) stage_flush<W>(b, s_w[wv], s_m[wv], cnt, lane);
     }
     stage_flush<W>(b, s_w[wv], s_m[wv], cnt, lane);
@@ -653,7 +720,8 @@ __global__ __launch_bounds__(BB) void k_b_pull(BatchDev b, int l) {
             sc[h] = (v == mL[h] || v == mR[h]) ? myc[h] : -1;
         }
         bool ovf = false;
-        sigma_sum<SI, W>(b, fr, N, b.sl_j0[s], b.sl_j1[s], acc, facc, ovf, sc, cm);
+        int seen = 0;
+        sigma_sum<SI, W>(b, fr, N, b.sl_j0[s], b.sl_j1[s], acc, facc, ovf, seen, sc, cm);
         const int pb = mbits<W>(N, lane);
 #pragma unroll
         for (int h = 0; h < W; ++h) {
