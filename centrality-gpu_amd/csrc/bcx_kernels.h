@@ -44,6 +44,7 @@ struct PlainArgs {
     const int32_t *slots;  // chain only: [2*count] row slots of L and R
     int32_t count;
     int32_t split;         // bfs: copies of the BC accumulator (bc holds split * n words)
+    int32_t sweep;         // 1: dependencies are added to bc in vertex order (plain_sweep)
     int32_t sigma_f64;     // 1: FP64 sigma by pull
     int32_t fp32;          // bfs: compensated FP32 terms (with integer sigma; no MODE_ROW)
     uint64_t limit;        // u64 overflow threshold (0 = 2^64)
@@ -59,6 +60,7 @@ struct PlainShape {
     bool lds_codes;
 };
 PlainShape plain_shape(int32_t n, bool fp32);
+bool plain_sweep(int32_t n, int64_t arcs);
 
 hipError_t launch_plain_bfs(const CompDev &c, const PlainArgs &a, const PlainScratch &sc,
                             const Rows &rows, const PlainShape &p, int grid, hipStream_t st);

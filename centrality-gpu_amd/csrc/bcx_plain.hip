@@ -134,6 +134,7 @@ struct PlainCtx {
     Codes<LG> lv;
     uint64_t *sg;   // path counts
     TT *tt;         // terms (FP64: the same words as sg, unless sg is kept)
+    double *dl;     // dependencies of the source, when they are added in vertex order
     int32_t *S;     // vertices in level order
     int32_t *off;   // level offsets past LDS_LEVELS
     int32_t *drow;  // levels, when the source's row is kept
@@ -489,11 +490,20 @@ __device__ __forceinline__ void plain_backward(const PlainCtx<LG, TT> &x, int ma
                 const double sum = rho.value();
                 const double delta = sv * sum;
                 x.tt[v] = (TT)(((double)rv + 1.0) / sv + sum);
-                if (delta != 0.0) unsafeAtomicAdd(&bc[v], ws * delta);
+                if (x.dl) x.dl[v] = delta;
+                else if (delta != 0.0) unsafeAtomicAdd(&bc[v], ws * delta);
                 if (probe) probe[v] = delta;
             }
         }
         pbarrier();
+    }
+    if (!x.dl) return;
+    // added in vertex order: neighbouring lanes' atomics share a line
+    if (tid == 0) x.dl[x.S[0]] = 0.0;
+    pbarrier();
+    for (int v = tid; v < x.n; v += nt) {
+        const double delta = x.dl[v];
+        if (delta != 0.0) unsafeAtomicAdd(&bc[v], ws * delta);
     }
 }
 
@@ -539,6 +549,7 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_bfs(CompDev c, PlainArgs a
         const bool row = mode & MODE_ROW;
         x.sg = row ? rows.sig + (int64_t)slot * rows.stride : sc.sig + base;
         x.tt = row || sizeof(TT) == 4 ? (TT *)(sc.dl + base) : (TT *)x.sg;
+        x.dl = row || !a.sweep ? nullptr : (sizeof(TT) == 4 ? (double *)x.sg : sc.dl + base);
         x.drow = row ? rows.d + (int64_t)slot * rows.stride : nullptr;
         const int maxlvl = plain_forward<F64>(x, s, a.limit);
         if (!F64 && maxlvl < 0) {
@@ -569,6 +580,7 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev 
     x.sh = &sh;
     x.sg = sg;
     x.tt = a.probe ? a.probe + c.n : (double *)sg;
+    x.dl = nullptr;
     x.drow = nullptr;
     while (true) {
         if (tid == 0) {
@@ -694,6 +706,16 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev 
         pbarrier();
     }
 }
+
+// Whether the sources' dependencies are stored and added to BC in vertex order,
+// a line's atomics together, instead of one by one as the backward makes them.
+// Sparse components have an atomic per few arcs (a grid of 26k: 330M for 16384
+// sources, two thirds of the bytes written); the row of dependencies costs cache
+// that larger components need.  One by one / in order: grids of 3.7k, 11k, 18.6k,
+// 22k and 26k vertices 1431 / 1261, 2553 / 2283, 3516 / 3176, 3973 / 3939 and
+// 25900 / 31000 us; power-law cores of 12.7k and 16.9k 1857 / 1894 and 2357 /
+// 2538; R-MAT core of 12k 7890 / 8084.
+bool plain_sweep(int32_t n, int64_t arcs) { return n <= 20000 && arcs <= 5 * (int64_t)n; }
 
 // Waves per source by the component's size: a barrier per level against the
 // vertices a level gives the waves.  4 / 8 / 16 waves (us; k sources): grid of

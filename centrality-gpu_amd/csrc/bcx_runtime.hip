@@ -392,6 +392,7 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
     a.bc = bc;
     a.probe = probe;
     a.fp32 = fp32;
+    a.sweep = plain_sweep(dc.n, dc.arcs);
     // Thousands of sources add into SPLIT copies of the accumulator, folded
     // afterwards: a vertex's sum is then SPLIT times shorter, and its rounding
     // error what the tiled kernels' is, which add a tile's sources first (16384

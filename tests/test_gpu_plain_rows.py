@@ -90,3 +90,20 @@ def test_deep(engine, n):
         assert st["max_level"] > 1024
         mx, _, zeros = relerr(got, want)
         assert mx < 1e-9 and zeros, (n, chains, mx)
+
+
+@pytest.mark.parametrize("n,chords", [(2500, 100), (2500, 3750), (2500, 3760), (20000, 900), (20001, 900)])
+@pytest.mark.parametrize("prec", [bcx.PREC_FP64, bcx.PREC_FP32C])
+def test_dependencies_in_vertex_order(engine, n, chords, prec):
+    """Sparse components up to 20000 vertices and 5 arcs per vertex add a
+    source's dependencies in vertex order; one over either line adds them one by
+    one.  Ragged source lists, the whole list twice (rows are used again)."""
+    c = csr(n, ring(n, chords, n + chords))
+    sub = np.unique(np.linspace(0, n - 1, 601).astype(np.int64))
+    want = oracle.component_bc(c.row_ptr, c.col, c.reach, sources=sub.astype(np.int32))
+    path = bcx.PATH_PLAIN if prec == bcx.PREC_FP64 else bcx.PATH_BATCHED
+    tol = 1e-9 if prec == bcx.PREC_FP64 else 1e-6
+    for _ in range(2):
+        (got,), st = engine.bc([c], subset=sub, path=path, precision=prec, flags=bcx.FLAG_NO_TUNE)
+        mx, _, zeros = relerr(got, want)
+        assert mx < tol and zeros, (n, chords, prec, mx)
