@@ -58,17 +58,21 @@ constexpr int NW = BB / 64;    // waves per block
 constexpr int UNR = 8;         // gathers in flight per lane in the sum loops (fewer for W = 4)
 constexpr int SMALL = 16;      // degree up to which one lane expands an entry
 // The level kernels wait on dependent gathers, so waves per SIMD (occupancy,
-// set by VGPRs and LDS per block) decide their speed.  The staging and window
-// sizes keep both kernels' LDS at <= 13.3 KB per block (12 blocks per CU);
-// uniform values live in scalar registers (readlane / readfirstlane), u32
-// counts in 32-bit registers, and the chain terms are made by their own
-// kernel, so with u32 counts and FP32 terms both kernels fit 80 VGPRs: 6
-// waves per SIMD.  On the 1M-vertex mixed graph: 176.1k MTEPS at 4 waves,
-// 198.6k at 5 (188.9k with the pull alone at 5), 221.7k at 6 (215.7k with
-// the same registers at 5).
+// set by VGPRs and LDS per block) decide their speed.  The staging keeps the
+// pull's LDS at <= 13.3 KB per block (12 blocks per CU), the backward's sums
+// take 8.2; uniform values live in scalar registers (readlane /
+// readfirstlane), u32 counts in 32-bit registers, and the chain terms are made
+// by their own kernel, so with u32 counts and FP32 terms both kernels fit 80
+// VGPRs: 6 waves per SIMD.  On the 1M-vertex mixed graph: 176.1k MTEPS at 4
+// waves, 198.6k at 5 (188.9k with the pull alone at 5), 221.7k at 6 (215.7k
+// with the same registers at 5).  With eight tiles in flight the vector ALUs are
+// busy half the time beside 2.1 TB/s of random lines, so the per-arc
+// instructions count too: source masks as scalar lane predicates (lane_in), not
+// 64-bit shifts by the lane, and the backward's triples read from their lanes,
+// not through a list in LDS, took 6144 sources of a 168k-vertex power-law core
+// from 44.6 to 42.5 ms and of a 165k-vertex R-MAT core from 87.1 to 84.2.
 constexpr int STAGE = 176, STAGE_FLUSH = 112;  // pull: list entries staged per wave, flush point
 constexpr int FEB = 8;         // list entries per wave block in the backward
-constexpr int WIN = 64;        // arcs per compaction window of a backward block
 
 __device__ __forceinline__ int gwave() { return (int)((blockIdx.x * (unsigned)blockDim.x + threadIdx.x) >> 6); }
 __device__ __forceinline__ int nwaves() { return (int)((gridDim.x * (unsigned)blockDim.x) >> 6); }
@@ -142,6 +146,25 @@ __device__ __forceinline__ int mbits(const Msk<W> &a, int k) {
     int r = 0;
 #pragma unroll
     for (int h = 0; h < W; ++h) r |= (int)((a.m[h] >> k) & 1) << h;
+    return r;
+}
+// Whether lane k is in a wave-uniform lane mask (bit k): the mask in scalar
+// registers is the predicate, where a shift by the lane would be a 64-bit
+// vector operation per word.
+__device__ __forceinline__ bool lane_in(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+template <int W>
+__device__ __forceinline__ uint64_t mall(const Msk<W> &a) {  // lanes with any source in a
+    uint64_t x = 0;
+#pragma unroll
+    for (int h = 0; h < W; ++h) x |= a.m[h];
+    return x;
+}
+// a mask that every lane holds, in scalar registers
+template <int W>
+__device__ __forceinline__ Msk<W> muni(const Msk<W> &a) {
+    Msk<W> r;
+#pragma unroll
+    for (int h = 0; h < W; ++h) r.m[h] = uni64(a.m[h]);
     return r;
 }
 template <int W>
@@ -494,12 +517,12 @@ __global__ __launch_bounds__(BB) void k_b_expand(BatchDev b, int l) {
 // (sc[h] == c); cm holds the tile's chain sources.
 template <int SM, int W>
 __device__ __forceinline__ void sigma_sum(const BatchDev &b, const uint64_t *fr, const Msk<W> &N, int a0, int a1,
-                                          SgW<SM> (&acc)[W], double (&facc)[W], bool &ovf, int &seen,
+                                          SgW<SM> (&acc)[W], double (&facc)[W], bool &ovf, Msk<W> &seen,
                                           const int (&sc)[W], const Msk<W> &cm) {
-    // gathers in flight (W words each): 2 at W = 4, where 4 in flight cost
-    // the pull a wave per SIMD (measured 165.0k against 175.2k MTEPS on the
-    // 1M-vertex mixed graph, 276.9k against 295.2k on R-MAT)
-    constexpr int UW = W == 4 ? UNR / 4 : UNR;
+    // gathers in flight (W words each): at W = 4, 1, 2, 3 and 4 ran 6144 sources
+    // of a 168k-vertex power-law core in 45.4, 43.4, 42.9 and 42.7 ms (78 VGPRs
+    // at 4; more would cost a wave per SIMD)
+    constexpr int UW = W == 1 ? UNR : (W == 2 ? UNR / (SM == SIG_U64 ? 2 : 1) : (SM == SIG_U32 ? UNR / 2 : UNR / 4));
     const int lane = threadIdx.x & 63;
     for (int c = a0; c < a1; c += 64) {
         const int j = c + lane;
@@ -512,43 +535,38 @@ __device__ __forceinline__ void sigma_sum(const BatchDev &b, const uint64_t *fr,
         uint64_t bal = __ballot(many<W>(f));
         while (bal) {
             SgW<SM> x[UW][W];
-            int use[UW];
+            Msk<W> use[UW];
 #pragma unroll
             for (int u = 0; u < UW; ++u) {
-                use[u] = 0;
+                use[u] = mzero<W>();
 #pragma unroll
                 for (int h = 0; h < W; ++h) x[u][h] = 0;
                 if (bal) {
                     const int src = __ffsll((long long)bal) - 1;
                     bal &= bal - 1;
                     const int vv = bcast(v, src);
-                    const int pb = mbits<W>(mshfl<W>(f, src), lane);
-                    if (pb) {
-                        if (vv >= 0) {
-                            use[u] = pb;
-                            sg_row<SM, W>(b, (int64_t)vv * 64 + lane, x[u]);
-                        } else {
+                    use[u] = mshfl<W>(f, src);
+                    if (vv >= 0) {
+                        if (lane_in(mall<W>(use[u]))) sg_row<SM, W>(b, (int64_t)vv * 64 + lane, x[u]);
+                    } else {
 #pragma unroll
-                            for (int h = 0; h < W; ++h)
-                                if (((pb >> h) & 1) && ~vv == sc[h]) {
-                                    use[u] |= 1 << h;
-                                    x[u][h] = (SgW<SM>)(SM == SIG_F64 ? d2u(1.0) : 1ull);
-                                }
+                        for (int h = 0; h < W; ++h) {
+                            use[u].m[h] = __ballot(lane_in(use[u].m[h]) && ~vv == sc[h]);
+                            x[u][h] = (SgW<SM>)(SM == SIG_F64 ? d2u(1.0) : 1ull);
                         }
                     }
                 }
             }
 #pragma unroll
-            for (int u = 0; u < UW; ++u) seen |= use[u];
-#pragma unroll
             for (int u = 0; u < UW; ++u)
 #pragma unroll
                 for (int h = 0; h < W; ++h) {
-                    if (!((use[u] >> h) & 1)) continue;
+                    seen.m[h] |= use[u].m[h];
+                    const SgW<SM> y = lane_in(use[u].m[h]) ? x[u][h] : 0;
                     if (SM == SIG_F64) {
-                        facc[h] += u2d(x[u][h]);
+                        facc[h] += u2d(y);
                     } else {
-                        const SgW<SM> s = acc[h] + x[u][h];  // (wrap: the word overflowed)
+                        const SgW<SM> s = acc[h] + y;  // (wrap: the word overflowed)
                         ovf |= (s < acc[h]);
                         acc[h] = s;
                     }
@@ -651,7 +669,6 @@ __global__ __launch_bounds__(BB) void k_b_pull(BatchDev b, int l) {
             const int a0 = bcast(r0, src), a1 = bcast(r1, src);
             const int ew = bcast(e0, src);
             const bool hub = is_hub(b, a1 - a0);
-            int pb = mbits<W>(N, lane);
             const int64_t cell = ((int64_t)w * 64 + lane) * W;
             if (!(split && hub)) {
                 SgW<SM> acc[W];
@@ -664,25 +681,23 @@ __global__ __launch_bounds__(BB) void k_b_pull(BatchDev b, int l) {
                     sc[h] = (w == mL[h] || w == mR[h]) ? myc[h] : -1;
                 }
                 bool ovf = false;
-                int seen = 0;
+                Msk<W> seen = mzero<W>();
                 sigma_sum<SM, W>(b, fr, N, a0, a1, acc, facc, ovf, seen, sc, cm);
                 if (up && !hub) {
-                    pb = seen;
-#pragma unroll
-                    for (int h = 0; h < W; ++h) N.m[h] = __ballot((seen >> h) & 1);
+                    N = seen;
                     if (!many<W>(N)) continue;
                     if (lane == 0) mst<W>(nx, w, N);
                 }
 #pragma unroll
                 for (int h = 0; h < W; ++h) {
-                    if (!((pb >> h) & 1)) continue;
+                    if (!lane_in(N.m[h])) continue;
                     sg_put<SM>(b, cell + h, F64 ? d2u(facc[h]) : acc[h]);
                     if (!F64 && (ovf || acc[h] > sg_max<SM>() || (b.limit && acc[h] >= b.limit))) b.ctr[1] = 1;
                 }
             }
 #pragma unroll
             for (int h = 0; h < W; ++h) {
-                if (!((pb >> h) & 1)) continue;
+                if (!lane_in(N.m[h])) continue;
                 if (b.lvl) b.lvl[cell + h] = l + 1;
                 if (ew >= 0) b.ep_lvl[((int64_t)ew * 64 + lane) * W + h] = l + 1;
             }
@@ -720,7 +735,7 @@ __global__ __launch_bounds__(BB) void k_b_pull(BatchDev b, int l) {
             sc[h] = (v == mL[h] || v == mR[h]) ? myc[h] : -1;
         }
         bool ovf = false;
-        int seen = 0;
+        Msk<W> seen = mzero<W>();
         sigma_sum<SI, W>(b, fr, N, b.sl_j0[s], b.sl_j1[s], acc, facc, ovf, seen, sc, cm);
         const int pb = mbits<W>(N, lane);
 #pragma unroll
@@ -818,25 +833,25 @@ __device__ __forceinline__ void rho_sum(const BatchDev &b, const uint64_t *succ,
         uint64_t bal = __ballot(many<W>(x));
         while (bal) {
             TT t[UW][W];
-            int use[UW];
+            Msk<W> use[UW];
 #pragma unroll
             for (int u = 0; u < UW; ++u) {
-                use[u] = 0;
+                use[u] = mzero<W>();
 #pragma unroll
                 for (int h = 0; h < W; ++h) t[u][h] = 0;
                 if (bal) {
                     const int src = __ffsll((long long)bal) - 1;
                     bal &= bal - 1;
                     const int ww = bcast(w, src);
-                    use[u] = mbits<W>(mshfl<W>(x, src), lane);
-                    if (use[u]) tt_row<TT, W>(b, (int64_t)ww * 64 + lane, t[u]);
+                    use[u] = mshfl<W>(x, src);
+                    if (lane_in(mall<W>(use[u]))) tt_row<TT, W>(b, (int64_t)ww * 64 + lane, t[u]);
                 }
             }
 #pragma unroll
             for (int u = 0; u < UW; ++u)
 #pragma unroll
                 for (int h = 0; h < W; ++h)
-                    if ((use[u] >> h) & 1) acc[h].add(t[u][h]);
+                    if (lane_in(use[u].m[h])) acc[h].add(t[u][h]);
         }
     }
 #pragma unroll
@@ -873,9 +888,6 @@ __device__ __forceinline__ void finish_vertex(const BatchDev &b, int v, int l, c
 template <int SM, typename TT, int W>
 __global__ __launch_bounds__(BB) void k_b_back(BatchDev b, int l) {
     constexpr bool F64 = SM == SIG_F64;
-    __shared__ int t_w[NW][WIN];
-    __shared__ Msk<W> t_x[NW][WIN];
-    __shared__ int t_k[NW][WIN];
     // entries per wave block: FEB / W, so a block holds FEB * 64 (entry, source) pairs
     constexpr int EB = FEB / W;
     constexpr int UW = W == 4 ? UNR / 2 : UNR;
@@ -892,13 +904,12 @@ __global__ __launch_bounds__(BB) void k_b_back(BatchDev b, int l) {
     uint64_t *clr = mbuf(b, l + 2);
     for (int i = c0 + blockIdx.x * BB + threadIdx.x; i < c1; i += gridDim.x * BB) mst<W>(clr, b.Q[i], mzero<W>());
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const uint64_t me = 1ull << lane;
     using Acc = typename std::conditional<sizeof(TT) == 4, KahanF, SumD>::type;
     // Blocks of EB list entries per wave.  The arcs of the block are walked
-    // as one flat range (lane per arc) in windows of WIN: successor masks
-    // are gathered for 64 arcs at once and the (entry, successor, sources)
-    // triples that matter are compacted in LDS; the t rows of those triples
-    // are then gathered UW at a time, accumulated per entry in arc order.
+    // as one flat range, a lane per arc: successor masks are gathered for 64
+    // arcs at once, and the t rows of the (entry, successor, sources) triples
+    // that matter, read from their lanes, UW at a time, accumulated per entry
+    // in arc order.
     for (int base = q0 + gwave() * EB; base < q1; base += nwaves() * EB) {
         const int e = base + lane;
         int v0 = 0, r0 = 0, r1 = 0, ep0 = -1;
@@ -938,53 +949,43 @@ __global__ __launch_bounds__(BB) void k_b_back(BatchDev b, int l) {
         }
         Acc acc[W];
         int kcur = -1;
-        for (int win = 0; win < T; win += WIN) {
-            const int wend = min(T, win + WIN);
-            int nrel = 0;
-            for (int c = win; c < wend; c += 64) {
-                const int g = c + lane;
-                int k = 0;
+        for (int win = 0; win < T; win += 64) {
+            const int g = win + lane;
+            int k = 0;
 #pragma unroll
-                for (int j = 1; j < EB; ++j) k += (P[j] <= g);
-                int a0k = A[0], pk = P[0];
-                Msk<W> mk = MM[0];
+            for (int j = 1; j < EB; ++j) k += (P[j] <= g);
+            int a0k = A[0] - P[0];
+            Msk<W> mk = MM[0];
 #pragma unroll
-                for (int j = 1; j < EB; ++j)
-                    if (k == j) {
-                        a0k = A[j];
-                        pk = P[j];
-                        mk = MM[j];
-                    }
-                int w = 0;
-                Msk<W> x = mzero<W>();
-                if (g < wend) {
-                    w = b.col[a0k + g - pk];
-                    if (w >= 0) x = mand<W>(mld<W>(succ, w), mk);  // (w < 0: a contracted chain)
+            for (int j = 1; j < EB; ++j)
+                if (k == j) {
+                    a0k = A[j] - P[j];
+                    mk = MM[j];
                 }
-                const uint64_t bal = __ballot(many<W>(x));
-                if (many<W>(x)) {
-                    const int pos = nrel + __popcll(bal & (me - 1));
-                    t_w[wv][pos] = w;
-                    t_x[wv][pos] = x;
-                    t_k[wv][pos] = k;
-                }
-                nrel += __popcll(bal);
+            int w = 0;
+            Msk<W> x = mzero<W>();
+            if (g < T) {
+                w = b.col[a0k + g];
+                if (w >= 0) x = mand<W>(mld<W>(succ, w), mk);  // (w < 0: a contracted chain)
             }
-            __builtin_amdgcn_wave_barrier();
-            for (int r = 0; r < nrel; r += UW) {
+            uint64_t bal = __ballot(many<W>(x));
+            while (bal) {
                 TT t[UW][W];
-                int kk[UW], use[UW];
+                int kk[UW];
+                Msk<W> use[UW];
 #pragma unroll
                 for (int u = 0; u < UW; ++u) {
-                    const int rr = r + u;
-                    use[u] = 0;
+                    use[u] = mzero<W>();
                     kk[u] = -1;
 #pragma unroll
                     for (int h = 0; h < W; ++h) t[u][h] = 0;
-                    if (rr < nrel) {
-                        kk[u] = __builtin_amdgcn_readfirstlane(t_k[wv][rr]);  // (uniform: a scalar register)
-                        use[u] = mbits<W>(t_x[wv][rr], lane);
-                        if (use[u]) tt_row<TT, W>(b, (int64_t)t_w[wv][rr] * 64 + lane, t[u]);
+                    if (bal) {
+                        const int src = __ffsll((long long)bal) - 1;
+                        bal &= bal - 1;
+                        kk[u] = bcast(k, src);
+                        const int ww = bcast(w, src);
+                        use[u] = mshfl<W>(x, src);
+                        if (lane_in(mall<W>(use[u]))) tt_row<TT, W>(b, (int64_t)ww * 64 + lane, t[u]);
                     }
                 }
 #pragma unroll
@@ -1000,10 +1001,9 @@ __global__ __launch_bounds__(BB) void k_b_back(BatchDev b, int l) {
                     }
 #pragma unroll
                     for (int h = 0; h < W; ++h)
-                        if ((use[u] >> h) & 1) acc[h].add(t[u][h]);
+                        if (lane_in(use[u].m[h])) acc[h].add(t[u][h]);
                 }
             }
-            __builtin_amdgcn_wave_barrier();
         }
         if (kcur >= 0)
 #pragma unroll
@@ -1012,10 +1012,9 @@ __global__ __launch_bounds__(BB) void k_b_back(BatchDev b, int l) {
 #pragma unroll
         for (int j = 0; j < EB; ++j) {
             if (!OWN[j] || EP[j] < 0) continue;
-            const int pb = mbits<W>(MM[j], lane);
 #pragma unroll
             for (int h = 0; h < W; ++h)
-                if ((pb >> h) & 1) r_rho[wv][j][h * 64 + lane] += b.ep_rho[((int64_t)EP[j] * 64 + lane) * W + h];
+                if (lane_in(MM[j].m[h])) r_rho[wv][j][h * 64 + lane] += b.ep_rho[((int64_t)EP[j] * 64 + lane) * W + h];
         }
         // finish every entry of the block (hubs excepted): sigma rows first
         SgW<SM> SX[EB][W];
@@ -1023,17 +1022,16 @@ __global__ __launch_bounds__(BB) void k_b_back(BatchDev b, int l) {
         for (int j = 0; j < EB; ++j) {
 #pragma unroll
             for (int h = 0; h < W; ++h) SX[j][h] = 0;
-            if (OWN[j] && mbits<W>(MM[j], lane)) sg_row<SM, W>(b, (int64_t)V[j] * 64 + lane, SX[j]);
+            if (OWN[j] && lane_in(mall<W>(MM[j]))) sg_row<SM, W>(b, (int64_t)V[j] * 64 + lane, SX[j]);
         }
 #pragma unroll
         for (int j = 0; j < EB; ++j) {
             if (!OWN[j]) continue;
             const int v = V[j];
-            const int pb = mbits<W>(MM[j], lane);
             double contrib = 0.0;
 #pragma unroll
             for (int h = 0; h < W; ++h) {
-                if (!((pb >> h) & 1)) continue;
+                if (!lane_in(MM[j].m[h])) continue;
                 const int64_t cell = ((int64_t)v * 64 + lane) * W + h;
                 const double sv = sg_val<SM>(SX[j][h]);
                 const double a = r_rho[wv][j][h * 64 + lane];  // rho_v
