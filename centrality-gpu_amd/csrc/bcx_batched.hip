@@ -66,7 +66,7 @@ constexpr int SMALL = 16;      // degree up to which one lane expands an entry
 // VGPRs: 6 waves per SIMD.  On the 1M-vertex mixed graph: 176.1k MTEPS at 4
 // waves, 198.6k at 5 (188.9k with the pull alone at 5), 221.7k at 6 (215.7k
 // with the same registers at 5).  With eight tiles in flight the vector ALUs are
-// busy half the time beside 2.1 TB/s of random lines, so the per-arc
+// busy half the time beside 3.9 TB/s of L2-fabric lines (a large copy: 4.6), so the per-arc
 // instructions count too: source masks as scalar lane predicates (lane_in), not
 // 64-bit shifts by the lane, and the backward's triples read from their lanes,
 // not through a list in LDS, took 6144 sources of a 168k-vertex power-law core

@@ -22,7 +22,9 @@
 // core, the same with 256 and 512 sources in flight), and the dependent loads
 // per level on deep graphs.  Against level words, list marks and count atomics
 // in global memory with a lane per vertex: 1000 sources of the 84k core 165 ->
-// 19 ms, 2049 sources of an 18.6k grid 27.4 -> 5.1 ms.
+// 19 ms, 2049 sources of an 18.6k grid 27.4 -> 5.1 ms; with chain sources run
+// directly, the core's BFS-ordered copy and dependencies added in vertex order
+// 11.5 and 3.2 ms.
 //
 // A wave takes 64 vertices of a level.  Short rows are walked by a lane each,
 // four arcs per step; longer ones as one flat range with a lane per arc, whose
