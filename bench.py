@@ -87,7 +87,7 @@ def copy_probe(mib):
     print(json.dumps({"copy_probe_mib": mib, "copies": 3}))
 
 
-BATCHED_KERNELS = ("bcx::k_b_", "bcx::k_small", "bcx::k_wg", "bcx::k_na_")
+BATCHED_KERNELS = ("bcx::k_b_", "bcx::k_src", "bcx::k_small", "bcx::k_plain", "bcx::k_wg", "bcx::k_na_")
 
 
 def _union(iv):
@@ -346,7 +346,7 @@ def main():
                      "launches_per_step": round(launches, 1),
                      "algorithmic_bytes_per_step": round(balg_b / K),
                      "kernel": "batched kernels of a step (k_b_expand, k_b_pull, k_b_back, the chain kernels; "
-                               "k_small; k_wg)"},
+                               "k_src; k_small; k_plain_bfs; k_wg)"},
         "cpu_baseline": cpu,
     }
     g.free()

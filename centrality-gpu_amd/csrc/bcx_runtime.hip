@@ -393,14 +393,14 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
     a.probe = probe;
     a.fp32 = fp32;
     a.sweep = plain_sweep(dc.n, dc.arcs);
-    // Thousands of sources add into SPLIT copies of the accumulator, folded
+    // Hundreds of sources and more add into SPLIT copies of the accumulator, folded
     // afterwards: a vertex's sum is then SPLIT times shorter, and its rounding
     // error what the tiled kernels' is, which add a tile's sources first (16384
     // sources of a 26k grid, error against 64 bits 1.5e-15 on tiles, 5.7e-15
     // with one accumulator).  Accumulators of the workgroups' own, without
     // atomics, ran 20-30% slower (8000 sources of that grid 13.6 -> 16.0 ms).
     constexpr int SPLIT = 16;
-    constexpr size_t SPLIT_SOURCES = 4096;
+    constexpr size_t SPLIT_SOURCES = 512;
     // (an ordered run folds its one copy back to the component's order)
     a.split = src.size() >= SPLIT_SOURCES ? SPLIT : 1;
     const size_t word = sizeof(double) * (size_t)dc.n;

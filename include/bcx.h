@@ -147,11 +147,13 @@ typedef struct bcx_dgraph bcx_dgraph;   /* device-resident component set */
 typedef struct {
     int32_t        path;          /* BCX_PATH_*                              */
     int32_t        precision;     /* BCX_PREC_*                              */
-    int32_t        use_chains;    /* 1: chain vertices via endpoint rows     */
+    int32_t        use_chains;    /* 1: chain vertices via endpoint rows where
+                                     that costs less than a run of their own */
     int32_t        batch_width;   /* batched: concurrent tiles, 1..8 (0 = 8) */
     const int64_t *src_subset;    /* NULL = all sources; else slots          */
     int64_t        n_src;         /* slot = comp_offset[c] + local vertex    */
-    int64_t        row_cap_bytes; /* endpoint-row slab cap (0 = auto)        */
+    int64_t        row_cap_bytes; /* endpoint-row slab cap (0 = auto; > 0 also
+                                     keeps every chain vertex on rows)       */
     int32_t        sigma_f64_threshold_log2; /* test hook: treat sigma >=
                                      2^k as overflow (0 = 64, i.e. uint64)  */
     int32_t        flags;         /* BCX_FLAG_* bits                          */
@@ -164,8 +166,10 @@ typedef struct {
 } bcx_opts;
 
 /* Batched path: run components of up to 2048 vertices through the
- * multi-launch tile path instead of the one-launch small-component kernel
- * (both compute the same; the flag exists for tests and measurements).     */
+ * multi-launch tile path instead of the one-launch small-component kernels: a
+ * wave per source where the component's arcs leave the LDS room for two
+ * sources or more (three with FP32 terms), else a workgroup per tile (all
+ * compute the same; the flag exists for tests and measurements).           */
 #define BCX_FLAG_NO_SMALL_KERNEL 1
 /* Batched path: launch every kernel eagerly instead of replaying captured
  * hipGraphs (the persistent small-component and workgroup passes, and the
@@ -173,9 +177,10 @@ typedef struct {
 #define BCX_FLAG_NO_GRAPH        2
 /* Batched path: components of 2049..131072 vertices whose BFS levels are
  * narrow (average level width at most 4096 vertices from the highest-degree
- * vertex) run one workgroup per tile through every level.  NO_WG_KERNEL
- * sends them to the multi-launch tiles; WG_KERNEL sends every component of
- * that size range to the workgroup kernel.                                 */
+ * vertex) run one workgroup per source, or per tile where the options ask for
+ * a tile width or FP32 terms meet counts past 64 bits.  NO_WG_KERNEL sends
+ * them to the multi-launch tiles; WG_KERNEL sends every component of that size
+ * range to the workgroup-per-tile kernel.                                  */
 #define BCX_FLAG_NO_WG_KERNEL    4
 #define BCX_FLAG_WG_KERNEL       8
 /* Batched path, multi-launch tiles: with use_chains, the chains that no
@@ -190,8 +195,9 @@ typedef struct {
 /* Batched path: components of at least 16384 vertices get a schedule
  * measured once on sample tiles and cached (no counterpart in the
  * reference, which switches schedule from sampled BFS depths,
- * Codes/kernels_free.cu:447-470): the workgroup or multi-launch kernel for
- * components of up to 131072 vertices, and for multi-launch components the
+ * Codes/kernels_free.cu:447-470): one workgroup per source, the multi-launch
+ * tiles or (up to 131072 vertices) the workgroup-per-tile kernel, by the number
+ * of sources of a run, and for multi-launch components the
  * sources per lane, the level kernels' blocks per CU, the tiles in flight
  * and chain contraction on or off.  NO_TUNE keeps the defaults (the
  * level-width rule, 4 sources per lane, 8 blocks per CU, 8 tiles,
@@ -222,8 +228,8 @@ typedef struct {
                                   list entries of the completed tiles         */
     int64_t n_tiles;           /* batched, multi-launch tiles completed       */
     int32_t n_comp_small;      /* batched: components run on the small-component */
-    int32_t n_comp_wg;         /*   kernel, the workgroup kernel and the      */
-    int32_t n_comp_multi;      /*   multi-launch tiles                        */
+    int32_t n_comp_wg;         /*   kernels, one workgroup per source or tile */
+    int32_t n_comp_multi;      /*   and the multi-launch tiles                */
     int32_t n_tuned;           /* batched: components whose schedule was measured
                                   (the schedule of each is measured once)     */
     int32_t sched_blocks_per_cu; /* batched: blocks per CU, tiles in flight and */
@@ -271,10 +277,10 @@ int  bcx_bc(bcx_ctx *ctx, const bcx_component *comps, int32_t n_comps,
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): the batched run (bcx_run, BCX_PATH_BATCHED, default
  * flags) of ONE component of at most BCX_NOALLOC_MAX_N vertices -- the
- * small-component kernel -- that allocates nothing.  Every buffer beyond the
- * inputs and the output (tile table, source weights, work counters, and the
+ * small-component kernels -- that allocates nothing.  Every buffer beyond the
+ * inputs and the output (tile tables, source weights, work counters, and the
  * path-count / term / list slabs of at most BCX_NOALLOC_MAX_WORKGROUPS
- * workgroups) lives in one static device array of BCX_NOALLOC_SCRATCH_BYTES
+ * workgroups of the kernel that needs them) lives in one static device array of BCX_NOALLOC_SCRATCH_BYTES
  * per GPU, held from the first bcx_create on that GPU until the process
  * ends.  Inputs and output are the caller's device memory: d_row_ptr[n+1],
  * d_col[arcs], d_reach[n] (NULL = all zero), d_srcs[n_src] (distinct local
@@ -308,7 +314,7 @@ int  bcx_debug_source(bcx_ctx *ctx, const bcx_component *comp, int32_t src,
                       double *sigma_f64, double *delta, int32_t *sigma_is_f64);
 
 /* Kernels of the batched path (bcx_debug_tile's *kernel_used).            */
-#define BCX_KERNEL_SMALL     1   /* workgroup per tile, state in LDS (n <= 2048)  */
+#define BCX_KERNEL_SMALL     1   /* state in LDS, one launch (n <= 2048)          */
 #define BCX_KERNEL_WG        2   /* workgroup per tile, state in HBM (deep BFS)   */
 #define BCX_KERNEL_MULTI     3   /* level launches across the device per tile     */
 
@@ -316,7 +322,8 @@ int  bcx_debug_source(bcx_ctx *ctx, const bcx_component *comp, int32_t src,
  * local vertices; 1 <= ns <= 64, or up to 64 W on the multi-launch tiles of
  * W sources per lane) run as the sources of one tile on the kernel that bcx_run
  * picks for this component under opts->flags (the flags force a kernel as
- * they do for a run), with that kernel's per-source probe arrays switched
+ * they do for a run; a component that a run takes source by source is probed
+ * on the workgroup-per-tile kernel), with that kernel's per-source probe arrays switched
  * on; every source is read back.  Outputs are [ns * n], row i for srcs[i]
  * (any pointer may be NULL): levels, path counts (both forms; the tile's
  * counts are FP64 when *sigma_is_f64 = 1, else exact integers) and
