@@ -820,7 +820,7 @@ static int64_t sample_work(const HostComp &hc, const std::vector<int32_t> &order
 // 1M-vertex mixed graph, 1.68 / 1.61 on an R-MAT core with chains, 1.82 /
 // 1.88 on a 519k-vertex Chung-Lu core without chains.  The choice is cached
 // and applied to every later source set of the component.
-std::vector<int32_t> tuned_sources(DComp &dc, const std::vector<int32_t> &srcs) {
+void tune_order(DComp &dc) {
     if (dc.tile_order < 0) {
         const HostComp &hc = dc.host;
         const int32_t n = hc.n;
@@ -856,6 +856,10 @@ std::vector<int32_t> tuned_sources(DComp &dc, const std::vector<int32_t> &srcs) 
             }
         }
     }
+}
+
+std::vector<int32_t> tuned_sources(DComp &dc, const std::vector<int32_t> &srcs) {
+    tune_order(dc);
     if (dc.tile_order == 1) return ball_sources(dc, srcs);
     if (dc.tile_order == 2) {
         std::vector<int32_t> o(srcs);
@@ -1953,16 +1957,14 @@ int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, int64_t n_src, 
     // the widest lanes, which narrower lanes cut into more tiles (a sample of
     // 64-source tiles left the wide candidates a few tiles for eight slots and
     // picked 128-source tiles where 256-source ones run 10% faster)
-    const std::vector<int32_t> samp =
-        rc ? std::vector<int32_t>() : sample_tiles(dc, TUNE_TILES, (int64_t)BATCH_W * MAX_SPL);
+    std::vector<int32_t> samp;
     double r_multi = 0.0;
     if (!rc && need_kind) {
         dc.rate_src = dc.rate_wg = dc.rate_multi = 0.0;
         if (source_fits && !valid_spl(o->sources_per_lane)) {
-            const std::vector<int32_t> order = batched_order(dc);
             std::vector<int32_t> ss;
             const int64_t k = std::min<int64_t>(dc.n <= WG_N ? TUNE_SOURCES : TUNE_SOURCES / 8, dc.n);
-            for (int64_t i = 0; i < k; ++i) ss.push_back(order[(size_t)(i * dc.n / k)]);
+            for (int64_t i = 0; i < k; ++i) ss.push_back((int32_t)(i * dc.n / k));
             bool overflow = false;
             rc = source_component(ctx, dc, ss, &to, bc + dc.offset, nullptr, &overflow);
             const double t = ctx->timer.collect();
@@ -1976,7 +1978,10 @@ int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, int64_t n_src, 
     }
     const double per_src = need_kind && dc.rate_src > 0 ? 1.0 / dc.rate_src : 0.0;
     const double launches = 3.0 * (dc.depth + 1) * LAUNCH_S / (MAX_SLOTS * BATCH_W * MAX_SPL);
-    if (!rc && !(per_src > 0 && dc.depth >= 0 && per_src < 2 * launches)) rc = time_multi(samp, base, &r_multi);
+    if (!rc && !(per_src > 0 && dc.depth >= 0 && per_src < 2 * launches)) {
+        samp = sample_tiles(dc, TUNE_TILES, (int64_t)BATCH_W * MAX_SPL);
+        rc = time_multi(samp, base, &r_multi);
+    }
     if (!rc && need_kind) {
         dc.rate_multi = r_multi;
         dc.kind_measured = true;

@@ -175,6 +175,7 @@ struct SmallJob {
 };
 std::vector<int32_t> batched_sources(bcx::DComp &dc, const int32_t *subset, int64_t n_sub, int64_t *n_chain);
 std::vector<int32_t> ball_sources(bcx::DComp &dc, const std::vector<int32_t> &srcs);
+void tune_order(bcx::DComp &dc);
 std::vector<int32_t> tuned_sources(bcx::DComp &dc, const std::vector<int32_t> &srcs);
 // Every vertex of the component in the order a full batched run tiles its
 // sources (64 consecutive entries per tile).
