@@ -368,11 +368,7 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
                         double *probe = nullptr, bool fp32 = false, bool ordered = false) {
     if (src.empty()) return BCX_OK;
     int rc;
-    ordered = ordered && dc.ord_state == 1;
-    std::vector<int32_t> ids;
-    if (ordered)
-        for (int32_t v : src) ids.push_back(dc.ord_inv[(size_t)v]);
-    if ((rc = upload(ctx, ordered ? ids.data() : src.data(), src.size() * 4, ctx->w_src, "work list"))) return rc;
+    if ((rc = ctx->w_src.ensure(ctx, src.size() * 4, "work list"))) return rc;
     if ((rc = upload(ctx, slot.data(), slot.size() * 4, ctx->w_aux, "work list"))) return rc;
     if ((rc = upload(ctx, mode.data(), mode.size(), ctx->w_mode, "work list"))) return rc;
     rc = ctx_hip(ctx, hipMemsetAsync(ctx->counters.p, 0, 4 * sizeof(int32_t), ctx->stream), "memset");
@@ -381,6 +377,28 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
     const int grid = plain_grid(ctx, dc.n, (int64_t)src.size(), shape);
     PlainScratch sc;
     if ((rc = ensure_plain_scratch(ctx, dc.n, grid, sc))) return rc;
+    // Hundreds of sources and more add into SPLIT copies of the accumulator, folded
+    // afterwards: a vertex's sum is then SPLIT times shorter, and its rounding
+    // error what the tiled kernels' is, which add a tile's sources first (16384
+    // sources of a 26k grid, error against 64 bits 1.5e-15 on tiles, 5.7e-15
+    // with one accumulator).  Accumulators of the workgroups' own, without
+    // atomics, ran 20-30% slower (8000 sources of that grid 13.6 -> 16.0 ms).
+    // Where a capacity has little room left beside the rows above, there is one
+    // accumulator, and without room for that an ordered run has the
+    // component's own order.
+    constexpr int SPLIT = 16;
+    constexpr size_t SPLIT_SOURCES = 512;
+    const size_t word = sizeof(double) * (size_t)dc.n;
+    const size_t room = ctx->mem_cap > ctx->mem_used ? ctx->mem_cap - ctx->mem_used : 0;
+    int split = src.size() >= SPLIT_SOURCES && ctx->bc_split.bytes + room / 16 >= word * SPLIT ? SPLIT : 1;
+    ordered = ordered && dc.ord_state == 1;
+    if (split > 1 && ctx->bc_split.ensure(ctx, word * SPLIT, "split accumulator") != BCX_OK) split = 1;
+    if (ordered && split == 1 && ctx->bc_split.ensure(ctx, word, "accumulator") != BCX_OK) ordered = false;
+    const bool fold = split > 1 || ordered;  // (an ordered run folds its one copy back to the component's order)
+    std::vector<int32_t> ids;
+    if (ordered)
+        for (int32_t v : src) ids.push_back(dc.ord_inv[(size_t)v]);
+    if ((rc = upload(ctx, ordered ? ids.data() : src.data(), src.size() * 4, ctx->w_src, "work list"))) return rc;
     PlainArgs a{};
     a.src = (const int32_t *)ctx->w_src.p;
     a.aux = (const int32_t *)ctx->w_aux.p;
@@ -393,23 +411,7 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
     a.probe = probe;
     a.fp32 = fp32;
     a.sweep = plain_sweep(dc.n, dc.arcs);
-    // Hundreds of sources and more add into SPLIT copies of the accumulator, folded
-    // afterwards: a vertex's sum is then SPLIT times shorter, and its rounding
-    // error what the tiled kernels' is, which add a tile's sources first (16384
-    // sources of a 26k grid, error against 64 bits 1.5e-15 on tiles, 5.7e-15
-    // with one accumulator).  Accumulators of the workgroups' own, without
-    // atomics, ran 20-30% slower (8000 sources of that grid 13.6 -> 16.0 ms).
-    constexpr int SPLIT = 16;
-    constexpr size_t SPLIT_SOURCES = 512;
-    // (an ordered run folds its one copy back to the component's order)
-    a.split = src.size() >= SPLIT_SOURCES ? SPLIT : 1;
-    const size_t word = sizeof(double) * (size_t)dc.n;
-    bool fold = a.split > 1 || ordered;
-    if (fold && ctx->bc_split.ensure(ctx, word * a.split, "split accumulator") != BCX_OK) {
-        a.split = 1;
-        if (ordered && (rc = ctx->bc_split.ensure(ctx, word, "accumulator"))) return rc;
-        fold = ordered;
-    }
+    a.split = split;
     if (fold) {
         a.bc = (double *)ctx->bc_split.p;
         if ((rc = ctx_hip(ctx, hipMemsetAsync(a.bc, 0, word * a.split, ctx->stream), "memset"))) return rc;
@@ -457,6 +459,10 @@ static int order_copy(bcx_ctx *ctx, DComp &dc) {
         top_arcs += arcs[k];
     }
     if (2 * top_arcs < h.arcs) return BCX_OK;
+    // (a capacity that has little left beside the rows of a run goes without)
+    const size_t copy = 4 * (4 * (size_t)n + 1 + h.col.size());
+    const size_t rows = (size_t)plain_stride(n) * PLAIN_WORD_BYTES * (size_t)plain_min_grid(ctx, n);
+    if (plain_room(ctx) < copy + rows + ctx->mem_cap / 4) return BCX_OK;
     int rc = run_bfs_list(ctx, dc, {root}, {-1}, {0}, true, 0, nullptr, Rows{}, nullptr);  // (forward only)
     PlainScratch sc;
     if (rc || (rc = ensure_plain_scratch(ctx, n, 1, sc))) return rc;

@@ -107,3 +107,22 @@ def test_dependencies_in_vertex_order(engine, n, chords, prec):
         (got,), st = engine.bc([c], subset=sub, path=path, precision=prec, flags=bcx.FLAG_NO_TUNE)
         mx, _, zeros = relerr(got, want)
         assert mx < tol and zeros, (n, chords, prec, mx)
+
+
+@pytest.mark.parametrize("spare", [2, 8, 400])
+def test_little_room_beside_the_rows(engine, spare):
+    """A capacity that holds the workgroups' rows and `spare` MiB: the run takes
+    what fits of the ordered copy and the split accumulators, and is never
+    refused for them.  Every vertex of a bipartite graph of 40 hubs."""
+    rng = np.random.default_rng(spare)
+    n, hubs_n = 5000, 40
+    e = [(h, v) for v in range(hubs_n, n) for h in rng.choice(hubs_n, size=3, replace=False)]
+    c = csr(n, e)
+    sub = np.sort(rng.permutation(n)[:700]).astype(np.int64)
+    rows = ((n + 2 + 63) // 64 * 64) * 28 * min(len(sub), 2 * engine.info()[0])
+    eng = bcx.Engine(0, mem_cap=rows + (spare << 20))
+    (got,), st = eng.bc([c], subset=sub)
+    eng.close()
+    want = oracle.component_bc(c.row_ptr, c.col, c.reach, sources=sub.astype(np.int32))
+    mx, _, zeros = relerr(got, want)
+    assert mx < 1e-9 and zeros, mx
