@@ -432,8 +432,8 @@ static int run_tiles(bcx_ctx *ctx, const DComp &dc, int64_t n_src, const TileJob
     return rc;
 }
 
-// Static hub slice tables and pull chunks of one component, n of whose
-// vertices are tile vertices.  A pull wave takes the entries of a chunk one
+// Static hub slice tables (without `split`: none, every row is walked whole)
+// and pull chunks of one component, n of whose vertices are tile vertices.  A pull wave takes the entries of a chunk one
 // after another, and in the BFS order of the tile graph the heavy vertices lie
 // together at the front: in chunks of 64 vertices a big level lasted as long as
 // the heaviest chunk.  Chunks of at most PULL_ARCS arcs took a tile's two big
@@ -441,12 +441,12 @@ static int run_tiles(bcx_ctx *ctx, const DComp &dc, int64_t n_src, const TileJob
 // (256 arcs: 280 and 380, with a scan of twice the chunks on small levels), the
 // core's 6144 sources from 80 to 53 ms.
 constexpr int64_t PULL_ARCS = 512;
-static int stage_hubs(bcx_ctx *ctx, const DComp &dc, int32_t n) {
+static int stage_hubs(bcx_ctx *ctx, const DComp &dc, int32_t n, bool split = true) {
     BatchedState &bs = *ctx->batched;
     const HostComp &hc = dc.host;
     const int64_t budget = (int64_t)HUB_SLICES_PER_CU * std::max(1, ctx->n_cu);
-    int64_t T = HUB_MIN;
-    for (;; T *= 2) {
+    int64_t T = split ? HUB_MIN : INT32_MAX;
+    for (; split; T *= 2) {
         int64_t ns = 0;
         for (int32_t v = 0; v < hc.n && ns <= budget; ++v) {
             const int64_t d = hc.rp[v + 1] - hc.rp[v];
@@ -1205,6 +1205,12 @@ static int cut_slots(bcx_ctx *ctx, const ChainCut *cut) {
 }
 
 static bool want_cut(const bcx_opts *o) { return o->use_chains && !(o->flags & BCX_FLAG_NO_CONTRACT); }
+// Set by batched_opts: chains contracted whatever the tuner found; rows whole
+// (no hub slices).
+constexpr int32_t FLAG_CONTRACT = 1 << 30, FLAG_ROWS = 1 << 29;
+static bool runs_cut(const DComp &dc, const bcx_opts *o) {
+    return want_cut(o) && (dc.sched_cut != 0 || (o->flags & FLAG_CONTRACT));
+}
 
 static int tile_graph(bcx_ctx *ctx, DComp &dc, bool want, DComp *&pc, ChainCut *&cut,
                       const std::vector<int32_t> *&inv, const int32_t *&perm);
@@ -1214,7 +1220,7 @@ int batched_prepare(bcx_ctx *ctx, DComp &dc, const bcx_opts *o) {
     ChainCut *cut = nullptr;
     const std::vector<int32_t> *inv = nullptr;
     const int32_t *perm = nullptr;
-    return tile_graph(ctx, dc, want_cut(o) && dc.sched_cut != 0, pc, cut, inv, perm);
+    return tile_graph(ctx, dc, runs_cut(dc, o), pc, cut, inv, perm);
 }
 
 // The tile graph of a multi-launch component: the copy with contracted
@@ -1264,7 +1270,7 @@ static int wg_spl(const bcx_opts *o) { return valid_spl(o->sources_per_lane) ? o
 
 static MultiSched multi_sched(const DComp &dc, const bcx_opts *o) {
     MultiSched m;
-    m.cut = want_cut(o) && dc.sched_cut != 0;
+    m.cut = runs_cut(dc, o);
     m.spl = valid_spl(o->sources_per_lane) ? o->sources_per_lane : (dc.sched_spl > 0 ? dc.sched_spl : DEFAULT_SPL);
     m.bpc = o->blocks_per_cu > 0 ? std::min(o->blocks_per_cu, 64) : (dc.sched_bpc > 0 ? dc.sched_bpc : DEFAULT_BPC);
     m.slots = o->batch_width > 0 ? std::max(1, std::min(MAX_SLOTS, o->batch_width))
@@ -1287,7 +1293,9 @@ static int multi_run(bcx_ctx *ctx, DComp &dc, const std::vector<int32_t> &srcs, 
     rc = bs_ensure(ctx, pc->n, (int32_t)(ntiles * tw), m.slots, false);
     if (rc) return rc;
     if (cut && (rc = cut_slots(ctx, cut))) return rc;
-    if ((rc = stage_sources(ctx, *pc, ps, tw)) || (rc = stage_hubs(ctx, *pc, cut ? cut->n_core : pc->n))) return rc;
+    if ((rc = stage_sources(ctx, *pc, ps, tw)) ||
+        (rc = stage_hubs(ctx, *pc, cut ? cut->n_core : pc->n, !(o->flags & FLAG_ROWS))))
+        return rc;
     TileJob j = make_job(ctx, *pc, o, bc, m.bpc);
     j.perm = perm;
     j.cut = cut;
@@ -1875,6 +1883,54 @@ constexpr int TUNE_TILES = 24;
 constexpr int64_t TUNE_SOURCES = 4096;
 constexpr double LAUNCH_S = 4e-6;  // of a level kernel that finds next to nothing to do
 
+// With FP32 terms the result shows the kernel: the multi-launch tiles carry the
+// interiors of contracted chains in FP64 closed form and sum a hub's row in
+// slices, every other kernel rounds a term at each vertex and sums a row in CSR
+// order (1e-10 to 7e-9 apart; FP64 terms: FP64 rounding).  So what a component
+// is decides alone which of the two its FP32C runs get, whatever the number of
+// sources, the calls before and the timing of samples: the parts of a job add
+// up, and a source gives the same in every call.  Below the line every row is
+// summed whole: one workgroup per source, the workgroup kernel, or tiles with
+// neither contracted chains nor hub slices, whichever is fastest (to 1e-15 the
+// same).  The line is where the rates of full jobs on the workgroup kernel and
+// the sliced tiles crossed (the former ahead / behind, vertices at levels:
+// contracted tiles, power-law cores 67.3k / 69.0k at 24 to 27, R-MAT 44.5k / 85.7k at
+// 7, a 74k grid of 510 ahead; tiles without chains, power-law cores 84.1k /
+// 92.5k at 31 and 40, core of a block graph 74.1k / 76.8k at 4): drawn
+// elsewhere, the results in between would change.
+enum { FP32_ANY = 0, FP32_ROWS = 1, FP32_TILES = 2 };
+static int64_t fp32_line(const DComp &dc, bool cut) { return (cut ? 58000 : 74000) + 400 * (int64_t)dc.depth; }
+static bool fp32_free(const DComp &dc, const bcx_opts *o) {
+    return !run_fp32(o) || dc.n < TUNE_N ||
+           (o->flags & (BCX_FLAG_NO_TUNE | BCX_FLAG_WG_KERNEL | BCX_FLAG_NO_WG_KERNEL));  // (fixed by the options)
+}
+static int fp32_route(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, int *route) {
+    *route = FP32_ANY;
+    if (fp32_free(dc, o)) return BCX_OK;
+    int8_t &r = dc.fp32_route[want_cut(o)];
+    if (r < 0 && dc.n <= WG_N) {
+        (void)batched_narrow(dc);  // (measures the depth)
+        ChainCut *cut = nullptr;
+        if (want_cut(o) && dc.n > fp32_line(dc, true) && dc.n <= fp32_line(dc, false)) {
+            const int rc = chain_cut(ctx, dc, cut);
+            if (rc) return rc;
+        }
+        r = dc.n > fp32_line(dc, cut != nullptr) ? FP32_TILES : FP32_ROWS;
+    }
+    if (r < 0) r = FP32_TILES;
+    *route = r;
+    return BCX_OK;
+}
+
+bcx_opts batched_opts(const DComp &dc, const bcx_opts &o) {
+    bcx_opts r = o;
+    r.flags &= ~(FLAG_CONTRACT | FLAG_ROWS);
+    const int route = fp32_free(dc, &o) ? FP32_ANY : dc.fp32_route[want_cut(&o)];
+    if (route == FP32_ROWS) r.flags |= BCX_FLAG_NO_CONTRACT | FLAG_ROWS;
+    if (route == FP32_TILES) r.flags |= FLAG_CONTRACT;
+    return r;
+}
+
 // Sources of k tiles of `width` evenly spaced over the component's tile order.
 static std::vector<int32_t> sample_tiles(DComp &dc, int64_t k, int64_t width) {
     const std::vector<int32_t> order = batched_order(dc);
@@ -1907,10 +1963,15 @@ static int measured_kind(bcx_ctx *ctx, const DComp &dc, int64_t n_src) {
     return kind;
 }
 
-int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, int64_t n_src, bcx_stats *st) {
-    const int kind0 = batched_kind(dc, o->flags);
+int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *opts, int64_t n_src, bcx_stats *st) {
+    int kind0 = batched_kind(dc, opts->flags);
     if (kind0 == BCX_KERNEL_SMALL) return kind0;
-    const bool kind_fixed = (o->flags & (BCX_FLAG_NO_WG_KERNEL | BCX_FLAG_WG_KERNEL)) != 0;
+    int route = FP32_ANY, rc = fp32_route(ctx, dc, opts, &route);
+    if (rc) return rc;
+    const bool sliced = route == FP32_TILES;
+    if (sliced) kind0 = BCX_KERNEL_MULTI;
+    const bcx_opts own = batched_opts(dc, *opts), *o = &own;
+    const bool kind_fixed = sliced || (o->flags & (BCX_FLAG_NO_WG_KERNEL | BCX_FLAG_WG_KERNEL)) != 0;
     // (the rows of the per-source kernel have to fit beside the tiles' buffers)
     const bool source_fits = plain_scratch_fits(ctx, dc.n, n_src);
     if ((o->flags & BCX_FLAG_NO_TUNE) || dc.n < TUNE_N)
@@ -1919,13 +1980,15 @@ int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, int64_t n_src, 
     const bool need_kind = !kind_fixed && !dc.kind_measured;
     int kind = kind_fixed ? kind0 : (dc.kind_measured ? measured_kind(ctx, dc, n_src) : -1);
     if (kind == KIND_SOURCE && !source_fits) kind = kind0;
-    const bool need_multi = !dc.sched_multi && (need_kind || kind == BCX_KERNEL_MULTI);
+    // (tiles of whole rows run under the defaults: six candidates twice cost more
+    // than a dozen full jobs of a component below the line)
+    const bool need_multi = !dc.sched_multi && (need_kind || kind == BCX_KERNEL_MULTI) && route != FP32_ROWS;
     if (!need_kind && !need_multi) return kind;
     // the run's timer is set aside: the samples are timed on their own
     Timer keep;
     std::swap(keep, ctx->timer);
     DBuf scratch;
-    int rc = scratch.ensure(ctx, 8 * ((size_t)dc.offset + (size_t)dc.n), "tuner scratch");
+    rc = scratch.ensure(ctx, 8 * ((size_t)dc.offset + (size_t)dc.n), "tuner scratch");
     bcx_opts to = *o;
     to.src_subset = nullptr;
     to.n_src = 0;
@@ -1994,7 +2057,7 @@ int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, int64_t n_src, 
         if (o->blocks_per_cu <= 0)
             for (int bpc : {4, 16}) cands.push_back({base.cut, bpc, base.slots, base.spl});
         if (o->batch_width <= 0) cands.push_back({base.cut, base.bpc, 4, base.spl});
-        if (base.cut) cands.push_back({false, base.bpc, base.slots, base.spl});
+        if (base.cut && !sliced) cands.push_back({false, base.bpc, base.slots, base.spl});
         if (!valid_spl(o->sources_per_lane))
             for (int w : {1, 2, 4})
                 if (w != base.spl) cands.push_back({base.cut, base.bpc, base.slots, w});

@@ -81,6 +81,9 @@ struct DComp {
     // cut_state -1 not yet tried, 0 the component has too few such chains)
     ChainCut *cut = nullptr;
     int8_t cut_state = -1;
+    // FP32C: rounding of the component's terms without and with chains to
+    // contract (FP32_ROWS or FP32_TILES; -1 not yet looked at)
+    int8_t fp32_route[2] = {-1, -1};
     // batched path: the schedule measured on sample sources, cached for every
     // later run of the component (sources per second on each kernel, 0: not a
     // candidate; round_wg: sources of a full round of workgroup tiles;
@@ -218,6 +221,9 @@ int source_component(bcx_ctx *ctx, bcx::DComp &dc, const std::vector<int32_t> &s
                      bcx_stats *st, bool *overflow);
 // Whether the context's cap leaves room for the per-source kernel's rows.
 bool plain_scratch_fits(bcx_ctx *ctx, int32_t n, int64_t count);
+// The options that a component's multi-launch tiles run under, once it has its
+// schedule: FP32C runs round the terms of a component alike in every call.
+bcx_opts batched_opts(const bcx::DComp &dc, const bcx_opts &o);
 // Blocks per CU, tiles in flight and sources per lane a multi-launch run of
 // dc uses.
 void batched_sched_report(const bcx::DComp &dc, const bcx_opts *o, int32_t *bpc, int32_t *slots, int32_t *spl);

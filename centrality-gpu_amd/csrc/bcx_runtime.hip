@@ -985,7 +985,8 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
             s->n_comp_wg++;
             (kind == KIND_SOURCE ? single : wg).push_back({&dc, std::move(tiles)});
         } else {
-            if ((rc = batched_prepare(ctx, dc, &o))) return rc;  // one-time work stays outside the timing
+            const bcx_opts own = batched_opts(dc, o);
+            if ((rc = batched_prepare(ctx, dc, &own))) return rc;  // one-time work stays outside the timing
             s->n_comp_multi++;
             if (dc.n > largest_multi) {
                 largest_multi = dc.n;
@@ -1027,9 +1028,11 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
             (rc = batched_persistent_start(ctx, small, &o, bc, s, PASS_SMALL, sp)) ||
             (rc = batched_persistent_start(ctx, wg, &o, bc, s, PASS_WG, sp)))
             return rc;
-        for (SmallJob &jb : multi)
-            if ((rc = batched_component(ctx, *const_cast<DComp *>(jb.dc), jb.srcs, &o, bc + jb.dc->offset, s)))
-                return rc;
+        for (SmallJob &jb : multi) {
+            DComp &dc = *const_cast<DComp *>(jb.dc);
+            const bcx_opts own = batched_opts(dc, o);
+            if ((rc = batched_component(ctx, dc, jb.srcs, &own, bc + dc.offset, s))) return rc;
+        }
         std::vector<SmallJob> again;  // FP32 terms, overflowed counts
         for (SmallJob &jb : single) {
             bool overflow = false;

@@ -1,0 +1,50 @@
+"""Which kernel a batched component runs on never shows in its FP32C result.
+
+Every kernel but the multi-launch tiles rounds the same terms to FP32 at the same
+points and sums them in the same order (1e-12 apart: FP64 rounding of the
+accumulated BC); those tiles contract chains and slice the rows of hubs (1e-10
+to 7e-9 apart).  So a component runs on them in every call or in none, and
+counts past 64 bits turn the same 64 sources to FP64 terms on whichever kernel
+they are met.
+"""
+import numpy as np
+import pytest
+
+import bcx
+
+pytestmark = pytest.mark.gpu
+
+B, F32 = bcx.PATH_BATCHED, bcx.PREC_FP32C
+SAME = 1e-12
+
+
+def giant(cfg, scale, seed=3):
+    n, uv = bcx.generate(cfg, 0, scale)
+    uv = np.random.default_rng(seed).permutation(n).astype(np.int32)[uv]
+    return max(bcx.Host.from_edges(n, uv).decompose().components(), key=lambda c: c.n)
+
+
+def far(a, b):
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+@pytest.mark.parametrize("chains", [True, False])
+@pytest.mark.parametrize("cfg,scale,flags", [(2, 0.022, bcx.FLAG_WG_KERNEL), (5, 0.06, bcx.FLAG_WG_KERNEL),
+                                             (2, 0.08, bcx.FLAG_WG_KERNEL), (2, 0.12, bcx.FLAG_NO_WG_KERNEL)])
+def test_fp32c_does_not_depend_on_the_number_of_sources(engine, cfg, scale, flags, chains):
+    """18.6k, 23k and 67k cores (rows whole) and a 101k core (sliced tiles): subsets of
+    every size, with the tuner's rates of each, equal the kernel that the flags
+    force."""
+    c = giant(cfg, scale)
+    order = np.random.default_rng(7).permutation(c.n).astype(np.int64)
+    g = engine.upload([c])
+    try:
+        for k in (64, 600, 4096, 20000):
+            kw = dict(path=B, precision=F32, subset=order[:k], use_chains=chains)
+            got, st = g.run(**kw)
+            want, _ = g.run(flags=flags, **kw)
+            print("case", cfg, scale, c.n, k, "multi", st["n_comp_multi"], "contracted", st["n_contracted"],
+                  far(got, want), flush=True)
+            assert far(got, want) < SAME
+    finally:
+        g.free()
