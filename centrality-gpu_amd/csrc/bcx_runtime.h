@@ -53,6 +53,7 @@ struct DComp {
     int64_t offset = 0;  // into the concatenated BC vector
     int32_t depth = -1;  // BFS depth from the highest-degree vertex (-1: not measured)
     double sigma_est = 0.0;  // largest path count of that BFS (measured with depth)
+    bool src_wrapped = false;  // a per-source FP32C run met counts past 64 bits
     std::vector<int32_t> rank;      // batched path: BFS rank of each vertex (built on first use)
     std::vector<uint8_t> on_chain;  // batched path: 1 for chain vertices (built on first use)
     std::vector<int32_t> ball;      // batched path: every vertex in ball-tile order (built on first use)

@@ -600,6 +600,7 @@ int source_component(bcx_ctx *ctx, DComp &dc, const std::vector<int32_t> &srcs, 
         if (!ctx->overflow) return BCX_OK;
         rc = ctx_hip(ctx, hipMemsetAsync(bc, 0, sizeof(double) * (size_t)dc.n, ctx->stream), "memset");
         if (rc || fp32) {
+            if (!limit) dc.src_wrapped = true;
             *overflow = true;
             return rc;
         }
@@ -1044,14 +1045,10 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
             (rc = batched_persistent_finish(ctx, s, PASS_WG)))
             return rc;
         for (SmallJob &jb : again) {
+            // (in the order of the tiles: those around an overflow turn to FP64)
             DComp &dc = *const_cast<DComp *>(jb.dc);
-            if (dc.n > WG_N) {
-                if ((rc = batched_prepare(ctx, dc, &o)) ||
-                    (rc = batched_component(ctx, dc, jb.srcs, &o, bc + dc.offset, s)))
-                    return rc;
-                continue;
-            }
-            if ((rc = batched_persistent_start(ctx, {jb}, &o, bc, s, PASS_WG, ctx->stream)) ||
+            const std::vector<SmallJob> tiles{{&dc, tuned_sources(dc, jb.srcs)}};
+            if ((rc = batched_persistent_start(ctx, tiles, &o, bc, s, PASS_WG, ctx->stream)) ||
                 (rc = batched_persistent_finish(ctx, s, PASS_WG)))
                 return rc;
         }

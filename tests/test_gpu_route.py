@@ -48,3 +48,25 @@ def test_fp32c_does_not_depend_on_the_number_of_sources(engine, cfg, scale, flag
             assert far(got, want) < SAME
     finally:
         g.free()
+
+
+@pytest.mark.parametrize("cfg,scale,seed,bits", [(4, 0.035, 0, 0), (4, 0.035, 2, 0), (4, 0.03, 5, 0),
+                                                 (2, 0.006, 3, 8), (2, 0.006, 3, 9)])
+def test_the_same_sources_turn_to_fp64(engine, cfg, scale, seed, bits):
+    """Components with counts past 64 bits (or a forced limit) from some sources
+    only: the sources that get FP64 terms are those of the workgroup kernel's
+    tiles, whether the counts were foreseen (grids whose hub's counts, by the
+    numbering, reach 2^43, 2^59 and 2^48) or met by a per-source run."""
+    c = giant(cfg, scale, seed)
+    assert c.n > 2048
+    sub = np.random.default_rng(11).permutation(c.n)[:2000].astype(np.int64)
+    g = engine.upload([c])
+    try:
+        kw = dict(path=B, precision=F32, subset=sub, sigma_threshold_log2=bits)
+        got = [g.run(**kw) for _ in range(2)]
+        want, ws = g.run(flags=bcx.FLAG_WG_KERNEL, **kw)
+        for bc, st in got:
+            print("case", cfg, scale, c.n, bits, "FP64", ws["n_f64_sigma"], st["n_f64_sigma"], far(bc, want), flush=True)
+            assert st["n_f64_sigma"] == ws["n_f64_sigma"] and far(bc, want) < SAME
+    finally:
+        g.free()
