@@ -91,6 +91,7 @@ SIGNATURES = {
     "bcx_dgraph_free": (None, [C.c_void_p, C.c_void_p]),
     "bcx_run": (C.c_int, [C.c_void_p, C.c_void_p, C.POINTER(Opts), C.POINTER(C.c_double),
                           C.POINTER(Stats)]),
+    "bcx_run_by_source": (C.c_int32, [C.c_void_p]),
     "bcx_bc": (C.c_int, [C.c_void_p, C.POINTER(Component), C.c_int32, C.POINTER(Opts),
                          C.POINTER(C.c_double), C.POINTER(Stats)]),
     "bcx_host_bc": (C.c_int, [C.c_void_p, C.c_void_p, C.POINTER(Opts), C.POINTER(C.c_double),
@@ -395,6 +396,10 @@ class Engine:
         if rc:
             self._err(rc, "host_bc")
         return bc, st.as_dict()
+
+    def run_by_source(self):
+        """Components that the last run took source by source (batched path)."""
+        return lib().bcx_run_by_source(self.h)
 
     def debug_source(self, comp, src, **kw):
         o, keep = make_opts(**kw)

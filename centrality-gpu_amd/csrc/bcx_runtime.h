@@ -140,6 +140,7 @@ struct bcx_ctx {
     double *bc_pin = nullptr;      // pinned host staging of the result download
     size_t bc_pin_bytes = 0;
     int32_t *up_pin = nullptr;     // pinned host staging of small uploads
+    int32_t by_source = 0;         // batched: components the last run took source by source
     bool busy = true;              // work may be in flight on the context stream
     BatchedState *batched = nullptr;
     SmallState *small = nullptr;

@@ -891,6 +891,7 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
     std::memset(s, 0, sizeof(*s));
     auto t0 = std::chrono::steady_clock::now();
     ctx->busy = true;
+    ctx->by_source = 0;
     // a run that failed part-way may have left work on the side stream and
     // timer intervals open or uncollected
     batched_persistent_reset(ctx);
@@ -1040,6 +1041,7 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
             if ((rc = source_component(ctx, *const_cast<DComp *>(jb.dc), jb.srcs, &o, bc + jb.dc->offset, s, &overflow)))
                 return rc;
             if (overflow) again.push_back(std::move(jb));
+            else ctx->by_source++;
         }
         if ((rc = batched_persistent_finish(ctx, s, PASS_SRC)) || (rc = batched_persistent_finish(ctx, s, PASS_SMALL)) ||
             (rc = batched_persistent_finish(ctx, s, PASS_WG)))
@@ -1073,6 +1075,8 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
     s->t_total_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     return BCX_OK;
 }
+
+int32_t bcx_run_by_source(const bcx_ctx *ctx) { return ctx ? ctx->by_source : 0; }
 
 int bcx_bc(bcx_ctx *ctx, const bcx_component *comps, int32_t n_comps, const bcx_opts *opts,
            double *bc_out, bcx_stats *st) {

@@ -269,6 +269,12 @@ int  bcx_batched_order(bcx_ctx *ctx, bcx_dgraph *g, int32_t c, int32_t *order);
 int  bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts,
              double *bc_out, bcx_stats *st);
 
+/* Components that the context's last bcx_run took source by source, one
+ * workgroup each (batched path; bcx_stats.n_comp_wg counts them together with
+ * those on the workgroup-per-tile kernel).  A component left to the tiles
+ * because its counts overflowed is not among them.                         */
+int32_t bcx_run_by_source(const bcx_ctx *ctx);
+
 /* Convenience: upload + run + free (one call per component set).          */
 int  bcx_bc(bcx_ctx *ctx, const bcx_component *comps, int32_t n_comps,
             const bcx_opts *opts, double *bc_out, bcx_stats *st);

@@ -50,6 +50,23 @@ def test_fp32c_does_not_depend_on_the_number_of_sources(engine, cfg, scale, flag
         g.free()
 
 
+def test_per_source_runs_are_told_apart(engine):
+    """The per-source kernel runs where it should: deep and mid-size components
+    in either precision, not where a flag or a lane width asks for tiles, nor
+    where an FP32C run met an overflow and went to the tiles."""
+    c = giant(2, 0.006)
+    g = engine.upload([c])
+    try:
+        for kw, want in ((dict(precision=F32), 1), (dict(precision=bcx.PREC_FP64), 1),
+                         (dict(precision=F32, flags=bcx.FLAG_WG_KERNEL), 0), (dict(precision=F32, sources_per_lane=2), 0),
+                         (dict(precision=bcx.PREC_FP64, sigma_threshold_log2=6), 1),
+                         (dict(precision=F32, sigma_threshold_log2=6), 0)):
+            _, st = g.run(path=B, subset=np.arange(64), **kw)
+            assert st["n_comp_wg"] == 1 and engine.run_by_source() == want, (kw, want)
+    finally:
+        g.free()
+
+
 @pytest.mark.parametrize("cfg,scale,seed,bits", [(4, 0.035, 0, 0), (4, 0.035, 2, 0), (4, 0.03, 5, 0),
                                                  (2, 0.006, 3, 8), (2, 0.006, 3, 9)])
 def test_the_same_sources_turn_to_fp64(engine, cfg, scale, seed, bits):
