@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "bcx_batched.h"
+#include "bcx_kernels.h"
 #include "bcx_small.h"
 #include "bcx_src.h"
 #include "bcx_runtime.h"
@@ -1856,31 +1857,29 @@ int batched_kind(DComp &dc, int flags) {
 }
 
 // ------------------------------------------------------------------------
-// Schedule tuner.  A component of at least TUNE_N vertices is run once on
-// sample sources (evenly spaced over its tile order, BC into a scratch
-// accumulator, timed with HIP events, outside the run's timing) under each
-// candidate schedule, and what was measured is cached for every later run:
-//  * kernel: the per-source kernel over TUNE_SOURCES sources and the
-//    multi-launch tiles over TUNE_TILES tiles, unless three launches per level
-//    alone would take those longer than half of what the per-source kernel
-//    takes (deep components); the workgroup kernel over min(tiles, CUs) tiles
-//    (its concurrent width) only where counts overflow the per-source kernel
-//    with FP32 terms.  A run takes the kernel with the least estimated time for
-//    its number of sources.  All sources, per source / multi-launch / workgroup
-//    (ms): 18.6k grid 22 / - / 97; 10.6k power-law core 11 / 26 / 40, 42k core
-//    - / 131 / 220, 84k core (20000 sources) - / 93 / 207; 2000 sources of the
-//    84k core 24 / 23 / 158;
+// Schedule tuner.  A component of at least TUNE_N vertices is run on sample
+// sources (evenly spaced over its tile order, BC into a scratch accumulator,
+// timed with HIP events, outside the run's timing), and what was measured is
+// cached with the options that it was measured under:
+//  * kernel: the time of a source on the per-source kernel, of one multi-launch
+//    tile alone and of a source of TUNE_TILES of them, of a round of workgroup
+//    tiles, each when a run's choice first depends on it.  A run takes the
+//    kernel with the least estimated time for its number of sources.  A tile
+//    alone lasts as long as one of eight in flight, so the first is charged
+//    whole.  Per source / multi-launch / workgroup, FP32C (ms; 64, 2048 and
+//    16384 sources): 18.6k power-law core 1.7, 5.5, 35 / 3.3, 18, 66 / 20, 90,
+//    92; 67k core 3.8, 28, 203 / 4.7, 24, 97 / 67, 234, 246; 23k R-MAT core 4.9,
+//    14, 90 / 3.8, 15, 73 / 40, 49, 56;
 //  * multi-launch: 8 / 4 / 16 level-kernel blocks per CU, 8 / 4 tiles in
 //    flight, chain contraction on / off, once a run takes them.
-// Each tiled candidate runs twice (the first run captures its graphs) and is
-// timed on the second; a multi-launch candidate replaces the default only when
-// its rate (sources per second) is at least 3% higher.  Options that fix a
-// choice are kept.  (The reference picks its schedule from sampled BFS depths
-// and frontier sizes, Codes/kernels_free.cu:447-470, 288, 381.)
+// Everything is timed on a second run (the first captures graphs and makes
+// copies); a multi-launch candidate replaces the default only when its rate
+// (sources per second) is at least 3% higher.  Options that fix a choice are
+// kept.  (The reference picks its schedule from sampled BFS depths and frontier
+// sizes, Codes/kernels_free.cu:447-470, 288, 381.)
 // ------------------------------------------------------------------------
 constexpr int32_t TUNE_N = 16384;
 constexpr int TUNE_TILES = 24;
-constexpr int64_t TUNE_SOURCES = 4096;
 constexpr double LAUNCH_S = 4e-6;  // of a level kernel that finds next to nothing to do
 
 // With FP32 terms the result shows the kernel: the multi-launch tiles carry the
@@ -1942,153 +1941,198 @@ static bool counts_may_wrap(const DComp &dc, const bcx_opts *o) {
     return run_fp32(o) && (dc.src_wrapped || (dc.sigma_est > 4294967296.0 && dc.sigma_est <= 4.6e18));
 }
 
-// Sources of k tiles of `width` evenly spaced over the component's tile order.
-static std::vector<int32_t> sample_tiles(DComp &dc, int64_t k, int64_t width) {
-    const std::vector<int32_t> order = batched_order(dc);
-    const int64_t T = ((int64_t)dc.n + width - 1) / width;
-    k = std::min(k, T);
-    std::vector<int32_t> out;
-    for (int64_t i = 0; i < k; ++i) {
-        const int64_t t = (2 * i + 1) * T / (2 * k);
-        for (int64_t v = t * width; v < std::min<int64_t>((t + 1) * width, dc.n); ++v)
-            out.push_back(order[(size_t)v]);
-    }
-    return out;
-}
-
-// The kernel with the least estimated time for n_src sources, from the rates
-// measured on the samples (0: not measured).
-static int measured_kind(bcx_ctx *ctx, const DComp &dc, int64_t n_src) {
-    const double cus = std::max(1, ctx->n_cu), s = (double)n_src;
-    int kind = BCX_KERNEL_MULTI;
-    // (one tile alone runs at 0.7 of the rate of eight)
-    double best = dc.rate_multi > 0 ? s / dc.rate_multi * (n_src < 8 * BATCH_W * MAX_SPL ? 1.4 : 1.0) : 1e30;
-    if (dc.rate_wg > 0) {
-        const double t = std::ceil(std::ceil(s / BATCH_W) / cus) * dc.round_wg / dc.rate_wg;
-        if (t < best) {
-            best = t;
-            kind = BCX_KERNEL_WG;
-        }
-    }
-    if (dc.rate_src > 0 && std::max(s, cus) / dc.rate_src < best) kind = KIND_SOURCE;
-    return kind;
-}
-
-int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *opts, int64_t n_src, bcx_stats *st) {
-    int kind0 = batched_kind(dc, opts->flags);
-    if (kind0 == BCX_KERNEL_SMALL) return kind0;
-    int route = FP32_ANY, rc = fp32_route(ctx, dc, opts, &route);
-    if (rc) return rc;
-    const bool sliced = route == FP32_TILES;
-    if (sliced) kind0 = BCX_KERNEL_MULTI;
-    const bcx_opts own = batched_opts(dc, *opts), *o = &own;
-    const bool kind_fixed = sliced || (o->flags & (BCX_FLAG_NO_WG_KERNEL | BCX_FLAG_WG_KERNEL)) != 0;
-    // (the rows of the per-source kernel have to fit beside the tiles' buffers)
-    const bool wraps = counts_may_wrap(dc, o);
-    const bool source_fits = !wraps && plain_scratch_fits(ctx, dc.n, n_src);
-    if (wraps && route == FP32_ROWS) return BCX_KERNEL_WG;
-    if ((o->flags & BCX_FLAG_NO_TUNE) || dc.n < TUNE_N)
-        return kind0 == BCX_KERNEL_WG && !kind_fixed && source_fits && !valid_spl(o->sources_per_lane) ? KIND_SOURCE
-                                                                                                       : kind0;
-    const bool need_kind = !kind_fixed && !dc.kind_measured;
-    int kind = kind_fixed ? kind0 : (dc.kind_measured ? measured_kind(ctx, dc, n_src) : -1);
-    if (kind == KIND_SOURCE && !source_fits) kind = kind0;
-    // (tiles of whole rows run under the defaults: six candidates twice cost more
-    // than a dozen full jobs of a component below the line)
-    const bool need_multi = !dc.sched_multi && (need_kind || kind == BCX_KERNEL_MULTI) && route != FP32_ROWS;
-    if (!need_kind && !need_multi) return kind;
-    // the run's timer is set aside: the samples are timed on their own
+namespace {
+// The samples of one component under one run's options.  The run's timer is
+// set aside while it lives: the samples are timed on their own.
+struct Tuner {
+    bcx_ctx *ctx;
+    DComp &dc;
+    bcx_opts o;
+    MultiSched base;  // the defaults, or what the options fix
     Timer keep;
-    std::swap(keep, ctx->timer);
     DBuf scratch;
-    rc = scratch.ensure(ctx, 8 * ((size_t)dc.offset + (size_t)dc.n), "tuner scratch");
-    bcx_opts to = *o;
-    to.src_subset = nullptr;
-    to.n_src = 0;
-    double *bc = (double *)scratch.p;
-    auto time_multi = [&](const std::vector<int32_t> &srcs, const MultiSched &m, double *rate) {
-        double t = 0.0;
-        int r = BCX_OK;
-        for (int rep = 0; rep < 2 && !r; ++rep) {
-            r = multi_run(ctx, dc, srcs, &to, m, bc + dc.offset, nullptr);
-            t = ctx->timer.collect();
+    std::vector<int32_t> order, samp;
+    bool on = false;
+    Tuner(bcx_ctx *c, DComp &d, const bcx_opts &opts) : ctx(c), dc(d), o(opts), base(multi_sched(d, &opts)) {
+        o.src_subset = nullptr;
+        o.n_src = 0;
+    }
+    ~Tuner() {
+        if (!on) return;
+        std::swap(keep, ctx->timer);
+        keep.destroy();
+        scratch.release(ctx);
+    }
+    int begin() {
+        if (on) return BCX_OK;
+        const int rc = scratch.ensure(ctx, 8 * ((size_t)dc.offset + (size_t)dc.n), "tuner scratch");
+        if (rc) return rc;
+        std::swap(keep, ctx->timer);
+        order = batched_order(dc);
+        on = true;
+        return BCX_OK;
+    }
+    double *bc() { return (double *)scratch.p; }
+    // Sources of k tiles of `width` evenly spaced over the component's tile order.
+    std::vector<int32_t> tiles(int64_t k, int64_t width) {
+        const int64_t T = ((int64_t)dc.n + width - 1) / width;
+        k = std::min(k, T);
+        std::vector<int32_t> out;
+        for (int64_t i = 0; i < k; ++i) {
+            const int64_t t = (2 * i + 1) * T / (2 * k);
+            for (int64_t v = t * width; v < std::min<int64_t>((t + 1) * width, dc.n); ++v)
+                out.push_back(order[(size_t)v]);
         }
-        *rate = t > 0 ? (double)srcs.size() / t : 0.0;
-        return r;
-    };
-    auto time_wg = [&](const std::vector<int32_t> &srcs, double *rate) {
-        double t = 0.0;
-        int r = BCX_OK;
-        std::vector<SmallJob> jobs{{&dc, srcs}};
-        for (int rep = 0; rep < 2 && !r; ++rep) {
-            r = persistent_start(ctx, jobs, &to, bc, nullptr, true, ctx->stream, false);
-            if (!r) r = persistent_finish(ctx, nullptr, true);
-            t = ctx->timer.collect();
+        return out;
+    }
+    // Seconds of the second of two runs.
+    template <typename F>
+    int timed(double *t, F run) {
+        int rc = begin();
+        for (int rep = 0; rep < 2 && !rc; ++rep) {
+            rc = run();
+            *t = ctx->timer.collect();
         }
-        *rate = t > 0 ? (double)srcs.size() / t : 0.0;
-        return r;
-    };
-    const MultiSched base = multi_sched(dc, o);  // the defaults, or what the options fix
+        return rc;
+    }
+    int multi(const std::vector<int32_t> &srcs, const MultiSched &m, double *t) {
+        return timed(t, [&] { return multi_run(ctx, dc, srcs, &o, m, bc() + dc.offset, nullptr); });
+    }
     // every multi-launch candidate runs the same sources: TUNE_TILES tiles of
     // the widest lanes, which narrower lanes cut into more tiles (a sample of
     // 64-source tiles left the wide candidates a few tiles for eight slots and
     // picked 128-source tiles where 256-source ones run 10% faster)
-    std::vector<int32_t> samp;
-    double r_multi = 0.0;
-    if (!rc && need_kind) {
-        dc.rate_src = dc.rate_wg = dc.rate_multi = 0.0;
-        if (source_fits && !valid_spl(o->sources_per_lane)) {
-            std::vector<int32_t> ss;
-            const int64_t k = std::min<int64_t>(dc.n <= WG_N ? TUNE_SOURCES : TUNE_SOURCES / 8, dc.n);
-            for (int64_t i = 0; i < k; ++i) ss.push_back((int32_t)(i * dc.n / k));
+    int multi(const MultiSched &m, double *t) {
+        const int rc = begin();
+        if (rc) return rc;
+        if (samp.empty()) samp = tiles(TUNE_TILES, (int64_t)BATCH_W * MAX_SPL);
+        return multi(samp, m, t);
+    }
+    int wg(double *t) {
+        const int rc = begin();
+        if (rc) return rc;
+        const std::vector<SmallJob> jobs{{&dc, tiles(std::max(1, ctx->n_cu), (int64_t)BATCH_W * wg_spl(&o))}};
+        return timed(t, [&] {
+            const int r = persistent_start(ctx, jobs, &o, bc(), nullptr, true, ctx->stream, false);
+            return r ? r : persistent_finish(ctx, nullptr, true);
+        });
+    }
+    int source(int64_t k, double *t, bool *overflow) {
+        std::vector<int32_t> ss;
+        for (int64_t i = 0; i < k; ++i) ss.push_back((int32_t)(i * dc.n / k));
+        return timed(t, [&] {
+            return *overflow ? BCX_OK
+                             : source_component(ctx, dc, ss, &o, bc() + dc.offset, nullptr, overflow);
+        });
+    }
+};
+}  // namespace
+
+// What was measured of a component under these options.
+static KindTimes &kind_times(DComp &dc, const bcx_opts *o) {
+    const std::array<int32_t, 5> key = {run_fp32(o), want_cut(o), valid_spl(o->sources_per_lane) ? o->sources_per_lane : 0,
+                                        o->batch_width, o->blocks_per_cu};
+    for (KindTimes &t : dc.times)
+        if (t.key == key) return t;
+    dc.times.emplace_back();
+    dc.times.back().key = key;
+    return dc.times.back();
+}
+
+// The kernel with the least estimated time for n_src sources.  by_source: the
+// per-source kernel is a candidate; rows: tiles sum whole rows.
+static int measured_kind(Tuner &t, int64_t n_src, bool by_source, bool rows, int *kind) {
+    KindTimes &r = kind_times(t.dc, &t.o);
+    const double cus = std::max(1, t.ctx->n_cu), s = (double)n_src;
+    const bool fp32 = run_fp32(&t.o);
+    double src = 1e30;
+    *kind = KIND_SOURCE;
+    int rc;
+    if (by_source) {
+        // (a round of the launch takes as long with fewer sources)
+        const int64_t round = (int64_t)cus * plain_shape(t.dc.n, fp32).per_cu, k = std::min<int64_t>(2 * round, t.dc.n);
+        if (r.src < 0 && plain_scratch_fits(t.ctx, t.dc.n, k)) {
+            double x = 0.0;
             bool overflow = false;
-            rc = source_component(ctx, dc, ss, &to, bc + dc.offset, nullptr, &overflow);
-            const double t = ctx->timer.collect();
-            dc.rate_src = t > 0 && !overflow ? (double)k / t : 0.0;
+            if ((rc = t.source(k, &x, &overflow))) return rc;
+            if (!overflow) r.src = x / (double)k;
+            if (overflow && rows) {  // (see counts_may_wrap)
+                *kind = BCX_KERNEL_WG;
+                return BCX_OK;
+            }
         }
-        if (!rc && dc.rate_src == 0.0 && dc.n <= WG_N) {
-            const std::vector<int32_t> ws = sample_tiles(dc, std::max(1, ctx->n_cu), (int64_t)BATCH_W * wg_spl(o));
-            rc = time_wg(ws, &dc.rate_wg);
-            dc.round_wg = (double)ws.size();
-        }
+        if (r.src >= 0) src = std::max(s, (double)round) * r.src;
+        // (deep components: three launches per level alone take the tiles longer
+        // than half of what the per-source kernel takes)
+        if (r.src >= 0 && t.dc.depth >= 0 &&
+            r.src < 6.0 * (t.dc.depth + 1) * LAUNCH_S / (MAX_SLOTS * BATCH_W * MAX_SPL))
+            return BCX_OK;
     }
-    const double per_src = need_kind && dc.rate_src > 0 ? 1.0 / dc.rate_src : 0.0;
-    const double launches = 3.0 * (dc.depth + 1) * LAUNCH_S / (MAX_SLOTS * BATCH_W * MAX_SPL);
-    if (!rc && !(per_src > 0 && dc.depth >= 0 && per_src < 2 * launches)) {
-        samp = sample_tiles(dc, TUNE_TILES, (int64_t)BATCH_W * MAX_SPL);
-        rc = time_multi(samp, base, &r_multi);
+    if (r.tile < 0) {
+        if ((rc = t.begin()) || (rc = t.multi(t.tiles(1, BATCH_W * MAX_SPL), t.base, &r.tile))) return rc;
     }
-    if (!rc && need_kind) {
-        dc.rate_multi = r_multi;
-        dc.kind_measured = true;
-        kind = measured_kind(ctx, dc, n_src);
+    if (src <= r.tile) return BCX_OK;
+    if (r.more < 0) {
+        double x = 0.0;
+        if ((rc = t.multi(t.base, &x))) return rc;
+        const double more = (double)t.samp.size() - BATCH_W * MAX_SPL;
+        r.more = more > 0 ? std::max(0.0, x - r.tile) / more : 0.0;
     }
-    MultiSched best = base;
-    const bool tune_multi = need_multi && kind == BCX_KERNEL_MULTI;
-    if (!rc && tune_multi) {
+    const double tiles = r.tile + r.more * std::max(0.0, s - BATCH_W * MAX_SPL);
+    if (tiles < src) *kind = BCX_KERNEL_MULTI;
+    // the workgroup tiles: a round of them lasts as long with fewer sources, so
+    // beside the per-source kernel they are looked at from half a round on, and
+    // only where tiles of whole rows are the alternative
+    const double wide = BATCH_W * wg_spl(&t.o);
+    if (t.dc.n <= WG_N && (src == 1e30 || (rows && s >= 0.5 * cus * wide))) {
+        if (r.wg < 0 && (rc = t.wg(&r.wg))) return rc;
+        if (std::ceil(std::ceil(s / wide) / cus) * r.wg < std::min(src, tiles)) *kind = BCX_KERNEL_WG;
+    }
+    return BCX_OK;
+}
+
+int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *opts, int64_t n_src, bcx_stats *st) {
+    const int kind0 = batched_kind(dc, opts->flags);
+    if (kind0 == BCX_KERNEL_SMALL) return kind0;
+    int route = FP32_ANY, rc = fp32_route(ctx, dc, opts, &route);
+    if (rc) return rc;
+    const bcx_opts own = batched_opts(dc, *opts), *o = &own;
+    const bool fixed = (o->flags & (BCX_FLAG_NO_WG_KERNEL | BCX_FLAG_WG_KERNEL)) != 0;
+    const bool wraps = counts_may_wrap(dc, o);
+    // (a lane width asks for tiles; the per-source kernel's rows have to fit)
+    const bool by_source = !fixed && route != FP32_TILES && !wraps && !valid_spl(o->sources_per_lane) &&
+                           plain_scratch_fits(ctx, dc.n, n_src);
+    if ((o->flags & BCX_FLAG_NO_TUNE) || dc.n < TUNE_N) return kind0 == BCX_KERNEL_WG && by_source ? KIND_SOURCE : kind0;
+    Tuner t(ctx, dc, own);
+    int kind = kind0;
+    if (!fixed) {
+        if (route == FP32_TILES || (dc.n > WG_N && !by_source)) kind = BCX_KERNEL_MULTI;
+        else if (wraps && route == FP32_ROWS) kind = BCX_KERNEL_WG;
+        else if ((rc = measured_kind(t, n_src, by_source, route == FP32_ROWS, &kind))) return rc;
+    }
+    // (tiles of whole rows run under the defaults: six candidates twice cost more
+    // than a dozen full jobs of a component below the line)
+    if (kind == BCX_KERNEL_MULTI && !dc.sched_multi && route != FP32_ROWS) {
+        const MultiSched base = t.base;
+        MultiSched best = base;
         std::vector<MultiSched> cands;
         if (o->blocks_per_cu <= 0)
             for (int bpc : {4, 16}) cands.push_back({base.cut, bpc, base.slots, base.spl});
         if (o->batch_width <= 0) cands.push_back({base.cut, base.bpc, 4, base.spl});
-        if (base.cut && !sliced) cands.push_back({false, base.bpc, base.slots, base.spl});
+        if (base.cut && route != FP32_TILES) cands.push_back({false, base.bpc, base.slots, base.spl});
         if (!valid_spl(o->sources_per_lane))
             for (int w : {1, 2, 4})
                 if (w != base.spl) cands.push_back({base.cut, base.bpc, base.slots, w});
-        double r_best = r_multi;
+        double t_best = 0.0;
+        if ((rc = t.multi(base, &t_best))) return rc;
         for (const MultiSched &m : cands) {
-            double r = 0.0;
-            if ((rc = time_multi(samp, m, &r))) break;
-            if (r > 1.03 * r_best) {
-                r_best = r;
+            double x = 0.0;
+            if ((rc = t.multi(m, &x))) return rc;
+            if (t_best > 1.03 * x) {
+                t_best = x;
                 best = m;
             }
         }
-    }
-    std::swap(keep, ctx->timer);
-    keep.destroy();
-    scratch.release(ctx);
-    if (rc) return rc;
-    if (tune_multi) {
         // (a choice the options fixed is not cached: later runs may leave it free)
         dc.sched_multi = true;
         dc.sched_cut = (base.cut && !best.cut) ? 0 : 1;
@@ -2096,7 +2140,7 @@ int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *opts, int64_t n_sr
         dc.sched_spl = (int8_t)(valid_spl(o->sources_per_lane) ? 0 : best.spl);
         dc.sched_slots = (int16_t)(o->batch_width > 0 ? 0 : best.slots);
     }
-    if (st) st->n_tuned++;
+    if (st && t.on) st->n_tuned++;
     return kind;
 }
 

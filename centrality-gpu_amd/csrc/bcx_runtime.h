@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <map>
 #include <string>
 #include <utility>
@@ -47,6 +48,17 @@ struct HostComp {
     std::vector<int32_t> ch_ptr, ch_nodes, ch_ends;
 };
 
+// Seconds measured on a component (negative: not yet), under the options of
+// `key` (FP32C, chains contracted, sources per lane, tiles in flight, blocks
+// per CU).
+struct KindTimes {
+    std::array<int32_t, 5> key{};
+    double src = -1.0;   // a source on the per-source kernel, of a full launch
+    double tile = -1.0;  // a multi-launch tile alone
+    double more = -1.0;  // each source past its own
+    double wg = -1.0;    // a round of the workgroup kernel's tiles
+};
+
 struct DComp {
     int32_t n = 0;
     int64_t arcs = 0;
@@ -85,12 +97,9 @@ struct DComp {
     // FP32C: rounding of the component's terms without and with chains to
     // contract (FP32_ROWS or FP32_TILES; -1 not yet looked at)
     int8_t fp32_route[2] = {-1, -1};
-    // batched path: the schedule measured on sample sources, cached for every
-    // later run of the component (sources per second on each kernel, 0: not a
-    // candidate; round_wg: sources of a full round of workgroup tiles;
-    // sched_multi: the multi-launch fields below were measured)
-    bool kind_measured = false;
-    double rate_multi = 0.0, rate_wg = 0.0, rate_src = 0.0, round_wg = 0.0;
+    // batched path: what was measured on sample sources, cached for every later
+    // run under the same options (sched_multi: the multi-launch fields below were)
+    std::vector<KindTimes> times;
     bool sched_multi = false;
     int8_t sched_cut = 1;     // multi-launch: 1 contracted chains, 0 the relabelled copy
     int16_t sched_bpc = 0;    // multi-launch: level-kernel blocks per CU (0: default)

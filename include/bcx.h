@@ -230,8 +230,9 @@ typedef struct {
     int32_t n_comp_small;      /* batched: components run on the small-component */
     int32_t n_comp_wg;         /*   kernels, one workgroup per source or tile */
     int32_t n_comp_multi;      /*   and the multi-launch tiles                */
-    int32_t n_tuned;           /* batched: components whose schedule was measured
-                                  (the schedule of each is measured once)     */
+    int32_t n_tuned;           /* batched: components run on samples before this
+                                  run (each sample is taken once, when a choice
+                                  first depends on it)                        */
     int32_t sched_blocks_per_cu; /* batched: blocks per CU, tiles in flight and */
     int32_t sched_slots;       /*   sources per lane of the largest           */
     int32_t sched_sources_per_lane; /* multi-launch component                 */

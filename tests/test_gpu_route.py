@@ -67,6 +67,44 @@ def test_per_source_runs_are_told_apart(engine):
         g.free()
 
 
+@pytest.mark.parametrize("prec", [bcx.PREC_FP64, F32])
+@pytest.mark.parametrize("width_first", [False, True])
+def test_lane_width_is_kept_and_keeps_nothing(engine, prec, width_first):
+    """A run that fixes the sources per lane gets tiles of that width, whatever
+    earlier runs of the component measured, and leaves no choice behind for
+    those that do not (a 17k grid: source by source)."""
+    c = giant(4, 0.23)
+    assert c.n >= 16384
+    sub = np.arange(0, c.n, 67)
+    g = engine.upload([c])
+    try:
+        seen = []
+        for width in ([1, 0, 1, 0] if width_first else [0, 1, 0, 1]):
+            bc, st = g.run(path=B, precision=prec, subset=sub, sources_per_lane=width)
+            seen.append(bc)
+            assert engine.run_by_source() == (0 if width else 1), (width, st)
+            assert not width or st["n_comp_wg"] == 1 or st["sched_sources_per_lane"] == width
+        for bc in seen[1:]:
+            assert far(bc, seen[0]) < SAME
+    finally:
+        g.free()
+
+
+def test_precisions_are_measured_apart(engine):
+    """Counts that leave 64 bits end FP32C's per-source runs of a component, not
+    those with FP64 terms, in either order; the overflow is met once."""
+    c = giant(4, 0.035, 0)
+    sub = np.arange(0, c.n, 2)
+    for order in ((F32, bcx.PREC_FP64), (bcx.PREC_FP64, F32)):
+        g = engine.upload([c])
+        try:
+            for prec in order + order:
+                g.run(path=B, precision=prec, subset=sub)
+                assert engine.run_by_source() == (prec == bcx.PREC_FP64)
+        finally:
+            g.free()
+
+
 @pytest.mark.parametrize("cfg,scale,seed,bits", [(4, 0.035, 0, 0), (4, 0.035, 2, 0), (4, 0.03, 5, 0),
                                                  (2, 0.006, 3, 8), (2, 0.006, 3, 9)])
 def test_the_same_sources_turn_to_fp64(engine, cfg, scale, seed, bits):
