@@ -2110,9 +2110,12 @@ int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *opts, int64_t n_sr
         else if (wraps && route == FP32_ROWS) kind = BCX_KERNEL_WG;
         else if ((rc = measured_kind(t, n_src, by_source, route == FP32_ROWS, &kind))) return rc;
     }
-    // (tiles of whole rows run under the defaults: six candidates twice cost more
-    // than a dozen full jobs of a component below the line)
-    if (kind == BCX_KERNEL_MULTI && !dc.sched_multi && route != FP32_ROWS) {
+    // (below the line the tiles run under the defaults: the candidates cost 200 to
+    // 300 ms and none gained on power-law cores of 34k and 67k vertices, 20.5 and
+    // 23.0 ms for 6144 sources against 21.9 and 24.2 tuned, nor on R-MAT cores of
+    // 23k and 45k, 13.3 and 19.8 against 13.9 and 22.1)
+    const bool below = !fixed && dc.n <= WG_N && dc.n <= fp32_line(dc, want_cut(opts));
+    if (kind == BCX_KERNEL_MULTI && !dc.sched_multi && !below) {
         const MultiSched base = t.base;
         MultiSched best = base;
         std::vector<MultiSched> cands;

@@ -7,6 +7,8 @@ to 7e-9 apart).  So a component runs on them in every call or in none, and
 counts past 64 bits turn the same 64 sources to FP64 terms on whichever kernel
 they are met.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -103,6 +105,28 @@ def test_precisions_are_measured_apart(engine):
                 assert engine.run_by_source() == (prec == bcx.PREC_FP64)
         finally:
             g.free()
+
+
+def test_first_call_on_a_mid_size_core(engine):
+    """The first run of a 23k R-MAT core takes the samples that its choice of
+    kernel needs; only a run that asks for the multi-launch tiles, and a core
+    above the line, pays for a tuned schedule (six candidates twice)."""
+    c = giant(5, 0.06)
+    g = engine.upload([c])
+    kw = dict(path=B, subset=np.arange(64))
+    g.run(**kw)  # (code objects, buffers)
+    g.free()
+    took = {}
+    for flags in (0, bcx.FLAG_NO_WG_KERNEL):
+        g = engine.upload([c])
+        try:
+            t = time.perf_counter()
+            g.run(flags=flags, **kw)
+            took[flags] = time.perf_counter() - t
+        finally:
+            g.free()
+    print("case first call", {k: round(1e3 * v, 1) for k, v in took.items()}, flush=True)
+    assert took[0] < 0.6 * took[bcx.FLAG_NO_WG_KERNEL]
 
 
 @pytest.mark.parametrize("cfg,scale,seed,bits", [(4, 0.035, 0, 0), (4, 0.035, 2, 0), (4, 0.03, 5, 0),
