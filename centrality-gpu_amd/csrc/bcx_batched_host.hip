@@ -129,7 +129,7 @@ static int bs_ensure(bcx_ctx *ctx, int32_t n, int32_t n_src, int want_slots, boo
     if (!ctx->batched) ctx->batched = new BatchedState();
     BatchedState &bs = *ctx->batched;
     const size_t per = (size_t)n * MAX_SPL * (8 + 24 + 512 + 512 + 8 * 12) + (1 << 20);
-    const size_t room = ctx->mem_cap > ctx->mem_used ? (ctx->mem_cap - ctx->mem_used) : 0;
+    const size_t room = ctx_room(ctx);
     int fit = (int)std::max<size_t>(1, std::min<size_t>(MAX_SLOTS, room / 2 / std::max<size_t>(per, 1)));
     bs.n_slots = std::max(1, std::min(want_slots, fit));
     int rc;
@@ -1543,7 +1543,7 @@ static int persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, con
     const int64_t per_cu = wg ? 1 : small_blocks_per_cu(nmax, csr);
     int64_t grid = std::max<int64_t>(1, std::min<int64_t>((int64_t)tiles.size(), per_cu * (int64_t)ctx->n_cu));
     if (wg) {
-        const size_t room = ctx->mem_cap > ctx->mem_used ? (ctx->mem_cap - ctx->mem_used) / 2 : 0;
+        const size_t room = ctx_room(ctx) / 2;
         grid = std::max<int64_t>(1, std::min<int64_t>(grid, (int64_t)(room / per_wg)));
     }
     if ((rc = ss.sig.ensure(ctx, 8 * slab * grid, "persistent sigma")) ||
@@ -2054,8 +2054,9 @@ static int measured_kind(Tuner &t, int64_t n_src, bool by_source, bool rows, int
         if (r.src < 0 && plain_scratch_fits(t.ctx, t.dc.n, k)) {
             double x = 0.0;
             bool overflow = false;
-            if ((rc = t.source(k, &x, &overflow))) return rc;
-            if (!overflow) r.src = x / (double)k;
+            rc = t.source(k, &x, &overflow);
+            if (rc && rc != BCX_E_NOMEM) return rc;  // (no room: the tiles)
+            if (!rc && !overflow) r.src = x / (double)k;
             if (overflow && rows) {  // (see counts_may_wrap)
                 *kind = BCX_KERNEL_WG;
                 return BCX_OK;
@@ -2080,11 +2081,11 @@ static int measured_kind(Tuner &t, int64_t n_src, bool by_source, bool rows, int
     }
     const double tiles = r.tile + r.more * std::max(0.0, s - BATCH_W * MAX_SPL);
     if (tiles < src) *kind = BCX_KERNEL_MULTI;
-    // the workgroup tiles: a round of them lasts as long with fewer sources, so
-    // beside the per-source kernel they are looked at from half a round on, and
-    // only where tiles of whole rows are the alternative
+    // the workgroup tiles, where a lane width asks for tiles; else a round of
+    // them lasts as long with fewer sources, so they are looked at from half a
+    // round on, beside the per-source kernel and tiles of whole rows
     const double wide = BATCH_W * wg_spl(&t.o);
-    if (t.dc.n <= WG_N && (src == 1e30 || (rows && s >= 0.5 * cus * wide))) {
+    if (t.dc.n <= WG_N && (valid_spl(t.o.sources_per_lane) || (rows && src < 1e30 && s >= 0.5 * cus * wide))) {
         if (r.wg < 0 && (rc = t.wg(&r.wg))) return rc;
         if (std::ceil(std::ceil(s / wide) / cus) * r.wg < std::min(src, tiles)) *kind = BCX_KERNEL_WG;
     }

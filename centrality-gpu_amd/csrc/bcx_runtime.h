@@ -149,6 +149,7 @@ struct bcx_ctx {
     double *bc_pin = nullptr;      // pinned host staging of the result download
     size_t bc_pin_bytes = 0;
     int32_t *up_pin = nullptr;     // pinned host staging of small uploads
+    int rows_held = 0;             // plain_scratch and bc_split belong to a launch being put together
     int32_t by_source = 0;         // batched: components the last run took source by source
     bool busy = true;              // work may be in flight on the context stream
     BatchedState *batched = nullptr;
@@ -172,6 +173,9 @@ int ctx_fail(bcx_ctx *ctx, int code, const std::string &msg);
 int ctx_hip(bcx_ctx *ctx, hipError_t e, const char *what);
 int dev_alloc(bcx_ctx *ctx, void **p, size_t bytes, const char *what);
 void dev_free(bcx_ctx *ctx, void *p);
+// Device memory that allocations can still get under the cap (what the idle
+// rows of the per-source kernel hold is given back for them).
+size_t ctx_room(const bcx_ctx *ctx);
 int upload(bcx_ctx *ctx, const void *host, size_t bytes, bcx::DBuf &buf, const char *what);
 int read_counters(bcx_ctx *ctx, bcx_stats *st);
 int64_t row_capacity(bcx_ctx *ctx, int32_t n, const bcx_opts *o);

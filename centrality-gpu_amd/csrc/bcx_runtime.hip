@@ -39,16 +39,36 @@ int ctx_hip(bcx_ctx *ctx, hipError_t e, const char *what) {
                     std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// The per-source kernel's rows and accumulators are kept from run to run for
+// speed alone: where an allocation finds no room beside them they are given
+// back (hipFree waits for what still runs on them).
+static bool give_rows_back(bcx_ctx *ctx) {
+    if (ctx->rows_held || (!ctx->plain_scratch.p && !ctx->bc_split.p)) return false;
+    ctx->plain_scratch.release(ctx);
+    ctx->bc_split.release(ctx);
+    return true;
+}
+
+size_t ctx_room(const bcx_ctx *ctx) {
+    const size_t rows = ctx->rows_held ? 0 : ctx->plain_scratch.bytes + ctx->bc_split.bytes;
+    return ctx->mem_cap + rows > ctx->mem_used ? ctx->mem_cap + rows - ctx->mem_used : 0;
+}
+
 int dev_alloc(bcx_ctx *ctx, void **p, size_t bytes, const char *what) {
     *p = nullptr;
     if (bytes == 0) bytes = 64;
     bytes = (bytes + 255) & ~(size_t)255;
+    if (ctx->mem_used + bytes > ctx->mem_cap && ctx_room(ctx) >= bytes) (void)give_rows_back(ctx);
     if (ctx->mem_used + bytes > ctx->mem_cap)
         return ctx_fail(ctx, BCX_E_NOMEM,
                         std::string("device memory cap exceeded allocating ") + what + " (" +
                             std::to_string(bytes) + " B, " + std::to_string(ctx->mem_used) +
                             " of " + std::to_string(ctx->mem_cap) + " B in use)");
     hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && give_rows_back(ctx)) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
     if (e != hipSuccess) {
         *p = nullptr;
         return ctx_hip(ctx, e, what);
@@ -327,6 +347,13 @@ static int plain_grid(bcx_ctx *ctx, int32_t n, int64_t count, const PlainShape &
     return (int)std::max(g, plain_min_grid(ctx, count));
 }
 
+// While it lives, the context's rows belong to a launch being put together.
+struct RowsHeld {
+    bcx_ctx *ctx;
+    explicit RowsHeld(bcx_ctx *c) : ctx(c) { ctx->rows_held++; }
+    ~RowsHeld() { ctx->rows_held--; }
+};
+
 static int ensure_plain_scratch(bcx_ctx *ctx, int32_t n, int grid, PlainScratch &sc) {
     const int64_t stride = plain_stride(n);
     const size_t per = (size_t)stride * PLAIN_WORD_BYTES;
@@ -368,6 +395,7 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
                         double *probe = nullptr, bool fp32 = false, bool ordered = false) {
     if (src.empty()) return BCX_OK;
     int rc;
+    const RowsHeld held(ctx);
     if ((rc = ctx->w_src.ensure(ctx, src.size() * 4, "work list"))) return rc;
     if ((rc = upload(ctx, slot.data(), slot.size() * 4, ctx->w_aux, "work list"))) return rc;
     if ((rc = upload(ctx, mode.data(), mode.size(), ctx->w_mode, "work list"))) return rc;
@@ -514,6 +542,7 @@ static int run_chain_list(bcx_ctx *ctx, const DComp &dc, const PlanBatch &b, boo
                           const Rows &rows, bcx_stats *st, double *probe = nullptr) {
     if (b.cci.empty()) return BCX_OK;
     int rc;
+    const RowsHeld held(ctx);
     if ((rc = upload(ctx, b.cci.data(), b.cci.size() * 4, ctx->w_src, "chain list"))) return rc;
     if ((rc = upload(ctx, b.cpos.data(), b.cpos.size() * 4, ctx->w_aux, "chain list"))) return rc;
     if ((rc = upload(ctx, b.cslots.data(), b.cslots.size() * 4, ctx->w_slots, "chain list"))) return rc;
@@ -1035,12 +1064,12 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
             const bcx_opts own = batched_opts(dc, o);
             if ((rc = batched_component(ctx, dc, jb.srcs, &own, bc + dc.offset, s))) return rc;
         }
-        std::vector<SmallJob> again;  // FP32 terms, overflowed counts
+        std::vector<SmallJob> again;  // FP32 terms with overflowed counts, or no room for rows beside the tiles
         for (SmallJob &jb : single) {
             bool overflow = false;
-            if ((rc = source_component(ctx, *const_cast<DComp *>(jb.dc), jb.srcs, &o, bc + jb.dc->offset, s, &overflow)))
-                return rc;
-            if (overflow) again.push_back(std::move(jb));
+            rc = source_component(ctx, *const_cast<DComp *>(jb.dc), jb.srcs, &o, bc + jb.dc->offset, s, &overflow);
+            if (rc && rc != BCX_E_NOMEM) return rc;
+            if (rc || overflow) again.push_back(std::move(jb));  // (nothing was added)
             else ctx->by_source++;
         }
         if ((rc = batched_persistent_finish(ctx, s, PASS_SRC)) || (rc = batched_persistent_finish(ctx, s, PASS_SMALL)) ||
@@ -1050,6 +1079,13 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
             // (in the order of the tiles: those around an overflow turn to FP64)
             DComp &dc = *const_cast<DComp *>(jb.dc);
             const std::vector<SmallJob> tiles{{&dc, tuned_sources(dc, jb.srcs)}};
+            if (dc.n > WG_N) {
+                const bcx_opts own = batched_opts(dc, o);
+                if ((rc = batched_prepare(ctx, dc, &own)) ||
+                    (rc = batched_component(ctx, dc, tiles[0].srcs, &own, bc + dc.offset, s)))
+                    return rc;
+                continue;
+            }
             if ((rc = batched_persistent_start(ctx, tiles, &o, bc, s, PASS_WG, ctx->stream)) ||
                 (rc = batched_persistent_finish(ctx, s, PASS_WG)))
                 return rc;

@@ -1,0 +1,88 @@
+"""Batched runs under a memory cap: the per-source kernel's rows are an option,
+so a job that the tiles alone have room for is never refused for them."""
+import numpy as np
+import pytest
+
+import bcx
+import oracle
+from helpers import relerr
+
+pytestmark = pytest.mark.gpu
+
+B = bcx.PATH_BATCHED
+
+
+def giant(cfg, scale):
+    n, uv = bcx.generate(cfg, 0, scale)
+    return max(bcx.Host.from_edges(n, uv).decompose().components(), key=lambda c: c.n)
+
+
+def rows(engine, c, sources):
+    """Bytes of the rows that a per-source run takes at least."""
+    return (c.n + 2 + 63) // 64 * 64 * 28 * min(sources, 2 * engine.info()[0])
+
+
+def slot(c):
+    """Bytes of a multi-launch tile in flight, about."""
+    return c.n * 4 * (8 + 24 + 512 + 512 + 96)
+
+
+def check(g, c, sub, tol, **kw):
+    got, st = g.run(path=B, subset=sub, **kw)
+    want = oracle.component_bc(c.row_ptr, c.col, c.reach, sources=sub.astype(np.int32), threads=16)
+    mx, _, zeros = relerr(got, want)
+    assert mx < tol and zeros, mx
+    return st
+
+
+@pytest.mark.parametrize("prec,tol", [(bcx.PREC_FP64, 1e-9), (bcx.PREC_FP32C, 1e-6)])
+def test_first_run_of_few_sources(engine, prec, tol):
+    """An 18.6k core, 64 sources first, under a cap with room for two tiles in
+    flight and the rows of 64 sources, not for those of the tuner's sample."""
+    c = giant(2, 0.022)
+    assert c.n >= 16384
+    cap = 2 * slot(c) + rows(engine, c, 64)
+    assert cap < rows(engine, c, c.n) + slot(c)
+    eng = bcx.Engine(0, mem_cap=cap)
+    try:
+        g = eng.upload([c])
+        for k in (64, 700):
+            check(g, c, np.linspace(0, c.n - 1, k).astype(np.int64), tol, precision=prec)
+        g.free()
+    finally:
+        eng.close()
+
+
+def test_rows_make_room_for_tiles(engine):
+    """A cap with room for a deep component's rows or one tile in flight, not
+    both: source by source, then on the tiles, then as there is room."""
+    c = giant(4, 0.23)
+    assert c.n >= 16384
+    eng = bcx.Engine(0, mem_cap=rows(engine, c, c.n) + slot(c) // 2 + (16 << 20))
+    sub = np.linspace(0, c.n - 1, 600).astype(np.int64)
+    try:
+        g = eng.upload([c])
+        for flags in (0, bcx.FLAG_NO_WG_KERNEL | bcx.FLAG_NO_TUNE, bcx.FLAG_NO_TUNE):
+            check(g, c, sub, 1e-9, flags=flags)
+            assert flags or eng.run_by_source() == 1
+        g.free()
+    finally:
+        eng.close()
+
+
+def test_tiles_and_rows_in_one_run(engine):
+    """Two components, one for the tiles and one for the per-source kernel, under
+    a cap that the tiles fill: the other goes to the tiles as well."""
+    a, b = giant(5, 0.12), giant(4, 0.2)
+    eng = bcx.Engine(0, mem_cap=int(1.15 * slot(a)) + rows(engine, b, b.n) // 2 + (20 << 20))
+    sub = np.concatenate([np.linspace(0, a.n - 1, 64).astype(np.int64), a.n + np.linspace(0, b.n - 1, 600).astype(np.int64)])
+    try:
+        g = eng.upload([a, b])
+        got, _ = g.run(path=B, subset=sub, flags=bcx.FLAG_NO_TUNE)
+        g.free()
+    finally:
+        eng.close()
+    for c, off, s in ((a, 0, sub[:64]), (b, a.n, sub[64:] - a.n)):
+        want = oracle.component_bc(c.row_ptr, c.col, c.reach, sources=s.astype(np.int32), threads=16)
+        mx, _, zeros = relerr(got[off:off + c.n], want)
+        assert mx < 1e-9 and zeros, mx
