@@ -208,6 +208,11 @@ __device__ __forceinline__ int plain_forward(const Ctx &x, int s, uint64_t limit
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wv = tid >> 6;
     PlainShared *sh = x.sh;
     for (int k = tid; k < (x.n + 15) / 16; k += nt) x.lv.w[k] = 0;
+    if (x.drow)  // (a kept row tells the vertices that the source does not reach)
+        for (int k = tid; k < x.n; k += nt) {
+            x.drow[k] = BCX_INF;
+            x.sg[k] = 0;
+        }
     if (tid < 3) sh->cnt[tid] = sh->ovf[tid] = 0;
     pbarrier();
     if (tid == 0) {
@@ -500,11 +505,12 @@ __device__ __forceinline__ void plain_backward(const PlainCtx<LG, TT> &x, int ma
         pbarrier();
     }
     if (!x.dl) return;
-    // added in vertex order: neighbouring lanes' atomics share a line
+    // added in vertex order: neighbouring lanes' atomics share a line (a vertex
+    // that the source does not reach has an earlier source's word)
     if (tid == 0) x.dl[x.S[0]] = 0.0;
     pbarrier();
     for (int v = tid; v < x.n; v += nt) {
-        const double delta = x.dl[v];
+        const double delta = x.lv.get(v) ? x.dl[v] : 0.0;
         if (delta != 0.0) unsafeAtomicAdd(&bc[v], ws * delta);
     }
 }
@@ -603,7 +609,8 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev 
         // combine (Codes/postprocesses.cu:329-351)
         int mymax = 0;
         for (int k = tid; k < c.n; k += nt) {
-            const int la = dL[k] + ld, lb = dR[k] + rd;
+            const int a0 = dL[k], b0 = dR[k];
+            const int la = a0 == BCX_INF ? BCX_INF : a0 + ld, lb = b0 == BCX_INF ? BCX_INF : b0 + rd;
             int lv;
             uint64_t sv;
             if (la < lb) { lv = la; sv = sL[k]; }
@@ -611,7 +618,7 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev 
             else { lv = lb; sv = F64 ? d2u(u2d(sL[k]) + u2d(sR[k])) : sL[k] + sR[k]; }
             d[k] = lv;
             sg[k] = sv;
-            mymax = max(mymax, lv);
+            if (lv != BCX_INF) mymax = max(mymax, lv);
         }
         mymax = wave_max(mymax);
         if (lane == 0) atomicMax(&sh.top, mymax);
@@ -636,6 +643,7 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev 
         // final levels are BFS distances (< n); the combine maximum can be
         // larger on the source's own chain before the walk above fixes it
         const int maxl = min(sh.top, c.n - 1);
+        // (a vertex that the endpoints do not reach lies past it and joins no level)
         const bool in_lds = maxl + 2 <= LDS_LEVELS;
         int *h = in_lds ? hist : off;  // off doubles as the histogram when deep
         for (int l = tid; l < maxl + 2; l += nt) h[l] = 0;
@@ -644,7 +652,7 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev 
         // once (most of a small-world component sits on a few levels)
         for (int k0 = 0; k0 < c.n; k0 += nt) {
             const int k = k0 + tid;
-            const int l = k < c.n ? d[k] : -1;
+            const int dk = k < c.n ? d[k] : -1, l = dk <= maxl ? dk : -1;
             if (l >= 0) x.lv.take(k, 1 + (uint32_t)(l % 3));
             for (uint64_t m = pbal(l >= 0); m;) {
                 const int src = __ffsll((long long)m) - 1;
@@ -669,12 +677,13 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev 
                     ast(&h[l], run);
                 }
             }
+            sh.stop = run;  // vertices in the list
         }
         pbarrier();
         // h[l] now = number of vertices with level < l; use as cursors
         for (int k0 = 0; k0 < c.n; k0 += nt) {
             const int k = k0 + tid;
-            const int l = k < c.n ? d[k] : -1;
+            const int dk = k < c.n ? d[k] : -1, l = dk <= maxl ? dk : -1;
             for (uint64_t m = pbal(l >= 0); m;) {
                 const int src = __ffsll((long long)m) - 1;
                 const int l0 = __builtin_amdgcn_readlane(l, src);
@@ -690,13 +699,14 @@ __global__ __launch_bounds__(64 * PMAXW) void k_plain_chain(CompDev c, ChainDev 
         if (!in_lds) {
             // every level's offset again from the sorted levels (the first
             // LDS_LEVELS of them in LDS)
+            const int total = sh.stop;
             if (tid == 0) x.set_off(0, 0);
-            for (int i = tid; i < c.n; i += nt) {
+            for (int i = tid; i < total; i += nt) {
                 const int li = d[x.S[i]];
                 const int lp = i ? d[x.S[i - 1]] : -1;
                 for (int l = lp + 1; l <= li; ++l) x.set_off(l, i);
-                if (i == c.n - 1)
-                    for (int l = li + 1; l <= maxl + 1; ++l) x.set_off(l, c.n);
+                if (i == total - 1)
+                    for (int l = li + 1; l <= maxl + 1; ++l) x.set_off(l, total);
             }
             pbarrier();
         }
