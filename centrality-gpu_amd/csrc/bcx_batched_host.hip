@@ -1824,9 +1824,14 @@ int batched_persistent_finish(bcx_ctx *ctx, bcx_stats *st, int pass, bool *again
 
 void batched_persistent_reset(bcx_ctx *ctx) {
     if (ctx->side) (void)hipStreamSynchronize(ctx->side);
-    if (ctx->small) ctx->small->pending = false;
-    if (ctx->wgk) ctx->wgk->pending = false;
-    if (ctx->srck) ctx->srck->pending = false;
+    // (a pass on the context's stream as well: its tables are copied from pinned
+    // memory that the next pass writes)
+    for (SmallState *ss : {ctx->small, ctx->wgk, ctx->srck})
+        if (ss && ss->pending) {
+            (void)hipStreamSynchronize(ctx->stream);
+            (void)hipStreamSynchronize(ss->run_stream);
+            ss->pending = false;
+        }
 }
 
 static void release_state(bcx_ctx *ctx, SmallState *&state) {

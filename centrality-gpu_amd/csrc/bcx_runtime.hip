@@ -846,6 +846,18 @@ struct Download {
     double *stage = nullptr;
 };
 
+// Waits for what a failing run has queued, before its host buffers go.
+struct Drain {
+    bcx_ctx *ctx;
+    bool done = false;
+    explicit Drain(bcx_ctx *c) : ctx(c) {}
+    ~Drain() {
+        if (done) return;
+        if (ctx->side) (void)hipStreamSynchronize(ctx->side);
+        (void)hipStreamSynchronize(ctx->stream);
+    }
+};
+
 // Starts the copy of the run's BC.  A run over a source subset leaves the
 // slices of components without sources at the zeros they were set to, so
 // only the other slices come back: gathered into one packed buffer on the
@@ -1033,6 +1045,7 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
     }
     const bool want = bc_out && g->total_n > 0;
     Download down;
+    Drain drain(ctx);
     bool downloaded = false;
     if (!srck.empty() && small.empty() && wg.empty() && single.empty() && multi.empty()) {
         // the one-launch pass alone: its counters and the result come back
@@ -1104,6 +1117,7 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
         if (want && (rc = download_start(ctx, g, bc, o.src_subset ? &touched : nullptr, down))) return rc;
         if ((rc = ctx_hip(ctx, hipStreamSynchronize(ctx->stream), "run"))) return rc;
     }
+    drain.done = true;
     if (want) download_add(down, bc_out);
     ctx->busy = false;
     s->t_chain_s = ctx->timer_chain.collect();

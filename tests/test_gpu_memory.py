@@ -86,3 +86,47 @@ def test_tiles_and_rows_in_one_run(engine):
         want = oracle.component_bc(c.row_ptr, c.col, c.reach, sources=s.astype(np.int32), threads=16)
         mx, _, zeros = relerr(got[off:off + c.n], want)
         assert mx < 1e-9 and zeros, mx
+
+
+def test_run_after_one_that_failed(engine):
+    """A run whose result download finds no room is refused after its kernel was
+    started; the next run of the context is not disturbed by what was queued."""
+    rng = np.random.default_rng(5)
+    comps = []
+    for i in range(40):
+        n = 100 + i
+        e = np.concatenate([np.stack([np.arange(n), (np.arange(n) + 1) % n], 1), np.stack([np.arange(n), (np.arange(n) + 2 + i % 7) % n], 1)])
+        e = np.unique(np.sort(e, axis=1), axis=0)
+        rp, col = oracle.csr_from_edges(n, e[rng.permutation(len(e))])
+        comps.append(bcx.HostComponent.from_csr(rp, col, rng.integers(0, 5, n).astype(np.int32)))
+    want = np.concatenate([oracle.component_bc(c.row_ptr, c.col, c.reach) for c in comps])
+    sub = np.arange(comps[0].n, len(want))  # (every component but the first)
+
+    def runs(cap):
+        eng = bcx.Engine(0, mem_cap=cap)
+        try:
+            eng.bc(comps, path=B)
+            return True
+        except bcx.BcxError as e:
+            assert e.code == -4
+            return False
+        finally:
+            eng.close()
+
+    lo, hi = 1 << 12, 1 << 22
+    while hi - lo > 256:  # the least cap that a whole run fits in
+        lo, hi = ((lo + hi) // 2, hi) if not runs((lo + hi) // 2) else (lo, (lo + hi) // 2)
+    eng = bcx.Engine(0, mem_cap=hi)
+    try:
+        g = eng.upload(comps)
+        g.run(path=B)
+        for _ in range(3):
+            with pytest.raises(bcx.BcxError) as e:
+                g.run(path=B, subset=sub)
+            assert e.value.code == -4
+            got, _ = g.run(path=B)
+            mx, _, zeros = relerr(got, want)
+            assert mx < 1e-9 and zeros, mx
+        g.free()
+    finally:
+        eng.close()
