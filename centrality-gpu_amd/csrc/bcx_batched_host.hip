@@ -1336,6 +1336,8 @@ struct SmallState {
     SrcArgs src{};  // (wave-per-source pass)
     std::vector<SmallTile> run_tiles;
     std::vector<std::pair<double *, int32_t>> run_slices;  // (wave-per-source pass) BC slice of each component
+    double *fold_bc = nullptr;     // (wave-per-source pass) the BC words from the first
+    int64_t fold_n = 0;            // component's to the last one's
     size_t run_narrow = 0;
     int run_grid = 0;
     hipStream_t run_stream = nullptr;
@@ -1401,8 +1403,9 @@ static int persistent_pass(bcx_ctx *ctx, SmallState &ss, bool wg, bool f64, bool
     return small_launch(ctx, ss, ss.run, wg, f64, ss.run_fp32, ss.run_grid, graph, ss.run_stream);
 }
 
-// The tables of a persistent pass: its components, tiles of tw sources,
-// sources and weights, and eight zeroed counters, in device memory.
+// The tables of a persistent pass: its components, tiles of width(sources of
+// the component) sources, sources and weights, and eight zeroed counters, in
+// device memory.
 struct PassTables {
     std::vector<SmallTile> tiles;
     const SmallComp *comps = nullptr;
@@ -1412,8 +1415,9 @@ struct PassTables {
     int32_t *counters = nullptr;
 };
 
+template <typename Width>
 static int stage_tables(bcx_ctx *ctx, SmallState &ss, const std::vector<const SmallJob *> &order, double *bc_base,
-                        size_t tw, PassTables &out) {
+                        Width width, PassTables &out) {
     std::vector<SmallComp> comps;
     std::vector<SmallTile> &tiles = out.tiles;
     std::vector<int32_t> srcs;
@@ -1432,6 +1436,7 @@ static int stage_tables(bcx_ctx *ctx, SmallState &ss, const std::vector<const Sm
         c.bc = bc_base + dc.offset;
         const int32_t ci = (int32_t)comps.size();
         comps.push_back(c);
+        const size_t tw = width(jb.srcs.size());
         for (size_t i = 0; i < jb.srcs.size(); i += tw) {
             SmallTile t{};
             t.comp = ci;
@@ -1525,7 +1530,7 @@ static int persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, con
     for (const SmallJob *jb : order)
         if (!wide(jb)) n_narrow_tiles += (jb->srcs.size() + TW - 1) / TW;
     PassTables tb;
-    int rc = stage_tables(ctx, ss, order, bc_base, TW, tb);
+    int rc = stage_tables(ctx, ss, order, bc_base, [&](size_t) { return TW; }, tb);
     if (rc) return rc;
     std::vector<SmallTile> &tiles = tb.tiles;
     if ((rc = ss.counter.ensure(ctx, 64, "small counters")) ||
@@ -1672,18 +1677,31 @@ bool src_takes(const DComp &dc, bool fp32) {
 
 static bool run_fp32(const bcx_opts *o) { return o->path == BCX_PATH_BATCHED && o->precision == BCX_PREC_FP32C; }
 
-// Queues the read-back of a launch's counters behind it.
-static int src_counters(bcx_ctx *ctx, SmallState &ss, const int32_t *from, hipStream_t sp) {
+static void src_counters_pin(SmallState &ss) {
     if (!ss.ctr_pin && hipHostMalloc((void **)&ss.ctr_pin, 64, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         ss.ctr_pin = nullptr;
     }
     ss.ctr_back = ss.ctr_pin ? ss.ctr_pin : ss.ctr_host;
+}
+
+// Queues the read-back of a launch's counters behind it.
+static int src_counters(bcx_ctx *ctx, SmallState &ss, const int32_t *from, hipStream_t sp) {
+    src_counters_pin(ss);
     return ctx_hip(ctx, hipMemcpyAsync(ss.ctr_back, from, 3 * sizeof(int32_t), hipMemcpyDeviceToHost, sp), "counter");
 }
 
-static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base,
-                     bcx_stats *st, hipStream_t sp, bool probe) {
+// Queues the sum of a launch's accumulators; to `out` as well, when given, and
+// the counters to their place.
+static int src_fold(bcx_ctx *ctx, const SmallState &ss, bcx_stats *st, hipStream_t sp, const int32_t *ctr = nullptr,
+                    double *out = nullptr) {
+    if (!ss.src.copy) return BCX_OK;
+    if (st) st->n_launches++;
+    return ctx_hip(ctx, launch_src_fold(ss.fold_bc, ss.src.copy, ss.fold_n, out, ctr, ss.ctr_back, sp), "source kernel");
+}
+
+static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base, int64_t copy,
+                     double *out, bcx_stats *st, hipStream_t sp, bool probe) {
     if (jobs.empty()) return BCX_OK;
     if (!ctx->srck) ctx->srck = new SmallState();
     SmallState &ss = *ctx->srck;
@@ -1707,8 +1725,17 @@ static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_
     const bool fp32 = run_fp32(o);
     const size_t per = n_src / (size_t)std::max(1, ctx->n_cu);
     const size_t tw = probe || per > 128 ? BATCH_W : (per > 64 ? 32 : (per > 8 ? 16 : (per > 4 ? 8 : 4)));
+    // With FP64 terms the sums over sources are to round no more than those of
+    // 64-source tiles added up in pairs (bcx_small.hip).  The w sources of a tile
+    // are added one by one, and the errors of the k / w tiles of a component sum to
+    // the square root of w^2 / 3k additions' worth: w^2 is kept at 3k or less.
     PassTables tb;
-    int rc = stage_tables(ctx, ss, order, bc_base, tw, tb);
+    int rc = stage_tables(ctx, ss, order, bc_base, [&](size_t k) {
+        if (fp32 || probe) return tw;
+        size_t w = 4;
+        while (w < tw && 4 * w * w <= 3 * k) w *= 2;
+        return w;
+    }, tb);
     if (rc || (rc = ss.redo.ensure(ctx, 4 * tb.tiles.size(), "source redo list"))) return rc;
     if (probe) {
         size_t cells = 0;
@@ -1729,12 +1756,20 @@ static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_
     a.limit = (o->sigma_f64_threshold_log2 > 0 && o->sigma_f64_threshold_log2 < 64)
                   ? (1ull << o->sigma_f64_threshold_log2) : 0;
     a.stop = fp32 && tw < BATCH_W;
+    a.copy = fp32 ? 0 : copy;
     a.psig = probe ? (uint64_t *)ss.psig.p : nullptr;
     a.lvl = probe ? (int32_t *)ss.lvl.p : nullptr;
     a.dbg = probe ? (double *)ss.dbg.p : nullptr;
     ss.src = a;
     ss.run_slices.clear();
-    for (const SmallJob *jb : order) ss.run_slices.push_back({bc_base + jb->dc->offset, jb->dc->n});
+    int64_t v0 = INT64_MAX, v1 = 0;
+    for (const SmallJob *jb : order) {
+        ss.run_slices.push_back({bc_base + jb->dc->offset, jb->dc->n});
+        v0 = std::min(v0, jb->dc->offset);
+        v1 = std::max(v1, jb->dc->offset + jb->dc->n);
+    }
+    ss.fold_bc = bc_base + v0;
+    ss.fold_n = v1 - v0;
     ss.run_fp32 = fp32;
     ss.run_tiles = std::move(tb.tiles);
     if (ss.occ_lds != a.lds) {
@@ -1747,9 +1782,12 @@ static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_
     if ((rc = follow_ctx_stream(ctx, sp))) return rc;
     ctx->timer.begin(ctx);
     rc = ctx_hip(ctx, launch_src(a, false, fp32, ss.run_grid, sp), "source kernel");
+    if (out) src_counters_pin(ss);
+    const bool back = out && ss.ctr_back == ss.ctr_pin;  // (the kernel stores the counters too)
+    if (!rc) rc = src_fold(ctx, ss, st, sp, back ? a.counter : nullptr, out ? out + v0 : nullptr);
     ctx->timer.end(ctx);
     if (st) st->n_launches++;
-    return rc ? rc : src_counters(ctx, ss, a.counter, sp);
+    return rc || back ? rc : src_counters(ctx, ss, a.counter, sp);
 }
 
 static int src_finish(bcx_ctx *ctx, bcx_stats *st, bool *reran = nullptr) {
@@ -1776,6 +1814,7 @@ static int src_finish(bcx_ctx *ctx, bcx_stats *st, bool *reran = nullptr) {
         a.stop = 0;
         ctx->timer.begin(ctx);
         r = ctx_hip(ctx, launch_src(a, f64, ss.run_fp32, std::min(ss.run_grid, a.n_tiles), sp), "source kernel");
+        if (!r) r = src_fold(ctx, ss, st, sp);
         ctx->timer.end(ctx);
         if (st) st->n_launches++;
         if (reran) *reran = true;
@@ -1813,8 +1852,8 @@ static int src_finish(bcx_ctx *ctx, bcx_stats *st, bool *reran = nullptr) {
 }
 
 int batched_persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base,
-                             bcx_stats *st, int pass, hipStream_t sp) {
-    if (pass == PASS_SRC) return src_start(ctx, jobs, o, bc_base, st, sp, false);
+                             bcx_stats *st, int pass, hipStream_t sp, int64_t copy, double *out) {
+    if (pass == PASS_SRC) return src_start(ctx, jobs, o, bc_base, copy, out, st, sp, false);
     return persistent_start(ctx, jobs, o, bc_base, st, pass == PASS_WG, sp, false);
 }
 
@@ -2193,7 +2232,7 @@ int batched_debug_tile(bcx_ctx *ctx, const bcx_component *comp, const int32_t *s
         if (!rc) {
             for (int32_t v = 0; v < n; ++v) at[v] = v;
             std::vector<SmallJob> jobs{{&dc, std::vector<int32_t>(srcs, srcs + ns)}};
-            rc = by_src ? src_start(ctx, jobs, o, bc, &st, ctx->stream, true)
+            rc = by_src ? src_start(ctx, jobs, o, bc, 0, nullptr, &st, ctx->stream, true)
                         : persistent_start(ctx, jobs, o, bc, &st, wg, ctx->stream, true);
             if (!rc) rc = by_src ? src_finish(ctx, &st) : persistent_finish(ctx, &st, wg);
         }

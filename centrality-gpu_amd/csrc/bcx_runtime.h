@@ -149,6 +149,8 @@ struct bcx_ctx {
     double *bc_pin = nullptr;      // pinned host staging of the result download
     size_t bc_pin_bytes = 0;
     int32_t *up_pin = nullptr;     // pinned host staging of small uploads
+    bcx::DBuf bc_copies;           // accumulators of a run with several (see SrcArgs::copy)
+    bool copies_held = false;      // a run is using them
     int rows_held = 0;             // plain_scratch and bc_split belong to a launch being put together
     int32_t by_source = 0;         // batched: components the last run took source by source
     bool busy = true;              // work may be in flight on the context stream
@@ -157,7 +159,7 @@ struct bcx_ctx {
     SmallState *wgk = nullptr;  // workgroup-per-tile kernel buffers
     SmallState *srck = nullptr;  // wave-per-source kernel buffers
     std::vector<bcx::DBuf *> all_bufs() {
-        return {&counters, &bc_acc, &plain_scratch, &rows_buf, &w_src, &w_aux, &w_mode, &w_slots, &bc_split, &bc_pack, &bc_chunks};
+        return {&counters, &bc_acc, &plain_scratch, &rows_buf, &w_src, &w_aux, &w_mode, &w_slots, &bc_split, &bc_copies, &bc_pack, &bc_chunks};
     }
 };
 
@@ -201,10 +203,13 @@ std::vector<int32_t> batched_order(bcx::DComp &dc);
 // One persistent launch over the tiles of `jobs`, started on stream sp
 // without waiting; _finish waits for it and reruns overflowed tiles in FP64.
 // The passes: 64-source tiles of small components, the workgroup-per-tile
-// kernel, and the wave-per-source kernel (components that src_takes accepts).
+// kernel, and the wave-per-source kernel (components that src_takes accepts;
+// copy: words from one of its zeroed accumulators to the next, 0: there is one;
+// out: pinned buffer for the sums of every component, with copy only).
 enum { PASS_SMALL = 0, PASS_WG = 1, PASS_SRC = 2 };
 int batched_persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_opts *o, double *bc_base,
-                             bcx_stats *st, int pass, hipStream_t sp);
+                             bcx_stats *st, int pass, hipStream_t sp, int64_t copy = 0,
+                             double *out = nullptr);
 // (*again, optional: some of it was rerun after the first launch)
 int batched_persistent_finish(bcx_ctx *ctx, bcx_stats *st, int pass, bool *again = nullptr);
 // Whether the wave-per-source kernel takes a component, with FP32 or FP64 terms.

@@ -19,6 +19,7 @@
 #include "bcx_batched.h"
 #include "bcx_device.h"
 #include "bcx_kernels.h"
+#include "bcx_src.h"
 #include "bcx_runtime.h"
 #include "bcx_small.h"
 
@@ -43,14 +44,22 @@ int ctx_hip(bcx_ctx *ctx, hipError_t e, const char *what) {
 // speed alone: where an allocation finds no room beside them they are given
 // back (hipFree waits for what still runs on them).
 static bool give_rows_back(bcx_ctx *ctx) {
-    if (ctx->rows_held || (!ctx->plain_scratch.p && !ctx->bc_split.p)) return false;
-    ctx->plain_scratch.release(ctx);
-    ctx->bc_split.release(ctx);
-    return true;
+    bool any = false;
+    auto give = [&](DBuf &b) {
+        any |= b.p != nullptr;
+        b.release(ctx);
+    };
+    if (!ctx->rows_held) {
+        give(ctx->plain_scratch);
+        give(ctx->bc_split);
+    }
+    if (!ctx->copies_held) give(ctx->bc_copies);
+    return any;
 }
 
 size_t ctx_room(const bcx_ctx *ctx) {
-    const size_t rows = ctx->rows_held ? 0 : ctx->plain_scratch.bytes + ctx->bc_split.bytes;
+    const size_t rows = (ctx->rows_held ? 0 : ctx->plain_scratch.bytes + ctx->bc_split.bytes) +
+                        (ctx->copies_held ? 0 : ctx->bc_copies.bytes);
     return ctx->mem_cap + rows > ctx->mem_used ? ctx->mem_cap + rows - ctx->mem_used : 0;
 }
 
@@ -839,6 +848,8 @@ __global__ void k_bc_gather(const double *bc, double *packed, const BcChunk *ch)
     for (int i = threadIdx.x; i < c.len; i += blockDim.x) packed[c.dst + i] = bc[c.src + i];
 }
 
+constexpr size_t OUT_BYTES = 1 << 20;  // results up to this size may be stored by a kernel
+
 // A result download in flight: the slices that come back and their staging.
 struct Download {
     std::vector<BcChunk> chunks;
@@ -858,12 +869,11 @@ struct Drain {
     }
 };
 
-// Starts the copy of the run's BC.  A run over a source subset leaves the
-// slices of components without sources at the zeros they were set to, so
-// only the other slices come back: gathered into one packed buffer on the
-// device and copied to pinned staging; download_add adds them slice by slice
-// once the stream has been waited for.
-static int download_start(bcx_ctx *ctx, bcx_dgraph *g, const double *bc, const std::vector<char> *touched, Download &d) {
+// The slices of a run's BC that come back, and their staging (packed, or as in
+// the accumulator); returns their words.  A run over a source subset leaves the
+// slices of components without sources at the zeros they were set to, so those
+// stay.
+static int64_t download_plan(bcx_ctx *ctx, bcx_dgraph *g, const std::vector<char> *touched, Download &d, bool pack) {
     std::vector<BcChunk> &chunks = d.chunks;
     chunks.clear();
     int64_t packed = 0;
@@ -873,15 +883,15 @@ static int download_start(bcx_ctx *ctx, bcx_dgraph *g, const double *bc, const s
         for (int64_t i = 0; i < dc.n; i += BC_CHUNK) {
             BcChunk c{};
             c.src = dc.offset + i;
-            c.dst = packed;
+            c.dst = pack ? packed : c.src;
             c.len = (int32_t)std::min<int64_t>(BC_CHUNK, dc.n - i);
             chunks.push_back(c);
             packed += c.len;
         }
     }
-    if (packed == 0) return BCX_OK;
+    if (!pack) packed = g->total_n;
     const size_t bytes = sizeof(double) * (size_t)packed;
-    if (ctx->bc_pin_bytes < bytes) {
+    if (packed && ctx->bc_pin_bytes < bytes) {
         if (ctx->bc_pin) (void)hipHostFree(ctx->bc_pin);
         ctx->bc_pin = nullptr;
         ctx->bc_pin_bytes = 0;
@@ -898,6 +908,17 @@ static int download_start(bcx_ctx *ctx, bcx_dgraph *g, const double *bc, const s
         d.pageable.resize((size_t)packed);
         d.stage = d.pageable.data();
     }
+    return packed;
+}
+
+// Starts the copy of the run's BC: gathered into one packed buffer on the device
+// and copied to the staging; download_add adds it slice by slice once the stream
+// has been waited for.
+static int download_start(bcx_ctx *ctx, bcx_dgraph *g, const double *bc, const std::vector<char> *touched, Download &d) {
+    const int64_t packed = download_plan(ctx, g, touched, d, true);
+    if (packed == 0) return BCX_OK;
+    const std::vector<BcChunk> &chunks = d.chunks;
+    const size_t bytes = sizeof(double) * (size_t)packed;
     const double *from = bc;
     int rc;
     if (packed < g->total_n) {
@@ -920,7 +941,7 @@ static void download_add(const Download &d, double *bc_out) {
     }
 }
 
-int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, bcx_stats *st) {
+static int run_graph(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, bcx_stats *st, bool copies) {
     if (!ctx || !g) return ctx_fail(ctx, BCX_E_ARG, "null context or graph");
     (void)hipSetDevice(ctx->device);
     bcx_opts o{};
@@ -940,12 +961,6 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
     ctx->timer.used = 0;
     ctx->timer_chain.depth = 0;
     ctx->timer_chain.used = 0;
-    int rc = ctx->bc_acc.ensure(ctx, sizeof(double) * (size_t)std::max<int64_t>(g->total_n, 1), "bc accumulator");
-    if (rc) return rc;
-    double *bc = (double *)ctx->bc_acc.p;
-    rc = ctx_hip(ctx, hipMemsetAsync(bc, 0, sizeof(double) * (size_t)std::max<int64_t>(g->total_n, 1), ctx->stream),
-                 "memset");
-    if (rc) return rc;
     // subset slots -> per-component local lists
     std::vector<std::vector<int32_t>> sub;
     if (o.src_subset) {
@@ -959,6 +974,26 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
             sub[ci - 1].push_back((int32_t)(slot - dc.offset));
         }
     }
+    // the accumulator; for small components with FP64 terms several, where the cap
+    // leaves plenty beside them
+    const size_t bc_bytes = sizeof(double) * (size_t)std::max<int64_t>(g->total_n, 1);
+    int64_t copy = 0;
+    if (o.path == BCX_PATH_PLAIN || o.precision != BCX_PREC_FP32C)
+        for (size_t ci = 0; ci < g->comps.size() && !copy; ++ci)
+            if ((!o.src_subset || !sub[ci].empty()) && src_takes(g->comps[ci], false)) copy = g->total_n;
+    if (copy && (!copies || ctx_room(ctx) / 16 < SRC_COPIES * bc_bytes ||
+                 ctx->bc_copies.ensure(ctx, SRC_COPIES * bc_bytes, "accumulators") != BCX_OK))
+        copy = 0;
+    ctx->copies_held = copy != 0;
+    struct Held {
+        bcx_ctx *ctx;
+        ~Held() { ctx->copies_held = false; }
+    } held{ctx};
+    int rc = copy ? BCX_OK : ctx->bc_acc.ensure(ctx, bc_bytes, "bc accumulator");
+    if (rc) return rc;
+    double *bc = (double *)(copy ? ctx->bc_copies.p : ctx->bc_acc.p);
+    rc = ctx_hip(ctx, hipMemsetAsync(bc, 0, copy ? SRC_COPIES * bc_bytes : bc_bytes, ctx->stream), "memset");
+    if (rc) return rc;
     std::vector<SmallJob> srck;   // small components for the wave-per-source kernel (both paths)
     std::vector<SmallJob> small;  // batched path: components for the one-launch small kernel
     std::vector<SmallJob> wg;     // batched path: deep components for the workgroup-per-tile kernel
@@ -1051,10 +1086,20 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
         // the one-launch pass alone: its counters and the result come back
         // behind it and the host waits once (with two more waits and a pageable
         // upload a 24-vertex call takes 88 us, so 75)
+        // With several accumulators, the kernel that adds them up stores a small
+        // result in the pinned buffer itself, in place of the two copies (host call
+        // of four blocks of 600 vertices: 152 us with one accumulator, 187 with
+        // that launch before the copies, 146 so; of 24 vertices 75 and 48).
+        double *out = nullptr;
+        const std::vector<char> *some = o.src_subset ? &touched : nullptr;
+        if (want && copy && bc_bytes <= OUT_BYTES) {
+            (void)download_plan(ctx, g, some, down, false);
+            if (down.pageable.empty()) out = down.stage;
+        }
         ctx->timer.begin(ctx);
-        rc = batched_persistent_start(ctx, srck, &o, bc, s, PASS_SRC, ctx->stream);
+        rc = batched_persistent_start(ctx, srck, &o, bc, s, PASS_SRC, ctx->stream, copy, out);
         ctx->timer.end(ctx);
-        if (rc || (want && (rc = download_start(ctx, g, bc, o.src_subset ? &touched : nullptr, down)))) return rc;
+        if (rc || (want && !out && (rc = download_start(ctx, g, bc, some, down)))) return rc;
         bool again = false;
         if ((rc = batched_persistent_finish(ctx, s, PASS_SRC, &again))) return rc;
         downloaded = want && !again;
@@ -1068,7 +1113,7 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
             return rc;
         const hipStream_t sp = overlap ? ctx->side : ctx->stream;
         ctx->timer.begin(ctx);
-        if ((rc = batched_persistent_start(ctx, srck, &o, bc, s, PASS_SRC, sp)) ||
+        if ((rc = batched_persistent_start(ctx, srck, &o, bc, s, PASS_SRC, sp, copy)) ||
             (rc = batched_persistent_start(ctx, small, &o, bc, s, PASS_SMALL, sp)) ||
             (rc = batched_persistent_start(ctx, wg, &o, bc, s, PASS_WG, sp)))
             return rc;
@@ -1124,6 +1169,15 @@ int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, b
     s->t_kernel_s = ctx->timer.collect() + s->t_chain_s;
     s->t_total_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     return BCX_OK;
+}
+
+int bcx_run(bcx_ctx *ctx, bcx_dgraph *g, const bcx_opts *opts, double *bc_out, bcx_stats *st) {
+    int rc = run_graph(ctx, g, opts, bc_out, st, true);
+    if (rc == BCX_E_NOMEM && ctx->bc_copies.p) {  // (nothing was added to bc_out)
+        ctx->bc_copies.release(ctx);
+        rc = run_graph(ctx, g, opts, bc_out, st, false);
+    }
+    return rc;
 }
 
 int32_t bcx_run_by_source(const bcx_ctx *ctx) { return ctx ? ctx->by_source : 0; }

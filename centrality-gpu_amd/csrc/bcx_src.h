@@ -17,6 +17,7 @@ namespace bcx {
 constexpr int SRC_N = 2048;                 // largest component (list entries are 15-bit ids and a flag)
 constexpr int SRC_WAVES = 16;               // waves of a workgroup
 constexpr int64_t SRC_LDS = 160 * 1024 - 512;  // dynamic LDS of a workgroup at most
+constexpr int SRC_COPIES = 16;              // BC accumulators of a launch with FP64 terms
 
 __host__ __device__ constexpr int64_t src_up16(int64_t x) { return (x + 15) & ~(int64_t)15; }
 // (groups: sum over the rows of ceil(arcs / 4))
@@ -43,6 +44,9 @@ struct SrcArgs {
     int32_t *redo;           // [n_tiles] those tiles
     uint64_t limit;          // u64 path-count threshold (0 = 2^64)
     int32_t stop;            // take no further tile once one has overflowed
+    // FP64 terms: words from one of SRC_COPIES accumulators to the next (0:
+    // there is one); launch_src_fold adds them up
+    int64_t copy;
     // probe only (null in runs): [n][64] per (vertex, source) of the last tile
     uint64_t *psig;
     int32_t *lvl;
@@ -51,6 +55,11 @@ struct SrcArgs {
 };
 
 hipError_t launch_src(const SrcArgs &a, bool f64, bool fp32, int grid, hipStream_t st);
+// The sum of the accumulators into the first, over n words from bc, and into out
+// (optional, host memory); clears the others.  ctr (optional): three counters that
+// go to ctr_out.
+hipError_t launch_src_fold(double *bc, int64_t copy, int64_t n, double *out, const int32_t *ctr, int32_t *ctr_out,
+                           hipStream_t st);
 int src_blocks_per_cu(int lds);
 
 }  // namespace bcx

@@ -449,8 +449,9 @@ __global__ __launch_bounds__(XB) void k_src(SrcArgs a) {
             if (tid == 0) a.redo[atomicAdd(&a.counter[1], 1)] = item;
         } else {
             if (tid == 0) atomicMax(&a.counter[2], s_depth);
+            gdbl *to = glb(cp.bc) + (item % SRC_COPIES) * a.copy;
             for (int v = tid; v < n; v += XB)
-                if (bc[v] != 0.0) gadd(glb(cp.bc) + v, bc[v]);
+                if (bc[v] != 0.0) gadd(to + v, bc[v]);
         }
         __syncthreads();
     }
@@ -463,6 +464,42 @@ hipError_t launch_src(const SrcArgs &a, bool f64, bool fp32, int grid, hipStream
     if (f64) hipLaunchKernelGGL((k_src<true, double>), dim3(grid), dim3(XB), a.lds, st, a);
     else if (fp32) hipLaunchKernelGGL((k_src<false, float>), dim3(grid), dim3(XB), a.lds, st, a);
     else hipLaunchKernelGGL((k_src<false, double>), dim3(grid), dim3(XB), a.lds, st, a);
+    return hipGetLastError();
+}
+
+// Rounded once: what each addition rounds off (exact by Knuth's two-sum) is added
+// at the end.  Words that no tile added to are left alone: other components' runs
+// may be adding to theirs.
+__global__ __launch_bounds__(256) void k_src_fold(double *bc, int64_t copy, int64_t n, double *out, const int32_t *ctr,
+                                                  int32_t *ctr_out) {
+    const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (ctr && v < 3) ctr_out[v] = ctr[v];
+    if (v >= n) return;
+    double x[SRC_COPIES];
+    bool any = false;
+#pragma unroll
+    for (int k = 0; k < SRC_COPIES; ++k) {
+        x[k] = bc[v + k * copy];
+        any |= k > 0 && x[k] != 0.0;
+    }
+    double s = x[0], e = 0.0;
+    if (any) {
+#pragma unroll
+        for (int k = 1; k < SRC_COPIES; ++k) {
+            const double t = s + x[k], y = t - s;
+            e += (s - (t - y)) + (x[k] - y);
+            s = t;
+            bc[v + k * copy] = 0.0;
+        }
+        if (isfinite(s)) s += e;
+        ast((uint64_t *)&bc[v], d2u(s));
+    }
+    if (out) out[v] = s;
+}
+
+hipError_t launch_src_fold(double *bc, int64_t copy, int64_t n, double *out, const int32_t *ctr, int32_t *ctr_out,
+                           hipStream_t st) {
+    hipLaunchKernelGGL(k_src_fold, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, bc, copy, n, out, ctr, ctr_out);
     return hipGetLastError();
 }
 

@@ -130,3 +130,31 @@ def test_run_after_one_that_failed(engine):
         g.free()
     finally:
         eng.close()
+
+
+def test_several_accumulators_make_room(engine):
+    """FP64 runs of small components take several accumulators; a cap that holds a
+    large component's rows, beside one accumulator alone, still does."""
+    n, k = 700, 4
+    e = np.concatenate([np.stack([np.arange(n), (np.arange(n) + s) % n], 1) for s in (1, 2, 9)])
+    rp, col = oracle.csr_from_edges(n, e)
+    small = bcx.HostComponent.from_csr(rp, col, np.zeros(n, np.int32))
+    one = oracle.component_bc(small.row_ptr, small.col, small.reach)
+    big = giant(4, 0.05)
+    sub = np.linspace(0, big.n - 1, 300).astype(np.int64)
+    part = oracle.component_bc(big.row_ptr, big.col, big.reach, sources=sub.astype(np.int32), threads=16)
+    eng = bcx.Engine(0, mem_cap=rows(engine, big, 300) + 800000)
+    assert 16 * 8 * (k * n + big.n) > 800000
+    try:
+        g = eng.upload([small] * k)
+        got, _ = g.run(path=B)
+        mx, _, zeros = relerr(got, np.tile(one, k))
+        assert mx < 1e-9 and zeros, mx
+        g.free()
+        g = eng.upload([small] * k + [big])
+        got, _ = g.run(path=bcx.PATH_PLAIN, subset=np.concatenate([np.arange(n), k * n + sub]))
+        mx, _, zeros = relerr(got, np.concatenate([one, np.zeros((k - 1) * n), part]))
+        assert mx < 1e-9 and zeros, mx
+        g.free()
+    finally:
+        eng.close()

@@ -1,0 +1,53 @@
+"""Rounding of the sums over sources on small components in FP64.
+
+The dependencies of every source come from the probe of a tile, which runs the
+same kernel, and their sum is exact in math.fsum; what a run is off by is the
+rounding of its own additions.  An addition errs by 0.29 ulp (uniform in half an
+ulp either way), one that has reached a part p of the sum by p times that.  The
+sums in tiles of 64, added up in pairs, and of 300 sources in 5 such tiles, have
+(0.2^2 + .. + 1) + 5 0.2^2 (1 + 1/2 + 1/4 + ..) = 2.6 of its squares: 0.47 ulp.
+The bound is 1.25 times that."""
+import math
+
+import numpy as np
+import pytest
+
+import bcx
+
+pytestmark = pytest.mark.gpu
+
+BOUND = 1.25 * math.sqrt(2.6 / 12)
+
+
+def component(n, seed):
+    rng = np.random.default_rng(seed)
+    e = {(min(i, (i + 1) % n), max(i, (i + 1) % n)) for i in range(n)}
+    while len(e) < 3 * n:
+        a, b = sorted(map(int, rng.integers(0, n, 2)))
+        if a != b:
+            e.add((a, b))
+    return bcx.Host.from_edges(n, sorted(e)).decompose().components()[0]
+
+
+def exact(engine, c):
+    rows = [engine.debug_tile(c, np.arange(s, min(s + 64, c.n)), precision=bcx.PREC_FP64)[3]
+            for s in range(0, c.n, 64)]
+    delta = np.concatenate(rows)
+    assert delta.shape == (c.n, c.n) and not np.any(c.reach)
+    return np.array([math.fsum(delta[:, v]) for v in range(c.n)])
+
+
+@pytest.mark.parametrize("path", [bcx.PATH_PLAIN, bcx.PATH_BATCHED])
+@pytest.mark.parametrize("n,copies", [(24, 1), (64, 1), (64, 100), (300, 1), (300, 120), (600, 4), (1100, 32),
+                                      (2047, 1)])
+def test_small_components(engine, n, copies, path):
+    # (components of few vertices: several, for the mean over as many)
+    comps = [component(n, 7 * n + k) for k in range(max(1, 400 // n))]
+    want = np.concatenate([exact(engine, c) for c in comps])
+    g = engine.upload(comps * copies)
+    got, st = g.run(path=path, precision=bcx.PREC_FP64)
+    g.free()
+    off = (got - np.tile(want, copies)) / np.spacing(np.tile(want, copies))
+    rms = math.sqrt(float(np.mean(off ** 2)))
+    print("n", n, "copies", copies, "path", path, "rms ulp", rms, flush=True)
+    assert rms < BOUND, rms
