@@ -423,13 +423,14 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
     // Where a capacity has little room left beside the rows above, there is one
     // accumulator, and without room for that an ordered run has the
     // component's own order.
-    constexpr int SPLIT = 16;
-    constexpr size_t SPLIT_SOURCES = 512;
+    constexpr int SPLIT = 32;
+    constexpr size_t SPLIT_FP32 = 512;
     const size_t word = sizeof(double) * (size_t)dc.n;
     const size_t room = ctx->mem_cap > ctx->mem_used ? ctx->mem_cap - ctx->mem_used : 0;
-    int split = src.size() >= SPLIT_SOURCES && ctx->bc_split.bytes + room / 16 >= word * SPLIT ? SPLIT : 1;
+    int split = fp32 && src.size() < SPLIT_FP32 ? 1 : SPLIT;
+    while (split > 1 && (8 * (size_t)split > src.size() || ctx->bc_split.bytes + room / 16 < word * split)) split /= 2;
     ordered = ordered && dc.ord_state == 1;
-    if (split > 1 && ctx->bc_split.ensure(ctx, word * SPLIT, "split accumulator") != BCX_OK) split = 1;
+    if (split > 1 && ctx->bc_split.ensure(ctx, word * split, "split accumulator") != BCX_OK) split = 1;
     if (ordered && split == 1 && ctx->bc_split.ensure(ctx, word, "accumulator") != BCX_OK) ordered = false;
     const bool fold = split > 1 || ordered;  // (an ordered run folds its one copy back to the component's order)
     std::vector<int32_t> ids;

@@ -1,4 +1,4 @@
-"""Rounding of the sums over sources on small components in FP64.
+"""Rounding of the sums over sources in FP64 where sources run one by one.
 
 The dependencies of every source come from the probe of a tile, which runs the
 same kernel, and their sum is exact in math.fsum; what a run is off by is the
@@ -50,4 +50,28 @@ def test_small_components(engine, n, copies, path):
     off = (got - np.tile(want, copies)) / np.spacing(np.tile(want, copies))
     rms = math.sqrt(float(np.mean(off ** 2)))
     print("n", n, "copies", copies, "path", path, "rms ulp", rms, flush=True)
+    assert rms < BOUND, rms
+
+
+@pytest.mark.parametrize("path", [bcx.PATH_PLAIN, bcx.PATH_BATCHED])
+@pytest.mark.parametrize("k", [64, 361, 1500])
+def test_per_source_kernel(engine, k, path):
+    """A grid of 3600 vertices, whose short rows are summed in one order by every
+    run of the kernel: k of its sources."""
+    w = 60
+    edges = [(y * w + x, y * w + x + 1) for y in range(w) for x in range(w - 1)]
+    edges += [(y * w + x, (y + 1) * w + x) for y in range(w - 1) for x in range(w)]
+    c = bcx.Host.from_edges(w * w, edges).decompose(use_chains=False).components()[0]
+    assert c.n == w * w and not np.any(c.reach)
+    sub = np.sort(np.random.default_rng(k).permutation(c.n)[:k]).astype(np.int64)
+    kw = dict(path=bcx.PATH_PLAIN, precision=bcx.PREC_FP64, use_chains=False)
+    delta = np.array([engine.debug_source(c, int(s), **kw)[3] for s in sub])
+    g = engine.upload([c])
+    got, _ = g.run(path=path, precision=bcx.PREC_FP64, use_chains=False, subset=sub)
+    g.free()
+    want = np.array([math.fsum(delta[:, v]) for v in range(c.n)])
+    pos = want > 0
+    off = (got[pos] - want[pos]) / np.spacing(want[pos])
+    rms = math.sqrt(float(np.mean(off ** 2)))
+    print("k", k, "path", path, "rms ulp", rms, flush=True)
     assert rms < BOUND, rms
