@@ -75,3 +75,50 @@ def test_per_source_kernel(engine, k, path):
     rms = math.sqrt(float(np.mean(off ** 2)))
     print("k", k, "path", path, "rms ulp", rms, flush=True)
     assert rms < BOUND, rms
+
+
+def dependencies(n, adj, s):
+    """Dependencies of source s in extended precision."""
+    level, order = {s: 0}, [s]
+    sigma = np.zeros(n, np.longdouble)
+    sigma[s] = 1
+    for v in order:
+        for w in adj[v]:
+            if w not in level:
+                level[w] = level[v] + 1
+                order.append(w)
+            if level[w] == level[v] + 1:
+                sigma[w] += sigma[v]
+    delta = np.zeros(n, np.longdouble)
+    for v in reversed(order):
+        for w in adj[v]:
+            if level[w] == level[v] + 1:
+                delta[v] += sigma[v] / sigma[w] * (1 + delta[w])
+    delta[s] = 0
+    return delta
+
+
+def test_rows_of_the_per_source_kernel(engine):
+    """Rows of 200 arcs, walked with a lane per arc: their sums are made of four
+    parts of at most 64 terms, (0.25 64 / 3 + 1.5) squares of 0.32 ulp, the terms'
+    own rounding is spread over 200, and the product with the count rounds once:
+    0.9 ulp.  The bound is 1.3 times that (one part of 200: 2.6)."""
+    rng = np.random.default_rng(11)
+    A, B, C = 40, 300, 600
+    n = 1 + A + B + C
+    e = [(0, 1 + a) for a in range(A)]
+    e += [(1 + a, 1 + A + int(b)) for a in range(A) for b in rng.choice(B, 200, replace=False)]
+    e += [(1 + A + b, 1 + A + B + int(c)) for b in range(B) for c in rng.choice(C, 7, replace=False)]
+    deg = np.bincount(np.array(e).ravel(), minlength=n)
+    e += [(1 + A + c % B, 1 + A + B + c) for c in range(C) if deg[1 + A + B + c] == 0]
+    adj = [[] for _ in range(n)]
+    for a, b in sorted(set(e)):
+        adj[a].append(b)
+        adj[b].append(a)
+    rp = np.concatenate([[0], np.cumsum([len(x) for x in adj])]).astype(np.int32)
+    comp = bcx.HostComponent.from_csr(rp, np.concatenate(adj).astype(np.int32), np.zeros(n, np.int32))
+    want = dependencies(n, adj, 0)[1:1 + A]
+    got = engine.debug_source(comp, 0, path=bcx.PATH_PLAIN, precision=bcx.PREC_FP64)[3][1:1 + A]
+    rms = math.sqrt(float(np.mean(((got - want) / np.spacing(want.astype(np.float64))) ** 2)))
+    print("rows: rms ulp", rms, flush=True)
+    assert rms < 1.2, rms
