@@ -581,6 +581,8 @@ bool batched_narrow(DComp &dc) {
         }
         dc.depth = depth;
         dc.sigma_est = smax;
+        for (int32_t v : hc.ch_nodes) lv[v] = 0;
+        dc.core_depth = *std::max_element(lv.begin(), lv.end());
     }
     return (int64_t)dc.n <= (int64_t)WG_WIDTH * (dc.depth + 1);
 }
@@ -695,11 +697,12 @@ std::vector<int32_t> ball_sources(DComp &dc, const std::vector<int32_t> &srcs) {
 }
 
 // Work of one tile of ns <= 64 sources: its (vertex, level) entries, each
-// weighted by the arcs the pull and the backward walk for it (degree + 1),
+// weighted by the arcs the pull and the backward walk for it (degree + row),
 // from a host 64-lane level-synchronous BFS (the tile kernels' own scheme,
 // on the CPU).  Stops early once the count passes `limit`.
 static int64_t tile_entries(const HostComp &hc, const int32_t *src, int ns, int64_t limit,
-                            std::vector<uint64_t> &vis, std::vector<uint64_t> &cur, std::vector<uint64_t> &nxt) {
+                            std::vector<uint64_t> &vis, std::vector<uint64_t> &cur, std::vector<uint64_t> &nxt,
+                            int row = 1) {
     std::vector<int32_t> fr, nf, seen;
     for (int k = 0; k < ns; ++k) {
         const int32_t v = src[k];
@@ -709,7 +712,7 @@ static int64_t tile_entries(const HostComp &hc, const int32_t *src, int ns, int6
     }
     seen = fr;
     int64_t entries = 0;
-    for (int32_t v : fr) entries += hc.rp[v + 1] - hc.rp[v] + 1;
+    for (int32_t v : fr) entries += hc.rp[v + 1] - hc.rp[v] + row;
     while (!fr.empty() && entries <= limit) {
         nf.clear();
         for (int32_t v : fr) {
@@ -728,7 +731,7 @@ static int64_t tile_entries(const HostComp &hc, const int32_t *src, int ns, int6
             vis[w] |= nxt[w];
             cur[w] = nxt[w];
             nxt[w] = 0;
-            entries += hc.rp[w + 1] - hc.rp[w] + 1;
+            entries += hc.rp[w + 1] - hc.rp[w] + row;
         }
         fr.swap(nf);
     }
@@ -785,26 +788,35 @@ static std::vector<int32_t> landmark_order(const HostComp &hc, const std::vector
     return order;
 }
 
-// Work of the tiles of `order` at nine evenly spaced positions, on host
-// threads (the work of single tiles varies by tens of percent).
-static int64_t sample_work(const HostComp &hc, const std::vector<int32_t> &order) {
-    const int64_t T = ((int64_t)hc.n + BATCH_W - 1) / BATCH_W;
-    constexpr int S = 9;
-    std::vector<int64_t> w(S, 0);
-    const unsigned nt = std::max(1u, std::min<unsigned>(S, std::thread::hardware_concurrency()));
+// Work of the tiles of `order` at `at`, on host threads.
+static std::vector<int64_t> tiles_work(const HostComp &hc, const std::vector<int32_t> &order,
+                                       const std::vector<int64_t> &at, int row) {
+    const int S = (int)at.size();
+    std::vector<int64_t> w((size_t)S, 0);
+    const unsigned nt = std::max(1u, std::min<unsigned>((unsigned)S, std::thread::hardware_concurrency()));
     std::vector<std::thread> th;
     for (unsigned t = 0; t < nt; ++t)
         th.emplace_back([&, t] {
             std::vector<uint64_t> vis((size_t)hc.n, 0), cur((size_t)hc.n, 0), nxt((size_t)hc.n, 0);
             for (int k = (int)t; k < S; k += (int)nt) {
-                const int64_t u = (k + 1) * T / (S + 1);
+                const int64_t u = at[(size_t)k];
                 const int ns = (int)std::min<int64_t>(BATCH_W, hc.n - u * BATCH_W);
-                w[k] = tile_entries(hc, order.data() + u * BATCH_W, ns, INT64_MAX, vis, cur, nxt);
+                w[(size_t)k] = tile_entries(hc, order.data() + u * BATCH_W, ns, INT64_MAX, vis, cur, nxt, row);
             }
         });
     for (auto &x : th) x.join();
+    return w;
+}
+
+// Work of the tiles of `order` at nine evenly spaced positions (the work of
+// single tiles varies by tens of percent).
+static int64_t sample_work(const HostComp &hc, const std::vector<int32_t> &order) {
+    const int64_t T = ((int64_t)hc.n + BATCH_W - 1) / BATCH_W;
+    constexpr int S = 9;
+    std::vector<int64_t> at;
+    for (int k = 0; k < S; ++k) at.push_back((k + 1) * T / (S + 1));
     int64_t sum = 0;
-    for (int64_t x : w) sum += x;
+    for (int64_t x : tiles_work(hc, order, at, 1)) sum += x;
     return sum;
 }
 
@@ -1932,37 +1944,53 @@ constexpr double LAUNCH_S = 4e-6;  // of a level kernel that finds next to nothi
 // order (1e-10 to 7e-9 apart; FP64 terms: FP64 rounding).  So what a component
 // is decides alone which of the two its FP32C runs get, whatever the number of
 // sources, the calls before and the timing of samples: the parts of a job add
-// up, and a source gives the same in every call.  Below the line every row is
+// up, and a source gives the same in every call.  With FP32_ROWS every row is
 // summed whole: one workgroup per source, the workgroup kernel, or tiles with
 // neither contracted chains nor hub slices, whichever is fastest (to 1e-15 the
-// same).  The line is where the rates of full jobs on the workgroup kernel and
-// the sliced tiles crossed (the former ahead / behind, vertices at levels:
-// contracted tiles, power-law cores 67.3k / 69.0k at 24 to 27, R-MAT 44.5k / 85.7k at
-// 7, a 74k grid of 510 ahead; tiles without chains, power-law cores 84.1k /
-// 92.5k at 31 and 40, core of a block graph 74.1k / 76.8k at 4): drawn
-// elsewhere, the results in between would change.
+// same).  Which of the two a component gets was settled by the rates of samples:
+// a round of 256 workgroup tiles against 24 sliced ones of 256 sources, on the
+// kernels as they then were.  Their times (ms) follow from the component, within
+// 6% and 10% (power-law cores of 17k to 126k vertices, R-MAT cores of 23k to 86k,
+// cores of block graphs of 17k to 116k; with and without chains):
+//   round   its slowest tile, 5.7e-6 (arcs walked + 58 entries), beside the
+//           component's arcs, 28e-6 each; the last sampled tile holds the deepest
+//           vertices, which reach the hubs on a level each (46.7k vertices: 9.2
+//           arcs walked per arc and 200 ms, or 4.5 and 109, by where it falls)
+//   tiles   38 + 6.5e-6 per arc + (0.55 + 4.5e-6 n) per level, of the vertices off
+//           chains where chains are contracted
+// Where both were timed their ratio and that of the rates lay on the same side of
+// 1.  Deep components (grids, 120 vertices a level: 5 to 10) never were near it.
 enum { FP32_ANY = 0, FP32_ROWS = 1, FP32_TILES = 2 };
-static int64_t fp32_line(const DComp &dc, bool cut) { return (cut ? 58000 : 74000) + 400 * (int64_t)dc.depth; }
+constexpr int32_t DEEP_WIDTH = 512;
 static bool fp32_free(const DComp &dc, const bcx_opts *o) {
     return !run_fp32(o) || dc.n < TUNE_N ||
            (o->flags & (BCX_FLAG_NO_TUNE | BCX_FLAG_WG_KERNEL | BCX_FLAG_NO_WG_KERNEL));  // (fixed by the options)
 }
-static int fp32_route(bcx_ctx *ctx, DComp &dc, const bcx_opts *o, int *route) {
-    *route = FP32_ANY;
-    if (fp32_free(dc, o)) return BCX_OK;
-    int8_t &r = dc.fp32_route[want_cut(o)];
-    if (r < 0 && dc.n <= WG_N) {
-        (void)batched_narrow(dc);  // (measures the depth)
-        ChainCut *cut = nullptr;
-        if (want_cut(o) && dc.n > fp32_line(dc, true) && dc.n <= fp32_line(dc, false)) {
-            const int rc = chain_cut(ctx, dc, cut);
-            if (rc) return rc;
-        }
-        r = dc.n > fp32_line(dc, cut != nullptr) ? FP32_TILES : FP32_ROWS;
+static double round_ms(DComp &dc) {
+    if (dc.round_ms < 0) {
+        const int64_t T = ((int64_t)dc.n + BATCH_W - 1) / BATCH_W, k = std::min<int64_t>(256, T);
+        std::vector<int64_t> at;
+        for (int64_t i : {25, 51, 76, 102, 127, 153, 179, 204, 230, 254, 255}) at.push_back((2 * std::min(i, k - 1) + 1) * T / (2 * k));
+        const std::vector<int64_t> w = tiles_work(dc.host, batched_order(dc), at, 58);
+        dc.round_ms = 5.7e-6 * (double)*std::max_element(w.begin(), w.end()) + 28e-6 * (double)dc.arcs;
     }
-    if (r < 0) r = FP32_TILES;
-    *route = r;
-    return BCX_OK;
+    return dc.round_ms;
+}
+static int fp32_route(DComp &dc, const bcx_opts *o) {
+    if (fp32_free(dc, o)) return FP32_ANY;
+    int8_t &r = dc.fp32_route[want_cut(o)];
+    if (r < 0) {
+        r = FP32_TILES;
+        if (dc.n <= WG_N) {
+            (void)batched_narrow(dc);  // (measures the depths)
+            const int32_t depth = want_cut(o) ? dc.core_depth : dc.depth;
+            const double tiles = 38.0 + 6.5e-6 * (double)dc.arcs + depth * (0.55 + 4.5e-6 * dc.n);
+            if (dc.n <= (int64_t)DEEP_WIDTH * (dc.depth + 1) ||
+                round_ms(dc) / (256 * BATCH_W) <= tiles / (TUNE_TILES * BATCH_W * MAX_SPL))
+                r = FP32_ROWS;
+        }
+    }
+    return r;
 }
 
 bcx_opts batched_opts(const DComp &dc, const bcx_opts &o) {
@@ -2139,8 +2167,8 @@ static int measured_kind(Tuner &t, int64_t n_src, bool by_source, bool rows, int
 int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *opts, int64_t n_src, bcx_stats *st) {
     const int kind0 = batched_kind(dc, opts->flags);
     if (kind0 == BCX_KERNEL_SMALL) return kind0;
-    int route = FP32_ANY, rc = fp32_route(ctx, dc, opts, &route);
-    if (rc) return rc;
+    const int route = fp32_route(dc, opts);
+    int rc = BCX_OK;
     const bcx_opts own = batched_opts(dc, *opts), *o = &own;
     const bool fixed = (o->flags & (BCX_FLAG_NO_WG_KERNEL | BCX_FLAG_WG_KERNEL)) != 0;
     const bool wraps = counts_may_wrap(dc, o);
@@ -2155,12 +2183,12 @@ int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *opts, int64_t n_sr
         else if (wraps && route == FP32_ROWS) kind = BCX_KERNEL_WG;
         else if ((rc = measured_kind(t, n_src, by_source, route == FP32_ROWS, &kind))) return rc;
     }
-    // (below the line the tiles run under the defaults: the candidates cost 200 to
+    // (mid-size components run under the defaults: the candidates cost 200 to
     // 300 ms and none gained on power-law cores of 34k and 67k vertices, 20.5 and
     // 23.0 ms for 6144 sources against 21.9 and 24.2 tuned, nor on R-MAT cores of
-    // 23k and 45k, 13.3 and 19.8 against 13.9 and 22.1)
-    const bool below = !fixed && dc.n <= WG_N && dc.n <= fp32_line(dc, want_cut(opts));
-    if (kind == BCX_KERNEL_MULTI && !dc.sched_multi && !below) {
+    // 23k and 45k, 13.3 and 19.8 against 13.9 and 22.1; tiles of whole rows likewise)
+    const bool defaults = !fixed && (route == FP32_ROWS || dc.n <= (want_cut(opts) ? 58000 : 74000) + 400 * dc.depth);
+    if (kind == BCX_KERNEL_MULTI && !dc.sched_multi && !defaults) {
         const MultiSched base = t.base;
         MultiSched best = base;
         std::vector<MultiSched> cands;

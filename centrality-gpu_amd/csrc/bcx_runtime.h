@@ -64,6 +64,8 @@ struct DComp {
     int64_t arcs = 0;
     int64_t offset = 0;  // into the concatenated BC vector
     int32_t depth = -1;  // BFS depth from the highest-degree vertex (-1: not measured)
+    int32_t core_depth = 0;  // deepest of its levels off the chains (measured with depth)
+    double round_ms = -1.0;  // batched path: a round of workgroup tiles, estimated (-1: not yet)
     double sigma_est = 0.0;  // largest path count of that BFS (measured with depth)
     bool src_wrapped = false;  // a per-source FP32C run met counts past 64 bits
     std::vector<int32_t> rank;      // batched path: BFS rank of each vertex (built on first use)

@@ -30,13 +30,20 @@ def far(a, b):
     return float(np.linalg.norm(a - b) / np.linalg.norm(b))
 
 
-@pytest.mark.parametrize("chains", [True, False])
-@pytest.mark.parametrize("cfg,scale,flags", [(2, 0.022, bcx.FLAG_WG_KERNEL), (5, 0.06, bcx.FLAG_WG_KERNEL),
-                                             (2, 0.08, bcx.FLAG_WG_KERNEL), (2, 0.12, bcx.FLAG_NO_WG_KERNEL)])
-def test_fp32c_does_not_depend_on_the_number_of_sources(engine, cfg, scale, flags, chains):
-    """18.6k, 23k and 67k cores (rows whole) and a 101k core (sliced tiles): subsets of
-    every size, with the tuner's rates of each, equal the kernel that the flags
-    force."""
+ROWS, SLICED = bcx.FLAG_WG_KERNEL, bcx.FLAG_NO_WG_KERNEL
+
+
+@pytest.mark.parametrize("cfg,scale,chains,flags", [
+    (2, 0.022, True, ROWS), (2, 0.022, False, ROWS), (5, 0.06, True, ROWS), (5, 0.06, False, ROWS),
+    (2, 0.047, True, SLICED), (2, 0.05547, True, SLICED), (2, 0.05547, False, SLICED), (2, 0.0555, True, ROWS),
+    (2, 0.08, True, ROWS), (2, 0.08, False, ROWS), (5, 0.17, True, SLICED), (2, 0.12, True, SLICED),
+    (2, 0.12, False, ROWS)])
+def test_fp32c_does_not_depend_on_the_number_of_sources(engine, cfg, scale, chains, flags):
+    """Power-law cores of 18.6k to 101k vertices and R-MAT cores: subsets of every
+    size, with the tuner's rates of each, equal the kernel that the flags force,
+    which is the one that full jobs of the component were given before the
+    per-source kernel was there (two cores of 46.7k: tiles over the last sources
+    that were sampled)."""
     c = giant(cfg, scale)
     order = np.random.default_rng(7).permutation(c.n).astype(np.int64)
     g = engine.upload([c])
