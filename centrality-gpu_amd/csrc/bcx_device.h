@@ -49,6 +49,18 @@ __device__ __forceinline__ void gadd(gdbl *p, double x) {
 __device__ __forceinline__ double u2d(uint64_t x) { return __longlong_as_double((long long)x); }
 __device__ __forceinline__ uint64_t d2u(double x) { return (uint64_t)__double_as_longlong(x); }
 
+// A sum that is rounded once: what each addition rounds off (exact by Knuth's
+// two-sum) is added at the end.
+struct ExactSum {
+    double s = 0.0, e = 0.0;
+    __device__ __forceinline__ void add(double x) {
+        const double t = s + x, y = t - s;
+        e += (s - (t - y)) + (x - y);
+        s = t;
+    }
+    __device__ __forceinline__ double value() const { return isfinite(s) ? s + e : s; }
+};
+
 // Wave64 reductions (fixed butterfly order: deterministic).
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll

@@ -179,9 +179,10 @@ __global__ __launch_bounds__(256) void k_na_add(unsigned char *b, double *bc, in
     const double *bc0 = (const double *)(b + O_BC);
     const int v = blockIdx.x * 256 + threadIdx.x;
     if (v >= n) return;
-    double sum = 0.0;
-    for (int k = 0; k < NA_COPIES; ++k) sum += bc0[k * NA_N + v];
-    if (sum != 0.0) bc[v] += sum;
+    ExactSum sum;
+#pragma unroll
+    for (int k = 0; k < NA_COPIES; ++k) sum.add(bc0[k * NA_N + v]);
+    if (sum.value() != 0.0) bc[v] += sum.value();
 }
 
 // The first pass listed the tiles whose 64-bit counts overflowed: they make

@@ -778,15 +778,9 @@ hipError_t launch_plain_bfs(const CompDev &c, const PlainArgs &a, const PlainScr
 __global__ void k_plain_fold(double *bc, const double *copies, const int32_t *perm, int n, int split) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= n) return;
-    // rounded once: what each addition rounds off (exact by Knuth's two-sum) is
-    // added at the end
-    double s = copies[v], e = 0.0;
-    for (int k = 1; k < split; ++k) {
-        const double x = copies[(int64_t)k * n + v], t = s + x, y = t - s;
-        e += (s - (t - y)) + (x - y);
-        s = t;
-    }
-    bc[perm ? perm[v] : v] += isfinite(s) ? s + e : s;
+    ExactSum s;
+    for (int k = 0; k < split; ++k) s.add(copies[(int64_t)k * n + v]);
+    bc[perm ? perm[v] : v] += s.value();
 }
 
 hipError_t launch_plain_fold(double *bc, const double *copies, const int32_t *perm, int n, int split, hipStream_t st) {

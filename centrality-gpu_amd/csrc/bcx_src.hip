@@ -467,9 +467,8 @@ hipError_t launch_src(const SrcArgs &a, bool f64, bool fp32, int grid, hipStream
     return hipGetLastError();
 }
 
-// Rounded once: what each addition rounds off (exact by Knuth's two-sum) is added
-// at the end.  Words that no tile added to are left alone: other components' runs
-// may be adding to theirs.
+// Words that no tile added to are left alone: other components' runs may be adding
+// to theirs.
 __global__ __launch_bounds__(256) void k_src_fold(double *bc, int64_t copy, int64_t n, double *out, const int32_t *ctr,
                                                   int32_t *ctr_out) {
     const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -482,19 +481,15 @@ __global__ __launch_bounds__(256) void k_src_fold(double *bc, int64_t copy, int6
         x[k] = bc[v + k * copy];
         any |= k > 0 && x[k] != 0.0;
     }
-    double s = x[0], e = 0.0;
+    ExactSum s;
+#pragma unroll
+    for (int k = 0; k < SRC_COPIES; ++k) s.add(x[k]);
     if (any) {
 #pragma unroll
-        for (int k = 1; k < SRC_COPIES; ++k) {
-            const double t = s + x[k], y = t - s;
-            e += (s - (t - y)) + (x[k] - y);
-            s = t;
-            bc[v + k * copy] = 0.0;
-        }
-        if (isfinite(s)) s += e;
-        ast((uint64_t *)&bc[v], d2u(s));
+        for (int k = 1; k < SRC_COPIES; ++k) bc[v + k * copy] = 0.0;
+        ast((uint64_t *)&bc[v], d2u(s.value()));
     }
-    if (out) out[v] = s;
+    if (out) out[v] = s.value();
 }
 
 hipError_t launch_src_fold(double *bc, int64_t copy, int64_t n, double *out, const int32_t *ctr, int32_t *ctr_out,

@@ -13,6 +13,7 @@ import numpy as np
 import pytest
 
 import bcx
+from test_zz_no_alloc import noalloc
 
 pytestmark = pytest.mark.gpu
 
@@ -50,6 +51,16 @@ def test_small_components(engine, n, copies, path):
     off = (got - np.tile(want, copies)) / np.spacing(np.tile(want, copies))
     rms = math.sqrt(float(np.mean(off ** 2)))
     print("n", n, "copies", copies, "path", path, "rms ulp", rms, flush=True)
+    assert rms < BOUND, rms
+
+
+@pytest.mark.parametrize("n", [40, 98, 300, 1000])
+def test_call_without_allocation(engine, n):
+    comps = [component(n, 7 * n + k) for k in range(max(1, 800 // n))]
+    want = np.concatenate([exact(engine, c) for c in comps])
+    got = np.concatenate([noalloc(engine, c, None, bcx.PREC_FP64) for c in comps])
+    rms = math.sqrt(float(np.mean(((got - want) / np.spacing(want)) ** 2)))
+    print("no allocation: n", n, "rms ulp", rms, flush=True)
     assert rms < BOUND, rms
 
 
