@@ -779,7 +779,13 @@ __global__ void k_plain_fold(double *bc, const double *copies, const int32_t *pe
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= n) return;
     ExactSum s;
-    for (int k = 0; k < split; ++k) s.add(copies[(int64_t)k * n + v]);
+    for (int k0 = 0; k0 < split; k0 += 8) {  // (eight loads in flight)
+        double x[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] = k0 + k < split ? copies[(int64_t)(k0 + k) * n + v] : 0.0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s.add(x[k]);
+    }
     bc[perm ? perm[v] : v] += s.value();
 }
 

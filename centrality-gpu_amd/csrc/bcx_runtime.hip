@@ -414,16 +414,19 @@ static int run_bfs_list(bcx_ctx *ctx, const DComp &dc, const std::vector<int32_t
     const int grid = plain_grid(ctx, dc.n, (int64_t)src.size(), shape);
     PlainScratch sc;
     if ((rc = ensure_plain_scratch(ctx, dc.n, grid, sc))) return rc;
-    // Hundreds of sources and more add into SPLIT copies of the accumulator, folded
-    // afterwards: a vertex's sum is then SPLIT times shorter, and its rounding
-    // error what the tiled kernels' is, which add a tile's sources first (16384
-    // sources of a 26k grid, error against 64 bits 1.5e-15 on tiles, 5.7e-15
-    // with one accumulator).  Accumulators of the workgroups' own, without
-    // atomics, ran 20-30% slower (8000 sources of that grid 13.6 -> 16.0 ms).
-    // Where a capacity has little room left beside the rows above, there is one
-    // accumulator, and without room for that an ordered run has the
+    // The sources add into copies of the accumulator, one per eight of them up to
+    // SPLIT, folded afterwards: a vertex's sum is then that much shorter, and its
+    // rounding error what the tiled kernels' is, which add a tile's sources in pairs
+    // (error in the sum alone on a grid of 3600 vertices, FP64 terms, with one
+    // accumulator / so: 64 sources 1.3 / 0.44 ulp, 361 sources 3.1 / 0.44, 1500
+    // sources - / 0.56; 32 copies 0.33 and 0.41 for the latter two, but 2049 sources
+    // of an 18.6k grid 3.20 -> 3.25 ms).  With FP32 terms the terms' own rounding
+    // hides it, and only hundreds of sources and more take copies.  Accumulators of
+    // the workgroups' own, without atomics, ran 20-30% slower (8000 sources of a 26k
+    // grid 13.6 -> 16.0 ms).  Where a capacity has little room left beside the rows
+    // above, there are fewer, and without room for one an ordered run has the
     // component's own order.
-    constexpr int SPLIT = 32;
+    constexpr int SPLIT = 16;
     constexpr size_t SPLIT_FP32 = 512;
     const size_t word = sizeof(double) * (size_t)dc.n;
     const size_t room = ctx->mem_cap > ctx->mem_used ? ctx->mem_cap - ctx->mem_used : 0;
