@@ -159,14 +159,6 @@ __device__ __forceinline__ uint64_t mall(const Msk<W> &a) {  // lanes with any s
     for (int h = 0; h < W; ++h) x |= a.m[h];
     return x;
 }
-// a mask that every lane holds, in scalar registers
-template <int W>
-__device__ __forceinline__ Msk<W> muni(const Msk<W> &a) {
-    Msk<W> r;
-#pragma unroll
-    for (int h = 0; h < W; ++h) r.m[h] = uni64(a.m[h]);
-    return r;
-}
 template <int W>
 __device__ __forceinline__ Msk<W> mshfl(const Msk<W> &a, int src) {
     Msk<W> r;
