@@ -8,7 +8,7 @@
 //           accumulators, so that the sum over many small tiles is as accurate
 //           as over 64-source ones (1000 sources, error against 64 bits: one
 //           accumulator 4.4e-16, k_small 1.8e-16)
-//   add     their sum into the caller's when no count left 64 bits
+//   add     their sum, rounded once, into the caller's when no count left 64 bits
 // followed by one read-back of the status words and a stream sync.  Components
 // with too many arcs for the LDS of k_src, and those with a count past 64 bits
 // (whose 64-source tiles turn to FP64 counts and terms as in bcx_run), go on:
@@ -17,7 +17,7 @@
 //   k_small FP64 path counts over those tiles (none: returns at once)
 // k_src holds its state in LDS, so its workgroups are not bound by the array's
 // slabs: a 1000-vertex component of average degree 8, every source: 2.48 ms on
-// 8 workgroups of k_small, 0.12 ms on 250 of k_src (the whole call).
+// 8 workgroups of k_small, 0.13 ms on 250 of k_src (the whole call).
 #include <algorithm>
 #include <mutex>
 #include <string>

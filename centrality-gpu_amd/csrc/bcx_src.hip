@@ -18,12 +18,12 @@
 // (Codes/kernels_free.cu:154-473 computes the same, one source per block with
 // its state in global memory.)
 //
-// What bounds it: vector issue (60% of the cycles with 16 waves per CU) and the
-// LDS round trips of a wave's arc steps; no step waits for another wave or for
-// global memory.  A step takes a group of four arcs of each lane's row (rows are
+// What bounds it: vector issue (61% of a busy compute unit's cycles with FP64
+// terms, 63% with FP32 ones) and the LDS round trips of a wave's arc steps; no
+// step waits for another wave or for global memory.  A step takes a group of four arcs of each lane's row (rows are
 // padded to whole groups, so no arc is tested for the row's end) and is free of
 // branches, so its accesses are in flight together.  Measured, 10k-vertex
-// workload of 16 blocks, all sources, whole run: 0.26 ms FP64 and 0.28 ms FP32C
+// workload of 16 blocks, all sources, whole run: 0.25 ms FP64 and 0.28 ms FP32C
 // (0.31 and 0.40 ms with single-arc bounds tests, 2-bit codes set by LDS
 // atomics and 64-source tiles), against 0.86 ms with 64 sources per wave, rows in
 // global memory and barriers per level (bcx_small.hip) and 10.1 ms with one

@@ -136,7 +136,13 @@ int  bcx_host_load(const char *path, const char *source_path, int use_chains, bc
 typedef struct bcx_ctx    bcx_ctx;
 typedef struct bcx_dgraph bcx_dgraph;   /* device-resident component set */
 
-/* Precision of the dependency (delta) arithmetic.                          */
+/* Precision of the dependency (delta) arithmetic.  With FP32C the terms are
+ * rounded to FP32 at every vertex, except that the multi-launch tiles carry the
+ * interiors of contracted chains in FP64 and sum a hub's row in slices; the two
+ * differ by 1e-10 to 7e-9.  Which of them a component gets follows from the
+ * component and use_chains alone, so the parts of a job add up and a source gives
+ * the same in every call; the flags below and, on the multi-launch tiles, their
+ * options can change it.                                                   */
 #define BCX_PREC_FP64        0   /* FP64 delta, FP64 BC                       */
 #define BCX_PREC_FP32C       1   /* FP32 compensated (Kahan) delta, FP64 BC   */
 
@@ -192,14 +198,16 @@ typedef struct {
  * Codes/postprocesses.cu:329-360).  NO_CONTRACT keeps every chain vertex in
  * the tile graph.                                                          */
 #define BCX_FLAG_NO_CONTRACT     16
-/* Batched path: components of at least 16384 vertices get a schedule
- * measured once on sample tiles and cached (no counterpart in the
- * reference, which switches schedule from sampled BFS depths,
+/* Batched path: components of at least 16384 vertices get a schedule from
+ * samples, each taken once, when a run's choice first depends on it, and cached
+ * with the options that it was taken under (no counterpart in the reference,
+ * which switches schedule from sampled BFS depths,
  * Codes/kernels_free.cu:447-470): one workgroup per source, the multi-launch
  * tiles or (up to 131072 vertices) the workgroup-per-tile kernel, by the number
- * of sources of a run, and for multi-launch components the
+ * of sources of a run, and for large multi-launch components the
  * sources per lane, the level kernels' blocks per CU, the tiles in flight
- * and chain contraction on or off.  NO_TUNE keeps the defaults (the
+ * and chain contraction on or off (FP32C: always on above 131072 vertices).
+ * NO_TUNE keeps the defaults (the
  * level-width rule, 4 sources per lane, 8 blocks per CU, 8 tiles,
  * contraction on).  Options that fix a choice (the kernel flags,
  * sources_per_lane, batch_width, blocks_per_cu, NO_CONTRACT) are kept and
@@ -216,7 +224,8 @@ typedef struct {
     int64_t n_launches;        /* kernel launches                             */
     int32_t max_level;         /* deepest BFS level seen                      */
     int32_t n_ball_tiles;      /* batched: components whose tiles the tile-order
-                                  tuner made graph balls (else BFS-rank runs) */
+                                  tuner makes graph balls (else BFS-rank or
+                                  landmark runs), those run by source too   */
     double  bytes_alg;         /* algorithmic HBM bytes of the work done      */
     double  teps_work;         /* sum over sources of component arcs/2        */
     double  t_chain_s;         /* part of t_kernel_s spent on chain sources   */
