@@ -1415,9 +1415,8 @@ static int persistent_pass(bcx_ctx *ctx, SmallState &ss, bool wg, bool f64, bool
     return small_launch(ctx, ss, ss.run, wg, f64, ss.run_fp32, ss.run_grid, graph, ss.run_stream);
 }
 
-// The tables of a persistent pass: its components, tiles of width(sources of
-// the component) sources, sources and weights, and eight zeroed counters, in
-// device memory.
+// The tables of a persistent pass: its components, tiles of width(job) sources,
+// sources and weights, and eight zeroed counters, in device memory.
 struct PassTables {
     std::vector<SmallTile> tiles;
     const SmallComp *comps = nullptr;
@@ -1448,7 +1447,7 @@ static int stage_tables(bcx_ctx *ctx, SmallState &ss, const std::vector<const Sm
         c.bc = bc_base + dc.offset;
         const int32_t ci = (int32_t)comps.size();
         comps.push_back(c);
-        const size_t tw = width(jb.srcs.size());
+        const size_t tw = width(jb);
         for (size_t i = 0; i < jb.srcs.size(); i += tw) {
             SmallTile t{};
             t.comp = ci;
@@ -1542,7 +1541,7 @@ static int persistent_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, con
     for (const SmallJob *jb : order)
         if (!wide(jb)) n_narrow_tiles += (jb->srcs.size() + TW - 1) / TW;
     PassTables tb;
-    int rc = stage_tables(ctx, ss, order, bc_base, [&](size_t) { return TW; }, tb);
+    int rc = stage_tables(ctx, ss, order, bc_base, [&](const SmallJob &) { return TW; }, tb);
     if (rc) return rc;
     std::vector<SmallTile> &tiles = tb.tiles;
     if ((rc = ss.counter.ensure(ctx, 64, "small counters")) ||
@@ -1739,13 +1738,16 @@ static int src_start(bcx_ctx *ctx, const std::vector<SmallJob> &jobs, const bcx_
     const size_t tw = probe || per > 128 ? BATCH_W : (per > 64 ? 32 : (per > 8 ? 16 : (per > 4 ? 8 : 4)));
     // With FP64 terms the sums over sources are to round no more than those of
     // 64-source tiles added up in pairs (bcx_small.hip).  The w sources of a tile
-    // are added one by one, and the errors of the k / w tiles of a component sum to
-    // the square root of w^2 / 3k additions' worth: w^2 is kept at 3k or less.
+    // are added to its a accumulators one by one, and the errors of the k / w tiles
+    // of a component sum to the square root of w^2 / 3k a^2 additions' worth, those of
+    // adding up the accumulators to that of 3 w / 2k: w^2 is kept at 3k a^2 or less and
+    // w at k / 4.
     PassTables tb;
-    int rc = stage_tables(ctx, ss, order, bc_base, [&](size_t k) {
+    int rc = stage_tables(ctx, ss, order, bc_base, [&](const SmallJob &jb) {
         if (fp32 || probe) return tw;
+        const size_t acc = (size_t)src_accs(jb.dc->n, jb.dc->groups, lds), k = jb.srcs.size();
         size_t w = 4;
-        while (w < tw && 4 * w * w <= 3 * k) w *= 2;
+        while (w < tw && 4 * w * w <= 3 * k * acc * acc && 8 * w <= k) w *= 2;
         return w;
     }, tb);
     if (rc || (rc = ss.redo.ensure(ctx, 4 * tb.tiles.size(), "source redo list"))) return rc;

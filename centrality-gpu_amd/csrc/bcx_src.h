@@ -33,6 +33,15 @@ __host__ __device__ constexpr int64_t src_waves(int64_t n, int64_t groups, int64
     return w < 0 ? 0 : (w > SRC_WAVES ? SRC_WAVES : w);
 }
 
+// BC accumulators of a workgroup with FP64 terms: 4, 2 or 1, those past the first
+// in what its waves leave of `lds`.  A wave adds to one of them, so a tile may be
+// that much wider for the same rounding (400 components of 3 to 2000 vertices and a
+// core, whole run: 7.40 ms with one, 7.25 so; a fifth of it: 1198 and 1150 us).
+__host__ __device__ constexpr int src_accs(int64_t n, int64_t groups, int64_t lds) {
+    const int64_t rest = lds - src_shared_bytes(n, groups) - src_waves(n, groups, lds) * src_wave_bytes(n);
+    return rest >= 3 * src_up16(8 * n) ? 4 : (rest >= src_up16(8 * n) ? 2 : 1);
+}
+
 struct SrcArgs {
     const SmallComp *comps;
     const SmallTile *tiles;  // at most 64 sources each

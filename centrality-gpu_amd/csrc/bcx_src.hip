@@ -392,7 +392,6 @@ __global__ __launch_bounds__(XB) void k_src(SrcArgs a) {
         double *bc = (double *)s_lds;
         int32_t *rp = (int32_t *)(s_lds + src_up16(8 * (int64_t)n));
         uint64_t *col = (uint64_t *)((unsigned char *)rp + src_up16(4 * ((int64_t)n + 1)));
-        for (int v = tid; v < n; v += XB) bc[v] = 0.0;
         // row pointers in groups of four arcs: a scan of the padded rows, XB at
         // a time
         int groups = 0;
@@ -418,6 +417,11 @@ __global__ __launch_bounds__(XB) void k_src(SrcArgs a) {
         if (tid == 0) rp[n] = groups;
         const int64_t wb = src_wave_bytes(n);
         const int waves = (int)src_waves(n, groups, a.lds);
+        const int accs = sizeof(TT) == 8 ? src_accs(n, groups, a.lds) : 1;
+        double *more = (double *)(s_lds + src_shared_bytes(n, groups) + waves * wb);  // the accumulators past the first
+        const int acc_words = (int)(src_up16(8 * (int64_t)n) / 8);
+        for (int v = tid; v < n; v += XB) bc[v] = 0.0;
+        for (int v = tid; v < (accs - 1) * acc_words; v += XB) more[v] = 0.0;
         for (int g = tid; g <= groups; g += XB) col[g] = 0x0001000100010001ull * (uint64_t)n;
         __syncthreads();
         for (int v = wv; v < n; v += SRC_WAVES) {  // (a wave per row)
@@ -431,13 +435,15 @@ __global__ __launch_bounds__(XB) void k_src(SrcArgs a) {
             x.st = (uint64_t *)p;
             x.lv = p + src_up16(8 * ((int64_t)n + 2));
             x.S = (uint16_t *)(x.lv + src_up16((int64_t)n + 2));
+            const int own = wv & (accs - 1);
+            double *acc = own ? more + (own - 1) * acc_words : bc;
             while (true) {
                 int i = 0;
                 if (lane == 0) i = atomicAdd(&s_next, 1);
                 i = __builtin_amdgcn_readlane(i, 0);
                 if (i >= tl.ns) break;
                 const int s = __builtin_amdgcn_readfirstlane(a.srcs[tl.src0 + i]);
-                if (!src_run<F64, TT>(a, n, s, a.ws[tl.src0 + i], rp, col, reach, bc, x, i,
+                if (!src_run<F64, TT>(a, n, s, a.ws[tl.src0 + i], rp, col, reach, acc, x, i,
                                          &s_depth)) {
                     if (lane == 0) s_ovf = 1;
                     break;
@@ -450,8 +456,12 @@ __global__ __launch_bounds__(XB) void k_src(SrcArgs a) {
         } else {
             if (tid == 0) atomicMax(&a.counter[2], s_depth);
             gdbl *to = glb(cp.bc) + (item % SRC_COPIES) * a.copy;
-            for (int v = tid; v < n; v += XB)
-                if (bc[v] != 0.0) gadd(to + v, bc[v]);
+            for (int v = tid; v < n; v += XB) {
+                double sum = bc[v];
+                if (accs == 2) sum += more[v];
+                if (accs == 4) sum = (sum + more[v]) + (more[acc_words + v] + more[2 * acc_words + v]);
+                if (sum != 0.0) gadd(to + v, sum);
+            }
         }
         __syncthreads();
     }

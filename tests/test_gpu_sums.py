@@ -54,6 +54,26 @@ def test_small_components(engine, n, copies, path):
     assert rms < BOUND, rms
 
 
+@pytest.mark.parametrize("path", [bcx.PATH_PLAIN, bcx.PATH_BATCHED])
+def test_sizes_beside_each_other(engine, path):
+    """Components that leave four, two and no accumulators' room beside their waves
+    (the launch's LDS is the largest one's), in tiles of up to 64 sources."""
+    comps = [component(n, n + k) for n, m in ((64, 6), (300, 1), (640, 1), (900, 1), (1100, 1)) for k in range(m)]
+    want = [exact(engine, c) for c in comps]
+    g = engine.upload(comps * 30)
+    got, _ = g.run(path=path, precision=bcx.PREC_FP64)
+    g.free()
+    got = got.reshape(30, -1)
+    at = 0
+    for n in (64, 300, 640, 900, 1100):
+        w = np.concatenate([x for x in want if len(x) == n])
+        off = (got[:, at:at + len(w)] - w) / np.spacing(w)
+        at += len(w)
+        rms = math.sqrt(float(np.mean(off ** 2)))
+        print("n", n, "path", path, "rms ulp", rms, flush=True)
+        assert rms < BOUND, (n, rms)
+
+
 @pytest.mark.parametrize("n", [40, 98, 300, 1000])
 def test_call_without_allocation(engine, n):
     comps = [component(n, 7 * n + k) for k in range(max(1, 800 // n))]
