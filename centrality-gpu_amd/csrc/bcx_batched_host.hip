@@ -2026,6 +2026,7 @@ struct Tuner {
     Timer keep;
     DBuf scratch;
     std::vector<int32_t> order, samp;
+    double base_s = -1.0;
     bool on = false;
     Tuner(bcx_ctx *c, DComp &d, const bcx_opts &opts) : ctx(c), dc(d), o(opts), base(multi_sched(d, &opts)) {
         o.src_subset = nullptr;
@@ -2081,6 +2082,12 @@ struct Tuner {
         if (rc) return rc;
         if (samp.empty()) samp = tiles(TUNE_TILES, (int64_t)BATCH_W * MAX_SPL);
         return multi(samp, m, t);
+    }
+    // the base schedule over the same sources, once
+    int multi_base(double *t) {
+        const int rc = base_s < 0 ? multi(base, &base_s) : BCX_OK;
+        *t = base_s;
+        return rc;
     }
     int wg(double *t) {
         const int rc = begin();
@@ -2149,7 +2156,7 @@ static int measured_kind(Tuner &t, int64_t n_src, bool by_source, bool rows, int
     if (src <= r.tile) return BCX_OK;
     if (r.more < 0) {
         double x = 0.0;
-        if ((rc = t.multi(t.base, &x))) return rc;
+        if ((rc = t.multi_base(&x))) return rc;
         const double more = (double)t.samp.size() - BATCH_W * MAX_SPL;
         r.more = more > 0 ? std::max(0.0, x - r.tile) / more : 0.0;
     }
@@ -2202,7 +2209,7 @@ int batched_schedule(bcx_ctx *ctx, DComp &dc, const bcx_opts *opts, int64_t n_sr
             for (int w : {1, 2, 4})
                 if (w != base.spl) cands.push_back({base.cut, base.bpc, base.slots, w});
         double t_best = 0.0;
-        if ((rc = t.multi(base, &t_best))) return rc;
+        if ((rc = t.multi_base(&t_best))) return rc;
         for (const MultiSched &m : cands) {
             double x = 0.0;
             if ((rc = t.multi(m, &x))) return rc;
